@@ -122,8 +122,10 @@ int st_mlp_forward_static(const void *x, int64_t B, int64_t H, const void *gate_
  *   scores  optional float [B,I] (NULL = not written)
  *   mask    uint8 [I]: mask[i] = any_b(score[b,i] >= thr)  (cmp_ge != 0)
  *                               any_b(score[b,i] >  thr)  (cmp_ge == 0)
- * H*sizeof(dtype) and r*sizeof(dtype) must be multiples of 16.  More than 64 rows
- * of x (fewer for ranks above 224) run as several passes over the predictor's weights.
+ * H*sizeof(dtype) and r*sizeof(dtype) must be multiples of 16.  Nine or more rows
+ * of x in fp16 / bf16 with r <= 512 run on the matrix cores in one pass (fp32
+ * accuracy of the scores all the same); otherwise more than 64 rows (fewer for
+ * ranks above 224) run as several passes over the predictor's weights.
  * ------------------------------------------------------------------------ */
 int st_predictor_mask(const void *x, int64_t B, int64_t H, const void *A, int64_t r, const void *Bm, int64_t I,
                       int dtype, float thr, int cmp_ge, float *t_ws, float *scores, uint8_t *mask, void *stream);

@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libsparse_mlp_amd.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
-SOURCES = ["capi.hip", "mlp_decode.hip", "mlp_batch.hip", "mlp_prefill.hip", "predictor.hip", "mask_select.hip",
+SOURCES = ["capi.hip", "mlp_decode.hip", "mlp_batch.hip", "mlp_prefill.hip", "predictor.hip", "predictor_mfma.hip", "mask_select.hip",
            "mlp_f64.hip", "cache.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -361,6 +361,9 @@ extern "C" int st_predictor_mask_ex(const void *x, int64_t B, int64_t H, const v
     ST_REQUIRE((flags & ~ST_PRED_ROUND_STORAGE) == 0, "st_predictor_mask_ex: unknown flags %d", flags);
     const int round_storage = (flags & ST_PRED_ROUND_STORAGE) && dtype != ST_F32 ? 1 : 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (predictor_mfma_supported(dtype, (int)B, (int)r))
+        return launch_predictor_mfma(dtype, x, (int)B, (int)H, A, (int)r, Bm, (int)I, thr, cmp_ge, t_ws, scores, mask,
+                                     round_storage, s);
     // Rows of x per pass: what the staging buffer of the second kernel holds, 64 at most.  Further passes reuse
     // the front of t_ws (the launches are ordered on the stream) and only ever switch mask bytes on.
     int64_t per = (56 * 1024) / (r * 4);

@@ -1,0 +1,407 @@
+// LoRA importance predictor for several rows of x (fp16 / bf16): both maps on the matrix cores.
+//
+//   kernel 1  t[b,k] = <x[b,:], A[k,:]>     tiles of (16 MI) x (16 NI), the block's waves split the hidden dimension;
+//                                           also clears the mask
+//   kernel 2  s[b,i] = <t[b,:], Bm[i,:]>    a wave keeps its rows of t in registers and walks over rows of Bm;
+//             mask[i] = 1 where any s[b,i] passes the cut (only ones are stored)
+//
+// The rank-r intermediate is fp32, and the matrix cores multiply 16-bit operands: kernel 2 splits t into parts of the
+// storage type that sum to it -- two fp16 parts or three bf16 parts, each rounding what the parts before it left over.
+// What is lost is below 2^-24 of t, half an ulp of fp32 (rows of fp16 parts are scaled by a power of two that puts their
+// largest element near 2^14, so that neither overflow nor the subnormals matter): the scores keep fp32 accuracy.
+//
+// Same contract as predictor.hip (src/modeling_skip.py:52-53,204-207,214).
+#include "st_mfma.h"
+
+namespace st {
+
+template <typename T> struct SplitParts;
+template <> struct SplitParts<f16_t> { static constexpr int value = 2; };
+template <> struct SplitParts<bf16_t> { static constexpr int value = 3; };
+
+// ---------------------------------------------------------------------------
+// kernel 1
+// ---------------------------------------------------------------------------
+// A tile of 16 MI rows of x by 16 NI rank rows per block.  Its W waves deal out pieces of 128 of the hidden dimension
+// among themselves; a wave loads the 256 bytes of every row of its next piece straight into a part of LDS of its own while
+// it multiplies the present one, so nothing waits for another wave until the sums meet at the end.  (Fragments loaded
+// from memory into registers, 16 rows x 64 bytes per instruction, went through a CU at 15 bytes per clock.)
+// LDS rows are 16 chunks of 16 bytes, chunk c of row k at c ^ (k % 16).
+constexpr int kPmPiece = 128;
+
+template <typename T, int MI, int NI, int W>
+__global__ __launch_bounds__(W * kWave) void predictor_down_mfma_kernel(const T *__restrict__ x, const T *__restrict__ A,
+                                                                        int B, int H, int r, int nt,
+                                                                        float *__restrict__ t, uint8_t *__restrict__ mask,
+                                                                        int I, int round_storage)
+{
+    constexpr int kThreads = W * kWave;
+    constexpr int kRows = 16 * (MI + NI), kBuf = kRows * 16, kDma = kRows / 4;   // a wave's buffer in chunks, its 1 KB loads
+    extern __shared__ __align__(16) uint4 lds[];   // [W][2][kRows][16]
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, q = lane >> 4;
+    const int m0 = (blockIdx.x / nt) * 16 * MI, k0 = (blockIdx.x % nt) * 16 * NI;
+    const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
+    const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint4 *)lds;
+
+    // load j fills LDS rows 4 j .. 4 j + 3, lane i position i % 16 of row i / 16.  Rows are clamped into range (what they
+    // feed is not stored), and so are columns past the end of a row (replaced by zeros below).
+    unsigned doff[kDma];
+#pragma unroll
+    for (int j = 0; j < kDma; ++j) {
+        const int row = 4 * j + (lane >> 4);
+        int g = row < 16 * MI ? m0 + row : k0 + row - 16 * MI;
+        const int last = row < 16 * MI ? B - 1 : r - 1;
+        g = g < last ? g : last;
+        doff[j] = (unsigned)g * (unsigned)H * (unsigned)sizeof(T);
+    }
+    const int pieces = (H + kPmPiece - 1) / kPmPiece;
+    auto dma = [&](int piece, int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < kDma; ++j) {
+            const int row = 4 * j + (lane >> 4), c = (lane & 15) ^ (row & 15);
+            const int h = piece * kPmPiece + 8 * c;
+            load_to_lds(lds_base + (unsigned)((wave * 2 + b) * kBuf + j * 64) * 16u, doff[j] + (unsigned)(h < H ? h : 0) * (unsigned)sizeof(T),
+                        reinterpret_cast<const char *>(4 * j < 16 * MI ? x : A));
+        }
+    };
+    f32x4_t acc[MI][NI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (wave < pieces) dma(wave, 0);
+    // the mask is cleared here, a kernel ahead of the one that switches bytes on
+    for (int i = blockIdx.x * kThreads + tid; i < I; i += gridDim.x * kThreads) mask[i] = 0;
+    int b = 0;
+    for (int piece = wave; piece < pieces; piece += W, b ^= 1) {
+        // (the loads of the next piece go out once the reads of the last use of their buffer are done)
+        ST_WAIT_VM_LGKM0(0);
+        asm volatile("" ::: "memory");
+        if (piece + W < pieces) dma(piece + W, b ^ 1);
+        const uint4 *buf = lds + (wave * 2 + b) * kBuf;
+#pragma unroll
+        for (int ks = 0; ks < kPmPiece / 32; ++ks) {
+            uint4 fa[MI], fb[NI];
+            const int c = (4 * ks + q) ^ l16;
+#pragma unroll
+            for (int i = 0; i < MI; ++i) fa[i] = buf[(16 * i + l16) * 16 + c];
+#pragma unroll
+            for (int j = 0; j < NI; ++j) fb[j] = buf[(16 * (MI + j) + l16) * 16 + c];
+            if (piece * kPmPiece + 32 * ks + 8 * q >= H) {   // (both operands: a product with zero must not meet an infinity)
+#pragma unroll
+                for (int i = 0; i < MI; ++i) fa[i] = zero4;
+#pragma unroll
+                for (int j = 0; j < NI; ++j) fb[j] = zero4;
+            }
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NI; ++j) acc[i][j] = Mfma<T>::run(fa[i], fb[j], acc[i][j]);
+        }
+    }
+    // (the sums go over the waves' own buffers, which nobody reads any more)
+    typedef float Red[MI * NI][256];
+    Red *red = reinterpret_cast<Red *>(lds);
+    static_assert(sizeof(Red) <= 2 * kBuf * 16, "a wave's sums exceed its buffers");
+    __syncthreads();
+
+    // D[m][n]: a lane holds rows 4 q + e of column l16
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) red[wave][i * NI + j][(4 * q + e) * 16 + l16] = acc[i][j][e];
+    __syncthreads();
+    for (int o = tid; o < MI * NI * 256; o += kThreads) {
+        float s = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) s += red[w][o >> 8][o & 255];
+        const int tile = o >> 8, m = m0 + 16 * (tile / NI) + ((o >> 4) & 15), k = k0 + 16 * (tile % NI) + (o & 15);
+        if (m < B && k < r) t[(size_t)m * r + k] = round_storage ? to_float<T>(from_float<T>(s)) : s;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// kernel 2
+// ---------------------------------------------------------------------------
+// Eight floats of t -> the parts of one A operand register quad each.
+template <typename T> __device__ __forceinline__ void split_parts(const float *v, uint4 *parts);
+template <> __device__ __forceinline__ void split_parts<bf16_t>(const float *v, uint4 *parts)
+{
+    bf16x8_t w[3];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        float rest = v[k];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const __bf16 b = (__bf16)rest;          // (the hardware's conversion: round to nearest even)
+            w[p][k] = b;
+            rest -= (float)b;
+            if (p == 0) rest = fabsf(rest) < 3.3e38f ? rest : 0.f;   // an infinity or NaN has nothing left over
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p) parts[p] = __builtin_bit_cast(uint4, w[p]);
+}
+template <> __device__ __forceinline__ void split_parts<f16_t>(const float *v, uint4 *parts)
+{
+    uint32_t w[2][8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const f16_t hi = from_float<f16_t>(v[k]);
+        const float left = v[k] - to_float<f16_t>(hi);
+        w[0][k] = hi.bits;
+        w[1][k] = from_float<f16_t>(left == left ? left : 0.f).bits;   // (infinity or NaN: nothing left over)
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+        parts[p] = make_uint4(w[p][0] | (w[p][1] << 16), w[p][2] | (w[p][3] << 16), w[p][4] | (w[p][5] << 16),
+                              w[p][6] | (w[p][7] << 16));
+}
+
+// A wave owns 16 MI rows of t (KS k steps of 32 of the rank, in registers as parts) and walks over rows of Bm, which the
+// block loads 64 rows (a stage) at a time straight into LDS, one stage ahead: its W waves share them (fragments loaded by
+// every wave on its own: 97 us for 2048 rows at rank 256, I 14336; now 54 us, of which the MFMAs are 18).  `wb` of the waves
+// own different rows of t, the other W / wb groups take different 16-row tiles of a stage (WB = W is a compile-time case:
+// every wave takes every tile); a block takes `per` stages.
+// LDS rows are 4 KS chunks of 16 bytes (the rank rounded up; the surplus chunks repeat others and are not used), chunk c of
+// row k sits at c ^ (k % 16): the 16 rows of a fragment read meet different banks.  Which indices a row switched on is
+// collected in LDS too: a store to memory inside the loop would have to be waited for together with the next stage.
+constexpr int kPmStage = 64;
+
+template <typename T, int KS, int MI, int W, bool ALL>
+__global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const float *__restrict__ t,
+                                                                      const T *__restrict__ Bm, int B, int r, int I,
+                                                                      int splits, int wb_rt, int per, float thr, int flags,
+                                                                      float *__restrict__ scores,
+                                                                      uint8_t *__restrict__ mask)
+{
+    constexpr int P = SplitParts<T>::value;
+    constexpr int kRow = 4 * KS, kBuf = kPmStage * kRow;      // 16-byte chunks
+    constexpr int kDma = kBuf / 64 / W;                       // 1 KB loads per wave and stage
+    extern __shared__ __align__(16) uint4 lds[];              // two buffers, then a byte per index of the block
+    uint8_t *hits = reinterpret_cast<uint8_t *>(lds + 2 * kBuf);
+    const int cmp_ge = flags & 1, round_storage = (flags >> 1) & 1;
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, q = lane >> 4;
+    const int wb = ALL ? W : wb_rt, ig = W / wb;              // wave groups that share a stage's tiles
+    // blocks of one XCD (ids equal modulo 8; `splits` is a multiple of 8 where it can be) work on the same rows of Bm
+    const int m0 = ((blockIdx.x / splits) * wb + wave % wb) * 16 * MI;
+    const int stages = (I + kPmStage - 1) / kPmStage;
+    const int s0 = (blockIdx.x % splits) * per, s1 = s0 + per < stages ? s0 + per : stages;
+    const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
+
+    const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint4 *)lds;
+    auto dma = [&](int stage, int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < kDma; ++j) {
+            const int at = (wave * kDma + j) * 64 + lane, row = at / kRow, pos = at % kRow;
+            int c = pos ^ (row & 15);
+            c = 8 * c < r ? c : 0;
+            int i = stage * kPmStage + row;
+            i = i < I ? i : I - 1;
+            const unsigned off = ((unsigned)i * (unsigned)r + 8u * (unsigned)c) * (unsigned)sizeof(T);
+            load_to_lds(lds_base + (unsigned)(b * kBuf + (wave * kDma + j) * 64) * 16u, off, reinterpret_cast<const char *>(Bm));
+        }
+    };
+    if (s0 >= s1) return;
+    dma(s0, 0);
+    for (int i = threadIdx.x; i < per * (kPmStage / 4); i += W * kWave) reinterpret_cast<uint32_t *>(hits)[i] = 0u;
+
+    uint4 tf[MI][P][KS];
+    float unscale[MI][4];    // of the rows this lane's results belong to
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const int m = m0 + 16 * i + l16;
+        const float *row = t + (size_t)(m < B ? m : B - 1) * r;
+        float v[KS][8];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int k = 32 * ks + 8 * q;
+            const float4 lo = *reinterpret_cast<const float4 *>(row + (k < r ? k : 0));
+            const float4 hi = *reinterpret_cast<const float4 *>(row + (k < r ? k + 4 : 0));
+            const float w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[ks][e] = k < r ? w[e] : 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) unscale[i][e] = 1.f;
+        if constexpr (P == 2) {
+            // a power of two per row that puts its largest finite element near 2^14
+            float big = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float a = fabsf(v[ks][e]);
+                    big = a < 3.0e38f ? fmaxf(big, a) : big;
+                }
+            big = fmaxf(big, __shfl_xor(big, 16, kWave));
+            big = fmaxf(big, __shfl_xor(big, 32, kWave));
+            int ex = (int)(__float_as_uint(big) >> 23) - 127;
+            ex = ex < -96 ? -96 : ex;                              // (also for a row of zeros)
+            const float scale = __uint_as_float((uint32_t)(127 + 13 - ex) << 23);
+            const float back = __uint_as_float((uint32_t)(127 - 13 + ex) << 23);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[ks][e] *= scale;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) unscale[i][e] = __shfl(back, 4 * q + e, kWave);
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            uint4 parts[P];
+            split_parts<T>(v[ks], parts);
+#pragma unroll
+            for (int p = 0; p < P; ++p) tf[i][p][ks] = parts[p];
+        }
+    }
+    // rows of t beyond B only exist in the last tiles: their scores do not count
+    unsigned live = 0u;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (m0 + 16 * i + 4 * q + e < B) live |= 1u << (4 * i + e);
+
+    for (int s = s0; s < s1; ++s) {
+        const int b = (s - s0) & 1;
+        ST_WAIT_VM_LGKM0(0);            // this wave's share of the stage has arrived (and the other buffer's reads are done)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (s + 1 < s1) dma(s + 1, b ^ 1);
+#pragma unroll
+        for (int j = 0; j < kPmStage / 16; ++j) {
+            if (!ALL && j % ig != wave / wb) continue;
+            uint4 bf[KS];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                bf[ks] = lds[b * kBuf + (16 * j + l16) * kRow + ((4 * ks + q) ^ l16)];
+                // (r > 32 (KS - 4): the launch picks KS; past the rank t is zero, and so must be what it meets)
+                if (ks >= KS - 4 && 32 * ks + 8 * q >= r) bf[ks] = zero4;
+            }
+            f32x4_t acc[MI][P];
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int p = 0; p < P; ++p) acc[i][p] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int p = 0; p < P; ++p)
+#pragma unroll
+                    for (int i = 0; i < MI; ++i) acc[i][p] = Mfma<T>::run(tf[i][p][ks], bf[ks], acc[i][p]);
+            const int col = s * kPmStage + 16 * j + l16;
+            bool any = false;
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float v = acc[i][P - 1][e];
+#pragma unroll
+                    for (int p = P - 2; p >= 0; --p) v += acc[i][p][e];   // smallest part first
+                    if constexpr (P == 2) v *= unscale[i][e];
+                    if (round_storage) v = to_float<T>(from_float<T>(v));
+                    const bool in = (live >> (4 * i + e)) & 1u;
+                    any = any || (in && (cmp_ge ? v >= thr : v > thr));
+                    if (scores && in && col < I) scores[(size_t)(m0 + 16 * i + 4 * q + e) * I + col] = v;
+                }
+            uint64_t hit = __builtin_amdgcn_ballot_w64(any);
+            hit |= hit >> 32;
+            hit |= hit >> 16;
+            if (lane < 16 && ((hit >> lane) & 1ull)) hits[(s - s0) * kPmStage + 16 * j + lane] = 1;
+        }
+    }
+    __syncthreads();
+    const int first = s0 * kPmStage, count = (I < s1 * kPmStage ? I : s1 * kPmStage) - first;
+    for (int i = threadIdx.x; i < count; i += W * kWave)
+        if (hits[i]) mask[first + i] = 1;
+}
+
+// From nine rows of x on.  The kernels of predictor.hip read every element of t from LDS for every row of x (about 1 us a
+// row at rank 256) and take x in passes of eight, sixteen and at last 64 rows; these take 7-14 us for any number up to 64.
+// Both kernels, replayed from a graph, there / here, at H 3072, rank 128, I 8192 (bf16): 7.5 / 8.4 us for 8 rows, 9.9 / 8.7
+// for 12, 17.0 / 9.6 for 32, 29.5 / 10.6 for 64, 233 / 15.6 for 512, 929 / 31 for 2048; at H 4096, rank 256, I 14336:
+// 10.6 / 10.6, 14.3 / 11.0, 25.0 / 12.1, 68.9 / 13.2, 538 / 29, 2236 / 78.  Ranks above 512 do not fit the registers.
+bool predictor_mfma_supported(int dtype, int B, int r) { return dtype != ST_F32 && B > 8 && r <= 512; }
+
+template <typename T>
+static int launch_t(const void *x, int B, int H, const void *A, int r, const void *Bm, int I, float thr, int cmp_ge,
+                    float *t_ws, float *scores, uint8_t *mask, int round_storage, hipStream_t stream)
+{
+    const int cus = device_cu_count();
+    {
+        ProfScope ps(ST_K_PRED_DOWN, stream);
+        auto go = [&](auto kern, int mi, int ni, int waves) -> int {
+            const int mt = (B + 16 * mi - 1) / (16 * mi), nt = (r + 16 * ni - 1) / (16 * ni);
+            const int lds = waves * 2 * 16 * (mi + ni) * 256;
+            const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
+            if (rc != ST_OK) return rc;
+            ST_LAUNCH(ps, kern, dim3(mt * nt), dim3(waves * kWave), lds, stream, static_cast<const T *>(x),
+                      static_cast<const T *>(A), B, H, r, nt, t_ws, mask, I, round_storage);
+            return ST_OK;
+        };
+        auto blocks = [&](int mi, int ni) { return ((B + 16 * mi - 1) / (16 * mi)) * ((r + 16 * ni - 1) / (16 * ni)); };
+        // 32 x 32 tiles (half the traffic from L2) once they make a block for three quarters of the CUs: 6.7 (16 x 16) against
+        // 8.6 us with 64 of them (512 rows, H 3072, rank 128), 17.8 against 11.8 us with 224, 40 against 26 us with 512
+        const int rc = 4 * blocks(2, 2) < 3 * cus ? go(predictor_down_mfma_kernel<T, 1, 1, 8>, 1, 1, 8)
+                                                  : go(predictor_down_mfma_kernel<T, 2, 2, 4>, 2, 2, 4);
+        if (rc != ST_OK) return rc;
+    }
+    ST_HIP(hipGetLastError());
+    {
+        ProfScope ps(ST_K_PRED_UP_MASK, stream);
+        // resident: blocks a CU holds at once (registers, LDS).  One round of blocks: every further one would split its
+        // rows of t into parts again.
+        auto go = [&](auto kern_all, auto kern, int ks, int mi, int waves, int resident) -> int {
+            int wb = 1;
+            while (wb < waves && B > 16 * mi * wb) wb *= 2;
+            const int mt = (B + 16 * mi * wb - 1) / (16 * mi * wb), stages = (I + kPmStage - 1) / kPmStage;
+            int splits = resident * cus / mt;
+            if (splits < 1) splits = 1;
+            int per = (stages + splits - 1) / splits;
+            per = per < 256 ? per : 256;                     // (the LDS bytes of a block's indices)
+            splits = (stages + per - 1) / per;
+            if (splits > kXcds) splits = (splits + kXcds - 1) / kXcds * kXcds;
+            const int lds = 2 * kPmStage * 4 * ks * 16 + per * kPmStage;
+            auto launch = [&](auto k) -> int {
+                const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(k), 2 * kPmStage * 4 * ks * 16 + 256 * kPmStage);
+                if (rc != ST_OK) return rc;
+                ST_LAUNCH(ps, k, dim3(mt * splits), dim3(waves * kWave), lds, stream, t_ws, static_cast<const T *>(Bm), B, r,
+                          I, splits, wb, per, thr, (cmp_ge ? 1 : 0) | (round_storage ? 2 : 0), scores, mask);
+                return ST_OK;
+            };
+            return wb == waves ? launch(kern_all) : launch(kern);
+        };
+#define ST_PM_UP(KS, MI, W, RES) go(predictor_up_mfma_kernel<T, KS, MI, W, true>, predictor_up_mfma_kernel<T, KS, MI, W, false>, KS, MI, W, RES)
+        int rc;
+        // (eight waves share a stage once there are rows of x for them: 16 rows in blocks of eight waves 5.2 us, of four 4.4)
+        if (B <= 64) {
+            if (r <= 128) rc = ST_PM_UP(4, 1, 4, 4);
+            else if (r <= 256) rc = ST_PM_UP(8, 1, 4, 2);
+            else if (r <= 384) rc = ST_PM_UP(12, 1, 4, 1);
+            else rc = ST_PM_UP(16, 1, 4, 1);
+        } else if (r <= 128) rc = ST_PM_UP(4, 1, 8, 2);
+        else if (r <= 256) rc = ST_PM_UP(8, 1, 8, 1);
+        else if (r <= 384) rc = ST_PM_UP(12, 1, 8, 1);
+        else rc = ST_PM_UP(16, 1, 4, 1);   // (eight waves of 256 registers cannot hold its parts)
+#undef ST_PM_UP
+        if (rc != ST_OK) return rc;
+    }
+    ST_HIP(hipGetLastError());
+    return ST_OK;
+}
+
+int launch_predictor_mfma(int dtype, const void *x, int B, int H, const void *A, int r, const void *Bm, int I, float thr,
+                          int cmp_ge, float *t_ws, float *scores, uint8_t *mask, int round_storage, hipStream_t stream)
+{
+    if (dtype == ST_F16)
+        return launch_t<f16_t>(x, B, H, A, r, Bm, I, thr, cmp_ge, t_ws, scores, mask, round_storage, stream);
+    return launch_t<bf16_t>(x, B, H, A, r, Bm, I, thr, cmp_ge, t_ws, scores, mask, round_storage, stream);
+}
+
+}  // namespace st

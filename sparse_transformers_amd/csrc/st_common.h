@@ -270,6 +270,11 @@ int launch_batch(int dtype, const void *x, int B, int H, const void *gate, const
                  const int *n_dev, void *out, void *comb, long ldc, void *workspace, int act, int has_gate,
                  hipStream_t stream);
 
+// Predictor on the matrix cores for several rows of x (fp16 / bf16, rank up to 512).
+bool predictor_mfma_supported(int dtype, int B, int r);
+int launch_predictor_mfma(int dtype, const void *x, int B, int H, const void *A, int r, const void *Bm, int I, float thr,
+                          int cmp_ge, float *t_ws, float *scores, uint8_t *mask, int round_storage, hipStream_t stream);
+
 // Double precision forward (plain kernels, for checking a model in fp64).
 int64_t f64_workspace_bytes(int64_t B, int64_t H, int64_t n);
 int launch_f64(const void *x, int B, int H, const void *gate, const void *up, const void *down, int n, const int *n_dev,

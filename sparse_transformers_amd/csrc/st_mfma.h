@@ -30,6 +30,24 @@ template <> struct Mfma<bf16_t> {
     }
 };
 
+constexpr int kXcds = 8;
+
+// s_waitcnt immediate: vmcnt in bits 3:0 (and 15:14), expcnt 6:4 left at "no wait", lgkmcnt 11:8 = 0
+#define ST_WAIT_VM_LGKM0(vm) __builtin_amdgcn_s_waitcnt(((vm) & 15) | (7 << 4) | (0 << 8) | (((vm) >> 4) << 14))
+
+// 64 lanes x 16 bytes from `base + off` (uniform base, per-lane byte offset) to the 1 KB of LDS at byte address
+// `dst` (uniform), lane i's 16 bytes at dst + 16 i.  The instruction takes the LDS address from M0; the compiler is not
+// told about M0 (it is a reserved register for inline assembly), so its value is put back, and the write of M0 is
+// followed by the wait state the instruction needs before it may read it.
+__device__ __forceinline__ void load_to_lds(unsigned dst, unsigned off, const char *base)
+{
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "s"(dst), "v"(off), "s"(base)
+                 : "memory");
+}
+
 __device__ __forceinline__ int device_count(int n_host, const int *n_dev)
 {
     int n = n_host;

@@ -53,6 +53,38 @@ def test_scores_and_mask(B, H, r, I, dtype, frac):
     assert near.sum() <= 3, f"guard band population {near.sum()}"      # expected 0, reported if not
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("B,H,r,I", [
+    (8, 64, 8, 17),          # one tile of everything, none of them full
+    (16, 72, 40, 50),        # H is not a multiple of a k step
+    (17, 1024, 128, 2048),   # one row into the second tile of rows
+    (33, 512, 136, 1000),    # ranks one chunk into the next register form: 128, 256, 384
+    (64, 768, 264, 1024),
+    (65, 768, 392, 777),
+    (130, 3072, 512, 4096),  # the largest rank of these kernels
+    (300, 640, 24, 333),
+    (515, 2048, 128, 8192),
+])
+def test_matrix_core_predictor(B, H, r, I, dtype):
+    """Several rows of x: fp32 accuracy of the scores although the rank-r intermediate goes through 16-bit operands,
+    also for rows of very different magnitude."""
+    x, A, Bm = _weights(B + r, B, H, r, I, dtype)
+    mag = torch.logspace(-3, 3, B)[:, None]
+    x = (x.float() * mag).to(x.dtype)
+    s_ref = oracle.predictor_scores(x.float().numpy(), A.float().numpy(), Bm.float().numpy())
+    m, s = st.predictor_mask(x.to(DEV), A.to(DEV), Bm.to(DEV), 0.0, True, return_scores=True)
+    scale = np.abs(s_ref).max(1, keepdims=True)                     # per row: each has its own magnitude
+    assert (np.abs(s.cpu().numpy() - s_ref) <= 2e-6 * scale + 1e-12).all()   # (the bound of test_scores_and_mask, per row)
+    # a cut that only a few indices pass in any row, so that every row decides some of them
+    thr = float(np.sort(s_ref.max(0))[-max(1, I // 3)]) * (1 - 1e-4)
+    near = (np.abs(s_ref - thr) < 8e-6 * scale).any(0)
+    for ge in (True, False):
+        got = st.predictor_mask(x.to(DEV), A.to(DEV), Bm.to(DEV), thr, ge).cpu().numpy()
+        assert np.array_equal(got[~near], oracle.mask_threshold(s_ref, thr, ge)[~near])
+    assert near.mean() < 0.01 + 2.0 / I
+    assert np.array_equal(m.cpu().numpy(), (s.cpu().numpy() >= 0).any(0))   # mask and scores come from the same sums
+
+
 def test_naive_threshold_is_score_ge_zero():
     x, A, Bm = _weights(1, 2, 256, 16, 512, "float32")
     # make some scores exactly zero: a zero row of Bm gives score 0 for every input row
