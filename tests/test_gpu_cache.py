@@ -93,6 +93,46 @@ def test_full_size_index_order(I, n, lo, hi):
     assert st_["n_active"] == n and st_["n_added"] == st_["n_removed"] > 0
 
 
+@pytest.mark.parametrize("I", [7, 1025, 8192, 14336, 16001, 22000])
+def test_surplus_removals(I):
+    """Updates that remove more than they add, in the stand-alone update kernel: everything but one index at once, a few
+    and a few thousand, removals that sit at the end of the list (each step's moved entry is itself removed later) or
+    spread over it, with additions beside them."""
+    H = 8
+    rng = np.random.default_rng(I)
+    g, u, d = (rng.standard_normal(s).astype(np.float32) for s in ((I, H), (I, H), (H, I)))
+    oc = oracle.OracleWeightCache(np.ones(I, bool), H, g, u, d, True)
+    wc = st.WeightCache(torch.ones(I, dtype=torch.bool, device=DEV), H, _t(g), _t(u), _t(d), True)
+    cur = np.ones(I, bool)
+
+    def step(m):
+        nonlocal cur
+        cur = m
+        oc.update_active_weights(m)
+        wc.update_active_weights_async(_t(m, torch.bool))
+        assert wc.get_active_indices().cpu().tolist() == oc.get_active_indices().tolist()
+
+    for frac in (0.35, 0.9, 0.2, 0.95, 0.6):
+        for _ in range(3):
+            step(rng.random(I) < frac)
+        for removed in (1, 3, 65, 1100, I // 3):      # from the end of the list, a few additions beside them
+            order = oc.get_active_indices()
+            m = cur.copy()
+            m[order[-removed:]] = False
+            off = np.flatnonzero(~cur)
+            m[off[: min(len(off), removed // 4)]] = True
+            if not m.any():
+                m[I // 2] = True
+            step(m)
+            m = cur | (rng.random(I) < 0.3)           # and room for the next one
+            step(m)
+    one = np.zeros(I, bool)
+    one[I // 2] = True
+    step(one)
+    step(np.ones(I, bool))
+    _check_layout(wc, oc.get_active_indices().tolist(), g, u, d, True)
+
+
 @pytest.mark.parametrize("I,has_gate", [(28672, True), (32768, False), (22016, True)])
 def test_large_intermediate_sizes(I, has_gate):
     """Intermediate sizes of the 70B-class models (28672), above what the index lists of the smaller kernels allow:
