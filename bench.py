@@ -6,9 +6,10 @@ predictor + threshold mask, the differential weight-cache update (driven by a pr
 with the workload's active fraction and per-step churn) and the fused sparse MLP.  All inputs (weights,
 predictor inputs, mask trace) are resident in HBM before the timed region starts.
 
-Prints ONE JSON line.  `roofline` is for the dominant kernel (the decode MLP with the cache update fused
-into it): algorithmic bytes per launch -- 3*n*H*s of active weights plus 2*3*k*H*s for the k changed rows
-of the update -- over its mean duration, measured with HIP events stamped at the kernel's begin and end
+Prints ONE JSON line.  `roofline` is for the dominant kernel (the decode MLP; in stacks of one or two layers the
+cache update is fused into it, in deeper ones the updates of all layers are one launch ahead of it): algorithmic
+bytes per launch -- 3*n*H*s of active weights, plus 2*3*k*H*s for the k changed rows of a fused update -- over its
+mean duration, measured with HIP events stamped at the kernel's begin and end
 in a second pass over the same workload.  `cpu_baseline` times the same path on the host cores on a
 bounded sample.
 """
@@ -86,7 +87,8 @@ def parse_args():
     ap.add_argument("--overlap", action="store_true",
                     help="run predictor/cache update on a side stream (measured slower inside a graph; off by default)")
     ap.add_argument("--no-fused", action="store_true",
-                    help="cache update and MLP as two kernels per layer instead of the fused update+decode kernel")
+                    help="cache update and MLP as two kernels per layer instead of the fused update+decode kernel or "
+                         "the launches shared between the layers of a stack")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-prefill-probe", action="store_true",
                     help="skip the short 512-row MFMA pass whose figures the decode line carries as `prefill_512`")
@@ -478,10 +480,14 @@ def decode_measure(args, wl, torch, st, _lib, syn, layers, B, K, W, P, count_wob
     wall_parts = None
     if wall and use_graph and not args.overlap and not from_predictor:
         def part_predictor():
+            if stack.fused and stack._batched():
+                return stack._predict_all()
             for l, layer in enumerate(stack.layers):
                 layer.predict_mask(stack.xp_stage[l], stack._t_ws)
 
         def part_update_mlp():
+            if stack.fused and stack._batched():
+                return stack._update_all_and_forward()
             x = stack.x_stage
             for l, layer in enumerate(stack.layers):
                 out = stack._pingpong[l & 1]
@@ -549,7 +555,8 @@ def decode_measure(args, wl, torch, st, _lib, syn, layers, B, K, W, P, count_wob
                    "churn": [wl.churn_lo, wl.churn_hi], "count_wobble": count_wobble, "mask_source": mask_source,
                    "changed_rows_mean": round(k_changed, 1),
                    "launch": "hip_graph" if use_graph else "eager",
-                   "streams": 2 if args.overlap else 1, "update_fused_into_decode": bool(stack.fused),
+                   "streams": 2 if args.overlap else 1, "update_fused_into_decode": bool(stack.fused and not stack._batched()),
+                   "launches_shared_between_layers": bool(stack.fused and stack._batched()),
                    "kernel_timing": "hip events stamped at kernel begin/end (hipExtLaunchKernelGGL), second pass launched call by call, each step queued behind a spin kernel so that its kernels run back to back"},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBPS, 4),
@@ -560,12 +567,13 @@ def decode_measure(args, wl, torch, st, _lib, syn, layers, B, K, W, P, count_wob
                      "bytes_mlp": alg_bytes, "bytes_cache_update": upd_bytes if dom == "cache_update_decode" else 0,
                      "frac_mlp_bytes_only": round(alg_bytes / (mlp_us * 1e-6) / 1e9 / HBM_PEAK_GBPS, 4)},
         "cache_update_us_per_layer": upd_us,
-        "cache_update_note": ("standalone cache_update_kernel, measured in a short unfused pass; the timed path "
-                              "runs it fused into the decode kernel") if unfused else "standalone kernel",
+        "cache_update_note": ("cache_update_kernel of a single layer, measured in a short unfused pass; the timed path runs "
+                              "it fused into the decode kernel or, from three layers on, as one launch for the stack")
+                             if unfused else "standalone kernel",
         "stack_hbm_gbps": round(layers * alg_bytes / (ms_per_step * 1e-3) / 1e9, 1),
         "host_wall_ms_per_step": round(host_s * 1e3 / K, 5),
         "wall_us_per_layer": wall_parts,
-        "wall_note": "graph replays of the predictor kernels alone, of update + MLP (+ reduce) alone, and of the whole step",
+        "wall_note": "graph replays of the predictor kernels alone, of update + MLP (+ reduce) alone, and of the whole step (staging copies included)",
         "kernels_us": per_kernel,
         "kernels_us_unfused": unfused,
         "churn_mean": churn_mean,

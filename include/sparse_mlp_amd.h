@@ -138,6 +138,19 @@ int st_predictor_mask_ex(const void *x, int64_t B, int64_t H, const void *A, int
                          int dtype, float thr, int cmp_ge, int flags, float *t_ws, float *scores, uint8_t *mask,
                          void *stream);
 
+/* The same for the L layers of a stack whose predictor inputs are all at hand (equal shapes, dtype and flags): what L
+ * calls of st_predictor_mask_ex without `scores` do, two launches for up to 32 layers.  `layers` is a HOST array,
+ * read before the call returns; the pointers in it are device pointers.  x [L,B,H]; t_ws float [L,B,r]. */
+typedef struct st_predictor_layer {
+    const void *A;    /* [r,H] */
+    const void *Bm;   /* [I,r] */
+    uint8_t *mask;    /* [I], different for every layer */
+    float thr;
+    int32_t cmp_ge;
+} st_predictor_layer;
+int st_predictor_mask_layers(const st_predictor_layer *layers, int64_t L, const void *x, int64_t B, int64_t H, int64_t r,
+                             int64_t I, int dtype, int flags, float *t_ws, void *stream);
+
 /* ------------------------------------------------------------------------
  * Mask methods that need a statistic of the whole score row, then the union
  * over rows.  Replaces the "topk" and "statistical_topk" branches and the
@@ -230,6 +243,11 @@ int st_cache_load_weights(st_cache *c, const void *gate, const void *up, const v
  * state[ST_STATE_STATUS] = ST_ERR_NO_ACTIVE and, like the reference, leaves
  * cur_mask unchanged. */
 int st_cache_update_async(st_cache *c, const uint8_t *mask, void *stream);
+
+/* st_cache_update_async for the caches of L different layers, one mask each (HOST arrays of handles and of device
+ * pointers, read before the call returns): caches of equal shape share a launch, up to 32 at a time.  The caches
+ * must be different ones. */
+int st_cache_update_layers(st_cache *const *caches, const uint8_t *const *masks, int64_t L, void *stream);
 
 /* Copies the state words to the host (waits for `stream`).  Returns
  * ST_ERR_NO_ACTIVE if the last update emptied the cache, else ST_OK.

@@ -32,6 +32,10 @@ class CacheBuffers(C.Structure):
     ]
 
 
+class PredictorLayer(C.Structure):
+    _fields_ = [("A", C.c_void_p), ("Bm", C.c_void_p), ("mask", C.c_void_p), ("thr", C.c_float), ("cmp_ge", C.c_int32)]
+
+
 # name -> (restype, argtypes); every symbol include/sparse_mlp_amd.h declares
 _vp, _i64, _ci, _f = C.c_void_p, C.c_int64, C.c_int, C.c_float
 SIGNATURES = {
@@ -45,6 +49,7 @@ SIGNATURES = {
     "st_mlp_forward_static": (_ci, [_vp, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _ci, _ci, _ci, _vp]),
     "st_predictor_mask": (_ci, [_vp, _i64, _i64, _vp, _i64, _vp, _i64, _ci, _f, _ci, _vp, _vp, _vp, _vp]),
     "st_predictor_mask_ex": (_ci, [_vp, _i64, _i64, _vp, _i64, _vp, _i64, _ci, _f, _ci, _ci, _vp, _vp, _vp, _vp]),
+    "st_predictor_mask_layers": (_ci, [C.POINTER(PredictorLayer), _i64, _vp, _i64, _i64, _i64, _i64, _ci, _ci, _vp, _vp]),
     "st_mask_select_workspace_bytes": (_i64, [_i64, _i64]),
     "st_mask_select": (_ci, [_vp, _i64, _i64, _ci, _i64, _f, _vp, _vp, _vp, _i64, _vp]),
     "st_approx_topk_threshold": (_ci, [_vp, _i64, _i64, _i64, _vp, _vp]),
@@ -54,6 +59,7 @@ SIGNATURES = {
     "st_cache_destroy": (None, [_vp]),
     "st_cache_load_weights": (_ci, [_vp, _vp, _vp, _vp, _vp]),
     "st_cache_update_async": (_ci, [_vp, _vp, _vp]),
+    "st_cache_update_layers": (_ci, [C.POINTER(_vp), C.POINTER(_vp), _i64, _vp]),
     "st_cache_update_forward": (_ci, [_vp, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _i64, _ci, _vp]),
     "st_cache_sync_state": (_ci, [_vp, _vp, _vp]),
     "st_cache_materialize_concat": (_ci, [_vp, _vp, _i64, _vp]),

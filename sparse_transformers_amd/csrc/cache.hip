@@ -109,14 +109,16 @@ struct FusedRows {
     int row_bytes, has_gate;
 };
 
-constexpr int kCopyUnroll = 4;  // rows a thread group keeps in flight
-
-constexpr int kPlanMaxWords = 4;  // 8-element words per thread in the vector path: I <= 32 * threads
-
 __device__ __forceinline__ uint64_t nonzero_bytes(uint64_t x)
 {
     x |= x >> 4; x |= x >> 2; x |= x >> 1;
     return x & 0x0101010101010101ull;
+}
+
+// 0x01-per-element bytes -> 8 bits (element k -> bit k)
+__device__ __forceinline__ uint32_t pack_bits8(uint64_t ones)
+{
+    return (uint32_t)((ones * 0x0102040810204080ull) >> 56);
 }
 
 // The plan as every block computes it, and the LDS arrays that hold it.
@@ -152,16 +154,16 @@ struct PlanShared {
 // list the previous one left, but where e_k is at its own step follows by chasing: it stays where it starts unless that is
 // a tail slot n-1-i of an earlier step i < k, which moved it to where e_i was, and so on.  Only the e_k that START in the
 // tail have to chase (about S^2 / n of them), and only through one another: they resolve in rounds, a thread each (a
-// chase that meets an unresolved one tries again in the next round; the smallest unresolved always gets through).  Then
-// every entry of the tail that stays follows the moves until one takes it below the tail, all of them at once.
-// One lane that took the steps in order needed 0.2 us for each (13 us of a 29 us update with 70 of them); this takes under
-// 2 us for any number.
-// surplus[-k] = e_k; overwritten.  *n_new: the count afterwards.  `dirty`: bits of the rewritten positions.
-template <int TPB, typename S>
-__device__ __forceinline__ void surplus_removals(uint16_t *idx_l, const uint16_t *pos_l, uint16_t *surplus, int S_all, int n,
-                                                 uint32_t *dirty, uint32_t *wave_tot, int *n_new, int tid, S sync)
+// chase that meets an unresolved one tries again in the next round; the smallest unresolved always gets through).  An
+// entry of the tail that stays, at slot n-1-j, then ends at place[j], followed on through place[n-1-q] while that is a
+// tail slot q.  One lane that took the steps in order needed 0.2 us for each (13 us of a 29 us update with 70 of them);
+// this takes under 2 us for any number.
+// place(k): in: where e_k starts (kNone: not in the list, no step at all: only after an update that failed; the others
+// move up); out: where it is at its step.  Returns the count after the steps (in every thread).
+template <int TPB, typename P, typename S>
+__device__ __forceinline__ int surplus_places(P place, int S_all, int n, uint32_t *wave_tot, int *shared_n, int tid, S sync)
 {
-    constexpr uint16_t kOpen = 0x8000u;    // (positions and indices stay below kPlanMaxI < 0x8000)
+    constexpr int kOpen = 0x8000;    // (positions stay below kPlanMaxI < 0x8000)
     const int lane = tid & (kWave - 1), wave = tid >> 6;
     auto any_of = [&](bool v) __attribute__((always_inline)) {   // over the block
         const bool w = __builtin_amdgcn_ballot_w64(v) != 0;
@@ -172,62 +174,48 @@ __device__ __forceinline__ void surplus_removals(uint16_t *idx_l, const uint16_t
         for (int k = 0; k < TPB / kWave; ++k) r |= wave_tot[k];
         return r != 0;
     };
-    // where each starts; indices that are not in the list are no step at all (only after an update that failed)
     bool missing = false;
-    for (int k = tid; k < S_all; k += TPB) {
-        const uint16_t p = pos_l[surplus[-k]];
-        surplus[-k] = p;
-        missing = missing || p == kNone;
-    }
+    for (int k = tid; k < S_all; k += TPB) missing = missing || place(k) == kNone;
     int S_ = S_all;
     if (any_of(missing)) {
         if (tid == 0) {
             int m = 0;
             for (int k = 0; k < S_all; ++k)
-                if (surplus[-k] != kNone) surplus[-m++] = surplus[-k];
-            *n_new = m;
+                if (place(k) != kNone) { const uint16_t v = place(k); place(m) = v; ++m; }
+            *shared_n = m;
         }
         sync();
-        S_ = *n_new;
+        S_ = *shared_n;
         sync();
     }
     const int base = n - S_;
     bool open = false;
     for (int k = tid; k < S_; k += TPB) {
-        const int p = surplus[-k];
+        const int p = place(k);
         if (p >= base) {
-            idx_l[p] |= kOpen;              // an entry of the tail that does not stay
-            surplus[-k] = (uint16_t)p | kOpen;
+            place(k) = (uint16_t)(p | kOpen);
             open = true;
         }
     }
     while (any_of(open)) {                  // (uniform; at least one resolves per round)
         open = false;
         for (int k = tid; k < S_; k += TPB) {
-            int q = surplus[-k];
+            int q = place(k);
             if (!(q & kOpen)) continue;
             q &= kOpen - 1;
             bool done = false;
             for (int hop = 0; hop <= S_; ++hop) {
                 const int i = n - 1 - q;
                 if (q < base || i >= k) { done = true; break; }   // stays there until its own step (i == k: it is the last entry)
-                const int d = surplus[-i];
+                const int d = place(i);
                 if (d & kOpen) break;
                 q = d;
             }
-            if (done) surplus[-k] = (uint16_t)q;
+            if (done) place(k) = (uint16_t)q;
             else open = true;
         }
     }
-    for (int j = tid; j < S_; j += TPB) {
-        const int v = idx_l[n - 1 - j];
-        if (v & kOpen) continue;
-        int q = surplus[-j];
-        for (int hop = 0; hop <= S_ && q >= base; ++hop) q = surplus[-(n - 1 - q)];
-        idx_l[q] = (uint16_t)v;
-        atomicOr(&dirty[q >> 5], 1u << (q & 31));
-    }
-    if (tid == 0) *n_new = base;
+    return base;
 }
 
 // Replays the bookkeeping of one update in LDS and publishes it (block 0 writes the other bookkeeping
@@ -237,13 +225,14 @@ __device__ __forceinline__ void surplus_removals(uint16_t *idx_l, const uint16_t
 // buffers are requested together with the ticket, so the front costs one memory round trip.  MARK: the
 // dirty bitmap is kept on the fast path too.  `after_issue()` runs right after the front loads have
 // been issued, `after_fill()` right after the first barrier (the front loads have arrived and been consumed).
+// NW: 8-element words per thread of the vector path (I <= 8 NW threads); the registers of the front loads follow from it.
 // idx_cap: only that many positions of the index lists are fetched up front (the rest follows if the count
 // turns out larger).
 //
 // Barrier sequence: 1 after the LDS fill; 2 in the diff scan;
 // [unchanged mask: done]; 1 after the lists; 1 after phases 1 and 2; [surplus removals: those of surplus_removals and 1
 // behind it, 2 in the compaction scan, 1 after the compaction].
-template <bool VEC, int PT, bool MARK, typename F, typename F2>
+template <bool VEC, int PT, int NW, bool MARK, typename F, typename F2>
 __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, PlanShared *ps,
                                            const uint8_t *__restrict__ new_mask, uint8_t *__restrict__ cur_mask2,
                                            int32_t *__restrict__ indices2, int32_t *__restrict__ state, int I,
@@ -279,12 +268,12 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
 
     // (several small arrays rather than one big one: each has to stay below the size up to which the
     // compiler keeps a private array in registers)
-    uint64_t v_new[kPlanMaxWords], v_cur0[kPlanMaxWords], v_cur1[kPlanMaxWords];
-    int4 v_i0a[kPlanMaxWords], v_i0b[kPlanMaxWords], v_i1a[kPlanMaxWords], v_i1b[kPlanMaxWords];
+    uint64_t v_new[NW], v_cur0[NW], v_cur1[NW];
+    int4 v_i0a[NW], v_i0b[NW], v_i1a[NW], v_i1b[NW];
     int n_both[2];
     if constexpr (VEC) {
 #pragma unroll
-        for (int w = 0; w < kPlanMaxWords; ++w) {
+        for (int w = 0; w < NW; ++w) {
             const int e = e0 + 8 * w;
             if (e < e1) {
                 v_new[w] = *reinterpret_cast<const uint64_t *>(new_mask + e);
@@ -309,11 +298,11 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
 
     int n;
     // VEC: new / current mask words as 0x01 bytes, kept in registers for the diff and for publishing
-    uint64_t w_new[kPlanMaxWords], w_cur[kPlanMaxWords];
+    uint64_t w_new[NW], w_cur[NW];
     if constexpr (VEC) {
         n = ep ? n_both[1] : n_both[0];
 #pragma unroll
-        for (int w = 0; w < kPlanMaxWords; ++w) {
+        for (int w = 0; w < NW; ++w) {
             const int e = e0 + 8 * w;
             w_new[w] = w_cur[w] = 0;
             if (e < e1) {
@@ -356,7 +345,7 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
     uint32_t cnt = 0;  // added in the low half, removed in the high half
     if constexpr (VEC) {
 #pragma unroll
-        for (int w = 0; w < kPlanMaxWords; ++w)
+        for (int w = 0; w < NW; ++w)
             cnt += (uint32_t)__popcll(w_new[w] & ~w_cur[w]) + ((uint32_t)__popcll(w_cur[w] & ~w_new[w]) << 16);
     } else {
         for (int i = e0; i < e1; ++i) {
@@ -385,7 +374,7 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
         int oa = (int)(off & 0xffffu), orr = (int)(off >> 16);
         if constexpr (VEC) {
 #pragma unroll
-            for (int w = 0; w < kPlanMaxWords; ++w) {
+            for (int w = 0; w < NW; ++w) {
                 const int e = e0 + 8 * w;
                 uint64_t a = w_new[w] & ~w_cur[w], r = w_cur[w] & ~w_new[w];   // one 0x01 byte per element, ascending
                 while (a) {
@@ -444,10 +433,26 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
         n_changed = (uint32_t)na;
         ST_TL(4);
     } else {
-        surplus_removals<TPB>(idx_l, pos_l, lists + I - 1 - pairs, nr - pairs, n, dirty, wave_tot, &n_new_s, tid, sync);
+        // (the places go over the removed indices, k-th surplus one at lists[I-1-pairs-k]; a surplus index is marked by
+        // having no position any more)
+        const int S_all = nr - pairs;
+        auto place = [&](int k) __attribute__((always_inline)) -> uint16_t & { return lists[I - 1 - pairs - k]; };
+        for (int k = tid; k < S_all; k += TPB) {
+            const int e = place(k);
+            place(k) = pos_l[e];
+            pos_l[e] = kNone;
+        }
+        n_new = surplus_places<TPB>(place, S_all, n, wave_tot, &n_new_s, tid, sync);
+        for (int j = tid; j < n - n_new; j += TPB) {
+            const int v = idx_l[n - 1 - j];
+            if (pos_l[v] == kNone) continue;
+            int q = place(j);
+            for (int hop = 0; hop <= S_all && q >= n_new; ++hop) q = place(n - 1 - q);
+            idx_l[q] = (uint16_t)v;
+            atomicOr(&dirty[q >> 5], 1u << (q & 31));
+        }
         sync();
         ST_TL(4);
-        n_new = n_new_s;
 
         // ---- compact the dirty positions below n_new into the copy list (in LDS, over the dead lists)
         uint32_t word = 0;
@@ -475,7 +480,7 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
         // the reference stores the new mask only when the rebuild did not throw (n_new > 0)
         if constexpr (VEC) {
 #pragma unroll
-            for (int w = 0; w < kPlanMaxWords; ++w) {
+            for (int w = 0; w < NW; ++w) {
                 const int e = e0 + 8 * w;
                 if (e < e1) *reinterpret_cast<uint64_t *>(mask_out + e) = n_new > 0 ? w_new[w] : w_cur[w];
             }
@@ -517,65 +522,332 @@ __device__ __forceinline__ void plan_finish(const PlanView &pv, int32_t *__restr
     }
 }
 
-// update = plan + this block's share of the row copies
-template <bool VEC, int TPB>
+// ---------------------------------------------------------------------------
+// update kernel
+// ---------------------------------------------------------------------------
+// The caches of one launch: several layers of equal shape (grid dimension y) or one.
+struct UpdateLayer {
+    const uint8_t *new_mask;
+    uint8_t *cur_mask2;
+    int32_t *indices2, *state;
+    const unsigned char *pool[3];
+    unsigned char *active[3];
+};
+struct UpdateLayers {
+    static constexpr bool kLayers = true;
+    UpdateLayer l[kMaxLayers];
+};
+
+// A work item: position `pos` is rewritten with pool row `idx` (kNone or a position past the new count: nothing to do).
+// This block's share of them, a wave per (item, matrix) with the whole row in flight (8 KB): at usual churn every wave has
+// at most one, so the copies cost one round trip.  (A thread group of 512 per row and four rows in flight left a quarter of
+// the lanes of a 6 KB row idle and took two dependent rounds from 1500 (item, matrix) pairs on: 11 us for 2600 of them.)
+template <int TPB>
+__device__ __forceinline__ void copy_items(const unsigned char *const (&pool)[3], unsigned char *const (&active)[3], int nmat,
+                                           int row_bytes, int tid, int items, int n_new, const uint16_t *pos,
+                                           const uint16_t *idx)
+{
+    constexpr int W = TPB / kWave;
+    const int lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int chunks = row_bytes >> 4;
+    const unsigned char *const pool0 = pool[0], *const pool1 = pool[1], *const pool2 = pool[2];
+    unsigned char *const act0 = active[0], *const act1 = active[1], *const act2 = active[2];
+    // the publishing block takes no copies when there are others to do them
+    const bool solo = gridDim.x == 1;
+    const int slots = (solo ? 1 : (int)gridDim.x - 1) * W;
+    const int work = items * nmat;
+    // (neighbouring items to different blocks: blocks own waves blk, blk + blocks, ...)
+    for (int w = solo ? wave : blockIdx.x == 0 ? work : (int)blockIdx.x - 1 + ((int)gridDim.x - 1) * wave; w < work; w += slots) {
+        const int j = w / nmat, m = w - j * nmat;
+        const int p = __builtin_amdgcn_readfirstlane((int)pos[j]), e = __builtin_amdgcn_readfirstlane((int)idx[j]);
+        if (p >= n_new) continue;
+        const unsigned char *from = (m == 0 ? pool0 : m == 1 ? pool1 : pool2) + (size_t)e * row_bytes;
+        unsigned char *to = (m == 0 ? act0 : m == 1 ? act1 : act2) + (size_t)p * row_bytes;
+        constexpr int U = 8;
+        for (int c0 = lane; c0 < chunks; c0 += U * kWave) {
+            uint4 v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int c = c0 + u * kWave;
+                v[u] = ld16_stream(from + ((size_t)(c < chunks ? c : chunks - 1) << 4));
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int c = c0 + u * kWave;
+                if (c < chunks) st16(to + ((size_t)c << 4), v[u]);
+            }
+        }
+    }
+}
+
+// LDS of the kernel below: two bytes per index for each of the items' indices, their positions and the surplus removals'
+// places, and three per eight indices for the ranks of the removed ones.
+constexpr size_t update_lds_bytes(int I)
+{
+    const size_t groups = (size_t)((I + 7) >> 3);
+    return (size_t)((I + 7) & ~7) * 6 + ((groups * 2 + 15) & ~(size_t)15) + ((groups + 15) & ~(size_t)15);
+}
+
+// The update by POSITION.  Which index a position holds afterwards follows from the old list and the two masks without an
+// index -> position map: a removed index has a rank among the removed ones (a prefix count per eight indices, and the
+// bits below it), the i-th of them hands its position to the i-th added index (phase 1), the surplus additions follow at
+// the end (phase 2), and a position of rank >= n_added is where a surplus removal starts (phase 3, surplus_places).  So
+// the plan is one scan, one pass over the list -- every thread keeps the positions it loaded in registers -- and two
+// barriers when removals do not outnumber additions.  Every block plans for itself (as a launch of its own the plan would
+// cost a kernel boundary) and copies its share of the items.
+// Masks in 8-byte words, lists in 16-byte vectors (I % 8 == 0, aligned buffers); I <= 8 NW TPB.
+template <int TPB, int NW, typename Tab>
 __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__restrict__ new_mask,
-                                                                    uint8_t *__restrict__ cur_mask2,
-                                                                    int32_t *__restrict__ indices2,
-                                                                    int32_t *__restrict__ state, int I, int gs_log2,
-                                                                    int idx_cap, CopyPlan cp)
+                                                           uint8_t *__restrict__ cur_mask2,
+                                                           int32_t *__restrict__ indices2, int32_t *__restrict__ state,
+                                                           int I, int idx_cap, CopyPlan cp, Tab tab)
+{
+    if constexpr (Tab::kLayers) {
+        const UpdateLayer &ly = tab.l[blockIdx.y];
+        new_mask = ly.new_mask;
+        cur_mask2 = ly.cur_mask2;
+        indices2 = ly.indices2;
+        state = ly.state;
+    }
+    constexpr int NV = 2 * NW;                 // vectors of four positions per thread
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ uint32_t wave_tot[TPB / kWave];
+    __shared__ int shared_n;
+    __shared__ uint32_t shared_changed;
+    const int Ip = (I + 7) & ~7;
+    uint16_t *const item_idx = reinterpret_cast<uint16_t *>(smem);   // added indices ascending; behind them the tail's entries
+    uint16_t *const item_pos = item_idx + Ip;
+    uint16_t *const place = item_pos + Ip;                           // k-th surplus index: where it starts, then where its step finds it
+    uint16_t *const rem_before = place + Ip;                         // per eight indices: removed ones below
+    uint8_t *const rem_bits = reinterpret_cast<uint8_t *>(rem_before) + ((((I + 7) >> 3) * 2 + 15) & ~15);
+    const int tid = threadIdx.x;
+    const bool writer = blockIdx.x == 0;
+    auto sync = [&]() __attribute__((always_inline)) { lds_barrier(); };
+
+    ST_TL(0);
+    // ---- everything the plan reads, in one round trip: both halves of the double buffers are requested before the epoch
+    // word has arrived.  (The epoch cannot flip before every block has arrived, and a block arrives -- one atomic, at the
+    // end of its plan -- after all its threads have consumed this load.)
+    const uint32_t tword = __hip_atomic_load(reinterpret_cast<const uint32_t *>(&state[ST_STATE_TICKET]), __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+    const int words = (I + 8 * TPB - 1) / (8 * TPB);   // per thread: a contiguous range, so that lists come out ascending
+    uint64_t v_new[NW], v_cur0[NW], v_cur1[NW];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const int e = 8 * (tid * words + w), ec = w < words && e < I ? e : 0;
+        v_new[w] = *reinterpret_cast<const uint64_t *>(new_mask + ec);
+        v_cur0[w] = *reinterpret_cast<const uint64_t *>(cur_mask2 + ec);
+        v_cur1[w] = *reinterpret_cast<const uint64_t *>(cur_mask2 + (size_t)I + ec);
+    }
+    int4 v_i0[NV], v_i1[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        const int p = 4 * (tid + TPB * q), pc = p < idx_cap ? p : 0;   // (idx_cap: a multiple of 8, or I)
+        v_i0[q] = *reinterpret_cast<const int4 *>(indices2 + pc);
+        v_i1[q] = *reinterpret_cast<const int4 *>(indices2 + (size_t)I + pc);
+    }
+    const int n_buf0 = state[ST_STATE_N_BUF0], n_buf1 = state[ST_STATE_N_BUF1];
+    if (tid == 0) shared_changed = 0;
+    const int ep = (int)((tword >> 16) & 1u);
+    const int n = ep ? n_buf1 : n_buf0;
+
+    // ---- diff: removed bits and their prefix counts per eight indices, added indices ascending
+    uint64_t w_new[NW], w_cur[NW];
+    uint32_t cnt = 0;   // added in the low half, removed in the high half
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const bool in = w < words && 8 * (tid * words + w) < I;
+        w_new[w] = in ? nonzero_bytes(v_new[w]) : 0ull;
+        w_cur[w] = in ? nonzero_bytes(ep ? v_cur1[w] : v_cur0[w]) : 0ull;
+        cnt += (uint32_t)__popcll(w_new[w] & ~w_cur[w]) + ((uint32_t)__popcll(w_cur[w] & ~w_new[w]) << 16);
+    }
+    ST_TL(1);
+    const int lane = tid & (kWave - 1), wave = tid >> 6;
+    const uint32_t incl = wave_incl_scan_dpp(cnt, lane);
+    if (lane == kWave - 1) wave_tot[wave] = incl;
+    sync();
+    uint32_t prefix = incl - cnt, total = 0;
+#pragma unroll
+    for (int w = 0; w < TPB / kWave; ++w) {
+        const uint32_t t = wave_tot[w];
+        if (w < wave) prefix += t;
+        total += t;
+    }
+    ST_TL(2);
+    const int na = (int)(total & 0xffffu), nr = (int)(total >> 16);
+    uint32_t arrival = 0;
+    int next_epoch = ep ^ 1;
+    if (na == 0 && nr == 0) {   // unchanged mask: nothing is touched (weight_cache.h:237-240)
+        if (tid == 0 && writer) {
+            state[ST_STATE_N_CHANGED] = 0;
+            state[ST_STATE_N_ADDED] = 0;
+            state[ST_STATE_N_REMOVED] = 0;
+        }
+        next_epoch = ep;
+        if (tid == 0) arrival = atomicAdd(reinterpret_cast<uint32_t *>(&state[ST_STATE_TICKET]), 1u);
+    } else {
+        const int pairs = na < nr ? na : nr, S_all = nr - pairs;
+        {
+            int oa = (int)(prefix & 0xffffu), orr = (int)(prefix >> 16);
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const int g = tid * words + w;
+                if (w < words && 8 * g < I) {
+                    uint64_t a = w_new[w] & ~w_cur[w];   // one 0x01 byte per element, ascending
+                    const uint64_t r = w_cur[w] & ~w_new[w];
+                    rem_before[g] = (uint16_t)orr;
+                    rem_bits[g] = (uint8_t)pack_bits8(r);
+                    orr += __popcll(r);
+                    while (a) {
+                        item_idx[oa++] = (uint16_t)(8 * g + ((__ffsll((long long)a) - 1) >> 3));
+                        a &= a - 1;
+                    }
+                }
+            }
+        }
+        // (removed indices that are not in the list -- only after an update that failed -- leave these untouched)
+        for (int i = tid; i < pairs; i += TPB) item_pos[i] = kNone;
+        for (int i = tid; i < S_all; i += TPB) place[i] = kNone;
+        for (int i = pairs + tid; i < na; i += TPB) {   // phase 2
+            const int p = n + (i - pairs);
+            item_pos[i] = p < I ? (uint16_t)p : kNone;
+        }
+        sync();
+        ST_TL(3);
+        // ---- the list: what every position holds after the paired replacements, in registers (kOut: a surplus index)
+        constexpr int kOut = 0xffff;
+        int32_t *const idx_out = indices2 + (size_t)(ep ^ 1) * I;
+        int held[NV][4];
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+            const int p0 = 4 * (tid + TPB * q);
+            int4 c = ep ? v_i1[q] : v_i0[q];
+            if (n > idx_cap && p0 >= idx_cap && p0 < n)   // more positions in use than the caller expected (one more round trip)
+                c = *reinterpret_cast<const int4 *>(indices2 + (size_t)ep * I + p0);
+            const int e4[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int p = p0 + k, e = p < n ? e4[k] & 0xffff : 0;
+                const uint32_t bits = rem_bits[e >> 3];
+                int h = e;
+                if (p < n && ((bits >> (e & 7)) & 1u)) {
+                    const int rank = (int)rem_before[e >> 3] + __popc(bits & ((1u << (e & 7)) - 1u));
+                    if (rank < na) {
+                        h = item_idx[rank];
+                        item_pos[rank] = (uint16_t)p;
+                    } else {
+                        h = kOut;
+                        place[rank - na] = (uint16_t)p;
+                    }
+                }
+                held[q][k] = h;
+            }
+        }
+        int n_new = n + (na - pairs) < I ? n + (na - pairs) : I, items = na;
+        if (S_all > 0) {
+            sync();
+            n_new = surplus_places<TPB>([&](int k) __attribute__((always_inline)) -> uint16_t & { return place[k]; }, S_all, n, wave_tot,
+                                        &shared_n, tid, sync);
+            // the entries of the tail, last first, behind the added indices: items like the others once their places are known
+#pragma unroll
+            for (int q = 0; q < NV; ++q)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int p = 4 * (tid + TPB * q) + k;
+                    if (p >= n_new && p < n) item_idx[na + (n - 1 - p)] = (uint16_t)held[q][k];
+                }
+            sync();
+            const int S_ = n - n_new;
+            items = na + S_;
+            for (int j = tid; j < S_; j += TPB) {
+                int to = kNone;
+                if (item_idx[na + j] != kOut) {
+                    to = place[j];
+                    for (int hop = 0; hop <= S_ && to >= n_new; ++hop) to = place[n - 1 - to];
+                    if (writer) idx_out[to] = item_idx[na + j];
+                }
+                item_pos[na + j] = (uint16_t)to;
+            }
+        }
+        sync();
+        ST_TL(4);
+        // ---- publish: one block writes the other bookkeeping buffer, the last arrival flips the epoch
+        if (writer) {
+            uint8_t *mask_out = cur_mask2 + (size_t)(ep ^ 1) * I;
+            const int kept = n < n_new ? n : n_new;
+#pragma unroll
+            for (int q = 0; q < NV; ++q)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int p = 4 * (tid + TPB * q) + k;
+                    if (p < kept && held[q][k] != kOut) idx_out[p] = held[q][k];
+                }
+            for (int i = pairs + tid; i < na; i += TPB)
+                if (item_pos[i] < n_new) idx_out[item_pos[i]] = item_idx[i];
+            // the reference stores the new mask only when the rebuild did not throw (n_new > 0)
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const int e = 8 * (tid * words + w);
+                if (w < words && e < I) *reinterpret_cast<uint64_t *>(mask_out + e) = n_new > 0 ? w_new[w] : w_cur[w];
+            }
+            uint32_t mine = 0;
+            if (S_all > 0)
+                for (int i = tid; i < items; i += TPB) mine += item_pos[i] < n_new ? 1u : 0u;
+            if (mine) atomicAdd(&shared_changed, mine);
+            sync();
+            if (tid == 0) {
+                state[ST_STATE_N_BUF0 + (ep ^ 1)] = n_new;
+                state[ST_STATE_N_ACTIVE] = n_new;
+                state[ST_STATE_N_CHANGED] = S_all > 0 ? (int)shared_changed : na;
+                state[ST_STATE_N_ADDED] = na;
+                state[ST_STATE_N_REMOVED] = nr;
+                state[ST_STATE_SERIAL] += 1;
+                state[ST_STATE_EPOCH] = ep ^ 1;
+                if (n_new > 0) {
+                    state[ST_STATE_STATUS] = 0;
+                    state[ST_STATE_VALID] = 1;
+                } else {
+                    state[ST_STATE_STATUS] = ST_ERR_NO_ACTIVE;
+                }
+            }
+        }
+        if (tid == 0) arrival = atomicAdd(reinterpret_cast<uint32_t *>(&state[ST_STATE_TICKET]), 1u);
+        ST_TL(5);
+        if constexpr (Tab::kLayers) {
+            const UpdateLayer &ly = tab.l[blockIdx.y];
+            copy_items<TPB>(ly.pool, ly.active, cp.nmat, cp.row_bytes, tid, items, n_new, item_pos, item_idx);
+        } else {
+            copy_items<TPB>(cp.pool, cp.active, cp.nmat, cp.row_bytes, tid, items, n_new, item_pos, item_idx);
+        }
+    }
+    // the block that arrived last resets the arrivals and sets the epoch (the atomic's result is first looked at here)
+    if (tid == 0) {
+        asm volatile("" : "+v"(arrival));
+        if ((arrival & 0xffffu) == gridDim.x - 1)
+            atomicExch(reinterpret_cast<uint32_t *>(&state[ST_STATE_TICKET]), (uint32_t)next_epoch << 16);
+    }
+    ST_TL(6);
+}
+
+// The same for masks that cannot be read in 8-byte words: cache_plan above, then the copies.
+template <int TPB>
+__global__ __launch_bounds__(TPB) void cache_update_bytes_kernel(const uint8_t *__restrict__ new_mask,
+                                                                 uint8_t *__restrict__ cur_mask2,
+                                                                 int32_t *__restrict__ indices2,
+                                                                 int32_t *__restrict__ state, int I, CopyPlan cp)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ PlanShared ps;
     const int tid = threadIdx.x;
     PlanView pv;
-    cache_plan<VEC, TPB, false>(pv, smem, &ps, new_mask, cur_mask2, indices2, state, I, idx_cap, tid, [] {}, [] {});
-    if (!pv.changed) {
-        plan_finish(pv, state);
-        return;
+    cache_plan<false, TPB, 1, false>(pv, smem, &ps, new_mask, cur_mask2, indices2, state, I, I, tid, [] {}, [] {});
+    if (pv.changed) {
+        // (the index of a rewritten position, beside the position: the map of the plan is not needed any more)
+        for (int i = tid; i < (int)pv.n_changed; i += TPB) pv.pos_l[i] = pv.lists[i] != kNone ? pv.idx_l[pv.lists[i]] : 0;
+        lds_barrier();
+        copy_items<TPB>(cp.pool, cp.active, cp.nmat, cp.row_bytes, tid, (int)pv.n_changed, pv.n_new, pv.lists, pv.pos_l);
     }
-    const uint16_t *lists = pv.lists, *idx_l = pv.idx_l;
-    const uint32_t n_changed = pv.n_changed;
-    const bool writer = pv.writer;
-    // ---- copy this block's share of the changed rows: active[m][p] <- pool[m][index at p]
-    {
-        const int nmat = cp.nmat, row_bytes = cp.row_bytes, chunks = row_bytes >> 4;
-        const int GS = 1 << gs_log2, ngrp = TPB >> gs_log2;
-        const int grp = tid >> gs_log2, cc = tid & (GS - 1);
-        // the publishing block takes no copies when there are others to do them
-        const bool solo = gridDim.x == 1;
-        const bool copies = solo || !writer;
-        const int slots = (solo ? 1 : (int)gridDim.x - 1) * ngrp;
-        const int slot = (solo ? 0 : (int)blockIdx.x - 1) * ngrp + grp;   // >= 0 whenever `copies`
-        const int work = (int)n_changed * nmat;
-        for (int w0 = copies ? slot : work; w0 < work; w0 += slots * kCopyUnroll) {
-            for (int c = cc; c < chunks; c += GS) {
-                uint4 v[kCopyUnroll];
-                unsigned char *dst[kCopyUnroll];
-#pragma unroll
-                for (int u = 0; u < kCopyUnroll; ++u) {
-                    const int w = w0 + u * slots;
-                    dst[u] = nullptr;
-                    if (w < work) {
-                        const int j = w / nmat, m = w - j * nmat;
-                        const int p = lists[j];
-                        if (p == kNone) continue;  // a removed index that was not in the cache: nothing to copy
-                        const int idx = idx_l[p];
-                        const unsigned char *pool = m == 0 ? cp.pool[0] : (m == 1 ? cp.pool[1] : cp.pool[2]);
-                        unsigned char *act = m == 0 ? cp.active[0] : (m == 1 ? cp.active[1] : cp.active[2]);
-                        v[u] = ld16(pool + (size_t)idx * row_bytes + ((size_t)c << 4));
-                        dst[u] = act + (size_t)p * row_bytes + ((size_t)c << 4);
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < kCopyUnroll; ++u)
-                    if (dst[u]) st16(dst[u], v[u]);
-            }
-        }
-    }
-
     plan_finish(pv, state);
-    ST_TL(6);
 }
 
 // ---------------------------------------------------------------------------
@@ -614,12 +886,6 @@ struct SparseShared {
     int src[kSparseMaxQ];
     int found, paired_tail, replay_ok, fast_ok, nchg;   // surplus removals (removed > added)
 };
-
-// 0x01-per-element bytes -> 8 bits (element k -> bit k)
-__device__ __forceinline__ uint32_t pack_bits8(uint64_t ones)
-{
-    return (uint32_t)((ones * 0x0102040810204080ull) >> 56);
-}
 
 template <typename T, int RB, int TPB, int NB = 1, int NW = 1, int SPECN = RB / 2>
 __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
@@ -1194,7 +1460,7 @@ __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
     } else {
         // ---- too many surplus removals for the replay above: the per-index plan
         PlanView pv;
-        cache_plan<true, TPB, true>(pv, smem, &plan_shared, new_mask, cur_mask2, indices2, state, I, I, tid,
+        cache_plan<true, TPB, NW, true>(pv, smem, &plan_shared, new_mask, cur_mask2, indices2, state, I, I, tid,
                                            [] {}, [] {});
         n = pv.n_new;
         if (plan_wave) {
@@ -1691,6 +1957,109 @@ extern "C" int st_cache_load_weights(st_cache *c, const void *gate, const void *
     return ST_OK;
 }
 
+// The pointers of one cache and the mask of its update.
+static st::UpdateLayer update_layer(const st_cache *c, const uint8_t *mask)
+{
+    st::UpdateLayer y;
+    y.new_mask = mask;
+    y.cur_mask2 = c->b.cur_mask;
+    y.indices2 = c->b.indices;
+    y.state = c->b.state;
+    int m = 0;
+    if (c->has_gate) {
+        y.pool[m] = static_cast<const unsigned char *>(c->b.gate_pool);
+        y.active[m++] = static_cast<unsigned char *>(c->b.gate_active);
+    }
+    y.pool[m] = static_cast<const unsigned char *>(c->b.up_pool);
+    y.active[m++] = static_cast<unsigned char *>(c->b.up_active);
+    y.pool[m] = static_cast<const unsigned char *>(c->b.downT_pool);
+    y.active[m++] = static_cast<unsigned char *>(c->b.down_active);
+    for (; m < 3; ++m) { y.pool[m] = y.pool[0]; y.active[m] = y.active[0]; }
+    return y;
+}
+
+// Masks as 8-byte words, index lists as 16-byte vectors?
+static bool update_is_aligned(const st_cache *c, const uint8_t *mask)
+{
+    return c->I % 8 == 0 && (uintptr_t)mask % 8 == 0 && (uintptr_t)c->b.cur_mask % 8 == 0 && (uintptr_t)c->b.indices % 16 == 0;
+}
+
+// How much of the index list the plan fetches up front: a quarter more than the count the host saw last
+// (st_cache_sync_state), everything when it has seen none.
+static int update_idx_cap(const st_cache *c)
+{
+    const int I = (int)c->I, seen = c->host_state[ST_STATE_N_ACTIVE];
+    return seen > 0 && seen + seen / 4 + 64 < I ? (seen + seen / 4 + 64 + 7) & ~7 : I;
+}
+
+// One update, or those of L > 1 caches of equal shape in one launch (I <= kPlanMaxI; 8-byte masks only).
+static int launch_update(st_cache *const *caches, const uint8_t *const *masks, int L, hipStream_t s)
+{
+    using namespace st;
+    const st_cache *c = caches[0];
+    const int I = (int)c->I;
+    static const int blocks = [] {
+        const char *v = getenv("ST_CACHE_BLOCKS");
+        const int b = v ? atoi(v) : 0;
+        return b >= 1 && b <= 1024 ? b : 0;
+    }();
+    static const int want_tpb = [] {
+        const char *v = getenv("ST_CACHE_TPB");
+        return v ? atoi(v) : 0;
+    }();
+    const bool aligned = update_is_aligned(c, masks[0]);
+    // 512-thread blocks (ST_CACHE_TPB=512) leave room on the CU for a kernel of another stream, but
+    // measure slower on their own; they cover I <= 12288.
+    const bool small = L == 1 && want_tpb == 512 && aligned && I <= 8 * 512 * 3;
+    const int tpb = small ? 512 : kPlanThreads, words = (I + 8 * tpb - 1) / (8 * tpb);
+    const UpdateLayer y = update_layer(c, masks[0]);
+    CopyPlan cp;
+    for (int m = 0; m < 3; ++m) { cp.pool[m] = y.pool[m]; cp.active[m] = y.active[m]; }
+    cp.nmat = c->has_gate ? 3 : 2;
+    cp.row_bytes = (int)(c->H * c->esz);
+    ProfScope ps(ST_K_CACHE_UPDATE, s);
+    auto launch = [&](auto kern, int grid, size_t lds, auto... rest) -> int {
+        const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), 160 * 1024 - 256);
+        if (rc != ST_OK) return rc;
+        ST_LAUNCH(ps, kern, dim3(grid, L), dim3(tpb), lds, s, masks[0], c->b.cur_mask, c->b.indices, c->b.state, I,
+                  rest...);
+        return ST_OK;
+    };
+    int rc;
+    if (L > 1) {
+        UpdateLayers tab;
+        int idx_cap = 0;
+        for (int l = 0; l < kMaxLayers; ++l) {
+            const int k = l < L ? l : 0;
+            tab.l[l] = update_layer(caches[k], masks[k]);
+            const int cap = update_idx_cap(caches[k]);
+            idx_cap = cap > idx_cap ? cap : idx_cap;
+        }
+        // A block per CU: every one of them plans (4 us), then the copies run at the rate of the memory (28 caches at
+        // H 3072, I 8192, 290 changed rows each: 300 MB in 55 us; two blocks per CU measured the same there, and 9 us
+        // slower for two caches at I 14336)
+        const size_t lds = update_lds_bytes(I);
+        const int most = device_cu_count() * 3 / 4;
+        int grid = blocks ? blocks : device_cu_count() / L;
+        grid = grid < 4 ? 4 : grid > most ? most : grid;
+        rc = words == 1   ? launch(cache_update_kernel<1024, 1, UpdateLayers>, grid, lds, idx_cap, cp, tab)
+             : words == 2 ? launch(cache_update_kernel<1024, 2, UpdateLayers>, grid, lds, idx_cap, cp, tab)
+                          : launch(cache_update_kernel<1024, 3, UpdateLayers>, grid, lds, idx_cap, cp, tab);
+    } else {
+        const int grid = blocks ? blocks : device_cu_count() * 3 / 4;   // (measured against 1/4, 3/8, 1/2 and all of the CUs)
+        const size_t lds = update_lds_bytes(I);
+        const int idx_cap = update_idx_cap(c);
+        rc = !aligned     ? launch(cache_update_bytes_kernel<1024>, grid, plan_lds_bytes(I), cp)
+             : small      ? launch(cache_update_kernel<512, 3, NoLayers>, grid, lds, idx_cap, cp, NoLayers{})
+             : words == 1 ? launch(cache_update_kernel<1024, 1, NoLayers>, grid, lds, idx_cap, cp, NoLayers{})
+             : words == 2 ? launch(cache_update_kernel<1024, 2, NoLayers>, grid, lds, idx_cap, cp, NoLayers{})
+                          : launch(cache_update_kernel<1024, 3, NoLayers>, grid, lds, idx_cap, cp, NoLayers{});
+    }
+    if (rc != ST_OK) return rc;
+    ST_HIP(hipGetLastError());
+    return ST_OK;
+}
+
 extern "C" int st_cache_update_async(st_cache *c, const uint8_t *mask, void *stream)
 {
     using namespace st;
@@ -1722,59 +2091,37 @@ extern "C" int st_cache_update_async(st_cache *c, const uint8_t *mask, void *str
         ST_HIP(hipGetLastError());
         return ST_OK;
     }
-    const size_t lds = plan_lds_bytes(I);
-    CopyPlan cp;
-    cp.nmat = 0;
-    if (c->has_gate) {
-        cp.pool[cp.nmat] = static_cast<const unsigned char *>(c->b.gate_pool);
-        cp.active[cp.nmat++] = static_cast<unsigned char *>(c->b.gate_active);
+    return launch_update(&c, &mask, 1, s);
+}
+
+extern "C" int st_cache_update_layers(st_cache *const *caches, const uint8_t *const *masks, int64_t L, void *stream)
+{
+    using namespace st;
+    ST_REQUIRE(caches && masks && L >= 1, "st_cache_update_layers: null pointer or no layers");
+    for (int64_t l = 0; l < L; ++l) {
+        ST_REQUIRE(caches[l] && masks[l], "st_cache_update_layers: null pointer in layer %lld", (long long)l);
+        for (int64_t k = 0; k < l; ++k)
+            ST_REQUIRE(caches[k] != caches[l], "st_cache_update_layers: layers %lld and %lld are the same cache", (long long)k, (long long)l);
     }
-    cp.pool[cp.nmat] = static_cast<const unsigned char *>(c->b.up_pool);
-    cp.active[cp.nmat++] = static_cast<unsigned char *>(c->b.up_active);
-    cp.pool[cp.nmat] = static_cast<const unsigned char *>(c->b.downT_pool);
-    cp.active[cp.nmat++] = static_cast<unsigned char *>(c->b.down_active);
-    for (int k = cp.nmat; k < 3; ++k) { cp.pool[k] = cp.pool[0]; cp.active[k] = cp.active[0]; }
-    cp.row_bytes = (int)(c->H * c->esz);
-    const int chunks = cp.row_bytes >> 4;
-    static const int blocks = [] {
-        const char *v = getenv("ST_CACHE_BLOCKS");
-        const int b = v ? atoi(v) : 0;
-        return b >= 1 && b <= 1024 ? b : 0;
-    }();
-    static const int want_tpb = [] {
-        const char *v = getenv("ST_CACHE_TPB");
-        return v ? atoi(v) : 0;
-    }();
-    const int grid = blocks ? blocks : device_cu_count() * 3 / 4;   // (measured against 1/4, 3/8, 1/2 and all of the CUs)
-    const bool aligned = (I % 8 == 0) && ((uintptr_t)mask % 8 == 0) && ((uintptr_t)c->b.cur_mask % 8 == 0) &&
-                         ((uintptr_t)c->b.indices % 16 == 0);
-    // 512-thread blocks (ST_CACHE_TPB=512) leave room on the CU for a kernel of another stream, but
-    // measure slower on their own; they cover I <= 12288 in the vector path.
-    const bool small = want_tpb == 512 && aligned && I <= 8 * 512 * kPlanMaxWords;
-    const int tpb = small ? 512 : 1024;
-    const bool vec = aligned && I <= 8 * tpb * kPlanMaxWords;
-    int gs_log2 = 6;
-    while ((1 << gs_log2) < chunks && (1 << gs_log2) < tpb) ++gs_log2;
-    // how much of the index list the blocks fetch up front: a quarter more than the count the host saw
-    // last (st_cache_sync_state), everything when it has seen none
-    const int seen = c->host_state[ST_STATE_N_ACTIVE];
-    const int idx_cap = seen > 0 && seen + seen / 4 + 64 < I ? (seen + seen / 4 + 64 + 7) & ~7 : I;
-    {
-        ProfScope ps(ST_K_CACHE_UPDATE, s);
-        auto launch = [&](auto kern) -> int {
-            const int arc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), 160 * 1024 - 256);
-            if (arc != ST_OK) return arc;
-            ST_LAUNCH(ps, kern, dim3(grid), dim3(tpb), lds, s, mask, c->b.cur_mask, c->b.indices, c->b.state,
-                               I, gs_log2, idx_cap, cp);
-            return ST_OK;
-        };
-        int rc;
-        if (small) rc = launch(cache_update_kernel<true, 512>);
-        else if (vec) rc = launch(cache_update_kernel<true, 1024>);
-        else rc = launch(cache_update_kernel<false, 1024>);
+    for (int64_t l0 = 0; l0 < L;) {
+        // as many neighbours of one shape as a launch takes
+        const st_cache *c = caches[l0];
+        int nl = 1;
+        while (nl < kMaxLayers && l0 + nl < L && caches[l0 + nl]->I == c->I && caches[l0 + nl]->H == c->H &&
+               caches[l0 + nl]->dtype == c->dtype && caches[l0 + nl]->has_gate == c->has_gate)
+            ++nl;
+        bool aligned = c->I <= kPlanMaxI;
+        for (int l = 0; l < nl; ++l) aligned = aligned && update_is_aligned(caches[l0 + l], masks[l0 + l]);
+        if (nl == 1 || !aligned) {
+            const int rc = st_cache_update_async(caches[l0], masks[l0], stream);
+            if (rc != ST_OK) return rc;
+            l0 += 1;
+            continue;
+        }
+        const int rc = launch_update(caches + l0, masks + l0, nl, static_cast<hipStream_t>(stream));
         if (rc != ST_OK) return rc;
+        l0 += nl;
     }
-    ST_HIP(hipGetLastError());
     return ST_OK;
 }
 

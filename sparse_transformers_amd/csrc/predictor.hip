@@ -18,11 +18,17 @@ constexpr int kPredDownUnroll = 2;  // chunks per thread issued together
 // One block per rank row k: all loads of the row (and of x) are issued before
 // any arithmetic, so the kernel costs one memory round trip.
 // BT = rows of x per pass (1 for single-row decode, so that nothing is requested twice).
-template <typename T, int BT>
+// (tab: several layers of equal shape at once, grid dimension y; x [layers,B,H], t [layers,B,r])
+template <typename T, int BT, typename Tab>
 __global__ __launch_bounds__(kPredDownThreads) void predictor_down_kernel(const T *__restrict__ x, int B, int H,
                                                                           const T *__restrict__ A, int r,
-                                                                          float *__restrict__ t, int round_storage)
+                                                                          float *__restrict__ t, int round_storage, Tab tab)
 {
+    if constexpr (Tab::kLayers) {
+        A = static_cast<const T *>(tab.l[blockIdx.y].A);
+        x += (size_t)blockIdx.y * B * H;
+        t += (size_t)blockIdx.y * B * r;
+    }
     constexpr int VEC = Elem<T>::kVec;
     __shared__ float red[kPredDownThreads / kWave][BT];
     const int k = blockIdx.x, tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
@@ -91,13 +97,21 @@ constexpr int kPredUpBTile = 8;
 // LPR lanes share one row of Bm (LPR >= r/VEC unless the row needs several
 // passes); a wave owns RPW consecutive rows and issues the loads of all of them
 // before the rank-r intermediate is staged in LDS.
-template <typename T, int LPR, int RPW>
+template <typename T, int LPR, int RPW, typename Tab>
 __global__ __launch_bounds__(kPredUpThreads) void predictor_up_mask_kernel(const float *__restrict__ t,
                                                                   const T *__restrict__ Bm,
                                                                   float *__restrict__ scores,
                                                                   uint8_t *__restrict__ mask, int B, int r, int I,
-                                                                  float thr, int flags)
+                                                                  float thr, int flags, Tab tab)
 {
+    if constexpr (Tab::kLayers) {
+        const st_predictor_layer &ly = tab.l[blockIdx.y];
+        Bm = static_cast<const T *>(ly.Bm);
+        mask = ly.mask;
+        thr = ly.thr;
+        flags = (flags & ~1) | (ly.cmp_ge ? 1 : 0);
+        t += (size_t)blockIdx.y * B * r;
+    }
     // (13 dwords of arguments, all of them in scalar registers when the wave starts; the three switches share one)
     const int cmp_ge = flags & 1, round_storage = (flags >> 1) & 1, accumulate = (flags >> 2) & 1;
     constexpr int VEC = Elem<T>::kVec;
@@ -197,13 +211,21 @@ __global__ __launch_bounds__(kPredUpThreads) void predictor_up_mask_kernel(const
 // once per (row of Bm, row of x) -- the first form of the kernel was bound by exactly those reads (32-byte
 // strides, half the banks idle) and took 1.3 us per additional row of x at r = 256.  All NITER row loads of a
 // wave are issued before anything else.
-template <typename T, int LPR, int NITER>
+template <typename T, int LPR, int NITER, typename Tab>
 __global__ __launch_bounds__(kPredUpThreads) void predictor_up_mask_rows_kernel(const float *__restrict__ t,
                                                                        const T *__restrict__ Bm,
                                                                        float *__restrict__ scores,
                                                                        uint8_t *__restrict__ mask, int B, int r, int I,
-                                                                       float thr, int flags)
+                                                                       float thr, int flags, Tab tab)
 {
+    if constexpr (Tab::kLayers) {
+        const st_predictor_layer &ly = tab.l[blockIdx.y];
+        Bm = static_cast<const T *>(ly.Bm);
+        mask = ly.mask;
+        thr = ly.thr;
+        flags = (flags & ~1) | (ly.cmp_ge ? 1 : 0);
+        t += (size_t)blockIdx.y * B * r;
+    }
     const int cmp_ge = flags & 1, round_storage = (flags >> 1) & 1, accumulate = (flags >> 2) & 1;   // (as above)
     constexpr int VEC = Elem<T>::kVec;
     constexpr int RPI = kWave / LPR;   // rows per iteration
@@ -277,65 +299,84 @@ __global__ __launch_bounds__(kPredUpThreads) void predictor_up_mask_rows_kernel(
     }
 }
 
-template <typename T, int LPR, int RPW>
-static void launch_up_rpw(ProfScope &ps, const float *t_ws, int B, int r, const void *Bm, int I, float thr, int cmp_ge,
-                          float *scores, uint8_t *mask, int round_storage, int accumulate, hipStream_t stream)
+// What the two kernels of one call (one layer, or several of equal shape) are launched with.
+struct PredLaunch {
+    const void *x; int B, H; const void *A; int r; const void *Bm; int I;
+    float thr; int flags;   // bit 0: >=, bit 1: round to storage, bit 2: later pass
+    float *t_ws, *scores; uint8_t *mask;
+    int layers; hipStream_t stream;
+};
+
+template <typename T, int LPR, typename Tab>
+static void launch_up(ProfScope &ps, const PredLaunch &a, const Tab &tab)
 {
     constexpr size_t batch = (size_t)kPredUpThreads * 2 * 16;   // the staging buffer is padded to whole batches
-    const size_t lds = ((size_t)B * r * sizeof(float) + batch - 1) / batch * batch;
-    constexpr int rows = RPW * (kPredUpThreads / kWave);
-    ST_LAUNCH(ps, (predictor_up_mask_kernel<T, LPR, RPW>), dim3((I + rows - 1) / rows), dim3(kPredUpThreads), lds,
-              stream, t_ws, static_cast<const T *>(Bm), scores, mask, B, r, I, thr,
-              (cmp_ge ? 1 : 0) | (round_storage ? 2 : 0) | (accumulate ? 4 : 0));
-}
-
-template <typename T, int LPR>
-static void launch_up(ProfScope &ps, const float *t_ws, int B, int r, const void *Bm, int I, float thr, int cmp_ge,
-                      float *scores, uint8_t *mask, int round_storage, int accumulate, hipStream_t stream)
-{
+    const size_t lds = ((size_t)a.B * a.r * sizeof(float) + batch - 1) / batch * batch;
+    auto go = [&](auto kern, int rows) {
+        ST_LAUNCH(ps, kern, dim3((a.I + rows - 1) / rows, a.layers), dim3(kPredUpThreads), lds, a.stream, a.t_ws,
+                  static_cast<const T *>(a.Bm), a.scores, a.mask, a.B, a.r, a.I, a.thr, a.flags, tab);
+    };
     constexpr int NITER = LPR >= 16 ? LPR / 16 : 1;   // about four rows of Bm per wave (measured against 1, 2 and 8 per lane)
-    if (B > 1 && r / Elem<T>::kVec <= LPR) {
-        constexpr size_t batch = (size_t)kPredUpThreads * 2 * 16;
-        const size_t lds = ((size_t)B * r * sizeof(float) + batch - 1) / batch * batch;
-        constexpr int rows = (kWave / LPR) * NITER * (kPredUpThreads / kWave);
-        ST_LAUNCH(ps, (predictor_up_mask_rows_kernel<T, LPR, NITER>), dim3((I + rows - 1) / rows), dim3(kPredUpThreads),
-                  lds, stream, t_ws, static_cast<const T *>(Bm), scores, mask, B, r, I, thr,
-                  (cmp_ge ? 1 : 0) | (round_storage ? 2 : 0) | (accumulate ? 4 : 0));
-        return;
-    }
-    launch_up_rpw<T, LPR, pred_rows_per_wave(LPR)>(ps, t_ws, B, r, Bm, I, thr, cmp_ge, scores, mask, round_storage,
-                                                   accumulate, stream);
+    constexpr int RPW = pred_rows_per_wave(LPR);
+    if (a.B > 1 && a.r / Elem<T>::kVec <= LPR)
+        go(predictor_up_mask_rows_kernel<T, LPR, NITER, Tab>, (kWave / LPR) * NITER * (kPredUpThreads / kWave));
+    else
+        go(predictor_up_mask_kernel<T, LPR, RPW, Tab>, RPW * (kPredUpThreads / kWave));
 }
 
-template <typename T>
-static int launch_predictor(const void *x, int B, int H, const void *A, int r, const void *Bm, int I, float thr,
-                            int cmp_ge, float *t_ws, float *scores, uint8_t *mask, int round_storage, int accumulate,
-                            hipStream_t stream)
+template <typename T, typename Tab>
+static int launch_predictor(const PredLaunch &a, const Tab &tab)
 {
-    constexpr int VEC = Elem<T>::kVec;
     {
-        ProfScope ps(ST_K_PRED_DOWN, stream);
-        if (B == 1)
-            ST_LAUNCH(ps, (predictor_down_kernel<T, 1>), dim3(r), dim3(kPredDownThreads), 0, stream,
-                      static_cast<const T *>(x), B, H, static_cast<const T *>(A), r, t_ws, round_storage);
-        else if (B <= kPredBTile)
-            ST_LAUNCH(ps, (predictor_down_kernel<T, kPredBTile>), dim3(r), dim3(kPredDownThreads), 0, stream,
-                      static_cast<const T *>(x), B, H, static_cast<const T *>(A), r, t_ws, round_storage);
-        else   // 9 to 16 rows of x in one pass (one memory round trip instead of two)
-            ST_LAUNCH(ps, (predictor_down_kernel<T, 2 * kPredBTile>), dim3(r), dim3(kPredDownThreads), 0, stream,
-                      static_cast<const T *>(x), B, H, static_cast<const T *>(A), r, t_ws, round_storage);
+        ProfScope ps(ST_K_PRED_DOWN, a.stream);
+        auto go = [&](auto kern) {
+            ST_LAUNCH(ps, kern, dim3(a.r, a.layers), dim3(kPredDownThreads), 0, a.stream, static_cast<const T *>(a.x), a.B,
+                      a.H, static_cast<const T *>(a.A), a.r, a.t_ws, (a.flags >> 1) & 1, tab);
+        };
+        if (a.B == 1) go(predictor_down_kernel<T, 1, Tab>);
+        else if (a.B <= kPredBTile) go(predictor_down_kernel<T, kPredBTile, Tab>);
+        else go(predictor_down_kernel<T, 2 * kPredBTile, Tab>);   // 9 to 16 rows of x in one pass (one memory round trip instead of two)
     }
     ST_HIP(hipGetLastError());
-    const int chunks = r / VEC;
+    const int chunks = a.r / Elem<T>::kVec;
     {
-        ProfScope ps(ST_K_PRED_UP_MASK, stream);
-        if (chunks <= 4) launch_up<T, 4>(ps, t_ws, B, r, Bm, I, thr, cmp_ge, scores, mask, round_storage, accumulate, stream);
-        else if (chunks <= 8) launch_up<T, 8>(ps, t_ws, B, r, Bm, I, thr, cmp_ge, scores, mask, round_storage, accumulate, stream);
-        else if (chunks <= 16) launch_up<T, 16>(ps, t_ws, B, r, Bm, I, thr, cmp_ge, scores, mask, round_storage, accumulate, stream);
-        else if (chunks <= 32) launch_up<T, 32>(ps, t_ws, B, r, Bm, I, thr, cmp_ge, scores, mask, round_storage, accumulate, stream);
-        else launch_up<T, 64>(ps, t_ws, B, r, Bm, I, thr, cmp_ge, scores, mask, round_storage, accumulate, stream);
+        ProfScope ps(ST_K_PRED_UP_MASK, a.stream);
+        if (chunks <= 4) launch_up<T, 4>(ps, a, tab);
+        else if (chunks <= 8) launch_up<T, 8>(ps, a, tab);
+        else if (chunks <= 16) launch_up<T, 16>(ps, a, tab);
+        else if (chunks <= 32) launch_up<T, 32>(ps, a, tab);
+        else launch_up<T, 64>(ps, a, tab);
     }
     ST_HIP(hipGetLastError());
+    return ST_OK;
+}
+
+template <typename Tab> static int launch_predictor_dtype(int dtype, const PredLaunch &a, const Tab &tab)
+{
+    switch (dtype) {
+    case ST_F32: return launch_predictor<float>(a, tab);
+    case ST_F16: return launch_predictor<f16_t>(a, tab);
+    default: return launch_predictor<bf16_t>(a, tab);
+    }
+}
+
+// Rows of x per pass of these kernels: what the staging buffer of the second one holds, 64 at most.
+static int64_t pred_rows_per_pass(int64_t r)
+{
+    const int64_t per = (56 * 1024) / (r * 4);
+    return per > 64 ? 64 : per;
+}
+
+static int check_predictor_args(const char *who, int64_t B, int64_t H, int64_t r, int64_t I, int dtype, int flags)
+{
+    ST_REQUIRE(dtype >= ST_F32 && dtype <= ST_BF16, "%s: unknown dtype %d", who, dtype);
+    const int esz = dtype == ST_F32 ? 4 : 2;
+    ST_REQUIRE(B >= 1 && B <= (1 << 20), "%s: B=%lld out of range", who, (long long)B);
+    ST_REQUIRE(H >= 1 && (H * esz) % 16 == 0, "%s: H=%lld rows are not 16-byte multiples", who, (long long)H);
+    ST_REQUIRE(r >= 1 && (r * esz) % 16 == 0, "%s: rank %lld rows are not 16-byte multiples", who, (long long)r);
+    ST_REQUIRE(I >= 1 && I <= (1 << 24), "%s: I=%lld out of range", who, (long long)I);
+    ST_REQUIRE(r * 4 <= 56 * 1024, "%s: rank %lld too large for the LDS staging buffer", who, (long long)r);
+    ST_REQUIRE((flags & ~ST_PRED_ROUND_STORAGE) == 0, "%s: unknown flags %d", who, flags);
     return ST_OK;
 }
 
@@ -347,37 +388,75 @@ extern "C" int st_predictor_mask_ex(const void *x, int64_t B, int64_t H, const v
 {
     using namespace st;
     ST_REQUIRE(x && A && Bm && t_ws && mask, "st_predictor_mask_ex: null pointer");
-    ST_REQUIRE(dtype >= ST_F32 && dtype <= ST_BF16, "st_predictor_mask_ex: unknown dtype %d", dtype);
+    const int arc = check_predictor_args("st_predictor_mask_ex", B, H, r, I, dtype, flags);
+    if (arc != ST_OK) return arc;
     const int esz = dtype == ST_F32 ? 4 : 2;
-    ST_REQUIRE(B >= 1 && B <= (1 << 20), "st_predictor_mask_ex: B=%lld out of range", (long long)B);
-    ST_REQUIRE(H >= 1 && (H * esz) % 16 == 0, "st_predictor_mask_ex: H=%lld rows are not 16-byte multiples",
-               (long long)H);
-    ST_REQUIRE(r >= 1 && (r * esz) % 16 == 0, "st_predictor_mask_ex: rank %lld rows are not 16-byte multiples",
-               (long long)r);
-    ST_REQUIRE(I >= 1 && I <= (1 << 24), "st_predictor_mask_ex: I=%lld out of range", (long long)I);
-    ST_REQUIRE(r * 4 <= 56 * 1024, "st_predictor_mask_ex: rank %lld too large for the LDS staging buffer", (long long)r);
     const uintptr_t align = (uintptr_t)x | (uintptr_t)A | (uintptr_t)Bm;
     ST_REQUIRE((align & 15) == 0, "st_predictor_mask_ex: pointers must be 16-byte aligned");
-    ST_REQUIRE((flags & ~ST_PRED_ROUND_STORAGE) == 0, "st_predictor_mask_ex: unknown flags %d", flags);
     const int round_storage = (flags & ST_PRED_ROUND_STORAGE) && dtype != ST_F32 ? 1 : 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (predictor_mfma_supported(dtype, (int)B, (int)r))
         return launch_predictor_mfma(dtype, x, (int)B, (int)H, A, (int)r, Bm, (int)I, thr, cmp_ge, t_ws, scores, mask,
                                      round_storage, s);
-    // Rows of x per pass: what the staging buffer of the second kernel holds, 64 at most.  Further passes reuse
-    // the front of t_ws (the launches are ordered on the stream) and only ever switch mask bytes on.
-    int64_t per = (56 * 1024) / (r * 4);
-    per = per > 64 ? 64 : per;
+    // Further passes reuse the front of t_ws (the launches are ordered on the stream) and only ever switch mask bytes on.
+    const int64_t per = pred_rows_per_pass(r);
     for (int64_t b0 = 0; b0 < B; b0 += per) {
-        const int bc = (int)(B - b0 < per ? B - b0 : per);
-        const void *xp = static_cast<const unsigned char *>(x) + (size_t)b0 * H * esz;
-        float *sp = scores ? scores + (size_t)b0 * I : nullptr;
-        const int acc = b0 > 0 ? 1 : 0;
+        PredLaunch a;
+        a.x = static_cast<const unsigned char *>(x) + (size_t)b0 * H * esz;
+        a.B = (int)(B - b0 < per ? B - b0 : per);
+        a.H = (int)H; a.A = A; a.r = (int)r; a.Bm = Bm; a.I = (int)I;
+        a.thr = thr;
+        a.flags = (cmp_ge ? 1 : 0) | (round_storage ? 2 : 0) | (b0 > 0 ? 4 : 0);
+        a.t_ws = t_ws;
+        a.scores = scores ? scores + (size_t)b0 * I : nullptr;
+        a.mask = mask; a.layers = 1; a.stream = s;
+        const int rc = launch_predictor_dtype(dtype, a, NoLayers{});
+        if (rc != ST_OK) return rc;
+    }
+    return ST_OK;
+}
+
+extern "C" int st_predictor_mask_layers(const st_predictor_layer *layers, int64_t L, const void *x, int64_t B, int64_t H,
+                                        int64_t r, int64_t I, int dtype, int flags, float *t_ws, void *stream)
+{
+    using namespace st;
+    ST_REQUIRE(layers && x && t_ws && L >= 1, "st_predictor_mask_layers: null pointer or no layers");
+    const int arc = check_predictor_args("st_predictor_mask_layers", B, H, r, I, dtype, flags);
+    if (arc != ST_OK) return arc;
+    const int esz = dtype == ST_F32 ? 4 : 2;
+    uintptr_t align = (uintptr_t)x | (uintptr_t)((size_t)B * H * esz) | (uintptr_t)t_ws;
+    for (int64_t l = 0; l < L; ++l) {
+        ST_REQUIRE(layers[l].A && layers[l].Bm && layers[l].mask, "st_predictor_mask_layers: null pointer in layer %lld", (long long)l);
+        align |= (uintptr_t)layers[l].A | (uintptr_t)layers[l].Bm;
+    }
+    ST_REQUIRE((align & 15) == 0, "st_predictor_mask_layers: pointers must be 16-byte aligned");
+    const int round_storage = (flags & ST_PRED_ROUND_STORAGE) && dtype != ST_F32 ? 1 : 0;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const bool mfma = predictor_mfma_supported(dtype, (int)B, (int)r);
+    if (!mfma && B > pred_rows_per_pass(r)) {   // several passes per layer: one layer at a time
+        for (int64_t l = 0; l < L; ++l) {
+            const st_predictor_layer &y = layers[l];
+            const int rc = st_predictor_mask_ex(static_cast<const unsigned char *>(x) + (size_t)l * B * H * esz, B, H, y.A, r,
+                                                y.Bm, I, dtype, y.thr, y.cmp_ge, flags, t_ws, nullptr, y.mask, stream);
+            if (rc != ST_OK) return rc;
+        }
+        return ST_OK;
+    }
+    for (int64_t l0 = 0; l0 < L; l0 += kMaxLayers) {
+        PredLayers tab;
+        const int nl = (int)(L - l0 < kMaxLayers ? L - l0 : kMaxLayers);
+        for (int l = 0; l < kMaxLayers; ++l) tab.l[l] = layers[l0 + (l < nl ? l : 0)];
+        const void *xl = static_cast<const unsigned char *>(x) + (size_t)l0 * B * H * esz;
+        float *tl = t_ws + (size_t)l0 * B * r;
         int rc;
-        switch (dtype) {
-        case ST_F32: rc = launch_predictor<float>(xp, bc, (int)H, A, (int)r, Bm, (int)I, thr, cmp_ge, t_ws, sp, mask, round_storage, acc, s); break;
-        case ST_F16: rc = launch_predictor<f16_t>(xp, bc, (int)H, A, (int)r, Bm, (int)I, thr, cmp_ge, t_ws, sp, mask, round_storage, acc, s); break;
-        default: rc = launch_predictor<bf16_t>(xp, bc, (int)H, A, (int)r, Bm, (int)I, thr, cmp_ge, t_ws, sp, mask, round_storage, acc, s); break;
+        if (mfma) {
+            rc = launch_predictor_mfma_layers(dtype, tab, nl, xl, (int)B, (int)H, (int)r, (int)I, tl, round_storage, s);
+        } else {
+            PredLaunch a;
+            a.x = xl; a.B = (int)B; a.H = (int)H; a.A = nullptr; a.r = (int)r; a.Bm = nullptr; a.I = (int)I;
+            a.thr = 0.f; a.flags = round_storage ? 2 : 0;
+            a.t_ws = tl; a.scores = nullptr; a.mask = nullptr; a.layers = nl; a.stream = s;
+            rc = launch_predictor_dtype(dtype, a, tab);
         }
         if (rc != ST_OK) return rc;
     }

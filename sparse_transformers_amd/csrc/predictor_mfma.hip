@@ -29,12 +29,18 @@ template <> struct SplitParts<bf16_t> { static constexpr int value = 3; };
 // LDS rows are 16 chunks of 16 bytes, chunk c of row k at c ^ (k % 16).
 constexpr int kPmPiece = 128;
 
-template <typename T, int MI, int NI, int W>
+template <typename T, int MI, int NI, int W, typename Tab>
 __global__ __launch_bounds__(W * kWave) void predictor_down_mfma_kernel(const T *__restrict__ x, const T *__restrict__ A,
                                                                         int B, int H, int r, int nt,
                                                                         float *__restrict__ t, uint8_t *__restrict__ mask,
-                                                                        int I, int round_storage)
+                                                                        int I, int round_storage, Tab tab)
 {
+    if constexpr (Tab::kLayers) {   // several layers of equal shape at once: x [layers,B,H], t [layers,B,r]
+        A = static_cast<const T *>(tab.l[blockIdx.y].A);
+        mask = tab.l[blockIdx.y].mask;
+        x += (size_t)blockIdx.y * B * H;
+        t += (size_t)blockIdx.y * B * r;
+    }
     constexpr int kThreads = W * kWave;
     constexpr int kRows = 16 * (MI + NI), kBuf = kRows * 16, kDma = kRows / 4;   // a wave's buffer in chunks, its 1 KB loads
     extern __shared__ __align__(16) uint4 lds[];   // [W][2][kRows][16]
@@ -171,13 +177,21 @@ template <> __device__ __forceinline__ void split_parts<f16_t>(const float *v, u
 // collected in LDS too: a store to memory inside the loop would have to be waited for together with the next stage.
 constexpr int kPmStage = 64;
 
-template <typename T, int KS, int MI, int W, bool ALL>
+template <typename T, int KS, int MI, int W, bool ALL, typename Tab>
 __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const float *__restrict__ t,
                                                                       const T *__restrict__ Bm, int B, int r, int I,
                                                                       int splits, int wb_rt, int per, float thr, int flags,
                                                                       float *__restrict__ scores,
-                                                                      uint8_t *__restrict__ mask)
+                                                                      uint8_t *__restrict__ mask, Tab tab)
 {
+    if constexpr (Tab::kLayers) {
+        const st_predictor_layer &ly = tab.l[blockIdx.y];
+        Bm = static_cast<const T *>(ly.Bm);
+        mask = ly.mask;
+        thr = ly.thr;
+        flags = (flags & ~1) | (ly.cmp_ge ? 1 : 0);
+        t += (size_t)blockIdx.y * B * r;
+    }
     constexpr int P = SplitParts<T>::value;
     constexpr int kRow = 4 * KS, kBuf = kPmStage * kRow;      // 16-byte chunks
     constexpr int kDma = kBuf / 64 / W;                       // 1 KB loads per wave and stage
@@ -329,11 +343,12 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
 // 10.6 / 10.6, 14.3 / 11.0, 25.0 / 12.1, 68.9 / 13.2, 538 / 29, 2236 / 78.  Ranks above 512 do not fit the registers.
 bool predictor_mfma_supported(int dtype, int B, int r) { return dtype != ST_F32 && B > 8 && r <= 512; }
 
-template <typename T>
-static int launch_t(const void *x, int B, int H, const void *A, int r, const void *Bm, int I, float thr, int cmp_ge,
-                    float *t_ws, float *scores, uint8_t *mask, int round_storage, hipStream_t stream)
+template <typename T, typename Tab>
+static int launch_t(const Tab &tab, int layers, const void *x, int B, int H, const void *A, int r, const void *Bm, int I,
+                    float thr, int cmp_ge, float *t_ws, float *scores, uint8_t *mask, int round_storage, hipStream_t stream)
 {
-    const int cus = device_cu_count();
+    // (the CUs a layer can count on when several share the launch)
+    const int cus = (device_cu_count() + layers - 1) / layers;
     {
         ProfScope ps(ST_K_PRED_DOWN, stream);
         auto go = [&](auto kern, int mi, int ni, int waves) -> int {
@@ -341,15 +356,16 @@ static int launch_t(const void *x, int B, int H, const void *A, int r, const voi
             const int lds = waves * 2 * 16 * (mi + ni) * 256;
             const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
             if (rc != ST_OK) return rc;
-            ST_LAUNCH(ps, kern, dim3(mt * nt), dim3(waves * kWave), lds, stream, static_cast<const T *>(x),
-                      static_cast<const T *>(A), B, H, r, nt, t_ws, mask, I, round_storage);
+            ST_LAUNCH(ps, kern, dim3(mt * nt, layers), dim3(waves * kWave), lds, stream, static_cast<const T *>(x),
+                      static_cast<const T *>(A), B, H, r, nt, t_ws, mask, I, round_storage, tab);
             return ST_OK;
         };
         auto blocks = [&](int mi, int ni) { return ((B + 16 * mi - 1) / (16 * mi)) * ((r + 16 * ni - 1) / (16 * ni)); };
         // 32 x 32 tiles (half the traffic from L2) once they make a block for three quarters of the CUs: 6.7 (16 x 16) against
         // 8.6 us with 64 of them (512 rows, H 3072, rank 128), 17.8 against 11.8 us with 224, 40 against 26 us with 512
-        const int rc = 4 * blocks(2, 2) < 3 * cus ? go(predictor_down_mfma_kernel<T, 1, 1, 8>, 1, 1, 8)
-                                                  : go(predictor_down_mfma_kernel<T, 2, 2, 4>, 2, 2, 4);
+        // (by the shape alone: how many layers share the launch must not change how the sums are split)
+        const int rc = 4 * blocks(2, 2) < 3 * device_cu_count() ? go(predictor_down_mfma_kernel<T, 1, 1, 8, Tab>, 1, 1, 8)
+                                                  : go(predictor_down_mfma_kernel<T, 2, 2, 4, Tab>, 2, 2, 4);
         if (rc != ST_OK) return rc;
     }
     ST_HIP(hipGetLastError());
@@ -371,13 +387,13 @@ static int launch_t(const void *x, int B, int H, const void *A, int r, const voi
             auto launch = [&](auto k) -> int {
                 const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(k), 2 * kPmStage * 4 * ks * 16 + 256 * kPmStage);
                 if (rc != ST_OK) return rc;
-                ST_LAUNCH(ps, k, dim3(mt * splits), dim3(waves * kWave), lds, stream, t_ws, static_cast<const T *>(Bm), B, r,
-                          I, splits, wb, per, thr, (cmp_ge ? 1 : 0) | (round_storage ? 2 : 0), scores, mask);
+                ST_LAUNCH(ps, k, dim3(mt * splits, layers), dim3(waves * kWave), lds, stream, t_ws, static_cast<const T *>(Bm), B, r,
+                          I, splits, wb, per, thr, (cmp_ge ? 1 : 0) | (round_storage ? 2 : 0), scores, mask, tab);
                 return ST_OK;
             };
             return wb == waves ? launch(kern_all) : launch(kern);
         };
-#define ST_PM_UP(KS, MI, W, RES) go(predictor_up_mfma_kernel<T, KS, MI, W, true>, predictor_up_mfma_kernel<T, KS, MI, W, false>, KS, MI, W, RES)
+#define ST_PM_UP(KS, MI, W, RES) go(predictor_up_mfma_kernel<T, KS, MI, W, true, Tab>, predictor_up_mfma_kernel<T, KS, MI, W, false, Tab>, KS, MI, W, RES)
         int rc;
         // (eight waves share a stage once there are rows of x for them: 16 rows in blocks of eight waves 5.2 us, of four 4.4)
         if (B <= 64) {
@@ -399,9 +415,15 @@ static int launch_t(const void *x, int B, int H, const void *A, int r, const voi
 int launch_predictor_mfma(int dtype, const void *x, int B, int H, const void *A, int r, const void *Bm, int I, float thr,
                           int cmp_ge, float *t_ws, float *scores, uint8_t *mask, int round_storage, hipStream_t stream)
 {
-    if (dtype == ST_F16)
-        return launch_t<f16_t>(x, B, H, A, r, Bm, I, thr, cmp_ge, t_ws, scores, mask, round_storage, stream);
-    return launch_t<bf16_t>(x, B, H, A, r, Bm, I, thr, cmp_ge, t_ws, scores, mask, round_storage, stream);
+    auto go = dtype == ST_F16 ? launch_t<f16_t, NoLayers> : launch_t<bf16_t, NoLayers>;
+    return go(NoLayers{}, 1, x, B, H, A, r, Bm, I, thr, cmp_ge, t_ws, scores, mask, round_storage, stream);
+}
+
+int launch_predictor_mfma_layers(int dtype, const PredLayers &tab, int layers, const void *x, int B, int H, int r, int I,
+                                 float *t_ws, int round_storage, hipStream_t stream)
+{
+    auto go = dtype == ST_F16 ? launch_t<f16_t, PredLayers> : launch_t<bf16_t, PredLayers>;
+    return go(tab, layers, x, B, H, nullptr, r, nullptr, I, 0.f, 0, t_ws, nullptr, nullptr, round_storage, stream);
 }
 
 }  // namespace st

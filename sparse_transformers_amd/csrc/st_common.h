@@ -270,10 +270,21 @@ int launch_batch(int dtype, const void *x, int B, int H, const void *gate, const
                  const int *n_dev, void *out, void *comb, long ldc, void *workspace, int act, int has_gate,
                  hipStream_t stream);
 
+// Several layers of equal shape in one launch: grid dimension y is the layer, whose pointers come from a table passed by
+// value (as the last argument; NoLayers takes its place in the single-layer kernels).
+constexpr int kMaxLayers = 32;   // of one launch: the largest table (80 bytes a layer) fits the 4 KB of kernel arguments
+struct NoLayers { static constexpr bool kLayers = false; };
+struct PredLayers {
+    static constexpr bool kLayers = true;
+    st_predictor_layer l[kMaxLayers];
+};
+
 // Predictor on the matrix cores for several rows of x (fp16 / bf16, rank up to 512).
 bool predictor_mfma_supported(int dtype, int B, int r);
 int launch_predictor_mfma(int dtype, const void *x, int B, int H, const void *A, int r, const void *Bm, int I, float thr,
                           int cmp_ge, float *t_ws, float *scores, uint8_t *mask, int round_storage, hipStream_t stream);
+int launch_predictor_mfma_layers(int dtype, const PredLayers &tab, int layers, const void *x, int B, int H, int r, int I,
+                                 float *t_ws, int round_storage, hipStream_t stream);
 
 // Double precision forward (plain kernels, for checking a model in fp64).
 int64_t f64_workspace_bytes(int64_t B, int64_t H, int64_t n);

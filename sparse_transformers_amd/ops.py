@@ -297,6 +297,30 @@ def predictor_scores(x: torch.Tensor, down_weight: torch.Tensor, up_weight: torc
                           round_to_storage=round_to_storage)[1]
 
 
+def predictor_mask_layers(x: torch.Tensor, layers, t_ws: torch.Tensor, round_to_storage: bool = False) -> None:
+    """``predictor_mask`` for the layers of a stack at once (two launches for up to 32 of them).
+
+    x: contiguous [L, B, H]; ``layers``: L tuples (down_weight [r,H], up_weight [I,r], mask bool[I], thr, ge) of equal
+    shapes in x's dtype, the masks different tensors; t_ws: float32, at least L*B*r elements."""
+    L, B, H = x.shape
+    r, I = layers[0][0].size(0), layers[0][1].size(0)
+    dev = require_gpu(x, t_ws)
+    if len(layers) != L or not x.is_contiguous() or t_ws.dtype != torch.float32 or t_ws.numel() < L * B * r:
+        raise ValueError("predictor_mask_layers: x must be contiguous [L,B,H] with one entry of `layers` per layer and "
+                         "t_ws a float32 tensor of L*B*r elements")
+    tab = (_lib.PredictorLayer * L)()
+    for i, (down, up, mask, thr, ge) in enumerate(layers):
+        if tuple(down.shape) != (r, H) or tuple(up.shape) != (I, r) or down.dtype != x.dtype or up.dtype != x.dtype or \
+                not down.is_contiguous() or not up.is_contiguous() or down.device != dev or up.device != dev:
+            raise ValueError(f"predictor_mask_layers: layer {i} differs in shape, dtype or device")
+        if mask.dtype != torch.bool or mask.numel() != I or not mask.is_contiguous() or mask.device != dev:
+            raise ValueError("masks must be contiguous bool[I] tensors on x's GPU")
+        tab[i] = _lib.PredictorLayer(down.data_ptr(), up.data_ptr(), mask.data_ptr(), float(thr), int(ge))
+    rc = _lib.lib().st_predictor_mask_layers(tab, L, x.data_ptr(), B, H, r, I, dtype_code(x), 1 if round_to_storage else 0,
+                                             t_ws.data_ptr(), current_stream_ptr(dev))
+    _lib.check(rc, "st_predictor_mask_layers")
+
+
 MASK_METHODS = {"topk": 0, "statistical_topk": 1}
 _select_workspaces: dict = {}
 

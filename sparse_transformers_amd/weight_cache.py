@@ -69,6 +69,23 @@ class ConcatWeightHandle(torch.Tensor):
         return func(*tree_map(real, args), **tree_map(real, kwargs or {}))
 
 
+def update_layers_async(caches, masks) -> None:
+    """``update_active_weights_async`` for the caches of several layers at once, one mask each: caches of equal shape share
+    their launches.  The caches must be different objects on one GPU."""
+    L = len(caches)
+    hs, ms, keep = (C.c_void_p * L)(), (C.c_void_p * L)(), []
+    for i, (c, mask) in enumerate(zip(caches, masks)):
+        m = c._mask_arg(mask)
+        keep.append(m)
+        c._flush_pending()
+        c._keep_snapshot()
+        hs[i], ms[i] = c._h, m.data_ptr()
+    rc = _lib.lib().st_cache_update_layers(hs, ms, L, current_stream_ptr(caches[0].device))
+    _lib.check(rc, "st_cache_update_layers")
+    for c in caches:
+        c._dirty = True
+
+
 class WeightCache:
     """Drop-in for the reference WeightCache, plus a zero-copy fast path.
 

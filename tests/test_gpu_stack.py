@@ -97,6 +97,42 @@ def test_graph_replay_equals_eager(overlap):
         _ = (xs[t].float() @ xs[t].float().t()).sum().item()   # unrelated eager work + a host sync between replays
 
 
+@pytest.mark.parametrize("dtype,L,H,I,r,B,trace_masks", [
+    ("float16", 3, 256, 640, 16, 1, False),      # as few layers as share launches
+    ("bfloat16", 35, 64, 120, 8, 1, True),       # more layers than one launch's table holds
+    ("float16", 4, 128, 1001, 24, 2, True),      # masks that are not 8-byte words
+    ("bfloat16", 4, 256, 9000, 72, 5, False),    # two mask words per thread of the update
+    ("bfloat16", 3, 256, 640, 40, 12, True),     # predictors on the matrix cores
+    ("float32", 3, 128, 320, 16, 70, False),     # more rows than one pass of the predictor takes
+])
+def test_staged_step_shares_launches_between_layers(dtype, L, H, I, r, B, trace_masks):
+    """A staged step runs all layers' predictors, then all their updates, as shared launches: masks, index order and output
+    are those of the layer-by-layer step, bit for bit, eagerly and replayed."""
+    a, _ = _build(dtype, L, H, I, r, B, seed=L)
+    b, _ = _build(dtype, L, H, I, r, B, seed=L)
+    trace = torch.from_numpy(syn.mask_trace(3, L, I, I // 3, 8, 0.05, 0.3, 0.3)).to(DEV)
+    tdt = getattr(torch, dtype)
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    for s in (a, b):
+        s.prepare(B, fused=s is a)
+        s.use_trace_masks = trace_masks
+        for l, layer in enumerate(s.layers):
+            layer.thr, layer.ge = 0.02 * (l % 3 - 1), l % 2 == 0
+    assert a._batched()
+    for t in range(6):
+        x, xp = torch.randn(B, H, device=DEV, generator=gen).to(tdt), torch.randn(L, B, H, device=DEV, generator=gen).to(tdt)
+        if t == 2:
+            torch.cuda.synchronize()
+            a.capture()
+        ya = a.step_staged(x, xp, trace[t], replay=t >= 2).clone()
+        yb = b.step_staged(x, xp, trace[t]).clone()
+        for la, lb in zip(a.layers, b.layers):
+            assert torch.equal(la.mask, lb.mask), t
+            lb.cache._dirty = la.cache._dirty = True
+            assert torch.equal(la.cache.get_active_indices(), lb.cache.get_active_indices()), t
+        assert torch.equal(ya, yb), t
+
+
 def test_skip_mlp_module_surface():
     """SkipMLP mirrors the reference module (src/modeling_skip.py:55-128): constructor arguments, sub-modules,
     registered buffers, state-dict keys, initialize_weight_cache / reset_cache, the three forwards."""
