@@ -6,8 +6,8 @@
  * passed as void* (NULL = the default stream).  All entry points return
  * ST_OK (0) or a negative st_status; st_last_error() gives a message for the
  * calling thread.  No entry point except st_cache_create/st_cache_destroy
- * (host memory only) and st_cache_sync_state (one small device-to-host copy)
- * allocates or synchronises: work is enqueued on `stream` and ordered with
+ * (host memory only), st_cache_sync_state (one small device-to-host copy) and
+ * st_cache_update_sync allocates or synchronises: work is enqueued on `stream` and ordered with
  * whatever else the caller enqueues there.
  *
  * Each entry point names the interface of NimbleEdge/sparse_transformers it
@@ -249,6 +249,15 @@ int st_cache_update_async(st_cache *c, const uint8_t *mask, void *stream);
  * must be different ones. */
 int st_cache_update_layers(st_cache *const *caches, const uint8_t *const *masks, int64_t L, void *stream);
 
+/* st_cache_update_async, then the state words of that update on the host: state_out (host int32[ST_STATE_WORDS], may be
+ * NULL) and the return value are those of st_cache_sync_state behind it, but the call only waits until the update's plan
+ * stands, not for its row copies (which later calls on `stream` follow anyway). */
+int st_cache_update_sync(st_cache *c, const uint8_t *mask, int32_t *state_out, void *stream);
+
+/* host; where updates leave the active count by themselves (pinned memory, 0 before the first one; the GPU may write it at
+ * any time until st_cache_destroy).  A guess for n_hint, never more. */
+const volatile int32_t *st_cache_seen_count(const st_cache *c);
+
 /* Copies the state words to the host (waits for `stream`).  Returns
  * ST_ERR_NO_ACTIVE if the last update emptied the cache, else ST_OK.
  * state_out: host int32[ST_STATE_WORDS], may be NULL. */
@@ -266,7 +275,8 @@ int st_cache_sync_state(st_cache *c, int32_t *state_out, void *stream);
  * ends in the same state and `out` holds the same bits as the two separate
  * calls.  x, out: [B,H] in the cache's dtype; combined: [B,ldc] or NULL;
  * workspace: st_mlp_workspace_bytes(B, H, I) bytes.  n_hint: the active count
- * the host last saw (0 = unknown); it picks the kernel variant, which rows are
+ * the host last saw (0 = unknown, negative = what the last update told the
+ * host, st_cache_seen_count); it picks the kernel variant, which rows are
  * requested before the plan is known and how much of the index list is
  * fetched up front, and never affects results.  An update that empties
  * the cache leaves status ST_ERR_NO_ACTIVE in the state words (reported by

@@ -60,6 +60,8 @@ SIGNATURES = {
     "st_cache_load_weights": (_ci, [_vp, _vp, _vp, _vp, _vp]),
     "st_cache_update_async": (_ci, [_vp, _vp, _vp]),
     "st_cache_update_layers": (_ci, [C.POINTER(_vp), C.POINTER(_vp), _i64, _vp]),
+    "st_cache_update_sync": (_ci, [_vp, _vp, _vp, _vp]),
+    "st_cache_seen_count": (_vp, [_vp]),
     "st_cache_update_forward": (_ci, [_vp, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _i64, _ci, _vp]),
     "st_cache_sync_state": (_ci, [_vp, _vp, _vp]),
     "st_cache_materialize_concat": (_ci, [_vp, _vp, _i64, _vp]),

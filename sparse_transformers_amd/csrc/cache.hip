@@ -24,8 +24,10 @@
 #include "st_common.h"
 
 #include <atomic>
+#include <chrono>
 
 #include <cstdlib>
+#include <cstring>
 #include <new>
 #include <type_traits>
 
@@ -525,6 +527,26 @@ __device__ __forceinline__ void plan_finish(const PlanView &pv, int32_t *__restr
 // ---------------------------------------------------------------------------
 // update kernel
 // ---------------------------------------------------------------------------
+// What an update tells the host on its own (pinned memory, written across the bus by the publishing block long before its
+// kernel ends): the count, as a guess for later launches, and for a caller that waits the state words, each beside the
+// number of the update so that the host sees without ordered stores when all of them are its own.
+struct HostWords {
+    int32_t count;
+    int32_t pad[15];
+    uint64_t state[8];   // (update number << 32) | value, in the order of kHostStateWords
+};
+constexpr int kHostStateWords[8] = {ST_STATE_N_ACTIVE, ST_STATE_N_CHANGED, ST_STATE_STATUS, ST_STATE_VALID,
+                                    ST_STATE_N_ADDED, ST_STATE_N_REMOVED, ST_STATE_SERIAL, ST_STATE_EPOCH};
+
+__device__ __forceinline__ void tell_count(HostWords *hw, int n)
+{
+    __hip_atomic_store(&hw->count, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void tell_state(HostWords *hw, uint32_t number, int k, int value)
+{
+    __hip_atomic_store(&hw->state[k], ((uint64_t)number << 32) | (uint32_t)value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The caches of one launch: several layers of equal shape (grid dimension y) or one.
 struct UpdateLayer {
     const uint8_t *new_mask;
@@ -532,6 +554,7 @@ struct UpdateLayer {
     int32_t *indices2, *state;
     const unsigned char *pool[3];
     unsigned char *active[3];
+    HostWords *host;
 };
 struct UpdateLayers {
     static constexpr bool kLayers = true;
@@ -600,10 +623,12 @@ template <int TPB, int NW, typename Tab>
 __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__restrict__ new_mask,
                                                            uint8_t *__restrict__ cur_mask2,
                                                            int32_t *__restrict__ indices2, int32_t *__restrict__ state,
-                                                           int I, int idx_cap, CopyPlan cp, Tab tab)
+                                                           int I, int idx_cap, CopyPlan cp, HostWords *host,
+                                                           uint32_t number, Tab tab)
 {
     if constexpr (Tab::kLayers) {
         const UpdateLayer &ly = tab.l[blockIdx.y];
+        host = ly.host;
         new_mask = ly.new_mask;
         cur_mask2 = ly.cur_mask2;
         indices2 = ly.indices2;
@@ -647,6 +672,7 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
         v_i1[q] = *reinterpret_cast<const int4 *>(indices2 + (size_t)I + pc);
     }
     const int n_buf0 = state[ST_STATE_N_BUF0], n_buf1 = state[ST_STATE_N_BUF1];
+    const int serial_old = state[ST_STATE_SERIAL], status_old = state[ST_STATE_STATUS], valid_old = state[ST_STATE_VALID];
     if (tid == 0) shared_changed = 0;
     const int ep = (int)((tword >> 16) & 1u);
     const int n = ep ? n_buf1 : n_buf0;
@@ -677,13 +703,23 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
     const int na = (int)(total & 0xffffu), nr = (int)(total >> 16);
     uint32_t arrival = 0;
     int next_epoch = ep ^ 1;
+    // the state words after the update, from one thread of the publishing block
+    auto tell_host = [&](int n_now, int n_changed, int status, int valid, int serial) __attribute__((always_inline)) {
+        tell_count(host, n_now);
+        if (number != 0) {
+            const int v[8] = {n_now, n_changed, status, valid, na, nr, serial, next_epoch};
+#pragma unroll
+            for (int k = 0; k < 8; ++k) tell_state(host, number, k, v[k]);
+        }
+    };
     if (na == 0 && nr == 0) {   // unchanged mask: nothing is touched (weight_cache.h:237-240)
+        next_epoch = ep;
         if (tid == 0 && writer) {
             state[ST_STATE_N_CHANGED] = 0;
             state[ST_STATE_N_ADDED] = 0;
             state[ST_STATE_N_REMOVED] = 0;
+            tell_host(n, 0, status_old, valid_old, serial_old);
         }
-        next_epoch = ep;
         if (tid == 0) arrival = atomicAdd(reinterpret_cast<uint32_t *>(&state[ST_STATE_TICKET]), 1u);
     } else {
         const int pairs = na < nr ? na : nr, S_all = nr - pairs;
@@ -798,17 +834,16 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
             if (tid == 0) {
                 state[ST_STATE_N_BUF0 + (ep ^ 1)] = n_new;
                 state[ST_STATE_N_ACTIVE] = n_new;
-                state[ST_STATE_N_CHANGED] = S_all > 0 ? (int)shared_changed : na;
+                const int n_changed = S_all > 0 ? (int)shared_changed : na;
+                const int status = n_new > 0 ? 0 : ST_ERR_NO_ACTIVE, valid = n_new > 0 ? 1 : valid_old;
+                state[ST_STATE_N_CHANGED] = n_changed;
                 state[ST_STATE_N_ADDED] = na;
                 state[ST_STATE_N_REMOVED] = nr;
-                state[ST_STATE_SERIAL] += 1;
+                state[ST_STATE_SERIAL] = serial_old + 1;
                 state[ST_STATE_EPOCH] = ep ^ 1;
-                if (n_new > 0) {
-                    state[ST_STATE_STATUS] = 0;
-                    state[ST_STATE_VALID] = 1;
-                } else {
-                    state[ST_STATE_STATUS] = ST_ERR_NO_ACTIVE;
-                }
+                state[ST_STATE_STATUS] = status;
+                state[ST_STATE_VALID] = valid;
+                tell_host(n_new, n_changed, status, valid, serial_old + 1);
             }
         }
         if (tid == 0) arrival = atomicAdd(reinterpret_cast<uint32_t *>(&state[ST_STATE_TICKET]), 1u);
@@ -891,7 +926,7 @@ template <typename T, int RB, int TPB, int NB = 1, int NW = 1, int SPECN = RB / 
 __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
     const uint8_t *__restrict__ new_mask, uint8_t *__restrict__ cur_mask2, int32_t *__restrict__ indices2,
     int32_t *__restrict__ state, int I, int launch_word, const T *__restrict__ x, int H, int n_hint,
-    T *__restrict__ combined, long ldc, float *__restrict__ partials, int act, int plan_bytes, FusedRows fr)
+    T *__restrict__ combined, long ldc, float *__restrict__ partials, int act, int plan_bytes, HostWords *host, FusedRows fr)
 {
     constexpr int VEC = Elem<T>::kVec;
     // Slots of the first batch that are requested ahead of the plan, on the caller's guess of the count and from the
@@ -1476,6 +1511,7 @@ __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
         speculate(std::integral_constant<int, 0>{}, std::integral_constant<int, SPEC>{});
         lds_barrier();
     }
+    if (blk == 0 && tid == 0) tell_count(host, n);
     ST_TL(4);
 
     float acc[NB][VEC];
@@ -1891,7 +1927,9 @@ struct st_cache {
     int64_t I, H;
     int dtype, has_gate;
     int esz;
-    int32_t *host_state;  // pinned
+    int32_t *host_state;   // pinned: ST_STATE_WORDS words as st_cache_sync_state last read them
+    st::HostWords *host;   // pinned, behind them: what updates write by themselves
+    uint32_t number;       // of the last update that a caller waited for
 };
 
 extern "C" int64_t st_cache_max_intermediate(void) { return st::kBigMaxI; }
@@ -1918,12 +1956,15 @@ extern "C" st_cache *st_cache_create(const st_cache_buffers *bufs, int64_t I, in
     c->b = *bufs;
     c->I = I; c->H = H; c->dtype = dtype; c->has_gate = has_gate ? 1 : 0; c->esz = esz;
     c->host_state = nullptr;
-    if (hipHostMalloc(reinterpret_cast<void **>(&c->host_state), ST_STATE_WORDS * sizeof(int32_t), hipHostMallocDefault) !=
-        hipSuccess) {
+    static_assert(ST_STATE_WORDS * sizeof(int32_t) == 64, "the host words keep a cache line of their own");
+    const size_t host_bytes = 64 + sizeof(HostWords);
+    if (hipHostMalloc(reinterpret_cast<void **>(&c->host_state), host_bytes, hipHostMallocDefault) != hipSuccess) {
         delete c;
         return fail("hipHostMalloc failed");
     }
-    for (int i = 0; i < ST_STATE_WORDS; ++i) c->host_state[i] = 0;
+    memset(c->host_state, 0, host_bytes);
+    c->host = reinterpret_cast<HostWords *>(reinterpret_cast<unsigned char *>(c->host_state) + 64);
+    c->number = 0;
     return c;
 }
 
@@ -1975,6 +2016,7 @@ static st::UpdateLayer update_layer(const st_cache *c, const uint8_t *mask)
     y.pool[m] = static_cast<const unsigned char *>(c->b.downT_pool);
     y.active[m++] = static_cast<unsigned char *>(c->b.down_active);
     for (; m < 3; ++m) { y.pool[m] = y.pool[0]; y.active[m] = y.active[0]; }
+    y.host = c->host;
     return y;
 }
 
@@ -1984,16 +2026,20 @@ static bool update_is_aligned(const st_cache *c, const uint8_t *mask)
     return c->I % 8 == 0 && (uintptr_t)mask % 8 == 0 && (uintptr_t)c->b.cur_mask % 8 == 0 && (uintptr_t)c->b.indices % 16 == 0;
 }
 
-// How much of the index list the plan fetches up front: a quarter more than the count the host saw last
-// (st_cache_sync_state), everything when it has seen none.
+// The count an update last told the host, 0 if none has yet.  A guess: later updates may be on their way.
+static int seen_count(const st_cache *c) { return *const_cast<const volatile int32_t *>(&c->host->count); }
+
+// How much of the index list the plan fetches up front: a quarter more than the count the host saw last, everything when
+// it has seen none.
 static int update_idx_cap(const st_cache *c)
 {
-    const int I = (int)c->I, seen = c->host_state[ST_STATE_N_ACTIVE];
+    const int I = (int)c->I, seen = seen_count(c);
     return seen > 0 && seen + seen / 4 + 64 < I ? (seen + seen / 4 + 64 + 7) & ~7 : I;
 }
 
 // One update, or those of L > 1 caches of equal shape in one launch (I <= kPlanMaxI; 8-byte masks only).
-static int launch_update(st_cache *const *caches, const uint8_t *const *masks, int L, hipStream_t s)
+// number: nonzero if the caller waits for the state words (L == 1).
+static int launch_update(st_cache *const *caches, const uint8_t *const *masks, int L, uint32_t number, hipStream_t s)
 {
     using namespace st;
     const st_cache *c = caches[0];
@@ -2042,18 +2088,18 @@ static int launch_update(st_cache *const *caches, const uint8_t *const *masks, i
         const int most = device_cu_count() * 3 / 4;
         int grid = blocks ? blocks : device_cu_count() / L;
         grid = grid < 4 ? 4 : grid > most ? most : grid;
-        rc = words == 1   ? launch(cache_update_kernel<1024, 1, UpdateLayers>, grid, lds, idx_cap, cp, tab)
-             : words == 2 ? launch(cache_update_kernel<1024, 2, UpdateLayers>, grid, lds, idx_cap, cp, tab)
-                          : launch(cache_update_kernel<1024, 3, UpdateLayers>, grid, lds, idx_cap, cp, tab);
+        rc = words == 1   ? launch(cache_update_kernel<1024, 1, UpdateLayers>, grid, lds, idx_cap, cp, c->host, 0u, tab)
+             : words == 2 ? launch(cache_update_kernel<1024, 2, UpdateLayers>, grid, lds, idx_cap, cp, c->host, 0u, tab)
+                          : launch(cache_update_kernel<1024, 3, UpdateLayers>, grid, lds, idx_cap, cp, c->host, 0u, tab);
     } else {
         const int grid = blocks ? blocks : device_cu_count() * 3 / 4;   // (measured against 1/4, 3/8, 1/2 and all of the CUs)
         const size_t lds = update_lds_bytes(I);
         const int idx_cap = update_idx_cap(c);
         rc = !aligned     ? launch(cache_update_bytes_kernel<1024>, grid, plan_lds_bytes(I), cp)
-             : small      ? launch(cache_update_kernel<512, 3, NoLayers>, grid, lds, idx_cap, cp, NoLayers{})
-             : words == 1 ? launch(cache_update_kernel<1024, 1, NoLayers>, grid, lds, idx_cap, cp, NoLayers{})
-             : words == 2 ? launch(cache_update_kernel<1024, 2, NoLayers>, grid, lds, idx_cap, cp, NoLayers{})
-                          : launch(cache_update_kernel<1024, 3, NoLayers>, grid, lds, idx_cap, cp, NoLayers{});
+             : small      ? launch(cache_update_kernel<512, 3, NoLayers>, grid, lds, idx_cap, cp, c->host, number, NoLayers{})
+             : words == 1 ? launch(cache_update_kernel<1024, 1, NoLayers>, grid, lds, idx_cap, cp, c->host, number, NoLayers{})
+             : words == 2 ? launch(cache_update_kernel<1024, 2, NoLayers>, grid, lds, idx_cap, cp, c->host, number, NoLayers{})
+                          : launch(cache_update_kernel<1024, 3, NoLayers>, grid, lds, idx_cap, cp, c->host, number, NoLayers{});
     }
     if (rc != ST_OK) return rc;
     ST_HIP(hipGetLastError());
@@ -2091,7 +2137,7 @@ extern "C" int st_cache_update_async(st_cache *c, const uint8_t *mask, void *str
         ST_HIP(hipGetLastError());
         return ST_OK;
     }
-    return launch_update(&c, &mask, 1, s);
+    return launch_update(&c, &mask, 1, 0, s);
 }
 
 extern "C" int st_cache_update_layers(st_cache *const *caches, const uint8_t *const *masks, int64_t L, void *stream)
@@ -2118,7 +2164,7 @@ extern "C" int st_cache_update_layers(st_cache *const *caches, const uint8_t *co
             l0 += 1;
             continue;
         }
-        const int rc = launch_update(caches + l0, masks + l0, nl, static_cast<hipStream_t>(stream));
+        const int rc = launch_update(caches + l0, masks + l0, nl, 0, static_cast<hipStream_t>(stream));
         if (rc != ST_OK) return rc;
         l0 += nl;
     }
@@ -2160,6 +2206,7 @@ extern "C" int st_cache_update_forward(st_cache *c, const uint8_t *mask, const v
                        I <= 32 * kSparseMaxW32 && I <= 8 * TPB * kSparseWords && chunks <= TPB && row_bytes % 16 == 0 &&
                        lds <= (size_t)(148 * 1024);
     if (!fused) {   // two launches: update, then the forward that reads the count on the device
+        if (n_hint < 0) n_hint = seen_count(c);
         const int rc = st_cache_update_async(c, mask, stream);
         if (rc != ST_OK) return rc;
         return st_mlp_forward(x, B, c->H, c->b.gate_active, c->b.up_active, c->b.down_active, c->I,
@@ -2176,7 +2223,8 @@ extern "C" int st_cache_update_forward(st_cache *c, const uint8_t *mask, const v
     fr.row_bytes = row_bytes;
     fr.has_gate = c->has_gate ? 1 : 0;
     float *partials = static_cast<float *>(workspace);
-    const int hint = (int)(n_hint < 0 ? 0 : (n_hint > c->I ? c->I : n_hint));
+    if (n_hint < 0) n_hint = seen_count(c);
+    const int hint = (int)(n_hint > c->I ? c->I : n_hint);
     {
         ProfScope ps(ST_K_CACHE_UPDATE_DECODE, s);
         auto launch = [&](auto kern, auto *xt, auto *ct) -> int {
@@ -2185,7 +2233,7 @@ extern "C" int st_cache_update_forward(st_cache *c, const uint8_t *mask, const v
             // (blocks, log2 of the thread-group size, gated or not, rows of x: one argument, see the kernel)
             const int launch_word = G | (gs_log2 << 16) | (fr.has_gate << 20) | ((int)B << 24);
             ST_LAUNCH(ps, kern, dim3(G), dim3(TPB), lds, s, mask, c->b.cur_mask, c->b.indices, c->b.state, I,
-                      launch_word, xt, H, hint, ct, (long)ldc, partials, act, (int)plan_bytes, fr);
+                      launch_word, xt, H, hint, ct, (long)ldc, partials, act, (int)plan_bytes, c->host, fr);
             return ST_OK;
         };
         int rc;
@@ -2224,15 +2272,12 @@ extern "C" int st_cache_update_forward(st_cache *c, const uint8_t *mask, const v
     return launch_mlp_reduce(c->dtype, partials, G, NBF, (int)B, H, out, s);
 }
 
-extern "C" int st_cache_sync_state(st_cache *c, int32_t *state_out, void *stream)
+extern "C" const volatile int32_t *st_cache_seen_count(const st_cache *c) { return c ? &c->host->count : nullptr; }
+
+// The outcome of an update from the host's copy of the state words.
+static int update_outcome(const st_cache *c)
 {
     using namespace st;
-    ST_REQUIRE(c, "st_cache_sync_state: null handle");
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    ST_HIP(hipMemcpyAsync(c->host_state, c->b.state, ST_STATE_WORDS * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    ST_HIP(hipStreamSynchronize(s));
-    if (state_out)
-        for (int i = 0; i < ST_STATE_WORDS; ++i) state_out[i] = c->host_state[i];
     if (c->host_state[ST_STATE_FAULT] != 0) {
         set_error("st_cache: the fault word of the state is set; the cache contents are undefined");
         return ST_ERR_HIP;
@@ -2242,6 +2287,55 @@ extern "C" int st_cache_sync_state(st_cache *c, int32_t *state_out, void *stream
         return ST_ERR_NO_ACTIVE;
     }
     return ST_OK;
+}
+
+extern "C" int st_cache_update_sync(st_cache *c, const uint8_t *mask, int32_t *state_out, void *stream)
+{
+    using namespace st;
+    ST_REQUIRE(c && mask, "st_cache_update_sync: null pointer");
+    if (c->I <= kPlanMaxI && update_is_aligned(c, mask)) {
+        if (++c->number == 0) c->number = 1;
+        const int rc = launch_update(&c, &mask, 1, c->number, static_cast<hipStream_t>(stream));
+        if (rc != ST_OK) return rc;
+        // The kernel's publishing block writes the words across the bus as soon as its plan stands; a copy of the state
+        // behind the kernel and a wait for the stream takes 10 us longer.  Bounded: with other work ahead of it on the
+        // stream the wait is the stream's.
+        const volatile uint64_t *w = c->host->state;
+        const auto begun = std::chrono::steady_clock::now();
+        for (int spins = 0;; ++spins) {
+            bool all = true;
+            int32_t v[8];
+            for (int k = 0; k < 8; ++k) {
+                const uint64_t x = w[k];
+                all = all && (uint32_t)(x >> 32) == c->number;
+                v[k] = (int32_t)(uint32_t)x;
+            }
+            if (all) {
+                for (int k = 0; k < 8; ++k) c->host_state[kHostStateWords[k]] = v[k];
+                if (state_out)
+                    for (int k = 0; k < ST_STATE_WORDS; ++k) state_out[k] = c->host_state[k];
+                return update_outcome(c);
+            }
+            __builtin_ia32_pause();
+            if ((spins & 63) == 63 && std::chrono::steady_clock::now() - begun > std::chrono::milliseconds(1)) break;
+        }
+    } else {
+        const int rc = st_cache_update_async(c, mask, stream);
+        if (rc != ST_OK) return rc;
+    }
+    return st_cache_sync_state(c, state_out, stream);
+}
+
+extern "C" int st_cache_sync_state(st_cache *c, int32_t *state_out, void *stream)
+{
+    using namespace st;
+    ST_REQUIRE(c, "st_cache_sync_state: null handle");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    ST_HIP(hipMemcpyAsync(c->host_state, c->b.state, ST_STATE_WORDS * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    ST_HIP(hipStreamSynchronize(s));
+    if (state_out)
+        for (int i = 0; i < ST_STATE_WORDS; ++i) state_out[i] = c->host_state[i];
+    return update_outcome(c);
 }
 
 extern "C" int st_cache_materialize_concat(st_cache *c, void *dst, int64_t n, void *stream)

@@ -157,6 +157,7 @@ class WeightCache:
                                      down_c.data_ptr(), current_stream_ptr(dev))
         _lib.check(rc, "st_cache_load_weights")
         self._host_state = (C.c_int32 * _lib.STATE_WORDS)()
+        self._seen = C.c_int32.from_address(L.st_cache_seen_count(self._h))   # the count the last finished update told the host
         self._host_serial = -1      # serial the host copy of the state belongs to
         self._dirty = True          # updates enqueued since the last read-back
         self.lazy_updates = False
@@ -211,16 +212,19 @@ class WeightCache:
             return
         known = not self._dirty
         serial = int(self._host_state[_lib.STATE_SERIAL])
-        self.update_active_weights_async(mask)
-        try:
-            self.sync_state()
-        except RuntimeError as exc:
-            # The "emptied" status stays in the state words until an update changes something.  An update with an
-            # unchanged mask touches nothing and returns silently in the reference (weight_cache.h:237-240), also
-            # right after the update that emptied the cache: only an update that did something may raise.
-            if str(exc) == "No active weights" and known and int(self._host_state[_lib.STATE_SERIAL]) == serial:
-                return
-            raise
+        m = self._mask_arg(mask)
+        self._flush_pending()
+        self._keep_snapshot()
+        self._dirty = True
+        rc = _lib.lib().st_cache_update_sync(self._h, m.data_ptr(), self._host_state, current_stream_ptr(self.device))
+        if rc in (_lib.ST_OK, _lib.ST_ERR_NO_ACTIVE):
+            self._dirty = False
+        # The "emptied" status stays in the state words until an update changes something.  An update with an
+        # unchanged mask touches nothing and returns silently in the reference (weight_cache.h:237-240), also
+        # right after the update that emptied the cache: only an update that did something may raise.
+        if rc == _lib.ST_ERR_NO_ACTIVE and known and int(self._host_state[_lib.STATE_SERIAL]) == serial:
+            return
+        _lib.check(rc, "st_cache_update_sync")
 
     def sync_state(self) -> dict:
         """Read the state words back (waits for the current stream)."""
@@ -282,7 +286,7 @@ class WeightCache:
         touching the host.  For one row of x this is a single kernel that takes the rows whose index
         changed straight from the pool (and writes them back to the active buffers on the way); the
         cache state and the result equal those of the two separate calls bit for bit.  ``n_hint`` (default:
-        the last count the host saw) only steers what the kernel requests before it knows the true count.
+        the last count an update told the host) only steers what the kernel requests before it knows the true count.
         ``workspace``: a caller-owned uint8 buffer of ``mlp_workspace_bytes(B, H, I)`` bytes (default: one
         kept per device and stream)."""
         m = self._mask_arg(mask)
@@ -302,7 +306,7 @@ class WeightCache:
         self._keep_snapshot()
         rc = _lib.lib().st_cache_update_forward(
             self._h, m.data_ptr(), x2.data_ptr(), B,
-            int(self._host_state[_lib.STATE_N_ACTIVE]) if n_hint is None else int(n_hint), out.data_ptr(),
+            -1 if n_hint is None else int(n_hint), out.data_ptr(),
             combined.data_ptr() if combined is not None else None, combined.stride(0) if combined is not None else 0,
             ws.data_ptr(), ws.numel(), _lib.ACT_CODES[act], current_stream_ptr(self.device))
         _lib.check(rc, "st_cache_update_forward")
@@ -322,9 +326,9 @@ class WeightCache:
         x2 = self._x_rows(x)
         if out is None:
             out = torch.empty_like(x2)
-        # the last count the host saw is only a prefetch hint; the kernels read the true one on the device
+        # the last count an update told the host is only a prefetch hint; the kernels read the true one on the device
         # (mlp_forward_rows checks out / combined against the cache's dtype, device and capacity I)
         mlp_forward_rows(x2, self.gate_active, self.up_active, self.down_active, self.intermediate_size,
                          self.n_active_dev, out, combined, act, self.has_gate,
-                         n_hint=int(self._host_state[_lib.STATE_N_ACTIVE]), workspace=workspace)
+                         n_hint=self._seen.value, workspace=workspace)
         return out.view(x.shape)
