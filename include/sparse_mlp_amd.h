@@ -236,6 +236,12 @@ void st_cache_destroy(st_cache *c);
  * gate/up [I,H], down [H,I], dtype of the cache; gate may be NULL when ungated. */
 int st_cache_load_weights(st_cache *c, const void *gate, const void *up, const void *down, void *stream);
 
+/* The reference's constructor as a whole (weight_cache.h:199-226): st_cache_load_weights, then st_cache_update_sync with
+ * the initial mask, in one pass over the weights.  state_out (may be NULL), the wait and the return value are those of
+ * st_cache_update_sync. */
+int st_cache_load_weights_masked(st_cache *c, const void *gate, const void *up, const void *down, const uint8_t *mask,
+                                 int32_t *state_out, void *stream);
+
 /* update_active_weights(mask): weight_cache.h:229-359 (diff :84-110, pairing
  * :248-277, append :280-307, swap-with-last :310-353).  mask: uint8/bool [I]
  * on the device.  Enqueues one kernel (bookkeeping + row copies); returns

@@ -58,6 +58,7 @@ SIGNATURES = {
     "st_cache_create": (_vp, [C.POINTER(CacheBuffers), _i64, _i64, _ci, _ci]),
     "st_cache_destroy": (None, [_vp]),
     "st_cache_load_weights": (_ci, [_vp, _vp, _vp, _vp, _vp]),
+    "st_cache_load_weights_masked": (_ci, [_vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "st_cache_update_async": (_ci, [_vp, _vp, _vp]),
     "st_cache_update_layers": (_ci, [C.POINTER(_vp), C.POINTER(_vp), _i64, _vp]),
     "st_cache_update_sync": (_ci, [_vp, _vp, _vp, _vp]),

@@ -28,6 +28,7 @@
 
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <type_traits>
 
@@ -1892,32 +1893,272 @@ __global__ __launch_bounds__(kBigThreads) void cache_update_big_kernel(const uin
         atomicExch(reinterpret_cast<uint32_t *>(&state[ST_STATE_TICKET]), (uint32_t)(ep ^ 1) << 16);
 }
 
-// in [R,C] -> out [C,R], 64x64 tiles through LDS.
-template <typename E>
-__global__ __launch_bounds__(256) void transpose_kernel(const E *__restrict__ in, E *__restrict__ out, int R, int C)
+// ---------------------------------------------------------------------------
+// construction
+// ---------------------------------------------------------------------------
+// The module's matrices [gate,] up [I,H] and down [H,I], the pools and the packed buffers.
+struct BuildMats {
+    const unsigned char *src[2], *down;
+    unsigned char *pool[2], *active[2], *downT_pool, *down_active;
+    int nrow;          // matrices copied by row: 2 gated, 1 ungated
+    int row_bytes;
+    int down_vec;      // rows of `down` may be read in 16-byte vectors
+};
+
+// Elements e .. e + 7 of a mask as 0x01 bytes (0 past I and for a null mask).
+__device__ __forceinline__ uint64_t mask8(const uint8_t *__restrict__ mask, int e, int I, bool vec)
 {
-    __shared__ E tile[64][65];
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int c0 = blockIdx.x * 64, r0 = blockIdx.y * 64;
-    for (int k = ty; k < 64; k += 4) {
-        const int r = r0 + k, c = c0 + tx;
-        if (r < R && c < C) tile[k][tx] = in[(size_t)r * C + c];
+    if (mask == nullptr || e >= I) return 0ull;
+    if (vec && e + 8 <= I) return nonzero_bytes(*reinterpret_cast<const uint64_t *>(mask + e));
+    uint64_t v = 0;
+    for (int k = 0; k < 8; ++k)
+        if (e + k < I && mask[e + k]) v |= 1ull << (8 * k);
+    return v;
+}
+
+constexpr int kBuildThreads = 256, kBuildRows = kBuildThreads / kWave;   // a wave per row
+template <int ESZ> struct BuildTile { static constexpr int rows = 256 / ESZ; };   // of a transposed tile, both ways: 256 bytes
+
+// Everything a new cache holds, in one pass over the module's weights: pools, packed rows of the initial mask in ascending
+// order (what the first update of an empty cache gives, weight_cache.h:199-226) and the bookkeeping of that update; with a
+// null mask the pools and an empty cache.  Bound by memory: each weight is read once and written to the pool and the packed
+// buffer from registers.  Block 0 does the bookkeeping, the next copy a row of gate or up per wave, the last transpose
+// 256 x 256 byte tiles of `down`, 8 x 8 (4 x 4) elements per thread in registers, so that a wave's loads and stores are
+// 128-byte lines on both sides and nothing goes through LDS.  A row's position is the number of set mask bytes before it,
+// counted by every block while its rows are on the way.
+// H 3072, I 8192, fp16, all rows (453 MB): 160 us as two copies, a transposing kernel (44 us), a reset and an update
+// (69 us, reading the pools back), @@ us as one.
+template <int ESZ>
+__global__ __launch_bounds__(kBuildThreads) void cache_build_kernel(const uint8_t *__restrict__ mask,
+                                                                    uint8_t *__restrict__ cur_mask2,
+                                                                    int32_t *__restrict__ indices2,
+                                                                    int32_t *__restrict__ state, int I, int H, int mask_vec,
+                                                                    HostWords *host, int tell, uint32_t number, BuildMats a)
+{
+    constexpr int kTile = BuildTile<ESZ>::rows, V = 16 / ESZ;
+    __shared__ uint32_t wave_tot[kBuildThreads / kWave];
+    __shared__ int tile_pos[kTile];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto sync = [&]() __attribute__((always_inline)) { lds_barrier(); };
+    // set mask bytes before element e0 (a multiple of 4); ends behind a barrier
+    auto rank_of = [&](int e0) __attribute__((always_inline)) -> int {
+        uint32_t c = 0;
+#pragma unroll 4
+        for (int e = 8 * tid; e < e0; e += 8 * kBuildThreads) {
+            uint64_t m = mask8(mask, e, I, mask_vec);
+            if (e + 8 > e0) m &= 0xffffffffull;
+            c += (uint32_t)__popcll(m);
+        }
+        const uint32_t incl = wave_incl_scan_dpp(c, lane);
+        if (lane == kWave - 1) wave_tot[wave] = incl;
+        sync();
+        uint32_t t = 0;
+#pragma unroll
+        for (int w = 0; w < kBuildThreads / kWave; ++w) t += wave_tot[w];
+        return (int)t;
+    };
+    const int row_groups = (I + kBuildRows - 1) / kBuildRows;
+    int unit = (int)blockIdx.x - 1;
+    if (unit < 0) {   // ---- bookkeeping: every thread a contiguous range of the mask
+        const int words = (I + 8 * kBuildThreads - 1) / (8 * kBuildThreads);
+        uint32_t cnt = 0;
+        for (int w = 0; w < words; ++w) cnt += (uint32_t)__popcll(mask8(mask, 8 * (tid * words + w), I, mask_vec));
+        uint32_t total;
+        int at = (int)block_excl_scan<kBuildThreads / kWave>(cnt, wave_tot, &total, tid, sync);
+        const int n = (int)total;
+        if (tid == 0) {
+            // an empty initial mask equals the empty cache's: nothing changes and nothing is valid (weight_cache.h:237-240)
+            const int some = n > 0 ? 1 : 0;
+            int w[ST_STATE_WORDS] = {};
+            w[ST_STATE_N_ACTIVE] = w[ST_STATE_N_CHANGED] = w[ST_STATE_N_ADDED] = w[ST_STATE_N_BUF1] = n;
+            w[ST_STATE_VALID] = w[ST_STATE_SERIAL] = w[ST_STATE_EPOCH] = some;
+            w[ST_STATE_TICKET] = some << 16;
+            for (int k = 0; k < ST_STATE_WORDS; ++k) state[k] = w[k];
+            if (tell) tell_count(host, n);
+            if (number != 0) {
+                const int v[8] = {n, n, 0, some, n, 0, some, some};   // kHostStateWords
+                for (int k = 0; k < 8; ++k) tell_state(host, number, k, v[k]);
+            }
+        }
+        for (int w = 0; w < words; ++w) {
+            const int e0 = 8 * (tid * words + w);
+            const uint64_t m = mask8(mask, e0, I, mask_vec);
+            for (int k = 0; k < 8 && e0 + k < I; ++k) {
+                const int e = e0 + k;
+                const bool set = (m >> (8 * k)) & 1u;
+                cur_mask2[e] = 0;
+                cur_mask2[(size_t)I + e] = set ? 1 : 0;
+                indices2[e] = -1;
+                if (set) indices2[(size_t)I + at++] = e;
+                if (e >= n) indices2[(size_t)I + e] = -1;
+            }
+        }
+        return;
     }
-    __syncthreads();
-    for (int k = ty; k < 64; k += 4) {
-        const int c = c0 + k, r = r0 + tx;
-        if (r < R && c < C) out[(size_t)c * R + r] = tile[tx][k];
+    if (unit < a.nrow * row_groups) {   // ---- rows of gate and up
+        const int m = unit >= row_groups ? 1 : 0, r0 = (unit - m * row_groups) * kBuildRows, r = r0 + wave;
+        const bool in = r < I;
+        const unsigned char *const from = (m ? a.src[1] : a.src[0]) + (size_t)(in ? r : r0) * a.row_bytes;
+        unsigned char *const pool = (m ? a.pool[1] : a.pool[0]) + (size_t)r * a.row_bytes;
+        const int chunks = a.row_bytes >> 4;
+        constexpr int U = 8;
+        uint4 v[U];
+        auto load = [&](int c0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int c = c0 + u * kWave;
+                v[u] = ld16_stream(from + ((size_t)(c < chunks ? c : chunks - 1) << 4));
+            }
+        };
+        load(lane);
+        int pos = -1;
+        if (mask != nullptr) {
+            const int before = rank_of(r0);
+            int mine = 0;
+            for (int k = 0; k < wave; ++k) mine += r0 + k < I && mask[r0 + k] ? 1 : 0;
+            if (in && mask[r]) pos = before + mine;
+        }
+        if (!in) return;
+        unsigned char *const act = (m ? a.active[1] : a.active[0]) + (size_t)(pos < 0 ? 0 : pos) * a.row_bytes;
+        for (int c0 = lane; c0 < chunks; c0 += U * kWave) {
+            if (c0 != lane) load(c0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int c = c0 + u * kWave;
+                if (c >= chunks) continue;
+                st16(pool + ((size_t)c << 4), v[u]);
+                if (pos >= 0) st16(act + ((size_t)c << 4), v[u]);
+            }
+        }
+        return;
+    }
+    // ---- a tile of down: waves 2 x 2, lanes 8 x 8, V x V elements each
+    unit -= a.nrow * row_groups;
+    const int ht = (H + kTile - 1) / kTile;
+    const int i0 = (unit / ht) * kTile, h0 = (unit % ht) * kTile;
+    const int il = (wave & 1) * 8 * V + (lane & 7) * V, h = h0 + (wave >> 1) * 8 * V + (lane >> 3) * V, i = i0 + il;
+    const bool in = h < H && i < I;   // (H is a multiple of V)
+    uint4 v[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        v[k] = make_uint4(0u, 0u, 0u, 0u);
+        if (!in) continue;
+        const unsigned char *const p = a.down + ((size_t)(h + k) * I + i) * ESZ;
+        if (a.down_vec) {
+            v[k] = ld16_stream(p);
+        } else {
+            uint32_t d[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                if (i + e >= I) continue;
+                if constexpr (ESZ == 2) d[e >> 1] |= (uint32_t)reinterpret_cast<const uint16_t *>(p)[e] << (16 * (e & 1));
+                else d[e] = reinterpret_cast<const uint32_t *>(p)[e];
+            }
+            v[k] = make_uint4(d[0], d[1], d[2], d[3]);
+        }
+    }
+    if (mask != nullptr) {
+        const int before = rank_of(i0);
+        const int e = i0 + tid;
+        if (tid < kTile) {   // (whole waves)
+            const bool set = e < I && mask[e] != 0;
+            const uint64_t b = __ballot(set);
+            int c = before + (int)__popcll(b & ((1ull << lane) - 1ull));
+            if (wave == 1) {   // behind the first wave's elements
+                const bool first = i0 + lane < I && mask[i0 + lane] != 0;
+                c += (int)__popcll(__ballot(first));
+            }
+            tile_pos[tid] = set ? c : -1;
+        }
+        sync();
+    }
+    if (!in) return;
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        if (i + k >= I) continue;
+        uint32_t o[4];
+        auto word = [&](const uint4 &q, int j) __attribute__((always_inline)) { return j == 0 ? q.x : j == 1 ? q.y : j == 2 ? q.z : q.w; };
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if constexpr (ESZ == 2)
+                o[j] = __builtin_amdgcn_perm(word(v[2 * j + 1], k >> 1), word(v[2 * j], k >> 1), k & 1 ? 0x07060302u : 0x05040100u);
+            else
+                o[j] = word(v[j], k);
+        }
+        const uint4 q = make_uint4(o[0], o[1], o[2], o[3]);
+        st16(a.downT_pool + (size_t)(i + k) * a.row_bytes + (size_t)h * ESZ, q);
+        if (mask != nullptr) {
+            const int p = tile_pos[il + k];
+            if (p >= 0) st16(a.down_active + (size_t)p * a.row_bytes + (size_t)h * ESZ, q);
+        }
     }
 }
 
-__global__ void cache_reset_kernel(uint8_t *cur_mask2, int32_t *indices2, int32_t *state, int I)
+// ---------------------------------------------------------------------------
+// the caches' pinned words
+// ---------------------------------------------------------------------------
+// A cache's copy of its state words and, behind them, what its updates write by themselves.
+struct HostSlot {
+    int32_t state[ST_STATE_WORDS];
+    HostWords words;
+};
+static_assert(ST_STATE_WORDS * sizeof(int32_t) == 64 && sizeof(HostSlot) == 192, "cache lines of their own");
+
+// Slots come from slabs that are kept between caches (allocating and freeing pinned memory waits for the device, and the
+// words of a model's caches share pages).  At most one slab per GPU stays without a user.  A kernel still on its way when
+// its cache is destroyed may write to the slot's next owner: its count is a guess there as everywhere, and the state words
+// carry the number of their update, which goes on from owner to owner.
+struct HostSlab {
+    static constexpr int kSlots = 64;
+    HostSlab *next;
+    int device;
+    HostSlot *base;
+    uint64_t used;
+    uint32_t number[kSlots];
+};
+static std::mutex host_slab_mutex;
+static HostSlab *host_slabs = nullptr;
+
+// A free slot of the current device, zeroed; false if there is no memory.
+static bool take_host_slot(HostSlab **slab, int *at)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < 2 * I) {
-        cur_mask2[i] = 0;
-        indices2[i] = -1;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lock(host_slab_mutex);
+    HostSlab *s = host_slabs;
+    while (s && (s->device != dev || s->used == ~0ull)) s = s->next;
+    if (!s) {
+        s = new (std::nothrow) HostSlab{};
+        if (!s) return false;
+        if (hipHostMalloc(reinterpret_cast<void **>(&s->base), HostSlab::kSlots * sizeof(HostSlot), hipHostMallocDefault) != hipSuccess) {
+            delete s;
+            return false;
+        }
+        s->device = dev;
+        s->next = host_slabs;
+        host_slabs = s;
     }
-    if (i < ST_STATE_WORDS) state[i] = 0;
+    *slab = s;
+    *at = __builtin_ctzll(~s->used);
+    s->used |= 1ull << *at;
+    memset(&s->base[*at], 0, sizeof(HostSlot));
+    return true;
+}
+
+static void give_host_slot_back(HostSlab *slab, int at, uint32_t number)
+{
+    std::lock_guard<std::mutex> lock(host_slab_mutex);
+    slab->number[at] = number;
+    slab->used &= ~(1ull << at);
+    if (slab->used != 0) return;
+    for (HostSlab **link = &host_slabs; *link; link = &(*link)->next) {   // another one without a user goes
+        HostSlab *s = *link;
+        if (s == slab || s->device != slab->device || s->used != 0) continue;
+        *link = s->next;
+        (void)hipHostFree(s->base);
+        delete s;
+        return;
+    }
 }
 
 }  // namespace st
@@ -1927,6 +2168,8 @@ struct st_cache {
     int64_t I, H;
     int dtype, has_gate;
     int esz;
+    st::HostSlab *slab;    // whose slot `slot` holds the next two
+    int slot;
     int32_t *host_state;   // pinned: ST_STATE_WORDS words as st_cache_sync_state last read them
     st::HostWords *host;   // pinned, behind them: what updates write by themselves
     uint32_t number;       // of the last update that a caller waited for
@@ -1955,24 +2198,66 @@ extern "C" st_cache *st_cache_create(const st_cache_buffers *bufs, int64_t I, in
     if (!c) return fail("out of host memory");
     c->b = *bufs;
     c->I = I; c->H = H; c->dtype = dtype; c->has_gate = has_gate ? 1 : 0; c->esz = esz;
-    c->host_state = nullptr;
-    static_assert(ST_STATE_WORDS * sizeof(int32_t) == 64, "the host words keep a cache line of their own");
-    const size_t host_bytes = 64 + sizeof(HostWords);
-    if (hipHostMalloc(reinterpret_cast<void **>(&c->host_state), host_bytes, hipHostMallocDefault) != hipSuccess) {
+    if (!take_host_slot(&c->slab, &c->slot)) {
         delete c;
         return fail("hipHostMalloc failed");
     }
-    memset(c->host_state, 0, host_bytes);
-    c->host = reinterpret_cast<HostWords *>(reinterpret_cast<unsigned char *>(c->host_state) + 64);
-    c->number = 0;
+    c->host_state = c->slab->base[c->slot].state;
+    c->host = &c->slab->base[c->slot].words;
+    c->number = c->slab->number[c->slot];
     return c;
 }
 
 extern "C" void st_cache_destroy(st_cache *c)
 {
     if (!c) return;
-    if (c->host_state) (void)hipHostFree(c->host_state);
+    st::give_host_slot_back(c->slab, c->slot, c->number);
     delete c;
+}
+
+// mask: of the rows that are active afterwards, in ascending order (null: none).  number: nonzero if the caller waits for
+// the state words.
+static int launch_build(st_cache *c, const void *gate, const void *up, const void *down, const uint8_t *mask, uint32_t number,
+                        hipStream_t s)
+{
+    using namespace st;
+    const size_t bytes = (size_t)c->I * c->H * c->esz;
+    BuildMats a;
+    a.row_bytes = (int)(c->H * c->esz);
+    a.nrow = 0;
+    auto rows = [&](const void *src, void *pool, void *active) -> int {
+        if ((uintptr_t)src & 15) {   // rows that cannot be read in vectors: into the pool first, the kernel reads them there
+            ST_HIP(hipMemcpyAsync(pool, src, bytes, hipMemcpyDeviceToDevice, s));
+            src = pool;
+        }
+        a.src[a.nrow] = static_cast<const unsigned char *>(src);
+        a.pool[a.nrow] = static_cast<unsigned char *>(pool);
+        a.active[a.nrow++] = static_cast<unsigned char *>(active);
+        return ST_OK;
+    };
+    int rc = c->has_gate ? rows(gate, c->b.gate_pool, c->b.gate_active) : ST_OK;
+    if (rc == ST_OK) rc = rows(up, c->b.up_pool, c->b.up_active);
+    if (rc != ST_OK) return rc;
+    if (a.nrow == 1) { a.src[1] = a.src[0]; a.pool[1] = a.pool[0]; a.active[1] = a.active[0]; }
+    a.down = static_cast<const unsigned char *>(down);
+    a.downT_pool = static_cast<unsigned char *>(c->b.downT_pool);
+    a.down_active = static_cast<unsigned char *>(c->b.down_active);
+    a.down_vec = ((uintptr_t)down & 15) == 0 && (c->I * c->esz) % 16 == 0;
+    const int tile = 256 / c->esz;
+    const int64_t blocks = 1 + (int64_t)a.nrow * ((c->I + kBuildRows - 1) / kBuildRows) +
+                           ((c->I + tile - 1) / tile) * ((c->H + tile - 1) / tile);
+    ST_REQUIRE(blocks <= 0x7fffffff, "st_cache: hidden size %lld out of range", (long long)c->H);
+    // the count is told where the updates that follow tell theirs (the guess must not stay behind)
+    const int tell = mask != nullptr && c->I <= kPlanMaxI && c->I % 8 == 0;
+    const int mask_vec = ((uintptr_t)mask & 7) == 0;
+    if (c->esz == 4)
+        hipLaunchKernelGGL(cache_build_kernel<4>, dim3((unsigned)blocks), dim3(kBuildThreads), 0, s, mask, c->b.cur_mask,
+                           c->b.indices, c->b.state, (int)c->I, (int)c->H, mask_vec, c->host, tell, number, a);
+    else
+        hipLaunchKernelGGL(cache_build_kernel<2>, dim3((unsigned)blocks), dim3(kBuildThreads), 0, s, mask, c->b.cur_mask,
+                           c->b.indices, c->b.state, (int)c->I, (int)c->H, mask_vec, c->host, tell, number, a);
+    ST_HIP(hipGetLastError());
+    return ST_OK;
 }
 
 extern "C" int st_cache_load_weights(st_cache *c, const void *gate, const void *up, const void *down, void *stream)
@@ -1980,22 +2265,7 @@ extern "C" int st_cache_load_weights(st_cache *c, const void *gate, const void *
     using namespace st;
     ST_REQUIRE(c && up && down, "st_cache_load_weights: null pointer");
     ST_REQUIRE(!c->has_gate || gate, "st_cache_load_weights: gated cache needs gate weights");
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const size_t bytes = (size_t)c->I * c->H * c->esz;
-    ST_HIP(hipMemcpyAsync(c->b.up_pool, up, bytes, hipMemcpyDeviceToDevice, s));
-    if (c->has_gate) ST_HIP(hipMemcpyAsync(c->b.gate_pool, gate, bytes, hipMemcpyDeviceToDevice, s));
-    const dim3 grid((unsigned)((c->I + 63) / 64), (unsigned)((c->H + 63) / 64));
-    if (c->esz == 4)
-        hipLaunchKernelGGL(transpose_kernel<uint32_t>, grid, dim3(256), 0, s, static_cast<const uint32_t *>(down),
-                           static_cast<uint32_t *>(c->b.downT_pool), (int)c->H, (int)c->I);
-    else
-        hipLaunchKernelGGL(transpose_kernel<uint16_t>, grid, dim3(256), 0, s, static_cast<const uint16_t *>(down),
-                           static_cast<uint16_t *>(c->b.downT_pool), (int)c->H, (int)c->I);
-    ST_HIP(hipGetLastError());
-    hipLaunchKernelGGL(cache_reset_kernel, dim3((unsigned)((2 * c->I + 255) / 256)), dim3(256), 0, s, c->b.cur_mask,
-                       c->b.indices, c->b.state, (int)c->I);
-    ST_HIP(hipGetLastError());
-    return ST_OK;
+    return launch_build(c, gate, up, down, nullptr, 0, static_cast<hipStream_t>(stream));
 }
 
 // The pointers of one cache and the mask of its update.
@@ -2289,6 +2559,35 @@ static int update_outcome(const st_cache *c)
     return ST_OK;
 }
 
+// The state words of update `c->number`, which is on its way on `stream`, into the host's copy and state_out.
+static int wait_for_state(st_cache *c, int32_t *state_out, void *stream)
+{
+    using namespace st;
+    // The publishing block writes the words across the bus as soon as its plan stands; a copy of the state behind the kernel
+    // and a wait for the stream takes 10 us longer.  Bounded: with other work ahead of it on the stream the wait is the
+    // stream's.
+    const volatile uint64_t *w = c->host->state;
+    const auto begun = std::chrono::steady_clock::now();
+    for (int spins = 0;; ++spins) {
+        bool all = true;
+        int32_t v[8];
+        for (int k = 0; k < 8; ++k) {
+            const uint64_t x = w[k];
+            all = all && (uint32_t)(x >> 32) == c->number;
+            v[k] = (int32_t)(uint32_t)x;
+        }
+        if (all) {
+            for (int k = 0; k < 8; ++k) c->host_state[kHostStateWords[k]] = v[k];
+            if (state_out)
+                for (int k = 0; k < ST_STATE_WORDS; ++k) state_out[k] = c->host_state[k];
+            return update_outcome(c);
+        }
+        __builtin_ia32_pause();
+        if ((spins & 63) == 63 && std::chrono::steady_clock::now() - begun > std::chrono::milliseconds(1)) break;
+    }
+    return st_cache_sync_state(c, state_out, stream);
+}
+
 extern "C" int st_cache_update_sync(st_cache *c, const uint8_t *mask, int32_t *state_out, void *stream)
 {
     using namespace st;
@@ -2296,34 +2595,21 @@ extern "C" int st_cache_update_sync(st_cache *c, const uint8_t *mask, int32_t *s
     if (c->I <= kPlanMaxI && update_is_aligned(c, mask)) {
         if (++c->number == 0) c->number = 1;
         const int rc = launch_update(&c, &mask, 1, c->number, static_cast<hipStream_t>(stream));
-        if (rc != ST_OK) return rc;
-        // The kernel's publishing block writes the words across the bus as soon as its plan stands; a copy of the state
-        // behind the kernel and a wait for the stream takes 10 us longer.  Bounded: with other work ahead of it on the
-        // stream the wait is the stream's.
-        const volatile uint64_t *w = c->host->state;
-        const auto begun = std::chrono::steady_clock::now();
-        for (int spins = 0;; ++spins) {
-            bool all = true;
-            int32_t v[8];
-            for (int k = 0; k < 8; ++k) {
-                const uint64_t x = w[k];
-                all = all && (uint32_t)(x >> 32) == c->number;
-                v[k] = (int32_t)(uint32_t)x;
-            }
-            if (all) {
-                for (int k = 0; k < 8; ++k) c->host_state[kHostStateWords[k]] = v[k];
-                if (state_out)
-                    for (int k = 0; k < ST_STATE_WORDS; ++k) state_out[k] = c->host_state[k];
-                return update_outcome(c);
-            }
-            __builtin_ia32_pause();
-            if ((spins & 63) == 63 && std::chrono::steady_clock::now() - begun > std::chrono::milliseconds(1)) break;
-        }
-    } else {
-        const int rc = st_cache_update_async(c, mask, stream);
-        if (rc != ST_OK) return rc;
+        return rc != ST_OK ? rc : wait_for_state(c, state_out, stream);
     }
-    return st_cache_sync_state(c, state_out, stream);
+    const int rc = st_cache_update_async(c, mask, stream);
+    return rc != ST_OK ? rc : st_cache_sync_state(c, state_out, stream);
+}
+
+extern "C" int st_cache_load_weights_masked(st_cache *c, const void *gate, const void *up, const void *down,
+                                            const uint8_t *mask, int32_t *state_out, void *stream)
+{
+    using namespace st;
+    ST_REQUIRE(c && up && down && mask, "st_cache_load_weights_masked: null pointer");
+    ST_REQUIRE(!c->has_gate || gate, "st_cache_load_weights_masked: gated cache needs gate weights");
+    if (++c->number == 0) c->number = 1;
+    const int rc = launch_build(c, gate, up, down, mask, c->number, static_cast<hipStream_t>(stream));
+    return rc != ST_OK ? rc : wait_for_state(c, state_out, stream);
 }
 
 extern "C" int st_cache_sync_state(st_cache *c, int32_t *state_out, void *stream)

@@ -153,19 +153,18 @@ class WeightCache:
         up_c = up_weight.detach().contiguous()
         down_c = down_weight.detach().contiguous()
         gate_c = gate_weight.detach().contiguous() if self.has_gate else None
-        rc = L.st_cache_load_weights(self._h, gate_c.data_ptr() if self.has_gate else None, up_c.data_ptr(),
-                                     down_c.data_ptr(), current_stream_ptr(dev))
-        _lib.check(rc, "st_cache_load_weights")
         self._host_state = (C.c_int32 * _lib.STATE_WORDS)()
         self._seen = C.c_int32.from_address(L.st_cache_seen_count(self._h))   # the count the last finished update told the host
-        self._host_serial = -1      # serial the host copy of the state belongs to
-        self._dirty = True          # updates enqueued since the last read-back
         self.lazy_updates = False
         self._pending_mask: Optional[torch.Tensor] = None
         self._concat_ref = None     # weak reference to the handle get_concat_weight() handed out last
         self._concat_serial = -1
-        # weight_cache.h:226: the constructor ends with update_active_weights(init_mask)
-        self.update_active_weights(init_mask)
+        # weight_cache.h:226: the constructor ends with update_active_weights(init_mask); here in one pass over the weights
+        mask = self._mask_arg(init_mask)
+        rc = L.st_cache_load_weights_masked(self._h, gate_c.data_ptr() if self.has_gate else None, up_c.data_ptr(),
+                                            down_c.data_ptr(), mask.data_ptr(), self._host_state, current_stream_ptr(dev))
+        self._dirty = rc != _lib.ST_OK   # updates enqueued since the last read-back
+        _lib.check(rc, "st_cache_load_weights_masked")
 
     def __del__(self):
         h, self._h = getattr(self, "_h", None), None

@@ -292,3 +292,59 @@ def test_fast_path_argument_errors():
     assert rc == _lib.ST_ERR_ARG and "ldc" in _lib.last_error()
     # nothing above changed the cache
     assert cache.get_num_active() == I
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("I,H", [(5, 8), (127, 136), (128, 64), (1000, 264), (2051, 48), (4104, 4160), (32768, 8)])
+def test_construction_equals_load_then_update(dtype, I, H):
+    """One pass over the weights gives what loading them and a first update give: pools, packed rows, lists, masks, state.
+    (tile edges both ways, sizes that cannot be read in vectors, rows of more than one pass, sources off their alignment)"""
+    import ctypes as C
+
+    from sparse_transformers_amd import _lib
+    tdt, L = getattr(torch, dtype), _lib.lib()
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(I + H)
+    for has_gate, fill, off in [(True, "some", 0), (False, "all", 0), (True, "none", 0), (True, "last", 1), (False, "some", 1)]:
+        def src(a, b):
+            return torch.randn(a * b + off, generator=gen, device=DEV).to(tdt)[off:].view(a, b)
+        gate, up, down = src(I, H) if has_gate else None, src(I, H), src(H, I)
+        mask = torch.zeros(I + off, dtype=torch.uint8, device=DEV)[off:]
+        if fill == "some":
+            mask.copy_(torch.randint(0, 3, (I,), generator=gen, device=DEV) * 64)   # any nonzero byte counts
+        elif fill != "none":
+            mask[0 if fill == "all" else I - 1:] = 1
+        one = st.WeightCache(mask, H, gate, up, down, has_gate)
+        two = st.WeightCache(torch.ones(I, dtype=torch.bool, device=DEV), H, gate, up, down, has_gate)
+        _lib.check(L.st_cache_load_weights(two._h, gate.data_ptr() if has_gate else None, up.data_ptr(), down.data_ptr(),
+                                           torch.cuda.current_stream().cuda_stream), "st_cache_load_weights")
+        two._dirty = True
+        assert two.get_num_active() == 0
+        m2 = mask.clone()
+        rc = L.st_cache_update_sync(two._h, m2.data_ptr(), two._host_state, torch.cuda.current_stream().cuda_stream)
+        assert rc == _lib.ST_OK, (fill, rc)
+        n = two.get_num_active()
+        assert n == int((mask != 0).sum()) and list(one._host_state)[:8] == list(two._host_state)[:8]
+        for name in ("gate_pool", "up_pool", "downT_pool", "gate_active", "up_active", "down_active", "indices", "cur_mask", "state"):
+            a, b = getattr(one, name), getattr(two, name)
+            if a is not None:
+                assert torch.equal(a[:n], b[:n]) if name.endswith("active") else torch.equal(a, b), (name, has_gate, fill)
+
+
+def test_host_words_are_shared_and_reused():
+    """More caches than one slab of pinned words holds, in any order of construction and destruction."""
+    w = torch.randn(64, 8, device=DEV)
+    down = torch.randn(8, 64, device=DEV)
+    for order in (1, -1):
+        caches = []
+        for k in range(150):
+            mask = torch.zeros(64, dtype=torch.bool, device=DEV)
+            mask[:1 + k % 64] = True
+            caches.append(st.WeightCache(mask, 8, w, w, down))
+            assert caches[-1].get_num_active() == 1 + k % 64
+        for k, c in enumerate(caches):
+            assert c._seen.value == 1 + k % 64
+            c.update_active_weights(torch.ones(64, dtype=torch.bool, device=DEV))
+            assert c.get_num_active() == 64
+        while caches:
+            caches.pop(0 if order == 1 else -1)
