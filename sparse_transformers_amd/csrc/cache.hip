@@ -1927,7 +1927,7 @@ template <int ESZ> struct BuildTile { static constexpr int rows = 256 / ESZ; }; 
 // 128-byte lines on both sides and nothing goes through LDS.  A row's position is the number of set mask bytes before it,
 // counted by every block while its rows are on the way.
 // H 3072, I 8192, fp16, all rows (453 MB): 160 us as two copies, a transposing kernel (44 us), a reset and an update
-// (69 us, reading the pools back), @@ us as one.
+// (69 us, reading the pools back), 79 us as one (5.7 TB/s).
 template <int ESZ>
 __global__ __launch_bounds__(kBuildThreads) void cache_build_kernel(const uint8_t *__restrict__ mask,
                                                                     uint8_t *__restrict__ cur_mask2,
