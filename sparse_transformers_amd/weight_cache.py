@@ -14,8 +14,8 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .ops import (_check_workspace, check_mlp_args, combined_for_launch, current_stream_ptr, dtype_code,
-                  mlp_forward_rows, mlp_workspace, mlp_workspace_bytes, require_gpu)
+from .ops import (_check_workspace, _kept_workspace, check_mlp_args, combined_for_launch, current_stream_ptr,
+                  dtype_code, mlp_forward_rows, mlp_workspace_bytes, require_gpu)
 
 
 class ConcatWeightHandle(torch.Tensor):
@@ -275,7 +275,7 @@ class WeightCache:
             raise ValueError(f"x must have {H} columns, got {tuple(x.shape)}")
         if x.dtype != self.dtype or x.device != self.device:
             raise TypeError(f"x must be {self.dtype} on {self.device}, got {x.dtype} on {x.device}")
-        x2 = x.reshape(-1, H)
+        x2 = x if x.dim() == 2 else x.reshape(-1, H)
         return x2 if x2.is_contiguous() else x2.contiguous()
 
     def update_and_forward(self, mask: torch.Tensor, x: torch.Tensor, act: str = "silu",
@@ -298,7 +298,7 @@ class WeightCache:
         # the count after the update is not known on the host: `combined` must hold the largest possible one
         check_mlp_args(x2, out, combined, self.dtype, self.device, H, (2 if self.has_gate else 1) * I)
         need = mlp_workspace_bytes(B, H, I)
-        ws = mlp_workspace(self.device, B, H, I) if workspace is None else _check_workspace(workspace, self.device, need)
+        ws = _kept_workspace(self.device, need) if workspace is None else _check_workspace(workspace, self.device, need)
         if act not in _lib.ACT_CODES:
             raise ValueError(f"unknown activation {act!r}; expected one of {sorted(_lib.ACT_CODES)}")
         combined, copy_back = combined_for_launch(combined, B, I)
@@ -312,7 +312,7 @@ class WeightCache:
         self._dirty = True
         if copy_back is not None:
             copy_back.copy_(combined)
-        return out.view(x.shape)
+        return out if x.dim() == 2 else out.view(x.shape)
 
     def forward(self, x: torch.Tensor, act: str = "silu", out: Optional[torch.Tensor] = None,
                 combined: Optional[torch.Tensor] = None, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -330,4 +330,4 @@ class WeightCache:
         mlp_forward_rows(x2, self.gate_active, self.up_active, self.down_active, self.intermediate_size,
                          self.n_active_dev, out, combined, act, self.has_gate,
                          n_hint=self._seen.value, workspace=workspace)
-        return out.view(x.shape)
+        return out if x.dim() == 2 else out.view(x.shape)
