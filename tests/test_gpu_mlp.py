@@ -284,6 +284,27 @@ def test_prefill_device_count(M):
     assert not out.any()                                       # empty active set -> zeros
 
 
+@pytest.mark.parametrize("M", [40, 130, 300])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 129, 1025, 3000, 6143, 6144])
+def test_prefill_tiles_follow_the_device_count(M, n):
+    """The tiles of weight rows are dealt out over the count the device holds: counts around the tile edges, from one row to
+    the capacity, in every form of the gate / up kernel; every column of the intermediate has to be written by some tile."""
+    I, H = 6144, 512
+    g = torch.Generator().manual_seed(n)
+    gate, up, dn = ((torch.randn(I, H, generator=g) * 0.05).half().to(DEV) for _ in range(3))
+    x = torch.randn(M, H, generator=g).half().to(DEV)
+    h = torch.nn.functional.silu(x.float() @ gate[:n].float().t()) * (x.float() @ up[:n].float().t())
+    want = h @ dn[:n].float()
+    for t in (gate, up, dn):
+        t[n:] = float("nan")
+    out = torch.full((M, H), float("nan"), dtype=torch.float16, device=DEV)
+    comb = torch.full((M, 2 * I), float("nan"), dtype=torch.float16, device=DEV)
+    mlp_forward_rows(x, gate, up, dn, I, torch.tensor([n], dtype=torch.int32, device=DEV), out, comb, "silu", True)
+    torch.cuda.synchronize()
+    assert_close(out.float().cpu().numpy(), want.cpu().numpy(), "float16", f"{M} rows, {n} active")
+    assert_close(comb[:, :n].float().cpu().numpy(), h.cpu().numpy(), "float16", f"intermediate, {M} rows, {n} active")
+
+
 def test_prefill_agrees_with_decode_kernel():
     """The MFMA path (B = 40) and the streaming path (the same rows, 4 at a time) agree to rounding."""
     x, cw, dn = _case(22, 40, 1024, 700, "float16", True)
