@@ -397,7 +397,7 @@ extern "C" int st_predictor_mask_ex(const void *x, int64_t B, int64_t H, const v
     ST_REQUIRE((align & 15) == 0, "st_predictor_mask_ex: pointers must be 16-byte aligned");
     const int round_storage = (flags & ST_PRED_ROUND_STORAGE) && dtype != ST_F32 ? 1 : 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (predictor_mfma_supported(dtype, (int)B, (int)r))
+    if (predictor_mfma_supported(dtype, (int)B, (int)H, (int)r))
         return launch_predictor_mfma(dtype, x, (int)B, (int)H, A, (int)r, Bm, (int)I, thr, cmp_ge, t_ws, scores, mask,
                                      round_storage, s);
     // Further passes reuse the front of t_ws (the launches are ordered on the stream) and only ever switch mask bytes on.
@@ -434,7 +434,7 @@ extern "C" int st_predictor_mask_layers(const st_predictor_layer *layers, int64_
     ST_REQUIRE((align & 15) == 0, "st_predictor_mask_layers: pointers must be 16-byte aligned");
     const int round_storage = (flags & ST_PRED_ROUND_STORAGE) && dtype != ST_F32 ? 1 : 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool mfma = predictor_mfma_supported(dtype, (int)B, (int)r);
+    const bool mfma = predictor_mfma_supported(dtype, (int)B, (int)H, (int)r);
     if (!mfma && B > pred_rows_per_pass(r)) {   // several passes per layer: one layer at a time
         for (int64_t l = 0; l < L; ++l) {
             const st_predictor_layer &y = layers[l];

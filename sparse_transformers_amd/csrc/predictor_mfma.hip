@@ -51,13 +51,16 @@ __global__ __launch_bounds__(W * kWave) void predictor_down_mfma_kernel(const T 
     const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint4 *)lds;
 
     // load j fills LDS rows 4 j .. 4 j + 3, lane i position i % 16 of row i / 16.  Rows are clamped into range (what they
-    // feed is not stored), and so are columns past the end of a row (replaced by zeros below).
+    // feed is not stored), and so are columns past the end of a row (replaced by zeros below).  Offsets of 32 bits only
+    // reach over the tile's own rows: x may be larger than 4 GiB.
+    const char *const x_tile = reinterpret_cast<const char *>(x + (size_t)m0 * H);
+    const char *const a_tile = reinterpret_cast<const char *>(A + (size_t)k0 * H);
     unsigned doff[kDma];
 #pragma unroll
     for (int j = 0; j < kDma; ++j) {
         const int row = 4 * j + (lane >> 4);
-        int g = row < 16 * MI ? m0 + row : k0 + row - 16 * MI;
-        const int last = row < 16 * MI ? B - 1 : r - 1;
+        int g = row < 16 * MI ? row : row - 16 * MI;
+        const int last = row < 16 * MI ? B - 1 - m0 : r - 1 - k0;
         g = g < last ? g : last;
         doff[j] = (unsigned)g * (unsigned)H * (unsigned)sizeof(T);
     }
@@ -68,7 +71,7 @@ __global__ __launch_bounds__(W * kWave) void predictor_down_mfma_kernel(const T 
             const int row = 4 * j + (lane >> 4), c = (lane & 15) ^ (row & 15);
             const int h = piece * kPmPiece + 8 * c;
             load_to_lds(lds_base + (unsigned)((wave * 2 + b) * kBuf + j * 64) * 16u, doff[j] + (unsigned)(h < H ? h : 0) * (unsigned)sizeof(T),
-                        reinterpret_cast<const char *>(4 * j < 16 * MI ? x : A));
+                        4 * j < 16 * MI ? x_tile : a_tile);
         }
     };
     f32x4_t acc[MI][NI];
@@ -209,15 +212,15 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
 
     const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint4 *)lds;
     auto dma = [&](int stage, int b) __attribute__((always_inline)) {
+        const T *const rows = Bm + (size_t)stage * kPmStage * r;   // (offsets within the stage: Bm may be larger than 4 GiB)
 #pragma unroll
         for (int j = 0; j < kDma; ++j) {
             const int at = (wave * kDma + j) * 64 + lane, row = at / kRow, pos = at % kRow;
             int c = pos ^ (row & 15);
             c = 8 * c < r ? c : 0;
-            int i = stage * kPmStage + row;
-            i = i < I ? i : I - 1;
+            const int last = I - 1 - stage * kPmStage, i = row < last ? row : last;
             const unsigned off = ((unsigned)i * (unsigned)r + 8u * (unsigned)c) * (unsigned)sizeof(T);
-            load_to_lds(lds_base + (unsigned)(b * kBuf + (wave * kDma + j) * 64) * 16u, off, reinterpret_cast<const char *>(Bm));
+            load_to_lds(lds_base + (unsigned)(b * kBuf + (wave * kDma + j) * 64) * 16u, off, reinterpret_cast<const char *>(rows));
         }
     };
     if (s0 >= s1) return;
@@ -340,8 +343,12 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
 // row at rank 256) and take x in passes of eight, sixteen and at last 64 rows; these take 7-14 us for any number up to 64.
 // Both kernels, replayed from a graph, there / here, at H 3072, rank 128, I 8192 (bf16): 7.5 / 8.4 us for 8 rows, 9.9 / 8.7
 // for 12, 17.0 / 9.6 for 32, 29.5 / 10.6 for 64, 233 / 15.6 for 512, 929 / 31 for 2048; at H 4096, rank 256, I 14336:
-// 10.6 / 10.6, 14.3 / 11.0, 25.0 / 12.1, 68.9 / 13.2, 538 / 29, 2236 / 78.  Ranks above 512 do not fit the registers.
-bool predictor_mfma_supported(int dtype, int B, int r) { return dtype != ST_F32 && B > 8 && r <= 512; }
+// 10.6 / 10.6, 14.3 / 11.0, 25.0 / 12.1, 68.9 / 13.2, 538 / 29, 2236 / 78.  Ranks above 512 do not fit the registers, and a
+// tile's 32 rows of x have to stay within 32-bit offsets.
+bool predictor_mfma_supported(int dtype, int B, int H, int r)
+{
+    return dtype != ST_F32 && B > 8 && r <= 512 && H < (1 << 26);
+}
 
 template <typename T, typename Tab>
 static int launch_t(const Tab &tab, int layers, const void *x, int B, int H, const void *A, int r, const void *Bm, int I,

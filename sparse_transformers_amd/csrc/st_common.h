@@ -280,7 +280,7 @@ struct PredLayers {
 };
 
 // Predictor on the matrix cores for several rows of x (fp16 / bf16, rank up to 512).
-bool predictor_mfma_supported(int dtype, int B, int r);
+bool predictor_mfma_supported(int dtype, int B, int H, int r);
 int launch_predictor_mfma(int dtype, const void *x, int B, int H, const void *A, int r, const void *Bm, int I, float thr,
                           int cmp_ge, float *t_ws, float *scores, uint8_t *mask, int round_storage, hipStream_t stream);
 int launch_predictor_mfma_layers(int dtype, const PredLayers &tab, int layers, const void *x, int B, int H, int r, int I,

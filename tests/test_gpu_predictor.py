@@ -85,6 +85,27 @@ def test_matrix_core_predictor(B, H, r, I, dtype):
     assert np.array_equal(m.cpu().numpy(), (s.cpu().numpy() >= 0).any(0))   # mask and scores come from the same sums
 
 
+def test_matrix_core_predictor_reads_beyond_4_gib():
+    """x and Bm of more than 4 GiB: the last row of either decides the mask (byte offsets of 32 bits would wrap)."""
+    H, r, I, B = 4096, 16, 64, 600_000                              # x: 4.9 GB
+    g = torch.Generator(device=DEV).manual_seed(3)
+    A, Bm = (torch.randn(a, b, generator=g, device=DEV).half() * 0.05 for a, b in ((r, H), (I, r)))
+    x = torch.zeros(B, H, dtype=torch.float16, device=DEV)
+    x[-1] = torch.randn(H, generator=g, device=DEV).half()
+    s = (x[-1:].float() @ A.float().t() @ Bm.float().t())[0]
+    hi = s.sort().values[I // 2:]
+    at = int((hi[1:] - hi[:-1]).argmax())
+    thr = float(hi[at] + hi[at + 1]) / 2
+    assert thr > 0 and torch.equal(st.predictor_mask(x, A, Bm, thr, True), s >= thr)
+    del x
+    H, r, I, B = 64, 136, 1 << 24, 9                                # Bm: 4.6 GB
+    A = torch.full((r, H), 0.125, dtype=torch.float16, device=DEV)
+    Bm = torch.zeros(I, r, dtype=torch.float16, device=DEV)
+    Bm[-1] = 0.125
+    x = torch.ones(B, H, dtype=torch.float16, device=DEV)
+    assert st.predictor_mask(x, A, Bm, 1.0, True).nonzero().flatten().tolist() == [I - 1]
+
+
 def test_naive_threshold_is_score_ge_zero():
     x, A, Bm = _weights(1, 2, 256, 16, 512, "float32")
     # make some scores exactly zero: a zero row of Bm gives score 0 for every input row
