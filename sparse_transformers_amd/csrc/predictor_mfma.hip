@@ -135,6 +135,8 @@ __global__ __launch_bounds__(W * kWave) void predictor_down_mfma_kernel(const T 
 // ---------------------------------------------------------------------------
 // kernel 2
 // ---------------------------------------------------------------------------
+constexpr float kMaxF32 = 3.402823466e+38f;
+
 // Eight floats of t -> the parts of one A operand register quad each.
 template <typename T> __device__ __forceinline__ void split_parts(const float *v, uint4 *parts);
 template <> __device__ __forceinline__ void split_parts<bf16_t>(const float *v, uint4 *parts)
@@ -145,10 +147,12 @@ template <> __device__ __forceinline__ void split_parts<bf16_t>(const float *v, 
         float rest = v[k];
 #pragma unroll
         for (int p = 0; p < 3; ++p) {
-            const __bf16 b = (__bf16)rest;          // (the hardware's conversion: round to nearest even)
+            __bf16 b = (__bf16)rest;                // (the hardware's conversion: round to nearest even)
+            if (p == 0 && fabsf(rest) <= kMaxF32 && fabsf((float)b) > kMaxF32)   // a finite value stays finite
+                b = __builtin_bit_cast(__bf16, (uint16_t)(rest > 0.f ? 0x7f7f : 0xff7f));
             w[p][k] = b;
             rest -= (float)b;
-            if (p == 0) rest = fabsf(rest) < 3.3e38f ? rest : 0.f;   // an infinity or NaN has nothing left over
+            if (p == 0) rest = fabsf(rest) <= kMaxF32 ? rest : 0.f;   // an infinity or NaN has nothing left over
         }
     }
 #pragma unroll
@@ -321,6 +325,9 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
                     float v = acc[i][P - 1][e];
 #pragma unroll
                     for (int p = P - 2; p >= 0; --p) v += acc[i][p][e];   // smallest part first
+                    // An infinite element of Bm decides the score by the sign of t, which its first part has; the others are
+                    // zero or of either sign and would make a NaN of it.
+                    v = fabsf(acc[i][0][e]) <= kMaxF32 ? v : acc[i][0][e];
                     if constexpr (P == 2) v *= unscale[i][e];
                     if (round_storage) v = to_float<T>(from_float<T>(v));
                     const bool in = (live >> (4 * i + e)) & 1u;

@@ -106,6 +106,46 @@ def test_matrix_core_predictor_reads_beyond_4_gib():
     assert st.predictor_mask(x, A, Bm, 1.0, True).nonzero().flatten().tolist() == [I - 1]
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("where", ["x", "A", "Bm"])
+@pytest.mark.parametrize("round_to_storage", [False, True])
+def test_matrix_core_predictor_infinities_and_nan(dtype, where, round_to_storage):
+    """Infinities, NaN and the largest finite values: every score is of the kind (NaN, either infinity, finite) that the
+    kernels for fewer rows of x, which multiply in fp32, give for the same row."""
+    B, H, r, I = 24, 256, 40, 300
+    x, A, Bm = (t.to(DEV) for t in _weights(11, B, H, r, I, dtype))
+    inf, nan, big = float("inf"), float("nan"), torch.finfo(x.dtype).max
+    x[7] = 0.0                                                   # 0 * inf
+    if where == "x":
+        x[2, 9], x[5, 200], x[19, 255] = inf, -inf, nan
+        x[11, :16] = big
+        A[8, 9], Bm[8] = 0.0, 0.0                                # inf * 0, once in either map
+        if dtype == "bfloat16":   # an element of the intermediate that is finite and would round to an infinity in 16 bits
+            A[30] = 0.0
+            A[30, 0] = A[30, 1] = 1.0
+            x[13] = 0.0
+            x[13, 0], x[13, 1] = big, 0.75 * 2.0 ** 120
+    elif where == "A":
+        A[3] = 0.0
+        A[20, 0], A[21, 255], A[22, 17] = inf, -inf, inf
+        Bm[10:, 20:23] = 0.0
+        x[12, 0] = x[12, 255] = 0.0
+    else:
+        Bm[3, 5], Bm[4, 6], Bm[5, 7] = inf, -inf, nan
+        Bm[6, 0], Bm[6, 1], Bm[7] = inf, -inf, inf
+        Bm[8], Bm[9, 39] = 0.0, big
+        A[3] = 0.0
+        Bm[11, 3] = inf                                          # meets t = 0
+    few = torch.cat([st.predictor_scores(x[b:b + 8].contiguous(), A, Bm, round_to_storage) for b in range(0, B, 8)])
+    m, s = st.predictor_mask(x, A, Bm, 0.5, True, return_scores=True, round_to_storage=round_to_storage)
+    for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(kind(s), kind(few)), (kind.__name__, (kind(s) != kind(few)).nonzero()[:8].tolist())
+    assert torch.isnan(s).any() and (where == "x" or torch.isposinf(s).any() and torch.isneginf(s).any())
+    assert torch.equal(m, (s >= 0.5).any(0))
+    near = torch.isfinite(few) & ((few - 0.5).abs() < 1e-4 + (1e-2 if round_to_storage else 0.0))
+    assert torch.equal(m[~near.any(0)], (few >= 0.5).any(0)[~near.any(0)])
+
+
 def test_naive_threshold_is_score_ge_zero():
     x, A, Bm = _weights(1, 2, 256, 16, 512, "float32")
     # make some scores exactly zero: a zero row of Bm gives score 0 for every input row
