@@ -6,9 +6,10 @@
  * passed as void* (NULL = the default stream).  All entry points return
  * ST_OK (0) or a negative st_status; st_last_error() gives a message for the
  * calling thread.  No entry point except st_cache_create/st_cache_destroy
- * (host memory only), st_cache_sync_state (one small device-to-host copy) and
- * st_cache_update_sync allocates or synchronises: work is enqueued on `stream` and ordered with
- * whatever else the caller enqueues there.
+ * (host memory only) and st_cache_sync_state, st_cache_update_sync and
+ * st_cache_load_weights_masked (which wait for `stream`) allocates or
+ * synchronises: work is enqueued on `stream` and ordered with whatever else
+ * the caller enqueues there.
  *
  * Each entry point names the interface of NimbleEdge/sparse_transformers it
  * replaces (paths relative to that repository).
@@ -255,9 +256,7 @@ int st_cache_update_async(st_cache *c, const uint8_t *mask, void *stream);
  * must be different ones. */
 int st_cache_update_layers(st_cache *const *caches, const uint8_t *const *masks, int64_t L, void *stream);
 
-/* st_cache_update_async, then the state words of that update on the host: state_out (host int32[ST_STATE_WORDS], may be
- * NULL) and the return value are those of st_cache_sync_state behind it, but the call only waits until the update's plan
- * stands, not for its row copies (which later calls on `stream` follow anyway). */
+/* st_cache_update_async, then st_cache_sync_state (state_out, the wait and the return value are its), by a shorter way. */
 int st_cache_update_sync(st_cache *c, const uint8_t *mask, int32_t *state_out, void *stream);
 
 /* host; where updates leave the active count by themselves (pinned memory, 0 before the first one; the GPU may write it at

@@ -324,11 +324,64 @@ def test_construction_equals_load_then_update(dtype, I, H):
         rc = L.st_cache_update_sync(two._h, m2.data_ptr(), two._host_state, torch.cuda.current_stream().cuda_stream)
         assert rc == _lib.ST_OK, (fill, rc)
         n = two.get_num_active()
-        assert n == int((mask != 0).sum()) and list(one._host_state)[:8] == list(two._host_state)[:8]
+        assert n == int((mask != 0).sum())
+        for c in (one, two):   # the words a wait leaves on the host are the device's, all of them
+            assert list(c._host_state) == c.state.tolist()
         for name in ("gate_pool", "up_pool", "downT_pool", "gate_active", "up_active", "down_active", "indices", "cur_mask", "state"):
             a, b = getattr(one, name), getattr(two, name)
             if a is not None:
                 assert torch.equal(a[:n], b[:n]) if name.endswith("active") else torch.equal(a, b), (name, has_gate, fill)
+
+
+@pytest.mark.parametrize("I,H,dtype", [(8192, 3072, "float16"), (2051, 1024, "float32"), (28672, 512, "bfloat16")])
+def test_waiting_calls_are_done_when_they_return(I, H, dtype):
+    """The constructor and update_active_weights wait: what they read (the mask, the module's weights) may be rewritten and
+    what they wrote (pools, packed rows) may be read on another stream right after they return, without an event."""
+    tdt = getattr(torch, dtype)
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(I)
+    side = torch.cuda.Stream(device=DEV)
+    want = [torch.randn(*s, generator=gen, device=DEV).to(tdt) for s in ((I, H), (I, H), (H, I))]
+    weights = [w.clone() for w in want]
+    rows = [torch.empty(I, H, dtype=tdt, device=DEV) for _ in range(3)]
+    want_rows = [want[0], want[1], want[2].t().contiguous()]
+
+    def take(wc):   # on the other stream: the packed rows as they are now, then the inputs are gone
+        with torch.cuda.stream(side):
+            for r, a in zip(rows, (wc.gate_active, wc.up_active, wc.down_active)):
+                r.copy_(a)
+
+    for _ in range(3):
+        mask = torch.rand(I, generator=gen, device=DEV) < 0.6
+        first = mask.clone()
+        for w, v in zip(weights, want):
+            w.copy_(v)
+        torch.cuda.synchronize()
+        wc = st.WeightCache(mask, H, *weights, True)
+        take(wc)
+        with torch.cuda.stream(side):
+            for t in (mask, *weights):
+                t.zero_()
+        torch.cuda.synchronize()
+        idx = torch.nonzero(first).flatten()
+        for r, w in zip(rows, want_rows):
+            assert torch.equal(r[: len(idx)], w[idx])
+        for pool, w in zip((wc.gate_pool, wc.up_pool, wc.downT_pool), want_rows):
+            assert torch.equal(pool, w)
+        for density in (0.55, 0.2, 0.9):
+            mask.copy_(torch.rand(I, generator=gen, device=DEV) < density)
+            second = mask.clone()
+            torch.cuda.synchronize()
+            wc.update_active_weights(mask)
+            take(wc)
+            with torch.cuda.stream(side):
+                mask.zero_()
+            torch.cuda.synchronize()
+            idx = wc.get_active_indices()
+            assert torch.equal(torch.sort(idx)[0], torch.nonzero(second).flatten())
+            for r, w in zip(rows, want_rows):
+                assert torch.equal(r[: len(idx)], w[idx])
+            assert list(wc._host_state) == wc.state.tolist()
 
 
 def test_host_words_are_shared_and_reused():
