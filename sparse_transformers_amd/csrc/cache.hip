@@ -8,7 +8,7 @@
 //   phase 1   i-th removed position <- i-th added  (:248-277)   parallel
 //   phase 2   surplus additions appended           (:280-307)   parallel
 //   phase 3   surplus removals, swap-with-last     (:310-353)   parallel: where
-//             each step moves what follows in closed form (surplus_removals)
+//             the entries of the tail go does not depend on the steps (surplus_ends)
 // and then copies its share of the changed rows with 16-byte loads/stores.
 // The plan only decides WHICH index ends up at WHICH position.  Because every
 // active row is a bit-copy of a pool row, the data movement never has to
@@ -97,6 +97,19 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t *wave_t
     return prefix + incl - v;
 }
 
+// Does any thread of the block see `v`?  (uniform)
+template <int TPB, typename S>
+__device__ __forceinline__ bool any_of_block(bool v, uint32_t *wave_tot, int tid, S sync)
+{
+    const bool w = __builtin_amdgcn_ballot_w64(v) != 0;
+    sync();
+    if ((tid & (kWave - 1)) == 0) wave_tot[tid >> 6] = w ? 1u : 0u;
+    sync();
+    uint32_t r = 0;
+    for (int k = 0; k < TPB / kWave; ++k) r |= wave_tot[k];
+    return r != 0;
+}
+
 struct CopyPlan {
     const unsigned char *pool[3];
     unsigned char *active[3];
@@ -154,33 +167,25 @@ struct PlanShared {
 
 // Phase 3 (weight_cache.h:310-353): S surplus indices e_0 < e_1 < ... leave the list of n entries one by one, step k moving
 // the entry that is last at the time (slot n-1-k, a "tail slot") to where e_k is at the time.  Every step depends on the
-// list the previous one left, but where e_k is at its own step follows by chasing: it stays where it starts unless that is
-// a tail slot n-1-i of an earlier step i < k, which moved it to where e_i was, and so on.  Only the e_k that START in the
-// tail have to chase (about S^2 / n of them), and only through one another: they resolve in rounds, a thread each (a
-// chase that meets an unresolved one tries again in the next round; the smallest unresolved always gets through).  An
-// entry of the tail that stays, at slot n-1-j, then ends at place[j], followed on through place[n-1-q] while that is a
-// tail slot q.  One lane that took the steps in order needed 0.2 us for each (13 us of a 29 us update with 70 of them);
-// this takes under 2 us for any number.
-// place(k): in: where e_k starts (kNone: not in the list, no step at all: only after an update that failed; the others
-// move up); out: where it is at its step.  Returns the count after the steps (in every thread).
+// list the previous one left, but the outcome does not need the steps: join tail slot n-1-k to the slot e_k starts in, for
+// every k.  No two tail slots are joined to the same slot, so the joins form paths (and closed loops of tail slots, all of
+// whose entries leave).  A step moves an entry only along its path, and a path begins at an entry of the tail that stays --
+// nothing is joined to its slot -- and ends at a slot in front of the tail: the only slot of the path that is left in the
+// end, so that is where the entry goes, whatever the order of the steps.  All paths are followed at once, a thread per tail
+// slot, every slot pointing at least twice as far along after each round (usual churn has paths of one or two slots, which
+// takes no round or one).
+// H 3072, I 8192, an update of 2000 removals with its copies, between events: one path through all of them 15 us (chased in
+// the order of the steps it took 1969 rounds, 1670 us), in random order 23 us (more rows to copy; 24 before).
+//
+// place(k): the position e_k starts at (kNone: not in the list, no step at all: only after an update that failed; the others
+// move up).  Returns the count after the steps (in every thread); ends behind a barrier.
 template <int TPB, typename P, typename S>
-__device__ __forceinline__ int surplus_places(P place, int S_all, int n, uint32_t *wave_tot, int *shared_n, int tid, S sync)
+__device__ __forceinline__ int surplus_count(P place, int S_all, int n, uint32_t *wave_tot, int *shared_n, int tid, S sync)
 {
-    constexpr int kOpen = 0x8000;    // (positions stay below kPlanMaxI < 0x8000)
-    const int lane = tid & (kWave - 1), wave = tid >> 6;
-    auto any_of = [&](bool v) __attribute__((always_inline)) {   // over the block
-        const bool w = __builtin_amdgcn_ballot_w64(v) != 0;
-        sync();
-        if (lane == 0) wave_tot[wave] = w ? 1u : 0u;
-        sync();
-        uint32_t r = 0;
-        for (int k = 0; k < TPB / kWave; ++k) r |= wave_tot[k];
-        return r != 0;
-    };
     bool missing = false;
     for (int k = tid; k < S_all; k += TPB) missing = missing || place(k) == kNone;
     int S_ = S_all;
-    if (any_of(missing)) {
+    if (any_of_block<TPB>(missing, wave_tot, tid, sync)) {
         if (tid == 0) {
             int m = 0;
             for (int k = 0; k < S_all; ++k)
@@ -189,36 +194,29 @@ __device__ __forceinline__ int surplus_places(P place, int S_all, int n, uint32_
         }
         sync();
         S_ = *shared_n;
-        sync();
     }
-    const int base = n - S_;
+    return n - S_;
+}
+
+// Behind a barrier after surplus_count (base: its result): place(k) becomes the slot the path of tail slot n-1-k ends at,
+// where stays(k): whether that slot's entry stays.
+template <int TPB, typename P, typename Q, typename S>
+__device__ __forceinline__ void surplus_ends(P place, Q stays, int base, int n, uint32_t *wave_tot, int tid, S sync)
+{
+    constexpr int kHops = 4, kRounds = 16;   // (2^16 slots; the bound is never met)
     bool open = false;
-    for (int k = tid; k < S_; k += TPB) {
-        const int p = place(k);
-        if (p >= base) {
-            place(k) = (uint16_t)(p | kOpen);
-            open = true;
-        }
-    }
-    while (any_of(open)) {                  // (uniform; at least one resolves per round)
+    for (int k = tid; k < n - base; k += TPB) open = open || (place(k) >= base && stays(k));
+    for (int round = 0; any_of_block<TPB>(open, wave_tot, tid, sync) && round < kRounds; ++round) {
         open = false;
-        for (int k = tid; k < S_; k += TPB) {
+        for (int k = tid; k < n - base; k += TPB) {
             int q = place(k);
-            if (!(q & kOpen)) continue;
-            q &= kOpen - 1;
-            bool done = false;
-            for (int hop = 0; hop <= S_; ++hop) {
-                const int i = n - 1 - q;
-                if (q < base || i >= k) { done = true; break; }   // stays there until its own step (i == k: it is the last entry)
-                const int d = place(i);
-                if (d & kOpen) break;
-                q = d;
-            }
-            if (done) place(k) = (uint16_t)q;
-            else open = true;
+            if (q < base) continue;
+            // (the others move on at the same time: whatever is read lies further along the same path)
+            for (int hop = 0; hop < kHops && q >= base; ++hop) q = place(n - 1 - q);
+            place(k) = (uint16_t)q;
+            open = open || (q >= base && stays(k));
         }
     }
-    return base;
 }
 
 // Replays the bookkeeping of one update in LDS and publishes it (block 0 writes the other bookkeeping
@@ -233,7 +231,7 @@ __device__ __forceinline__ int surplus_places(P place, int S_all, int n, uint32_
 // turns out larger).
 //
 // Barrier sequence: 1 after the LDS fill; 2 in the diff scan;
-// [unchanged mask: done]; 1 after the lists; 1 after phases 1 and 2; [surplus removals: those of surplus_removals and 1
+// [unchanged mask: done]; 1 after the lists; 1 after phases 1 and 2; [surplus removals: those of surplus_count and surplus_ends and 1
 // behind it, 2 in the compaction scan, 1 after the compaction].
 template <bool VEC, int PT, int NW, bool MARK, typename F, typename F2>
 __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, PlanShared *ps,
@@ -445,13 +443,13 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
             place(k) = pos_l[e];
             pos_l[e] = kNone;
         }
-        n_new = surplus_places<TPB>(place, S_all, n, wave_tot, &n_new_s, tid, sync);
+        n_new = surplus_count<TPB>(place, S_all, n, wave_tot, &n_new_s, tid, sync);
+        auto stays = [&](int k) __attribute__((always_inline)) { return pos_l[idx_l[n - 1 - k]] != kNone; };
+        surplus_ends<TPB>(place, stays, n_new, n, wave_tot, tid, sync);
         for (int j = tid; j < n - n_new; j += TPB) {
-            const int v = idx_l[n - 1 - j];
-            if (pos_l[v] == kNone) continue;
-            int q = place(j);
-            for (int hop = 0; hop <= S_all && q >= n_new; ++hop) q = place(n - 1 - q);
-            idx_l[q] = (uint16_t)v;
+            if (!stays(j)) continue;
+            const int q = place(j);
+            idx_l[q] = idx_l[n - 1 - j];
             atomicOr(&dirty[q >> 5], 1u << (q & 31));
         }
         sync();
@@ -620,7 +618,7 @@ constexpr size_t update_lds_bytes(int I)
 // The update by POSITION.  Which index a position holds afterwards follows from the old list and the two masks without an
 // index -> position map: a removed index has a rank among the removed ones (a prefix count per eight indices, and the
 // bits below it), the i-th of them hands its position to the i-th added index (phase 1), the surplus additions follow at
-// the end (phase 2), and a position of rank >= n_added is where a surplus removal starts (phase 3, surplus_places).  So
+// the end (phase 2), and a position of rank >= n_added is where a surplus removal starts (phase 3, surplus_ends).  So
 // the plan is one scan, one pass over the list -- every thread keeps the positions it loaded in registers -- and two
 // barriers when removals do not outnumber additions.  Every block plans for itself (as a launch of its own the plan would
 // cost a kernel boundary) and copies its share of the items.
@@ -647,7 +645,7 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
     const int Ip = (I + 7) & ~7;
     uint16_t *const item_idx = reinterpret_cast<uint16_t *>(smem);   // added indices ascending; behind them the tail's entries
     uint16_t *const item_pos = item_idx + Ip;
-    uint16_t *const place = item_pos + Ip;                           // k-th surplus index: where it starts, then where its step finds it
+    uint16_t *const place = item_pos + Ip;                           // k-th surplus index: where it starts; then the end of its tail slot's path
     uint16_t *const rem_before = place + Ip;                         // per eight indices: removed ones below
     uint8_t *const rem_bits = reinterpret_cast<uint8_t *>(rem_before) + ((((I + 7) >> 3) * 2 + 15) & ~15);
     const int tid = threadIdx.x;
@@ -778,9 +776,9 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
         int n_new = n + (na - pairs) < I ? n + (na - pairs) : I, items = na;
         if (S_all > 0) {
             sync();
-            n_new = surplus_places<TPB>([&](int k) __attribute__((always_inline)) -> uint16_t & { return place[k]; }, S_all, n, wave_tot,
-                                        &shared_n, tid, sync);
-            // the entries of the tail, last first, behind the added indices: items like the others once their places are known
+            auto place_of = [&](int k) __attribute__((always_inline)) -> uint16_t & { return place[k]; };
+            n_new = surplus_count<TPB>(place_of, S_all, n, wave_tot, &shared_n, tid, sync);
+            // the entries of the tail, last first, behind the added indices: items like the others once their paths' ends are known
 #pragma unroll
             for (int q = 0; q < NV; ++q)
 #pragma unroll
@@ -789,13 +787,14 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
                     if (p >= n_new && p < n) item_idx[na + (n - 1 - p)] = (uint16_t)held[q][k];
                 }
             sync();
+            auto stays = [&](int j) __attribute__((always_inline)) { return item_idx[na + j] != kOut; };
+            surplus_ends<TPB>(place_of, stays, n_new, n, wave_tot, tid, sync);
             const int S_ = n - n_new;
             items = na + S_;
             for (int j = tid; j < S_; j += TPB) {
                 int to = kNone;
-                if (item_idx[na + j] != kOut) {
+                if (stays(j)) {
                     to = place[j];
-                    for (int hop = 0; hop <= S_ && to >= n_new; ++hop) to = place[n - 1 - to];
                     if (writer) idx_out[to] = item_idx[na + j];
                 }
                 item_pos[na + j] = (uint16_t)to;

@@ -133,6 +133,39 @@ def test_surplus_removals(I):
     _check_layout(wc, oc.get_active_indices().tolist(), g, u, d, True)
 
 
+@pytest.mark.parametrize("I,unaligned", [(64, 0), (8192, 0), (8192, 1), (16001, 0), (22000, 0), (28672, 0)])
+def test_surplus_removals_in_one_chain(I, unaligned):
+    """A block of removals leaves the end of the list in descending order; removing index 0 and that end then moves every
+    step's entry to where the next step takes it from again.  With a few additions beside them, and once more behind."""
+    H, k = 8, max(8, I // 4)
+    rng = np.random.default_rng(I)
+    g, u, d = (rng.standard_normal(s).astype(np.float32) for s in ((I, H), (I, H), (H, I)))
+    oc = oracle.OracleWeightCache(np.ones(I, bool), H, g, u, d, True)
+    wc, fused = (st.WeightCache(torch.ones(I, dtype=torch.bool, device=DEV), H, _t(g), _t(u), _t(d), True) for _ in range(2))
+    x = torch.ones(1, H, device=DEV)
+
+    def step(m):
+        oc.update_active_weights(m)
+        buf = torch.zeros(I + unaligned, dtype=torch.bool, device=DEV)[unaligned:]
+        buf.copy_(_t(m, torch.bool))
+        wc.update_active_weights_async(buf)
+        fused.update_and_forward(buf, x)
+        want = oc.get_active_indices().tolist()
+        assert wc.get_active_indices().cpu().tolist() == want and fused.get_active_indices().cpu().tolist() == want
+
+    for added in (0, 3):
+        m = np.ones(I, bool)
+        step(m)
+        m[I // 2:I // 2 + k] = False
+        step(m)
+        m = m.copy()
+        m[0] = False
+        m[oc.get_active_indices()[-k:]] = False
+        m[I // 2:I // 2 + added] = True
+        step(m)
+    _check_layout(wc, oc.get_active_indices().tolist(), g, u, d, True)
+
+
 @pytest.mark.parametrize("I,has_gate", [(28672, True), (32768, False), (22016, True)])
 def test_large_intermediate_sizes(I, has_gate):
     """Intermediate sizes of the 70B-class models (28672), above what the index lists of the smaller kernels allow:
