@@ -862,13 +862,15 @@ template <int TPB>
 __global__ __launch_bounds__(TPB) void cache_update_bytes_kernel(const uint8_t *__restrict__ new_mask,
                                                                  uint8_t *__restrict__ cur_mask2,
                                                                  int32_t *__restrict__ indices2,
-                                                                 int32_t *__restrict__ state, int I, CopyPlan cp)
+                                                                 int32_t *__restrict__ state, int I, CopyPlan cp,
+                                                                 HostWords *host)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ PlanShared ps;
     const int tid = threadIdx.x;
     PlanView pv;
     cache_plan<false, TPB, 1, false>(pv, smem, &ps, new_mask, cur_mask2, indices2, state, I, I, tid, [] {}, [] {});
+    if (tid == 0 && pv.writer) tell_count(host, pv.n_new);
     if (pv.changed) {
         // (the index of a rewritten position, beside the position: the map of the plan is not needed any more)
         for (int i = tid; i < (int)pv.n_changed; i += TPB) pv.pos_l[i] = pv.lists[i] != kNone ? pv.idx_l[pv.lists[i]] : 0;
@@ -1689,7 +1691,8 @@ __device__ __forceinline__ int big_select(const uint32_t *bits, const uint32_t *
 __global__ __launch_bounds__(kBigThreads) void cache_update_big_kernel(const uint8_t *__restrict__ new_mask,
                                                                       uint8_t *__restrict__ cur_mask2,
                                                                       int32_t *__restrict__ indices2,
-                                                                      int32_t *__restrict__ state, int I, FusedRows fr)
+                                                                      int32_t *__restrict__ state, int I, FusedRows fr,
+                                                                      HostWords *host)
 {
     constexpr int TPB = kBigThreads;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -1744,6 +1747,7 @@ __global__ __launch_bounds__(kBigThreads) void cache_update_big_kernel(const uin
             state[ST_STATE_N_CHANGED] = 0;
             state[ST_STATE_N_ADDED] = 0;
             state[ST_STATE_N_REMOVED] = 0;
+            tell_count(host, n);
         }
         if (tid == 0) {
             arrival = atomicAdd(reinterpret_cast<uint32_t *>(&state[ST_STATE_TICKET]), 1u);
@@ -1856,6 +1860,7 @@ __global__ __launch_bounds__(kBigThreads) void cache_update_big_kernel(const uin
             } else {
                 state[ST_STATE_STATUS] = ST_ERR_NO_ACTIVE;
             }
+            tell_count(host, n_new);
         }
     }
     if (tid == 0) arrival = atomicAdd(reinterpret_cast<uint32_t *>(&state[ST_STATE_TICKET]), 1u);
@@ -1925,7 +1930,7 @@ __global__ __launch_bounds__(kBuildThreads) void cache_build_kernel(const uint8_
                                                                     uint8_t *__restrict__ cur_mask2,
                                                                     int32_t *__restrict__ indices2,
                                                                     int32_t *__restrict__ state, int I, int H, int mask_vec,
-                                                                    HostWords *host, int tell, BuildMats a)
+                                                                    HostWords *host, BuildMats a)
 {
     constexpr int kTile = BuildTile<ESZ>::rows, V = 16 / ESZ;
     __shared__ uint32_t wave_tot[kBuildThreads / kWave];
@@ -1966,7 +1971,7 @@ __global__ __launch_bounds__(kBuildThreads) void cache_build_kernel(const uint8_
             w[ST_STATE_VALID] = w[ST_STATE_SERIAL] = w[ST_STATE_EPOCH] = some;
             w[ST_STATE_TICKET] = some << 16;
             for (int k = 0; k < ST_STATE_WORDS; ++k) state[k] = w[k];
-            if (tell) tell_count(host, n);
+            tell_count(host, n);
         }
         for (int w = 0; w < words; ++w) {
             const int e0 = 8 * (tid * words + w);
@@ -2233,15 +2238,13 @@ static int launch_build(st_cache *c, const void *gate, const void *up, const voi
     const int64_t blocks = 1 + (int64_t)a.nrow * ((c->I + kBuildRows - 1) / kBuildRows) +
                            ((c->I + tile - 1) / tile) * ((c->H + tile - 1) / tile);
     ST_REQUIRE(blocks <= 0x7fffffff, "st_cache: hidden size %lld out of range", (long long)c->H);
-    // the count is told where the updates that follow tell theirs (the guess must not stay behind)
-    const int tell = mask != nullptr && c->I <= kPlanMaxI && c->I % 8 == 0;
     const int mask_vec = ((uintptr_t)mask & 7) == 0;
     if (c->esz == 4)
         hipLaunchKernelGGL(cache_build_kernel<4>, dim3((unsigned)blocks), dim3(kBuildThreads), 0, s, mask, c->b.cur_mask,
-                           c->b.indices, c->b.state, (int)c->I, (int)c->H, mask_vec, c->host, tell, a);
+                           c->b.indices, c->b.state, (int)c->I, (int)c->H, mask_vec, c->host, a);
     else
         hipLaunchKernelGGL(cache_build_kernel<2>, dim3((unsigned)blocks), dim3(kBuildThreads), 0, s, mask, c->b.cur_mask,
-                           c->b.indices, c->b.state, (int)c->I, (int)c->H, mask_vec, c->host, tell, a);
+                           c->b.indices, c->b.state, (int)c->I, (int)c->H, mask_vec, c->host, a);
     ST_HIP(hipGetLastError());
     return ST_OK;
 }
@@ -2350,7 +2353,7 @@ static int launch_update(st_cache *const *caches, const uint8_t *const *masks, i
         const int grid = blocks ? blocks : device_cu_count() * 3 / 4;   // (measured against 1/4, 3/8, 1/2 and all of the CUs)
         const size_t lds = update_lds_bytes(I);
         const int idx_cap = update_idx_cap(c);
-        rc = !aligned     ? launch(cache_update_bytes_kernel<1024>, grid, plan_lds_bytes(I), cp)
+        rc = !aligned     ? launch(cache_update_bytes_kernel<1024>, grid, plan_lds_bytes(I), cp, c->host)
              : small      ? launch(cache_update_kernel<512, 3, NoLayers>, grid, lds, idx_cap, cp, c->host, NoLayers{})
              : words == 1 ? launch(cache_update_kernel<1024, 1, NoLayers>, grid, lds, idx_cap, cp, c->host, NoLayers{})
              : words == 2 ? launch(cache_update_kernel<1024, 2, NoLayers>, grid, lds, idx_cap, cp, c->host, NoLayers{})
@@ -2388,7 +2391,7 @@ extern "C" int st_cache_update_async(st_cache *c, const uint8_t *mask, void *str
         }
         ProfScope ps(ST_K_CACHE_UPDATE, s);
         ST_LAUNCH(ps, cache_update_big_kernel, dim3(device_cu_count()), dim3(kBigThreads), lds_big, s, mask,
-                  c->b.cur_mask, c->b.indices, c->b.state, I, fr);
+                  c->b.cur_mask, c->b.indices, c->b.state, I, fr, c->host);
         ST_HIP(hipGetLastError());
         return ST_OK;
     }

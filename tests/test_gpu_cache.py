@@ -434,3 +434,19 @@ def test_host_words_are_shared_and_reused():
             assert c.get_num_active() == 64
         while caches:
             caches.pop(0 if order == 1 else -1)
+
+
+@pytest.mark.parametrize("I,unaligned", [(64, 0), (8192, 1), (2051, 0), (28672, 0), (32768, 0)])
+def test_every_update_tells_its_count(I, unaligned):
+    """The count that launches take as their guess is the last update's in every form of the update, and after construction."""
+    H = 8
+    g, u, d = (torch.randn(*s, device=DEV) for s in ((I, H), (I, H), (H, I)))
+    masks = [torch.rand(I, device=DEV) < f for f in (0.5, 0.3, 0.3, 0.8)]
+    masks.append(masks[-1].clone())   # an unchanged mask
+    wc = st.WeightCache(masks[0], H, g, u, d, True)
+    assert wc._seen.value == int(masks[0].sum())
+    for m in masks[1:]:
+        buf = torch.zeros(I + unaligned, dtype=torch.bool, device=DEV)[unaligned:]
+        wc._seen.value = -1
+        wc.update_active_weights(buf.copy_(m))
+        assert wc._seen.value == int(m.sum())
