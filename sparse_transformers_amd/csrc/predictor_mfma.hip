@@ -5,19 +5,20 @@
 //   kernel 2  s[b,i] = <t[b,:], Bm[i,:]>    a wave keeps its rows of t in registers and walks over rows of Bm;
 //             mask[i] = 1 where any s[b,i] passes the cut (only ones are stored)
 //
-// The rank-r intermediate is fp32, and the matrix cores multiply 16-bit operands: kernel 2 splits t into parts of the
-// storage type that sum to it -- two fp16 parts or three bf16 parts, each rounding what the parts before it left over.
-// What is lost is below 2^-24 of t, half an ulp of fp32 (rows of fp16 parts are scaled by a power of two that puts their
-// largest element near 2^14, so that neither overflow nor the subnormals matter): the scores keep fp32 accuracy.
+// The rank-r intermediate is fp32, and the matrix cores multiply 16-bit operands: kernel 2 splits t into three parts of the
+// storage type that sum to it, each rounding what the parts before it left over.  Three parts hold all 24 bits (two of fp16
+// hold 23, which a quarter of all values exceed).  Rows of fp16 parts are scaled by a power of two that puts their largest
+// element near 2^14; only of elements below 2^-15 of that one something may be lost to the subnormals, less than 2^-38 of
+// the largest.  In kernel 2 every product is exact and the sums are fp32: the scores keep fp32 accuracy.
 //
 // Same contract as predictor.hip (src/modeling_skip.py:52-53,204-207,214).
 #include "st_mfma.h"
 
+#include <type_traits>
+
 namespace st {
 
-template <typename T> struct SplitParts;
-template <> struct SplitParts<f16_t> { static constexpr int value = 2; };
-template <> struct SplitParts<bf16_t> { static constexpr int value = 3; };
+constexpr int kSplitParts = 3;
 
 // ---------------------------------------------------------------------------
 // kernel 1
@@ -141,12 +142,12 @@ constexpr float kMaxF32 = 3.402823466e+38f;
 template <typename T> __device__ __forceinline__ void split_parts(const float *v, uint4 *parts);
 template <> __device__ __forceinline__ void split_parts<bf16_t>(const float *v, uint4 *parts)
 {
-    bf16x8_t w[3];
+    bf16x8_t w[kSplitParts];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
         float rest = v[k];
 #pragma unroll
-        for (int p = 0; p < 3; ++p) {
+        for (int p = 0; p < kSplitParts; ++p) {
             __bf16 b = (__bf16)rest;                // (the hardware's conversion: round to nearest even)
             if (p == 0 && fabsf(rest) <= kMaxF32 && fabsf((float)b) > kMaxF32)   // a finite value stays finite
                 b = __builtin_bit_cast(__bf16, (uint16_t)(rest > 0.f ? 0x7f7f : 0xff7f));
@@ -156,20 +157,24 @@ template <> __device__ __forceinline__ void split_parts<bf16_t>(const float *v, 
         }
     }
 #pragma unroll
-    for (int p = 0; p < 3; ++p) parts[p] = __builtin_bit_cast(uint4, w[p]);
+    for (int p = 0; p < kSplitParts; ++p) parts[p] = __builtin_bit_cast(uint4, w[p]);
 }
 template <> __device__ __forceinline__ void split_parts<f16_t>(const float *v, uint4 *parts)
 {
-    uint32_t w[2][8];
+    uint32_t w[kSplitParts][8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-        const f16_t hi = from_float<f16_t>(v[k]);
-        const float left = v[k] - to_float<f16_t>(hi);
-        w[0][k] = hi.bits;
-        w[1][k] = from_float<f16_t>(left == left ? left : 0.f).bits;   // (infinity or NaN: nothing left over)
+        float rest = v[k];
+#pragma unroll
+        for (int p = 0; p < kSplitParts; ++p) {
+            const f16_t h = from_float<f16_t>(rest);
+            w[p][k] = h.bits;
+            rest -= to_float<f16_t>(h);
+            if (p == 0) rest = rest == rest ? rest : 0.f;   // an infinity or NaN has nothing left over
+        }
     }
 #pragma unroll
-    for (int p = 0; p < 2; ++p)
+    for (int p = 0; p < kSplitParts; ++p)
         parts[p] = make_uint4(w[p][0] | (w[p][1] << 16), w[p][2] | (w[p][3] << 16), w[p][4] | (w[p][5] << 16),
                               w[p][6] | (w[p][7] << 16));
 }
@@ -199,7 +204,8 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
         flags = (flags & ~1) | (ly.cmp_ge ? 1 : 0);
         t += (size_t)blockIdx.y * B * r;
     }
-    constexpr int P = SplitParts<T>::value;
+    constexpr int P = kSplitParts;
+    constexpr bool kScaled = std::is_same<T, f16_t>::value;
     constexpr int kRow = 4 * KS, kBuf = kPmStage * kRow;      // 16-byte chunks
     constexpr int kDma = kBuf / 64 / W;                       // 1 KB loads per wave and stage
     extern __shared__ __align__(16) uint4 lds[];              // two buffers, then a byte per index of the block
@@ -249,7 +255,7 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) unscale[i][e] = 1.f;
-        if constexpr (P == 2) {
+        if constexpr (kScaled) {
             // a power of two per row that puts its largest finite element near 2^14
             float big = 0.f;
 #pragma unroll
@@ -328,7 +334,7 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
                     // An infinite element of Bm decides the score by the sign of t, which its first part has; the others are
                     // zero or of either sign and would make a NaN of it.
                     v = fabsf(acc[i][0][e]) <= kMaxF32 ? v : acc[i][0][e];
-                    if constexpr (P == 2) v *= unscale[i][e];
+                    if constexpr (kScaled) v *= unscale[i][e];
                     if (round_storage) v = to_float<T>(from_float<T>(v));
                     const bool in = (live >> (4 * i + e)) & 1u;
                     any = any || (in && (cmp_ge ? v >= thr : v > thr));

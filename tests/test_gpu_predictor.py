@@ -55,7 +55,7 @@ def test_scores_and_mask(B, H, r, I, dtype, frac):
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("B,H,r,I", [
-    (8, 64, 8, 17),          # one tile of everything, none of them full
+    (9, 64, 8, 17),          # one tile of everything, none of them full; the fewest rows these kernels take
     (16, 72, 40, 50),        # H is not a multiple of a k step
     (17, 1024, 128, 2048),   # one row into the second tile of rows
     (33, 512, 136, 1000),    # ranks one chunk into the next register form: 128, 256, 384
@@ -83,6 +83,22 @@ def test_matrix_core_predictor(B, H, r, I, dtype):
         assert np.array_equal(got[~near], oracle.mask_threshold(s_ref, thr, ge)[~near])
     assert near.mean() < 0.01 + 2.0 / I
     assert np.array_equal(m.cpu().numpy(), (s.cpu().numpy() >= 0).any(0))   # mask and scores come from the same sums
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("B,H,r", [(9, 64, 8), (40, 3072, 128), (100, 512, 392)])
+def test_matrix_core_predictor_keeps_every_bit_of_the_intermediate(dtype, B, H, r):
+    """With a unit matrix as the second map the scores are the fp32 intermediate, all 24 bits of it: 16-bit parts of it that
+    sum to less would show.  (fp16 parts reach down to 2^-24 on a scale where a row's largest element is at least 2^13: what
+    lies below that, at most 2^-25 of 2^13, may be lost.)"""
+    x, A, _ = _weights(B, B, H, r, r, dtype)
+    t_ws = torch.empty(B, r, dtype=torch.float32, device=DEV)
+    _, s = st.predictor_mask(x.to(DEV), A.to(DEV), torch.eye(r, dtype=x.dtype, device=DEV), 0.0, True, t_ws=t_ws,
+                             return_scores=True)
+    want = x.double() @ A.double().t()                               # (and the intermediate is the first map's)
+    assert (t_ws.cpu() - want).abs().max() <= 2e-6 * want.abs().max()
+    lost = 2.0 ** -38 * t_ws.abs().amax(1, keepdim=True) if dtype == "float16" else 0.0
+    assert ((s - t_ws).abs() <= lost).all(), ((s != t_ws).float().mean(), ((s - t_ws) / t_ws).abs().max())
 
 
 def test_matrix_core_predictor_reads_beyond_4_gib():
