@@ -320,16 +320,19 @@ class SparseMLPStack:
 
     def _batched(self) -> bool:
         """True when the stack's layers can share launches: equal shapes and threshold masks, every layer with a cache and
-        a mask of its own."""
+        a mask of its own, predictors whose weights (which may have been replaced since) the kernels can read in place."""
         ls = self.layers
         c0, p0 = ls[0].cache, ls[0].predictor
 
         def like_first(layer):
             c, p = layer.cache, layer.predictor
-            return (layer.method in ("naive", "threshold") and c.hidden_size == c0.hidden_size
+            return (type(layer) is SparseDecodeLayer and type(p) is FastLoRAProjection
+                    and layer.method in ("naive", "threshold") and c.hidden_size == c0.hidden_size
                     and c.intermediate_size == c0.intermediate_size and c.dtype == c0.dtype and c.device == c0.device
-                    and p.lora_size == p0.lora_size and p.round_to_storage == p0.round_to_storage
-                    and p.down_weight.dtype == c0.dtype and p.up_weight.dtype == c0.dtype)
+                    and p.round_to_storage == p0.round_to_storage
+                    and p.down_weight.shape == p0.down_weight.shape and p.up_weight.shape == p0.up_weight.shape
+                    and p.down_weight.dtype == c0.dtype and p.up_weight.dtype == c0.dtype
+                    and p.down_weight.is_contiguous() and p.up_weight.is_contiguous())
         least = self._shared_launch_layers if self.x_stage.size(0) <= 2 else 2
         return (len(ls) >= least and all(map(like_first, ls))
                 and len({id(layer.cache) for layer in ls}) == len(ls) and len({layer.mask.data_ptr() for layer in ls}) == len(ls))

@@ -133,6 +133,37 @@ def test_staged_step_shares_launches_between_layers(dtype, L, H, I, r, B, trace_
         assert torch.equal(ya, yb), t
 
 
+def test_staged_step_takes_predictors_replaced_after_construction():
+    """Weights that are no longer contiguous, of another rank, and a predictor with a mask of its own: the staged step goes
+    layer by layer for them, as an eager step does."""
+    class Inverted(st.FastLoRAProjection):
+        def mask(self, x, *args, out=None, **kw):
+            return torch.logical_not(super().mask(x, *args, out=out, **kw), out=out)
+
+    L, H, I, r = 4, 128, 320, 16
+    gen = torch.Generator(device=DEV).manual_seed(2)
+    for kind in ("strided", "rank", "subclass"):
+        a, _ = _build("float16", L, H, I, r, seed=5)
+        b, _ = _build("float16", L, H, I, r, seed=5)
+        for s in (a, b):
+            s.prepare(1, fused=s is a)
+            s.use_trace_masks = False
+            p = s.layers[2].predictor
+            if kind == "strided":
+                p.down_weight = p.down_weight.t().contiguous().t()
+            elif kind == "rank":
+                p.down_weight, p.up_weight = p.down_weight[:8].contiguous(), p.up_weight[:, :8].contiguous()
+            else:
+                s.layers[2].predictor = Inverted(p.down_weight, p.up_weight)
+        assert not a._batched()
+        for t in range(3):
+            x, xp = torch.randn(1, H, device=DEV, generator=gen).half(), torch.randn(L, 1, H, device=DEV, generator=gen).half()
+            ya, yb = a.step_staged(x, xp).clone(), b.step_staged(x, xp).clone()
+            for la, lb in zip(a.layers, b.layers):
+                assert torch.equal(la.mask, lb.mask), (kind, t)
+            assert torch.equal(ya, yb), (kind, t)
+
+
 def test_skip_mlp_module_surface():
     """SkipMLP mirrors the reference module (src/modeling_skip.py:55-128): constructor arguments, sub-modules,
     registered buffers, state-dict keys, initialize_weight_cache / reset_cache, the three forwards."""
