@@ -224,20 +224,17 @@ __device__ __forceinline__ void surplus_ends(P place, Q stays, int base, int n, 
 // contains block barriers.  VEC: I % 8 == 0 and the mask is
 // 8-byte aligned, so masks are read as 8-byte words and indices as 16-byte vectors; both bookkeeping
 // buffers are requested together with the ticket, so the front costs one memory round trip.  MARK: the
-// dirty bitmap is kept on the fast path too.  `after_issue()` runs right after the front loads have
-// been issued, `after_fill()` right after the first barrier (the front loads have arrived and been consumed).
+// dirty bitmap is kept on the fast path too.
 // NW: 8-element words per thread of the vector path (I <= 8 NW threads); the registers of the front loads follow from it.
-// idx_cap: only that many positions of the index lists are fetched up front (the rest follows if the count
-// turns out larger).
 //
 // Barrier sequence: 1 after the LDS fill; 2 in the diff scan;
 // [unchanged mask: done]; 1 after the lists; 1 after phases 1 and 2; [surplus removals: those of surplus_count and surplus_ends and 1
 // behind it, 2 in the compaction scan, 1 after the compaction].
-template <bool VEC, int PT, int NW, bool MARK, typename F, typename F2>
+template <bool VEC, int PT, int NW, bool MARK>
 __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, PlanShared *ps,
                                            const uint8_t *__restrict__ new_mask, uint8_t *__restrict__ cur_mask2,
                                            int32_t *__restrict__ indices2, int32_t *__restrict__ state, int I,
-                                           const int idx_cap, const int tid, F after_issue, F2 after_fill)
+                                           const int tid)
 {
     constexpr int TPB = PT;
     uint16_t *pos_l = reinterpret_cast<uint16_t *>(smem);  // index -> position
@@ -280,18 +277,15 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
                 v_new[w] = *reinterpret_cast<const uint64_t *>(new_mask + e);
                 v_cur0[w] = *reinterpret_cast<const uint64_t *>(cur_mask2 + e);
                 v_cur1[w] = *reinterpret_cast<const uint64_t *>(cur_mask2 + (size_t)I + e);
-                if (e < idx_cap) {   // positions the caller expects to be in use (a multiple of 8, or all)
-                    v_i0a[w] = *reinterpret_cast<const int4 *>(indices2 + e);
-                    v_i0b[w] = *reinterpret_cast<const int4 *>(indices2 + e + 4);
-                    v_i1a[w] = *reinterpret_cast<const int4 *>(indices2 + (size_t)I + e);
-                    v_i1b[w] = *reinterpret_cast<const int4 *>(indices2 + (size_t)I + e + 4);
-                }
+                v_i0a[w] = *reinterpret_cast<const int4 *>(indices2 + e);
+                v_i0b[w] = *reinterpret_cast<const int4 *>(indices2 + e + 4);
+                v_i1a[w] = *reinterpret_cast<const int4 *>(indices2 + (size_t)I + e);
+                v_i1b[w] = *reinterpret_cast<const int4 *>(indices2 + (size_t)I + e + 4);
             }
         }
         n_both[0] = state[ST_STATE_N_BUF0];
         n_both[1] = state[ST_STATE_N_BUF1];
     }
-    after_issue();
     for (int w = tid; w < dirty_words; w += TPB) dirty[w] = 0u;
     const int ep = (int)((tword >> 16) & 1u);
     const bool writer = blockIdx.x == 0;
@@ -309,15 +303,13 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
             if (e < e1) {
                 w_new[w] = nonzero_bytes(v_new[w]);
                 w_cur[w] = nonzero_bytes(ep ? v_cur1[w] : v_cur0[w]);
-                if (e < idx_cap) {
-                    const int4 a = ep ? v_i1a[w] : v_i0a[w], b4 = ep ? v_i1b[w] : v_i0b[w];
-                    uint4 packed;
-                    packed.x = (uint32_t)(a.x & 0xffff) | ((uint32_t)a.y << 16);
-                    packed.y = (uint32_t)(a.z & 0xffff) | ((uint32_t)a.w << 16);
-                    packed.z = (uint32_t)(b4.x & 0xffff) | ((uint32_t)b4.y << 16);
-                    packed.w = (uint32_t)(b4.z & 0xffff) | ((uint32_t)b4.w << 16);
-                    *reinterpret_cast<uint4 *>(idx_l + e) = packed;
-                }
+                const int4 a = ep ? v_i1a[w] : v_i0a[w], b4 = ep ? v_i1b[w] : v_i0b[w];
+                uint4 packed;
+                packed.x = (uint32_t)(a.x & 0xffff) | ((uint32_t)a.y << 16);
+                packed.y = (uint32_t)(a.z & 0xffff) | ((uint32_t)a.w << 16);
+                packed.z = (uint32_t)(b4.x & 0xffff) | ((uint32_t)b4.y << 16);
+                packed.w = (uint32_t)(b4.z & 0xffff) | ((uint32_t)b4.w << 16);
+                *reinterpret_cast<uint4 *>(idx_l + e) = packed;
                 *reinterpret_cast<uint4 *>(pos_l + e) = make_uint4(0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu);
             }
         }
@@ -333,13 +325,7 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
     }
     ST_TL(1);
     sync();
-    after_fill();
     ST_TL(2);
-    if (VEC && n > idx_cap) {   // more positions in use than the caller expected: fetch the rest (one more round trip)
-        const int32_t *indices = indices2 + (size_t)ep * I;
-        for (int p = idx_cap + tid; p < n; p += TPB) idx_l[p] = (uint16_t)indices[p];
-        sync();
-    }
     for (int p = tid; p < n; p += TPB) pos_l[idx_l[p]] = (uint16_t)p;
 
     // ---- diff: contiguous element range per thread keeps the lists ascending
@@ -869,7 +855,7 @@ __global__ __launch_bounds__(TPB) void cache_update_bytes_kernel(const uint8_t *
     __shared__ PlanShared ps;
     const int tid = threadIdx.x;
     PlanView pv;
-    cache_plan<false, TPB, 1, false>(pv, smem, &ps, new_mask, cur_mask2, indices2, state, I, I, tid, [] {}, [] {});
+    cache_plan<false, TPB, 1, false>(pv, smem, &ps, new_mask, cur_mask2, indices2, state, I, tid);
     if (tid == 0 && pv.writer) tell_count(host, pv.n_new);
     if (pv.changed) {
         // (the index of a rewritten position, beside the position: the map of the plan is not needed any more)
@@ -1490,8 +1476,7 @@ __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
     } else {
         // ---- too many surplus removals for the replay above: the per-index plan
         PlanView pv;
-        cache_plan<true, TPB, NW, true>(pv, smem, &plan_shared, new_mask, cur_mask2, indices2, state, I, I, tid,
-                                           [] {}, [] {});
+        cache_plan<true, TPB, NW, true>(pv, smem, &plan_shared, new_mask, cur_mask2, indices2, state, I, tid);
         n = pv.n_new;
         if (plan_wave) {
             int s = -1;

@@ -68,7 +68,7 @@ def mlp_workspace_bytes(B: int, H: int, n: int, dtype: Optional[torch.dtype] = N
     return int(_lib.lib().st_mlp_workspace_bytes(B, H, n))
 
 
-def mlp_workspace(device: torch.device, B: int, H: int, n: int, dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+def _kept_workspace(device: torch.device, need: int) -> torch.Tensor:
     """Scratch for one forward on the current stream of ``device``.
 
     One list of buffers per (device, stream): two streams never share scratch, and a buffer that has been
@@ -76,10 +76,6 @@ def mlp_workspace(device: torch.device, B: int, H: int, n: int, dtype: Optional[
     baked in, so growing must not free it.  Callers that replay graphs or know their largest batch should
     own a buffer instead (``torch.empty(mlp_workspace_bytes(B, H, I), dtype=torch.uint8)``) and pass it as
     ``workspace=``."""
-    return _kept_workspace(device, mlp_workspace_bytes(B, H, n, dtype))
-
-
-def _kept_workspace(device: torch.device, need: int) -> torch.Tensor:
     bufs = _workspaces.setdefault((_device_index(device), current_stream_ptr(device)), [])
     if not bufs or bufs[-1].numel() < need:
         grow = max(need, 2 * bufs[-1].numel() if bufs else 0)
