@@ -110,7 +110,7 @@ __global__ __launch_bounds__(W * kWave) void predictor_down_mfma_kernel(const T 
                 for (int j = 0; j < NI; ++j) acc[i][j] = Mfma<T>::run(fa[i], fb[j], acc[i][j]);
         }
     }
-    // (the sums go over the waves' own buffers, which nobody reads any more)
+    // (the sums lie over the front of the buffers, the first waves': behind the barrier nobody reads those any more)
     typedef float Red[MI * NI][256];
     Red *red = reinterpret_cast<Red *>(lds);
     static_assert(sizeof(Red) <= 2 * kBuf * 16, "a wave's sums exceed its buffers");

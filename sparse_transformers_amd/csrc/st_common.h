@@ -272,7 +272,7 @@ int launch_batch(int dtype, const void *x, int B, int H, const void *gate, const
 
 // Several layers of equal shape in one launch: grid dimension y is the layer, whose pointers come from a table passed by
 // value (as the last argument; NoLayers takes its place in the single-layer kernels).
-constexpr int kMaxLayers = 32;   // of one launch: the largest table (80 bytes a layer) fits the 4 KB of kernel arguments
+constexpr int kMaxLayers = 32;   // of one launch: the largest table (88 bytes a layer) fits the 4 KB of kernel arguments
 struct NoLayers { static constexpr bool kLayers = false; };
 struct PredLayers {
     static constexpr bool kLayers = true;

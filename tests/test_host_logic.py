@@ -200,6 +200,60 @@ def test_surplus_removal_closed_form():
         assert closed_form(order, list(drop)) == oc.get_active_indices().tolist(), trial
 
 
+def test_surplus_removal_paths():
+    """The form of the surplus removals in the stand-alone update kernels, against the reference's sequential rule
+    (weight_cache.h:310-353): every tail slot is joined to the slot its step's index starts in, and an entry of the tail
+    that stays goes to the end of the path that begins at its slot.  All slots move along at once, in any interleaving,
+    four links at a time and through what others have reached: few rounds, also for one path through all of them."""
+    rng = np.random.default_rng(5)
+
+    def sequential(order, surplus):
+        lst = list(order)
+        pos = {e: p for p, e in enumerate(lst)}
+        for e in surplus:
+            p = pos.pop(e)
+            if p != len(lst) - 1:
+                lst[p] = lst[-1]
+                pos[lst[p]] = p
+            lst.pop()
+        return lst
+
+    def paths(order, surplus):
+        n, S = len(order), len(surplus)
+        base, pos, gone = n - S, {e: p for p, e in enumerate(order)}, set(surplus)
+        place = [pos[e] for e in surplus]
+        stays = [order[n - 1 - k] not in gone for k in range(S)]
+        rounds = 0
+        while any(s and p >= base for s, p in zip(stays, place)):
+            rounds += 1
+            for k in rng.permutation(S):
+                q = place[k]
+                for _ in range(4):
+                    q = place[n - 1 - q] if q >= base else q
+                place[k] = q
+        out = list(order[:base])
+        for k in range(S):
+            if stays[k]:
+                assert place[k] < base
+                out[place[k]] = order[n - 1 - k]
+        return out, rounds
+
+    for trial in range(3000):
+        n = int(rng.integers(2, 48))
+        order = rng.permutation(64)[:n].tolist()
+        if trial % 4 == 0:
+            order.sort(reverse=trial % 8 == 0)
+        surplus = sorted(rng.choice(order, int(rng.integers(1, n)), replace=False).tolist())
+        out, rounds = paths(order, surplus)
+        assert out == sequential(order, surplus), (trial, order, surplus)
+        assert rounds <= 3
+    for n, cut in ((64, 16), (8192, 2000), (22000, 5500)):     # a descending end of the list, removed with index 0
+        order = sequential(list(range(n)), list(range(n // 2, n // 2 + cut)))
+        surplus = sorted([0] + order[-cut:])
+        out, rounds = paths(order, surplus)
+        assert out == sequential(order, surplus) and rounds <= 7
+
+
 def test_surplus_removal_tail_only_form():
     """The form of the surplus removals that one wave of the fused update + decode kernel works out from the tail of
     the list alone (S surplus indices: the last S entries), against the reference's sequential rule
