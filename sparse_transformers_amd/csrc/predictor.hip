@@ -237,7 +237,6 @@ __global__ __launch_bounds__(kPredUpThreads) void predictor_up_mask_rows_kernel(
     const int chunks = r / VEC;
     const int cl = lane & (LPR - 1), gidx = lane / LPR;
     const int tile = (blockIdx.x * (kPredUpThreads / kWave) + wave) * (RPI * NITER);
-    const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
     const bool has_chunk = cl < chunks;
 
     uint4 w[NITER];
@@ -245,7 +244,6 @@ __global__ __launch_bounds__(kPredUpThreads) void predictor_up_mask_rows_kernel(
     for (int it = 0; it < NITER; ++it) {
         const int row = tile + it * RPI + gidx;
         w[it] = ld16(Bm + (size_t)(row < I ? row : I - 1) * r + (size_t)(has_chunk ? cl : 0) * VEC);
-        if (!has_chunk) w[it] = zero4;
     }
     {   // stage t: 16-byte pieces, two per thread requested together (the buffer is padded to whole batches)
         const float4 *t4 = reinterpret_cast<const float4 *>(t);
@@ -279,14 +277,15 @@ __global__ __launch_bounds__(kPredUpThreads) void predictor_up_mask_rows_kernel(
         for (int it = 0; it < NITER; ++it) {
             const int row = tile + it * RPI + gidx;
             float fw[VEC];
-            unpack<T>(w[it], fw);   // zeros in lanes without a chunk
+            unpack<T>(w[it], fw);
 #pragma unroll
             for (int b = 0; b < kPredUpBTile; ++b) {
                 if (b0 + b < B) {   // uniform
                     float acc = 0.f;
 #pragma unroll
                     for (int e = 0; e < VEC; ++e) acc = fmaf(fw[e], tr[b][e], acc);
-                    float v = group_sum_dpp<LPR>(acc);
+                    // (lanes without a chunk multiplied the first one: not by zero weights, which an infinity makes NaN of)
+                    float v = group_sum_dpp<LPR>(has_chunk ? acc : 0.f);
                     if (round_storage) v = to_float<T>(from_float<T>(v));
                     if (cmp_ge ? (v >= thr) : (v > thr)) any |= 1u << it;
                     if (scores && cl == 0 && row < I) scores[(size_t)(b0 + b) * I + row] = v;

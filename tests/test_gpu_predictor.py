@@ -162,6 +162,22 @@ def test_matrix_core_predictor_infinities_and_nan(dtype, where, round_to_storage
     assert torch.equal(m[~near.any(0)], (few >= 0.5).any(0)[~near.any(0)])
 
 
+@pytest.mark.parametrize("dtype,r", [("float32", 12), ("float16", 40), ("bfloat16", 72), ("float16", 512), ("float32", 264)])
+@pytest.mark.parametrize("B", [1, 2, 8])
+def test_infinite_intermediate_decides_by_sign(dtype, r, B):
+    """Ranks that leave lanes of a group without a part of the row: an infinity at either end of the intermediate gives
+    infinities of the weights' signs, not NaN."""
+    H, I = 64, 200
+    x, A, Bm = (t.to(DEV) for t in _weights(r, B, H, r, I, dtype))
+    x[:, 3] = 1.0
+    for at in (0, 7, r - 1):
+        Ai = A.clone()
+        Ai[at, 3] = float("inf")
+        m, s = st.predictor_mask(x, Ai, Bm, 0.0, True, return_scores=True)
+        assert torch.equal(s, torch.where(Bm[:, at] > 0, float("inf"), -float("inf")).expand(B, I)), (at, s[0, :4])
+        assert torch.equal(m, Bm[:, at] > 0)
+
+
 def test_naive_threshold_is_score_ge_zero():
     x, A, Bm = _weights(1, 2, 256, 16, 512, "float32")
     # make some scores exactly zero: a zero row of Bm gives score 0 for every input row
