@@ -6,7 +6,7 @@
 //             mask[i] = 1 where any s[b,i] passes the cut (only ones are stored)
 //
 // The rank-r intermediate is fp32, and the matrix cores multiply 16-bit operands: kernel 2 splits t into three parts of the
-// storage type that sum to it, each rounding what the parts before it left over.  Three parts hold all 24 bits (two of fp16
+// storage type that sum to it, each made of what the parts before it left over.  Three parts hold all 24 bits (two of fp16
 // hold 23, which a quarter of all values exceed).  Rows of fp16 parts are scaled by a power of two that puts their largest
 // element near 2^14; only of elements below 2^-15 of that one something may be lost to the subnormals, less than 2^-38 of
 // the largest.  In kernel 2 every product is exact and the sums are fp32: the scores keep fp32 accuracy.
@@ -138,45 +138,49 @@ __global__ __launch_bounds__(W * kWave) void predictor_down_mfma_kernel(const T 
 // ---------------------------------------------------------------------------
 constexpr float kMaxF32 = 3.402823466e+38f;
 
-// Eight floats of t -> the parts of one A operand register quad each.
-template <typename T> __device__ __forceinline__ void split_parts(const float *v, uint4 *parts);
-template <> __device__ __forceinline__ void split_parts<bf16_t>(const float *v, uint4 *parts)
+// Eight floats of t -> the parts of one A operand register quad each.  TINY (fp16): some are too small for a first part.
+template <typename T, bool TINY> __device__ __forceinline__ void split_parts(const float *v, uint4 *parts)
 {
-    bf16x8_t w[kSplitParts];
+    if constexpr (std::is_same<T, bf16_t>::value) {
+        // The first part is the upper half of the float: no finite value becomes an infinity (rounding it did, above
+        // 3.396e38), and what it leaves over has 16 bits, which two rounded parts hold.
+        uint32_t hi[4];
+        bf16x8_t w[kSplitParts - 1];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        float rest = v[k];
+        for (int k = 0; k < 8; ++k) {
+            float rest = v[k] - __uint_as_float(__float_as_uint(v[k]) & 0xffff0000u);
+            rest = rest == rest ? rest : 0.f;           // an infinity or NaN has nothing left over
 #pragma unroll
-        for (int p = 0; p < kSplitParts; ++p) {
-            __bf16 b = (__bf16)rest;                // (the hardware's conversion: round to nearest even)
-            if (p == 0 && fabsf(rest) <= kMaxF32 && fabsf((float)b) > kMaxF32)   // a finite value stays finite
-                b = __builtin_bit_cast(__bf16, (uint16_t)(rest > 0.f ? 0x7f7f : 0xff7f));
-            w[p][k] = b;
-            rest -= (float)b;
-            if (p == 0) rest = fabsf(rest) <= kMaxF32 ? rest : 0.f;   // an infinity or NaN has nothing left over
+            for (int p = 0; p < kSplitParts - 1; ++p) {
+                const __bf16 b = (__bf16)rest;          // (the hardware's conversion: round to nearest even)
+                w[p][k] = b;
+                rest -= (float)b;
+            }
+            if (k & 1) hi[k >> 1] = __builtin_amdgcn_perm(__float_as_uint(v[k]), __float_as_uint(v[k - 1]), 0x07060302u);
         }
-    }
+        parts[0] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
 #pragma unroll
-    for (int p = 0; p < kSplitParts; ++p) parts[p] = __builtin_bit_cast(uint4, w[p]);
-}
-template <> __device__ __forceinline__ void split_parts<f16_t>(const float *v, uint4 *parts)
-{
-    uint32_t w[kSplitParts][8];
+        for (int p = 1; p < kSplitParts; ++p) parts[p] = __builtin_bit_cast(uint4, w[p - 1]);
+    } else {
+        uint32_t w[kSplitParts][8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        float rest = v[k];
+        for (int k = 0; k < 8; ++k) {
+            float rest = v[k];
 #pragma unroll
-        for (int p = 0; p < kSplitParts; ++p) {
-            const f16_t h = from_float<f16_t>(rest);
-            w[p][k] = h.bits;
-            rest -= to_float<f16_t>(h);
-            if (p == 0) rest = rest == rest ? rest : 0.f;   // an infinity or NaN has nothing left over
+            for (int p = 0; p < kSplitParts; ++p) {
+                f16_t h = from_float<f16_t>(rest);
+                // (the first part keeps the sign of what is too small for it: it decides what an infinite weight gives)
+                if (TINY && p == 0 && (h.bits & 0x7fffu) == 0u && rest != 0.f) h.bits |= 1u;
+                w[p][k] = h.bits;
+                rest -= to_float<f16_t>(h);
+                if (p == 0) rest = rest == rest ? rest : 0.f;   // an infinity or NaN has nothing left over
+            }
         }
-    }
 #pragma unroll
-    for (int p = 0; p < kSplitParts; ++p)
-        parts[p] = make_uint4(w[p][0] | (w[p][1] << 16), w[p][2] | (w[p][3] << 16), w[p][4] | (w[p][5] << 16),
-                              w[p][6] | (w[p][7] << 16));
+        for (int p = 0; p < kSplitParts; ++p)
+            parts[p] = make_uint4(w[p][0] | (w[p][1] << 16), w[p][2] | (w[p][3] << 16), w[p][4] | (w[p][5] << 16),
+                                  w[p][6] | (w[p][7] << 16));
+    }
 }
 
 // A wave owns 16 MI rows of t (KS k steps of 32 of the rank, in registers as parts) and walks over rows of Bm, which the
@@ -278,12 +282,29 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
 #pragma unroll
             for (int e = 0; e < 4; ++e) unscale[i][e] = __shfl(back, 4 * q + e, kWave);
         }
+        auto split = [&](auto tiny) __attribute__((always_inline)) {
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            uint4 parts[P];
-            split_parts<T>(v[ks], parts);
+            for (int ks = 0; ks < KS; ++ks) {
+                uint4 parts[P];
+                split_parts<T, decltype(tiny)::value>(v[ks], parts);
 #pragma unroll
-            for (int p = 0; p < P; ++p) tf[i][p][ks] = parts[p];
+                for (int p = 0; p < P; ++p) tf[i][p][ks] = parts[p];
+            }
+        };
+        if constexpr (kScaled) {
+            // elements of up to 2^-25 that are not zero have no first part (the smallest of them all, zeros last)
+            uint32_t least = ~0u;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const uint32_t m = (__float_as_uint(v[ks][e]) << 1) - 1u;
+                    least = m < least ? m : least;
+                }
+            if (__builtin_amdgcn_ballot_w64(least < (uint32_t)(127 - 25) << 24) != 0) split(std::true_type{});
+            else split(std::false_type{});
+        } else {
+            split(std::false_type{});
         }
     }
     // rows of t beyond B only exist in the last tiles: their scores do not count

@@ -152,6 +152,8 @@ def test_matrix_core_predictor_infinities_and_nan(dtype, where, round_to_storage
         Bm[8], Bm[9, 39] = 0.0, big
         A[3] = 0.0
         Bm[11, 3] = inf                                          # meets t = 0
+        A[0, 0], A[38], x[15] = 6e4, 0.0, 0.0                    # meets an element 2^-60 of its row's largest one
+        x[15, 0], x[15, 1], A[38, 1], Bm[12, 38] = 6e4, 2.0 ** -14, 2.0 ** -14, inf
     few = torch.cat([st.predictor_scores(x[b:b + 8].contiguous(), A, Bm, round_to_storage) for b in range(0, B, 8)])
     m, s = st.predictor_mask(x, A, Bm, 0.5, True, return_scores=True, round_to_storage=round_to_storage)
     for kind in (torch.isnan, torch.isposinf, torch.isneginf):
