@@ -305,6 +305,40 @@ def test_prefill_tiles_follow_the_device_count(M, n):
     assert_close(comb[:, :n].float().cpu().numpy(), h.cpu().numpy(), "float16", f"intermediate, {M} rows, {n} active")
 
 
+@pytest.mark.parametrize("M,H,I,n,gated", [
+    # 256-row tiles of x by 128 (gated) or 256 active rows: t of them; rest = t modulo the CUs (256)
+    (1030, 384, 8192, 3000, True),     # t = 120: all halved
+    (1030, 384, 8192, 3201, True),     # t = 130: all big, the last row tile of x nearly empty
+    (1030, 128, 8192, 6527, True),     # t = 255; two K stages
+    (1030, 256, 8192, 6529, True),     # t = 260: 256 big, 4 halved
+    (1030, 256, 8192, 8192, True),     # t = 320: 256 big, 64 halved
+    (2030, 256, 8448, 8200, False),    # t = 264: 256 big, 8 halved, of which the second halves are past the padded count
+    (2030, 384, 8448, 8447, False),    # the same with both halves
+    (2030, 128, 8448, 4000, False),    # t = 128: all halved
+    (2030, 640, 8448, 4200, False),    # t = 136: all big
+])
+def test_prefill_big_tiles(M, H, I, n, gated):
+    """The 256 x 256 tiles of the gate / up kernel and the halves of those that do not fill a round of CUs: every element of
+    the output and of the intermediate, rows past the device's count NaN.  Bounds as in the tests above (fp32 sums of the
+    same fp16 operands, a rounding of the intermediate and of the output)."""
+    g = torch.Generator().manual_seed(n)
+    gate, up, dn = ((torch.randn(I, H, generator=g) * 0.05).half().to(DEV) for _ in range(3))
+    x = torch.randn(M, H, generator=g).half().to(DEV)
+    h = torch.nn.functional.silu((x.float() @ (gate if gated else up)[:n].float().t()))
+    if gated:
+        h = h * (x.float() @ up[:n].float().t())
+    want = h @ dn[:n].float()
+    for t in (gate, up, dn):
+        t[n:] = float("nan")
+    out = torch.full((M, H), float("nan"), dtype=torch.float16, device=DEV)
+    comb = torch.full((M, (2 if gated else 1) * I), float("nan"), dtype=torch.float16, device=DEV)
+    mlp_forward_rows(x, gate if gated else None, up, dn, I, torch.tensor([n], dtype=torch.int32, device=DEV), out, comb, "silu",
+                     gated)
+    torch.cuda.synchronize()
+    assert_close(out.float().cpu().numpy(), want.cpu().numpy(), "float16", f"{M} rows, {n} active")
+    assert_close(comb[:, :n].float().cpu().numpy(), h.cpu().numpy(), "float16", f"intermediate, {M} rows, {n} active")
+
+
 def test_prefill_agrees_with_decode_kernel():
     """The MFMA path (B = 40) and the streaming path (the same rows, 4 at a time) agree to rounding."""
     x, cw, dn = _case(22, 40, 1024, 700, "float16", True)
