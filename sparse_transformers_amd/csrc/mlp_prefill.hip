@@ -30,17 +30,6 @@ constexpr int kPfBM = 128;   // rows of x per block
 constexpr int kPfBN = 128;   // output columns per block (kernel 1: 64 gate + 64 up rows)
 constexpr int kPfBK = 128;   // columns of Hh are padded to a multiple of this
 
-// Workgroups are handed to the 8 XCDs round-robin by their linear id, and each XCD has its own L2.
-// This maps the linear id to a tile id such that every XCD works through one contiguous range of tile
-// ids; tile ids are ordered so that neighbours share an operand tile (the same weight rows for all row
-// tiles of x), which then comes from that XCD's L2 instead of HBM.  Returns -1 for the padding ids.
-__device__ __forceinline__ int xcd_tile_id(int bid, int ntiles)
-{
-    const int per = (ntiles + kXcds - 1) / kXcds;
-    const int t = (bid % kXcds) * per + bid / kXcds;
-    return (bid / kXcds < per && t < ntiles) ? t : -1;
-}
-
 // The gate / up kernels' tiles that hold active rows.  The grid covers the cache's capacity (`jt` tiles of weight rows); the
 // ranges are dealt out over the device's count, so that every XCD has its share of the work.  Dealt out over the capacity the
 // tiles of a half-active cache all fell to four of the eight: gate / up at H 4096, I 14336, 55 % active, 2048 rows 401 us

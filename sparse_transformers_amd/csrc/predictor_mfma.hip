@@ -23,56 +23,65 @@ constexpr int kSplitParts = 3;
 // ---------------------------------------------------------------------------
 // kernel 1
 // ---------------------------------------------------------------------------
-// A tile of 16 MI rows of x by 16 NI rank rows per block.  Its W waves deal out pieces of 128 of the hidden dimension
-// among themselves; a wave loads the 256 bytes of every row of its next piece straight into a part of LDS of its own while
-// it multiplies the present one, so nothing waits for another wave until the sums meet at the end.  (Fragments loaded
-// from memory into registers, 16 rows x 64 bytes per instruction, went through a CU at 15 bytes per clock.)
-// LDS rows are 16 chunks of 16 bytes, chunk c of row k at c ^ (k % 16).
-constexpr int kPmPiece = 128;
-
-template <typename T, int MI, int NI, int W, typename Tab>
+// A tile of 16 MI rows of x by 16 NI rank rows per block.  Its W waves deal out pieces of 8 PC of the hidden dimension among
+// themselves; a wave loads the 16 PC bytes of every row of its next pieces straight into a ring of NB buffers of its own in
+// LDS while it multiplies the present one, so nothing waits for another wave until the sums meet at the end.  (Fragments
+// loaded from memory into registers, 16 rows x 64 bytes per instruction, went through a CU at 15 bytes per clock.)
+// Bound by what a CU pulls through its L2, so by the rows of a tile per result and by the bytes in flight: 2048 rows, H 4096,
+// rank 256, bf16: 32 x 32 tiles with rank tiles fastest (every XCD read all of x) 25.2 us, 64 x 32 by XCD 12.1.
+// LDS rows are PC chunks of 16 bytes; chunk c of row k at c ^ (k % 16), or c ^ (k / 2 % 8) for rows of 128 bytes: the 16 rows
+// of a fragment read meet every bank alike.
+template <typename T, int MI, int NI, int W, int PC, int NB, typename Tab>
 __global__ __launch_bounds__(W * kWave) void predictor_down_mfma_kernel(const T *__restrict__ x, const T *__restrict__ A,
-                                                                        int B, int H, int r, int nt,
+                                                                        int B, int H, int r,
                                                                         float *__restrict__ t, uint8_t *__restrict__ mask,
-                                                                        int I, int round_storage, Tab tab)
+                                                                        int I, int launch_word, int blocks, Tab tab)
 {
     if constexpr (Tab::kLayers) {   // several layers of equal shape at once: x [layers,B,H], t [layers,B,r]
-        A = static_cast<const T *>(tab.l[blockIdx.y].A);
-        mask = tab.l[blockIdx.y].mask;
-        x += (size_t)blockIdx.y * B * H;
-        t += (size_t)blockIdx.y * B * r;
+        A = static_cast<const T *>(tab.l[blockIdx.z].A);
+        mask = tab.l[blockIdx.z].mask;
+        x += (size_t)blockIdx.z * B * H;
+        t += (size_t)blockIdx.z * B * r;
     }
-    constexpr int kThreads = W * kWave;
-    constexpr int kRows = 16 * (MI + NI), kBuf = kRows * 16, kDma = kRows / 4;   // a wave's buffer in chunks, its 1 KB loads
-    extern __shared__ __align__(16) uint4 lds[];   // [W][2][kRows][16]
+    // (14 dwords of arguments, all in scalar registers when the wave starts; the grid's size would arrive by a load)
+    const int gx = launch_word >> 1, round_storage = launch_word & 1;
+    constexpr int kThreads = W * kWave, kPiece = 8 * PC;
+    constexpr int kRows = 16 * (MI + NI), kBuf = kRows * PC, kDma = kBuf / 64;   // a wave's buffer in chunks, its 1 KB loads
+    static_assert((PC == 16 || PC == 8) && (NB - 1) * kDma < 64, "swizzle; waits count to 63");
+    extern __shared__ __align__(16) uint4 lds[];   // [W][NB][kRows][PC]
+    auto swz = [](int row) __attribute__((always_inline)) { return PC == 16 ? row & 15 : (row >> 1) & 7; };
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, q = lane >> 4;
-    const int m0 = (blockIdx.x / nt) * 16 * MI, k0 = (blockIdx.x % nt) * 16 * NI;
+    // (tiles of x fastest, their number padded to a multiple of the XCDs: a tile's rows come through one L2 only; no division,
+    // which takes a launch of this size 0.3 us)
+    const int m0 = blockIdx.x * 16 * MI, k0 = blockIdx.y * 16 * NI;
+    const bool live = m0 < B;
     const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
     const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint4 *)lds;
 
-    // load j fills LDS rows 4 j .. 4 j + 3, lane i position i % 16 of row i / 16.  Rows are clamped into range (what they
+    // load j fills 64 / PC LDS rows, lane i position i % PC of row i / PC.  Rows are clamped into range (what they
     // feed is not stored), and so are columns past the end of a row (replaced by zeros below).  Offsets of 32 bits only
     // reach over the tile's own rows: x may be larger than 4 GiB.
+    constexpr int kLoadRows = 64 / PC;
     const char *const x_tile = reinterpret_cast<const char *>(x + (size_t)m0 * H);
     const char *const a_tile = reinterpret_cast<const char *>(A + (size_t)k0 * H);
     unsigned doff[kDma];
 #pragma unroll
     for (int j = 0; j < kDma; ++j) {
-        const int row = 4 * j + (lane >> 4);
+        const int row = kLoadRows * j + lane / PC;
         int g = row < 16 * MI ? row : row - 16 * MI;
         const int last = row < 16 * MI ? B - 1 - m0 : r - 1 - k0;
         g = g < last ? g : last;
         doff[j] = (unsigned)g * (unsigned)H * (unsigned)sizeof(T);
     }
-    const int pieces = (H + kPmPiece - 1) / kPmPiece;
+    const int pieces = (H + kPiece - 1) / kPiece;
     auto dma = [&](int piece, int b) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < kDma; ++j) {
-            const int row = 4 * j + (lane >> 4), c = (lane & 15) ^ (row & 15);
-            const int h = piece * kPmPiece + 8 * c;
-            load_to_lds(lds_base + (unsigned)((wave * 2 + b) * kBuf + j * 64) * 16u, doff[j] + (unsigned)(h < H ? h : 0) * (unsigned)sizeof(T),
-                        4 * j < 16 * MI ? x_tile : a_tile);
+            const int row = kLoadRows * j + lane / PC, c = (lane % PC) ^ swz(row);
+            const int h = piece * kPiece + 8 * c;
+            load_to_lds(lds_base + (unsigned)((wave * NB + b) * kBuf + j * 64) * 16u, doff[j] + (unsigned)(h < H ? h : 0) * (unsigned)sizeof(T),
+                        kLoadRows * j < 16 * MI ? x_tile : a_tile);
         }
     };
     f32x4_t acc[MI][NI];
@@ -80,25 +89,31 @@ __global__ __launch_bounds__(W * kWave) void predictor_down_mfma_kernel(const T 
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NI; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    if (wave < pieces) dma(wave, 0);
-    // the mask is cleared here, a kernel ahead of the one that switches bytes on
-    for (int i = blockIdx.x * kThreads + tid; i < I; i += gridDim.x * kThreads) mask[i] = 0;
+#pragma unroll
+    for (int p = 0; p < NB - 1; ++p)
+        if (live && wave + p * W < pieces) dma(wave + p * W, p);
+    // the mask is cleared here, a kernel ahead of the one that switches bytes on (the stores are newer than the loads that are
+    // counted below: the first wait lets that many fewer of the second piece's loads be outstanding)
+    for (int i = (blockIdx.y * gx + blockIdx.x) * kThreads + tid; i < I; i += blocks * kThreads) mask[i] = 0;
+    if (!live) return;
     int b = 0;
-    for (int piece = wave; piece < pieces; piece += W, b ^= 1) {
-        // (the loads of the next piece go out once the reads of the last use of their buffer are done)
-        ST_WAIT_VM_LGKM0(0);
+    for (int piece = wave; piece < pieces; piece += W) {
+        // this piece has arrived once all but the newer ones' loads have; the next loads go out once the reads of the last
+        // use of their buffer are done
+        if (NB > 2 && piece + W < pieces) ST_WAIT_VM_LGKM0((NB - 2) * kDma); else ST_WAIT_VM_LGKM0(0);
         asm volatile("" ::: "memory");
-        if (piece + W < pieces) dma(piece + W, b ^ 1);
-        const uint4 *buf = lds + (wave * 2 + b) * kBuf;
+        const int before = b == 0 ? NB - 1 : b - 1;
+        if (piece + (NB - 1) * W < pieces) dma(piece + (NB - 1) * W, before);
+        const uint4 *buf = lds + (wave * NB + b) * kBuf;
 #pragma unroll
-        for (int ks = 0; ks < kPmPiece / 32; ++ks) {
+        for (int ks = 0; ks < kPiece / 32; ++ks) {
             uint4 fa[MI], fb[NI];
-            const int c = (4 * ks + q) ^ l16;
+            const int c = (4 * ks + q) ^ swz(l16);
 #pragma unroll
-            for (int i = 0; i < MI; ++i) fa[i] = buf[(16 * i + l16) * 16 + c];
+            for (int i = 0; i < MI; ++i) fa[i] = buf[(16 * i + l16) * PC + c];
 #pragma unroll
-            for (int j = 0; j < NI; ++j) fb[j] = buf[(16 * (MI + j) + l16) * 16 + c];
-            if (piece * kPmPiece + 32 * ks + 8 * q >= H) {   // (both operands: a product with zero must not meet an infinity)
+            for (int j = 0; j < NI; ++j) fb[j] = buf[(16 * (MI + j) + l16) * PC + c];
+            if (piece * kPiece + 32 * ks + 8 * q >= H) {   // (both operands: a product with zero must not meet an infinity)
 #pragma unroll
                 for (int i = 0; i < MI; ++i) fa[i] = zero4;
 #pragma unroll
@@ -109,11 +124,12 @@ __global__ __launch_bounds__(W * kWave) void predictor_down_mfma_kernel(const T 
 #pragma unroll
                 for (int j = 0; j < NI; ++j) acc[i][j] = Mfma<T>::run(fa[i], fb[j], acc[i][j]);
         }
+        b = b == NB - 1 ? 0 : b + 1;
     }
     // (the sums lie over the front of the buffers, the first waves': behind the barrier nobody reads those any more)
     typedef float Red[MI * NI][256];
     Red *red = reinterpret_cast<Red *>(lds);
-    static_assert(sizeof(Red) <= 2 * kBuf * 16, "a wave's sums exceed its buffers");
+    static_assert(sizeof(Red) <= NB * kBuf * 16, "a wave's sums exceed its buffers");
     __syncthreads();
 
     // D[m][n]: a lane holds rows 4 q + e of column l16
@@ -183,30 +199,34 @@ template <typename T, bool TINY> __device__ __forceinline__ void split_parts(con
     }
 }
 
-// A wave owns 16 MI rows of t (KS k steps of 32 of the rank, in registers as parts) and walks over rows of Bm, which the
+// A wave owns 16 rows of t (KS k steps of 32 of the rank, in registers as parts) and walks over rows of Bm, which the
 // block loads 64 rows (a stage) at a time straight into LDS, one stage ahead: its W waves share them (fragments loaded by
-// every wave on its own: 97 us for 2048 rows at rank 256, I 14336; now 54 us, of which the MFMAs are 18).  `wb` of the waves
-// own different rows of t, the other W / wb groups take different 16-row tiles of a stage (WB = W is a compile-time case:
-// every wave takes every tile); a block takes `per` stages.
+// every wave on its own: 97 us for 2048 rows at rank 256, I 14336).  W / IG of the waves own different rows of t, the IG
+// groups take different 16-row tiles of a stage; a block takes `per` stages.
+// MFMA bound: a tile of 16 indices is 3 KS of them, and while they run each fragment they have consumed is replaced by the
+// next tile's, so that no read is waited for.  What is left of a tile's work is the decision.  Unless scores are written or
+// rounded, rows of t past B are copies of the last one and columns past I are dropped at the end, so that a
+// lane's four scores become one comparison of their maximum.  Rows 2048, rank 256, I 14336, bf16 (45 GFLOP with the parts, 23
+// us of MFMAs): 58.8 us with reads just ahead of their use and a decision per score, now 39.5.
 // LDS rows are 4 KS chunks of 16 bytes (the rank rounded up; the surplus chunks repeat others and are not used), chunk c of
 // row k sits at c ^ (k % 16): the 16 rows of a fragment read meet different banks.  Which indices a row switched on is
 // collected in LDS too: a store to memory inside the loop would have to be waited for together with the next stage.
 constexpr int kPmStage = 64;
 
-template <typename T, int KS, int MI, int W, bool ALL, typename Tab>
+template <typename T, int KS, int W, int IG, typename Tab>
 __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const float *__restrict__ t,
                                                                       const T *__restrict__ Bm, int B, int r, int I,
-                                                                      int splits, int wb_rt, int per, float thr, int flags,
+                                                                      int per, float thr, int flags,
                                                                       float *__restrict__ scores,
                                                                       uint8_t *__restrict__ mask, Tab tab)
 {
     if constexpr (Tab::kLayers) {
-        const st_predictor_layer &ly = tab.l[blockIdx.y];
+        const st_predictor_layer &ly = tab.l[blockIdx.z];
         Bm = static_cast<const T *>(ly.Bm);
         mask = ly.mask;
         thr = ly.thr;
         flags = (flags & ~1) | (ly.cmp_ge ? 1 : 0);
-        t += (size_t)blockIdx.y * B * r;
+        t += (size_t)blockIdx.z * B * r;
     }
     constexpr int P = kSplitParts;
     constexpr bool kScaled = std::is_same<T, f16_t>::value;
@@ -217,35 +237,39 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
     const int cmp_ge = flags & 1, round_storage = (flags >> 1) & 1;
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, q = lane >> 4;
-    const int wb = ALL ? W : wb_rt, ig = W / wb;              // wave groups that share a stage's tiles
-    // blocks of one XCD (ids equal modulo 8; `splits` is a multiple of 8 where it can be) work on the same rows of Bm
-    const int m0 = ((blockIdx.x / splits) * wb + wave % wb) * 16 * MI;
+    constexpr int WB = W / IG, NT = kPmStage / 16 / IG;       // waves with rows of t of their own, tiles of a wave per stage
+    const int j0 = wave / WB;                                 // first of them: j0, j0 + IG, ...
+    // blocks of one XCD (ids equal modulo 8; the grid's x is a multiple of 8 where it can be) work on the same rows of Bm
+    const int m0 = (blockIdx.y * WB + wave % WB) * 16;
     const int stages = (I + kPmStage - 1) / kPmStage;
-    const int s0 = (blockIdx.x % splits) * per, s1 = s0 + per < stages ? s0 + per : stages;
+    const int s0 = blockIdx.x * per, s1 = s0 + per < stages ? s0 + per : stages;
     const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
 
     const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint4 *)lds;
+    unsigned doff[kDma];
+    auto lane_off = [&](int j, int last) __attribute__((always_inline)) {
+        const int at = (wave * kDma + j) * 64 + lane, row = at / kRow, c = (at % kRow) ^ (row & 15);
+        return ((unsigned)(row < last ? row : last) * (unsigned)r + (unsigned)(8 * c < r ? 8 * c : 0)) * (unsigned)sizeof(T);
+    };
+#pragma unroll
+    for (int j = 0; j < kDma; ++j) doff[j] = lane_off(j, kPmStage);
     auto dma = [&](int stage, int b) __attribute__((always_inline)) {
         const T *const rows = Bm + (size_t)stage * kPmStage * r;   // (offsets within the stage: Bm may be larger than 4 GiB)
+        const int last = I - 1 - stage * kPmStage;
+        const bool clip = last < kPmStage - 1;                      // uniform: the last row is repeated
 #pragma unroll
-        for (int j = 0; j < kDma; ++j) {
-            const int at = (wave * kDma + j) * 64 + lane, row = at / kRow, pos = at % kRow;
-            int c = pos ^ (row & 15);
-            c = 8 * c < r ? c : 0;
-            const int last = I - 1 - stage * kPmStage, i = row < last ? row : last;
-            const unsigned off = ((unsigned)i * (unsigned)r + 8u * (unsigned)c) * (unsigned)sizeof(T);
-            load_to_lds(lds_base + (unsigned)(b * kBuf + (wave * kDma + j) * 64) * 16u, off, reinterpret_cast<const char *>(rows));
-        }
+        for (int j = 0; j < kDma; ++j)
+            load_to_lds(lds_base + (unsigned)(b * kBuf + (wave * kDma + j) * 64) * 16u, clip ? lane_off(j, last) : doff[j],
+                        reinterpret_cast<const char *>(rows));
     };
     if (s0 >= s1) return;
     dma(s0, 0);
     for (int i = threadIdx.x; i < per * (kPmStage / 4); i += W * kWave) reinterpret_cast<uint32_t *>(hits)[i] = 0u;
 
-    uint4 tf[MI][P][KS];
-    float unscale[MI][4];    // of the rows this lane's results belong to
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-        const int m = m0 + 16 * i + l16;
+    uint4 tf[P][KS];
+    float unscale[4];        // of the rows this lane's results belong to
+    {
+        const int m = m0 + l16;
         const float *row = t + (size_t)(m < B ? m : B - 1) * r;
         float v[KS][8];
 #pragma unroll
@@ -258,7 +282,7 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
             for (int e = 0; e < 8; ++e) v[ks][e] = k < r ? w[e] : 0.f;
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) unscale[i][e] = 1.f;
+        for (int e = 0; e < 4; ++e) unscale[e] = 1.f;
         if constexpr (kScaled) {
             // a power of two per row that puts its largest finite element near 2^14
             float big = 0.f;
@@ -280,7 +304,7 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[ks][e] *= scale;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) unscale[i][e] = __shfl(back, 4 * q + e, kWave);
+            for (int e = 0; e < 4; ++e) unscale[e] = __shfl(back, 4 * q + e, kWave);
         }
         auto split = [&](auto tiny) __attribute__((always_inline)) {
 #pragma unroll
@@ -288,7 +312,7 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
                 uint4 parts[P];
                 split_parts<T, decltype(tiny)::value>(v[ks], parts);
 #pragma unroll
-                for (int p = 0; p < P; ++p) tf[i][p][ks] = parts[p];
+                for (int p = 0; p < P; ++p) tf[p][ks] = parts[p];
             }
         };
         if constexpr (kScaled) {
@@ -307,65 +331,96 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
             split(std::false_type{});
         }
     }
-    // rows of t beyond B only exist in the last tiles: their scores do not count
-    unsigned live = 0u;
+    const bool gen = scores != nullptr || round_storage;
+    // v > thr as v >= the next number up (none above infinity: nothing passes)
+    float least_in = thr;
+    if (!cmp_ge) {
+        const uint32_t u = __float_as_uint(thr);
+        const uint32_t up = (u << 1) == 0u ? 1u : (u >> 31) ? u - 1u : u + 1u;
+        least_in = thr < __builtin_inff() ? __uint_as_float(up) : __uint_as_float(0x7fc00000u);
+    }
+    // A lane's score: the parts' sums, smallest first.  An infinite element of Bm decides the score by the sign of t, which
+    // its first part has; the others are zero or of either sign and would make a NaN of it: they are kept finite (the median
+    // with a NaN among them is the least of the others).
+    auto score = [&](const f32x4_t (&acc)[P], int e) __attribute__((always_inline)) {
+        float rest = acc[P - 1][e];
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+        for (int p = P - 2; p >= 1; --p) rest += acc[p][e];
+        float v = __builtin_amdgcn_fmed3f(rest, -kMaxF32, kMaxF32) + acc[0][e];
+        if constexpr (kScaled) v *= unscale[e];
+        return v;
+    };
+    auto decide = [&](const f32x4_t (&acc)[P], int col) __attribute__((always_inline)) -> bool {
+        if (__builtin_expect(!gen, 1)) {
+            const float v = fmaxf(fmaxf(score(acc, 0), score(acc, 1)), fmaxf(score(acc, 2), score(acc, 3)));
+            return v >= least_in;   // (a NaN never passes, and the maximum is one only if all four are)
+        }
+        bool any = false;
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (m0 + 16 * i + 4 * q + e < B) live |= 1u << (4 * i + e);
+        for (int e = 0; e < 4; ++e) {
+            float v = score(acc, e);
+            if (round_storage) v = to_float<T>(from_float<T>(v));
+            const bool in = m0 + 4 * q + e < B;
+            any = any || (in && v >= least_in);
+            if (scores && in && col < I) scores[(size_t)(m0 + 4 * q + e) * I + col] = v;
+        }
+        return any;
+    };
 
+    const bool ragged = r < 32 * KS;   // (r > 32 (KS - 4): the launch picks KS; past the rank t is zero, and so must be what it meets)
+    uint4 bf[KS];
+    // (a lane's fragments of the wave's first tile in the stage that is read: everything else is a constant offset)
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    const __attribute__((address_space(3))) u32x4_t *at[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+        at[ks] = (const __attribute__((address_space(3))) u32x4_t *)lds + (16 * j0 + l16) * kRow + ((4 * ks + q) ^ l16);
+    ST_WAIT_VM_LGKM0(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (s0 + 1 < s1) dma(s0 + 1, 1);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) bf[ks] = __builtin_bit_cast(uint4, *at[ks]);
     for (int s = s0; s < s1; ++s) {
         const int b = (s - s0) & 1;
-        ST_WAIT_VM_LGKM0(0);            // this wave's share of the stage has arrived (and the other buffer's reads are done)
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        if (s + 1 < s1) dma(s + 1, b ^ 1);
+        uint64_t stage_hits = 0;
 #pragma unroll
-        for (int j = 0; j < kPmStage / 16; ++j) {
-            if (!ALL && j % ig != wave / wb) continue;
-            uint4 bf[KS];
+        for (int i = 0; i < NT; ++i) {
+            if (i == NT - 1 && s + 1 < s1) {
+                // the wave's last tile of the stage is in registers: behind the barrier the next stage is in LDS, and the
+                // buffer of this one is free for the one after it
+                ST_WAIT_VM_LGKM0(0);
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                if (s + 2 < s1) dma(s + 2, b);
+            }
+            if (ragged) {
+#pragma unroll
+                for (int ks = KS - 4; ks < KS; ++ks)
+                    if (32 * ks + 8 * q >= r) bf[ks] = zero4;
+            }
+            f32x4_t acc[P];
+#pragma unroll
+            for (int p = 0; p < P; ++p) acc[p] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
-                bf[ks] = lds[b * kBuf + (16 * j + l16) * kRow + ((4 * ks + q) ^ l16)];
-                // (r > 32 (KS - 4): the launch picks KS; past the rank t is zero, and so must be what it meets)
-                if (ks >= KS - 4 && 32 * ks + 8 * q >= r) bf[ks] = zero4;
+#pragma unroll
+                for (int p = 0; p < P; ++p) acc[p] = Mfma<T>::run(tf[p][ks], bf[ks], acc[p]);
+                __builtin_amdgcn_sched_barrier(0);
+                // (past the last stage: a stale buffer, not used)
+                if (i == NT - 1) at[ks] += b ? -kBuf : kBuf;
+                bf[ks] = __builtin_bit_cast(uint4, at[ks][i == NT - 1 ? 0 : 16 * IG * (i + 1) * kRow]);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            f32x4_t acc[MI][P];
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int p = 0; p < P; ++p) acc[i][p] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-                for (int p = 0; p < P; ++p)
-#pragma unroll
-                    for (int i = 0; i < MI; ++i) acc[i][p] = Mfma<T>::run(tf[i][p][ks], bf[ks], acc[i][p]);
-            const int col = s * kPmStage + 16 * j + l16;
-            bool any = false;
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float v = acc[i][P - 1][e];
-#pragma unroll
-                    for (int p = P - 2; p >= 0; --p) v += acc[i][p][e];   // smallest part first
-                    // An infinite element of Bm decides the score by the sign of t, which its first part has; the others are
-                    // zero or of either sign and would make a NaN of it.
-                    v = fabsf(acc[i][0][e]) <= kMaxF32 ? v : acc[i][0][e];
-                    if constexpr (kScaled) v *= unscale[i][e];
-                    if (round_storage) v = to_float<T>(from_float<T>(v));
-                    const bool in = (live >> (4 * i + e)) & 1u;
-                    any = any || (in && (cmp_ge ? v >= thr : v > thr));
-                    if (scores && in && col < I) scores[(size_t)(m0 + 16 * i + 4 * q + e) * I + col] = v;
-                }
-            uint64_t hit = __builtin_amdgcn_ballot_w64(any);
+            const int j = j0 + IG * i;
+            uint64_t hit = __builtin_amdgcn_ballot_w64(decide(acc, s * kPmStage + 16 * j + l16));
             hit |= hit >> 32;
             hit |= hit >> 16;
-            if (lane < 16 && ((hit >> lane) & 1ull)) hits[(s - s0) * kPmStage + 16 * j + lane] = 1;
+            stage_hits |= (hit & 0xffffull) << (16 * j);
         }
+        if ((stage_hits >> lane) & 1ull) hits[(s - s0) * kPmStage + lane] = 1;
     }
     __syncthreads();
     const int first = s0 * kPmStage, count = (I < s1 * kPmStage ? I : s1 * kPmStage) - first;
@@ -392,21 +447,27 @@ static int launch_t(const Tab &tab, int layers, const void *x, int B, int H, con
     const int cus = (device_cu_count() + layers - 1) / layers;
     {
         ProfScope ps(ST_K_PRED_DOWN, stream);
-        auto go = [&](auto kern, int mi, int ni, int waves) -> int {
-            const int mt = (B + 16 * mi - 1) / (16 * mi), nt = (r + 16 * ni - 1) / (16 * ni);
-            const int lds = waves * 2 * 16 * (mi + ni) * 256;
+        auto go = [&](auto kern, int mi, int ni, int waves, int row_chunks) -> int {
+            int mt = (B + 16 * mi - 1) / (16 * mi);
+            const int nt = (r + 16 * ni - 1) / (16 * ni);
+            if (mt > kXcds) mt = (mt + kXcds - 1) / kXcds * kXcds;
+            const int lds = waves * 16 * (mi + ni) * row_chunks * 16;
             const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
             if (rc != ST_OK) return rc;
-            ST_LAUNCH(ps, kern, dim3(mt * nt, layers), dim3(waves * kWave), lds, stream, static_cast<const T *>(x),
-                      static_cast<const T *>(A), B, H, r, nt, t_ws, mask, I, round_storage, tab);
+            ST_LAUNCH(ps, kern, dim3(mt, nt, layers), dim3(waves * kWave), lds, stream, static_cast<const T *>(x),
+                      static_cast<const T *>(A), B, H, r, t_ws, mask, I, mt << 1 | (round_storage ? 1 : 0), mt * nt, tab);
             return ST_OK;
         };
         auto blocks = [&](int mi, int ni) { return ((B + 16 * mi - 1) / (16 * mi)) * ((r + 16 * ni - 1) / (16 * ni)); };
-        // 32 x 32 tiles (half the traffic from L2) once they make a block for three quarters of the CUs: 6.7 (16 x 16) against
-        // 8.6 us with 64 of them (512 rows, H 3072, rank 128), 17.8 against 11.8 us with 224, 40 against 26 us with 512
-        // (by the shape alone: how many layers share the launch must not change how the sums are split)
-        const int rc = 4 * blocks(2, 2) < 3 * device_cu_count() ? go(predictor_down_mfma_kernel<T, 1, 1, 8, Tab>, 1, 1, 8)
-                                                  : go(predictor_down_mfma_kernel<T, 2, 2, 4, Tab>, 2, 2, 4);
+        // The largest tile of which there is one for three quarters of the CUs (by the shape alone: how many layers share the
+        // launch must not change how the sums are split).  32 x 32 tiles have half the traffic from L2: 6.7 (16 x 16) against
+        // 8.6 us with 64 of them (512 rows, H 3072, rank 128), 17.8 against 11.8 us with 224, 40 against 26 us with 512.  64 x
+        // 32 tiles a quarter less again and 96 KB of loads in flight instead of 64, both kernels, 32 x 32 / 64 x 32: 33.7 / 35.0
+        // us with 128 of them (1024 rows, H 4096, rank 256), 57.4 / 52.0 with 192, 54.9 / 48.4 with 256 (2048 rows).
+        const int want = 3 * device_cu_count();
+        const int rc = 4 * blocks(4, 2) >= want   ? go(predictor_down_mfma_kernel<T, 4, 2, 4, 8, 3, Tab>, 4, 2, 4, 24)
+                       : 4 * blocks(2, 2) >= want ? go(predictor_down_mfma_kernel<T, 2, 2, 4, 16, 2, Tab>, 2, 2, 4, 32)
+                                                  : go(predictor_down_mfma_kernel<T, 1, 1, 8, 16, 2, Tab>, 1, 1, 8, 32);
         if (rc != ST_OK) return rc;
     }
     ST_HIP(hipGetLastError());
@@ -414,38 +475,38 @@ static int launch_t(const Tab &tab, int layers, const void *x, int B, int H, con
         ProfScope ps(ST_K_PRED_UP_MASK, stream);
         // resident: blocks a CU holds at once (registers, LDS).  One round of blocks: every further one would split its
         // rows of t into parts again.
-        auto go = [&](auto kern_all, auto kern, int ks, int mi, int waves, int resident) -> int {
-            int wb = 1;
-            while (wb < waves && B > 16 * mi * wb) wb *= 2;
-            const int mt = (B + 16 * mi * wb - 1) / (16 * mi * wb), stages = (I + kPmStage - 1) / kPmStage;
-            int splits = resident * cus / mt;
+        auto go = [&](auto kern, int ks, int wb, int waves, int resident) -> int {
+            const int mt = (B + 16 * wb - 1) / (16 * wb), stages = (I + kPmStage - 1) / kPmStage;
+            // (as many per XCD as its CUs hold: 19 splits of 12 row tiles, three on some XCDs, took two rounds there: 1536 rows,
+            // rank 256, I 8192: both kernels 52 us, with two on each 34.9)
+            const int per_xcd = resident * cus / (kXcds * mt);
+            int splits = per_xcd > 0 ? per_xcd * kXcds : resident * cus / mt;
             if (splits < 1) splits = 1;
             int per = (stages + splits - 1) / splits;
             per = per < 256 ? per : 256;                     // (the LDS bytes of a block's indices)
             splits = (stages + per - 1) / per;
             if (splits > kXcds) splits = (splits + kXcds - 1) / kXcds * kXcds;
             const int lds = 2 * kPmStage * 4 * ks * 16 + per * kPmStage;
-            auto launch = [&](auto k) -> int {
-                const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(k), 2 * kPmStage * 4 * ks * 16 + 256 * kPmStage);
-                if (rc != ST_OK) return rc;
-                ST_LAUNCH(ps, k, dim3(mt * splits, layers), dim3(waves * kWave), lds, stream, t_ws, static_cast<const T *>(Bm), B, r,
-                          I, splits, wb, per, thr, (cmp_ge ? 1 : 0) | (round_storage ? 2 : 0), scores, mask, tab);
-                return ST_OK;
-            };
-            return wb == waves ? launch(kern_all) : launch(kern);
+            const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), 2 * kPmStage * 4 * ks * 16 + 256 * kPmStage);
+            if (rc != ST_OK) return rc;
+            ST_LAUNCH(ps, kern, dim3(splits, mt, layers), dim3(waves * kWave), lds, stream, t_ws, static_cast<const T *>(Bm), B, r,
+                      I, per, thr, (cmp_ge ? 1 : 0) | (round_storage ? 2 : 0), scores, mask, tab);
+            return ST_OK;
         };
-#define ST_PM_UP(KS, MI, W, RES) go(predictor_up_mfma_kernel<T, KS, MI, W, true, Tab>, predictor_up_mfma_kernel<T, KS, MI, W, false, Tab>, KS, MI, W, RES)
+#define ST_PM_UP(KS, W, IG, RES) go(predictor_up_mfma_kernel<T, KS, W, IG, Tab>, KS, W / IG, W, RES)
+#define ST_PM_UP4(KS, RES) (B <= 16 ? ST_PM_UP(KS, 4, 4, RES) : B <= 32 ? ST_PM_UP(KS, 4, 2, RES) : ST_PM_UP(KS, 4, 1, RES))
         int rc;
         // (eight waves share a stage once there are rows of x for them: 16 rows in blocks of eight waves 5.2 us, of four 4.4)
         if (B <= 64) {
-            if (r <= 128) rc = ST_PM_UP(4, 1, 4, 4);
-            else if (r <= 256) rc = ST_PM_UP(8, 1, 4, 2);
-            else if (r <= 384) rc = ST_PM_UP(12, 1, 4, 1);
-            else rc = ST_PM_UP(16, 1, 4, 1);
-        } else if (r <= 128) rc = ST_PM_UP(4, 1, 8, 2);
-        else if (r <= 256) rc = ST_PM_UP(8, 1, 8, 1);
-        else if (r <= 384) rc = ST_PM_UP(12, 1, 8, 1);
-        else rc = ST_PM_UP(16, 1, 4, 1);   // (eight waves of 256 registers cannot hold its parts)
+            if (r <= 128) rc = ST_PM_UP4(4, 4);
+            else if (r <= 256) rc = ST_PM_UP4(8, 2);
+            else if (r <= 384) rc = ST_PM_UP4(12, 1);
+            else rc = ST_PM_UP4(16, 1);
+        } else if (r <= 128) rc = ST_PM_UP(4, 8, 1, 2);
+        else if (r <= 256) rc = ST_PM_UP(8, 8, 1, 1);
+        else if (r <= 384) rc = ST_PM_UP(12, 8, 1, 1);
+        else rc = ST_PM_UP(16, 4, 1, 1);   // (eight waves of 256 registers cannot hold its parts)
+#undef ST_PM_UP4
 #undef ST_PM_UP
         if (rc != ST_OK) return rc;
     }

@@ -32,6 +32,17 @@ template <> struct Mfma<bf16_t> {
 
 constexpr int kXcds = 8;
 
+// Workgroups are handed to the 8 XCDs round-robin by their linear id, and each XCD has its own L2.
+// This maps the linear id to a tile id such that every XCD works through one contiguous range of tile
+// ids; tile ids are ordered so that neighbours share an operand tile (the same weight rows for all row
+// tiles of x), which then comes from that XCD's L2 instead of HBM.  Returns -1 for the padding ids.
+__device__ __forceinline__ int xcd_tile_id(int bid, int ntiles)
+{
+    const int per = (ntiles + kXcds - 1) / kXcds;
+    const int t = (bid % kXcds) * per + bid / kXcds;
+    return (bid / kXcds < per && t < ntiles) ? t : -1;
+}
+
 // s_waitcnt immediate: vmcnt in bits 3:0 (and 15:14), expcnt 6:4 left at "no wait", lgkmcnt 11:8 = 0
 #define ST_WAIT_VM_LGKM0(vm) __builtin_amdgcn_s_waitcnt(((vm) & 15) | (7 << 4) | (0 << 8) | (((vm) >> 4) << 14))
 

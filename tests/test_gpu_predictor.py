@@ -180,6 +180,33 @@ def test_infinite_intermediate_decides_by_sign(dtype, r, B):
         assert torch.equal(m, Bm[:, at] > 0)
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("B,H,r,I", [
+    (9, 64, 16, 200), (20, 1000, 128, 8192), (33, 520, 200, 5001), (64, 256, 256, 1000),      # four waves, 4 / 2 / 1 groups
+    (77, 520, 104, 5001), (130, 128, 384, 777), (300, 264, 440, 8191), (257, 64, 512, 640),   # eight (four above rank 384)
+    (2100, 200, 200, 5001), (2100, 1000, 224, 1000),                                         # 64 x 32 tiles of the intermediate
+])
+def test_matrix_core_mask_without_scores(dtype, B, H, r, I):
+    """Masks decided in registers against the scores the same kernels write: every rank and group form, thresholds that are a
+    score (>= and > differ there), infinities and NaN; and the scores against float64 (fp32 sums: 4e-6 of the largest)."""
+    x, A, Bm = (t.to(DEV) for t in _weights(r + B, B, H, r, I, dtype))
+    s = st.predictor_scores(x, A, Bm)
+    want = (x.double() @ A.double().t()) @ Bm.double().t()
+    assert (s.double() - want).abs().max() <= 4e-6 * want.abs().max()
+    cases = [(x, Bm, s)]
+    Bi, xi = Bm.clone(), x.clone()
+    Bi[3, 5], Bi[4, 6], Bi[5, 7], Bi[I - 1] = float("inf"), float("-inf"), float("nan"), float("inf")
+    cases.append((x, Bi, st.predictor_scores(x, A, Bi)))
+    xi[B - 1, 0], xi[0, 1] = float("inf"), float("nan")
+    cases.append((xi, Bm, st.predictor_scores(xi, A, Bm)))
+    for xc, Bc, sc in cases:
+        top = torch.where(torch.isnan(sc), -float("inf"), sc).amax(0)       # a NaN never passes
+        for thr in (0.0, float(top.sort().values[I // 2]), float("inf"), float("-inf"), float("nan")):
+            for ge in (True, False):
+                got = st.predictor_mask(xc, A, Bc, thr, ge)
+                assert torch.equal(got, ((sc >= thr) if ge else (sc > thr)).any(0)), (thr, ge)
+
+
 def test_naive_threshold_is_score_ge_zero():
     x, A, Bm = _weights(1, 2, 256, 16, 512, "float32")
     # make some scores exactly zero: a zero row of Bm gives score 0 for every input row
