@@ -617,7 +617,8 @@ extern "C" int st_mlp_forward(const void *x, int64_t B, int64_t H, const void *g
 
     const bool batch = B >= batch_min_rows() && B <= kBatchMaxRows && batch_supported(dtype, (int)H);
     if (B >= kPrefillMinRows && !batch && dtype != ST_F32 && H % 128 == 0 && n >= 1)
-        return launch_prefill(dtype, x, (int)B, (int)H, gate_rows, up_rows, down_rows, (int)n, n_dev, out, combined,
+        return launch_prefill(dtype, x, (int)B, (int)H, gate_rows, up_rows, down_rows, (int)n, n_dev,
+                              (int)(n_hint < 0 ? 0 : n_hint > n ? n : n_hint), out, combined,
                               (long)ldc, workspace, act, has_gate ? 1 : 0, static_cast<hipStream_t>(stream));
 
     if (batch)

@@ -45,13 +45,13 @@ __device__ __forceinline__ int live_tiles(int n_pad, int rows, int jt, int mt)
 // ---------------------------------------------------------------------------
 // D[m][j] of a 16 x 16 MFMA block: a lane holds rows 4 q + e (e = 0..3) of column l16.
 //
-// Kernel 1: the activation on a wave's 64 x 16 JN gate / up sums, and the product stored into Hh (and `comb`).
+// Kernel 1: the activation on a wave's 16 MI x 16 JN gate / up sums, and the product stored into Hh (and `comb`).
 // Columns n .. n_pad are written as zeros so that kernel 2 can run whole K stages.  The results go through a tile
-// of the wave's own in LDS (`stg`, 64 rows of 16 JN + 8 elements; the stage buffers are free by then) and leave as
+// of the wave's own in LDS (`stg`, 16 MI rows of 16 JN + 8 elements; the stage buffers are free by then) and leave as
 // whole 16-byte chunks, 64 bytes of a row per four lanes; storing every element by itself took 5.2 us of the 57
 // the kernel ran.
-template <typename T, bool HG, int JN, int ACT>
-__device__ __forceinline__ void pf_store_hidden_as(const f32x4_t (&ag)[4][JN], const f32x4_t (&au)[4][JN], T *stg,
+template <typename T, bool HG, int JN, int ACT, int MI>
+__device__ __forceinline__ void pf_store_hidden_as(const f32x4_t (&ag)[MI][JN], const f32x4_t (&au)[MI][JN], T *stg,
                                                    int lane, int mrow0, int colw, int M, int n, int n_pad, T *Hh,
                                                    long ldh, T *comb, long ldc)
 {
@@ -59,7 +59,7 @@ __device__ __forceinline__ void pf_store_hidden_as(const f32x4_t (&ag)[4][JN], c
     const int l16 = lane & 15, q = lane >> 4;
     const bool comb16 = comb && ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(comb) & 15) == 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < JN; ++j) {
             const int col = colw + 16 * j + l16;
@@ -74,10 +74,10 @@ __device__ __forceinline__ void pf_store_hidden_as(const f32x4_t (&ag)[4][JN], c
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-    for (int c = 0; c < 2 * JN; ++c) {
+    for (int c = 0; c < (MI * JN + 1) / 2; ++c) {
         const int idx = lane + 64 * c, row = idx / (2 * JN), ch = idx % (2 * JN);
         const int m = mrow0 + row, col0 = colw + 8 * ch;
-        if (m < M && col0 < n_pad) {
+        if (row < 16 * MI && m < M && col0 < n_pad) {
             const uint4 v = *reinterpret_cast<const uint4 *>(stg + row * kSP + 8 * ch);
             *reinterpret_cast<uint4 *>(Hh + (size_t)m * ldh + col0) = v;
             if (comb16 && col0 + 8 <= n) {
@@ -94,8 +94,8 @@ __device__ __forceinline__ void pf_store_hidden_as(const f32x4_t (&ag)[4][JN], c
 
 // One copy per activation, chosen once per block: with the activation switched per element the whole kernel was
 // 4 us slower (all five bodies live in the loop's register budget).
-template <typename T, bool HG, int JN>
-__device__ __forceinline__ void pf_store_hidden(int act, const f32x4_t (&ag)[4][JN], const f32x4_t (&au)[4][JN], T *stg,
+template <typename T, bool HG, int JN, int MI>
+__device__ __forceinline__ void pf_store_hidden(int act, const f32x4_t (&ag)[MI][JN], const f32x4_t (&au)[MI][JN], T *stg,
                                                 int lane, int mrow0, int colw, int M, int n, int n_pad, T *Hh, long ldh,
                                                 T *comb, long ldc)
 {
@@ -108,17 +108,17 @@ __device__ __forceinline__ void pf_store_hidden(int act, const f32x4_t (&ag)[4][
     }
 }
 
-// Kernel 2: a wave's 64 x 64 sums, either straight into Out (no K split) or as fp32 partial sums of split z through
-// a tile of the wave's own in LDS (`stg`, 64 rows of 68 floats), 256 bytes of a row per 16 lanes.
+// Kernel 2: a wave's 16 MI x 64 sums, either straight into Out (no K split) or as fp32 partial sums of split z through
+// a tile of the wave's own in LDS (`stg`, 16 MI rows of 68 floats), 256 bytes of a row per 16 lanes.
 constexpr int kPfStgF = 64 + 4;   // floats per staged row
-template <typename T>
-__device__ __forceinline__ void pf_store_out(const f32x4_t (&f)[4][4], float *stg, int lane, int mrow0, int colw, int M,
+template <typename T, int MI>
+__device__ __forceinline__ void pf_store_out(const f32x4_t (&f)[MI][4], float *stg, int lane, int mrow0, int colw, int M,
                                              int H, T *Out, float *partial_z)
 {
     const int l16 = lane & 15, q = lane >> 4;
     if (!partial_z) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int col = colw + 16 * j + l16;
@@ -131,7 +131,7 @@ __device__ __forceinline__ void pf_store_out(const f32x4_t (&f)[4][4], float *st
         return;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -140,7 +140,7 @@ __device__ __forceinline__ void pf_store_out(const f32x4_t (&f)[4][4], float *st
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-    for (int c = 0; c < 16; ++c) {
+    for (int c = 0; c < 4 * MI; ++c) {
         const int row = 4 * c + q, m = mrow0 + row, col = colw + 4 * l16;
         if (m < M && col < H)
             *reinterpret_cast<float4 *>(partial_z + (size_t)m * H + col) =
@@ -734,6 +734,157 @@ __global__ __launch_bounds__(kPwThreads) void prefill_gateup_wide_kernel(const T
 }
 
 // ---------------------------------------------------------------------------
+// kernel 1 for up to 128 rows of x
+// ---------------------------------------------------------------------------
+// One row of tiles: what takes the time is a block's own K loop, i.e. the bytes a CU has in flight, and the number of CUs
+// that have active rows.  A block takes all rows of x (16 MT) and 32 JN active rows (JN from the host's guess of the count:
+// the fewest that make no more blocks than CUs; it changes neither which products are summed nor in which order), and the
+// whole LDS is one ring of stages of 64 of K that are requested as far ahead as it reaches.  The eight waves are two K halves
+// of every stage x two halves of the rows of x x two halves of the active rows; a stage's fragments are read under the MFMAs
+// of the one ahead of it, which frees its slot at once.  H 2560, 6144 of 10240 active rows, ungated, 77 rows: 20.4 us
+// with two 64-row LDS buffers and register staging on the 96 blocks that had active rows, now 14.1.
+template <bool HG, int MT, int JN> struct FewTile {
+    static constexpr int kWRows = (HG ? 64 : 32) * JN;                       // weight rows
+    static constexpr int kRows = (16 * MT + kWRows + 63) / 64 * 64;          // LDS rows of a stage: x, gate, up; eight waves' whole loads
+    static constexpr int kBuf = kRows * kPfLd1;                              // in 16-byte units
+    static constexpr int kSlots = kPwLds / kBuf < 8 ? kPwLds / kBuf : 8;
+};
+
+template <typename T, bool HG, int MT, int JN>
+__global__ __launch_bounds__(kPwThreads) void prefill_gateup_few_kernel(const T *__restrict__ X, const T *__restrict__ gate,
+                                                                        const T *__restrict__ up,
+                                                                        const int *__restrict__ n_dev, int M, int H,
+                                                                        int n_host, T *__restrict__ Hh, long ldh,
+                                                                        T *__restrict__ comb, long ldc, int act)
+{
+    typedef FewTile<HG, MT, JN> Tile;
+    constexpr int kWR = 32 * JN, MI = MT / 2, kBuf = Tile::kBuf, kSlots = Tile::kSlots;
+    constexpr int kDma = Tile::kRows / 64;                // 1 KB loads per wave and stage
+    constexpr int kGRow = 16 * MT, kURow = kGRow + (HG ? kWR : 0);
+    __shared__ uint4 lds[kSlots * kBuf];
+    const int n = device_count(n_host, n_dev);
+    const int n_pad = (n + kPfBK - 1) / kPfBK * kPfBK;
+    const int j0 = blockIdx.x * kWR;
+    if (j0 >= n_pad) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kh = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+    const int l16 = lane & 15, q = lane >> 4;
+    const int fsw = pf_swz(l16);
+    const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint4 *)lds;
+
+    // loads (as in the tiles above): rows past M, the count and the weight rows repeat the last one.  Offsets of 32 bits only
+    // reach over the block's own weight rows.
+    const int row0 = j0 < n ? j0 : n - 1;
+    const char *dbase[kDma];
+    unsigned doff[kDma];
+#pragma unroll
+    for (int j = 0; j < kDma; ++j) {
+        const int L = 8 * (wave * kDma + j), r = L + (lane >> 3), c = (lane & 7) ^ pf_swz(r);
+        int g;
+        if (L < kGRow || L >= kGRow + Tile::kWRows) {
+            g = r < M ? r : M - 1;
+            dbase[j] = reinterpret_cast<const char *>(X);
+        } else {
+            const bool isg = HG && L < kURow;
+            g = j0 + r - (isg ? kGRow : kURow);
+            g = (g < n ? g : n - 1) - row0;
+            dbase[j] = reinterpret_cast<const char *>((isg ? gate : up) + (size_t)row0 * H);
+        }
+        doff[j] = ((unsigned)g * (unsigned)H + (unsigned)c * 8u) * (unsigned)sizeof(T);
+    }
+    const int nk = H / kPfBK1;   // (even: H is a multiple of 128)
+    auto dma = [&](int stage, int slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < kDma; ++j)
+            load_to_lds((unsigned)(slot * kBuf + (wave * kDma + j) * 64) * 16u + lds_base, doff[j], dbase[j] + (size_t)stage * kPfBK1 * sizeof(T));
+    };
+
+    f32x4_t ag[MI][JN], au[MI][JN];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < JN; ++j) {
+            ag[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            au[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    struct Frag { uint4 a[MI], g[JN], u[JN]; };
+    Frag F0, F1;
+    const int chunk = (4 * kh + q) ^ fsw;   // (the kh-th 32 of the stage's 64)
+    auto rd = [&](Frag &F, int slot) __attribute__((always_inline)) {
+        const uint4 *b = lds + slot * kBuf + l16 * kPfLd1 + chunk;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) F.a[i] = b[(16 * (MI * wm + i)) * kPfLd1];
+#pragma unroll
+        for (int j = 0; j < JN; ++j) {
+            if (HG) F.g[j] = b[(kGRow + 16 * (JN * wn + j)) * kPfLd1];
+            F.u[j] = b[(kURow + 16 * (JN * wn + j)) * kPfLd1];
+        }
+    };
+    auto mm = [&](const Frag &F) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < JN; ++j) {
+                au[i][j] = Mfma<T>::run(F.a[i], F.u[j], au[i][j]);
+                if (HG) ag[i][j] = Mfma<T>::run(F.a[i], F.g[j], ag[i][j]);
+            }
+    };
+    // behind the barrier stage s + 1 is in LDS and every wave has stage s in registers: its slot takes stage s + kSlots
+    auto stage = [&](int s, int slot, const Frag &Fc, Frag &Fn) __attribute__((always_inline)) {
+        const int next = slot == kSlots - 1 ? 0 : slot + 1;
+        if (s + kSlots <= nk) ST_WAIT_VM_LGKM0((kSlots - 2) * kDma); else ST_WAIT_VM_LGKM0(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        rd(Fn, next);   // (past the last stage: a stale slot, not used)
+        __builtin_amdgcn_sched_barrier(0);
+        if (s + kSlots < nk) dma(s + kSlots, slot);   // (loads that wait to be accepted do not hold up the reads)
+        mm(Fc);
+        __builtin_amdgcn_sched_barrier(0);
+        return next;
+    };
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s)
+        if (s < nk) dma(s, s);
+    if (nk >= kSlots) ST_WAIT_VM_LGKM0((kSlots - 1) * kDma); else ST_WAIT_VM_LGKM0(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    rd(F0, 0);
+    int slot = 0;
+    for (int s = 0; s < nk; s += 2) {
+        slot = stage(s, slot, F0, F1);
+        slot = stage(s + 1, slot, F1, F0);
+    }
+
+    // the second K half's sums to the first, which stores (behind the barrier nobody reads the stages any more)
+    constexpr int kRed = (HG ? 2 : 1) * MI * JN * 64;     // quads of a wave
+    f32x4_t *red = reinterpret_cast<f32x4_t *>(lds) + (wave & 3) * kRed + lane;
+    static_assert(4 * kRed + 4 * 16 * MI * (16 * JN + 8) / 8 <= kSlots * kBuf, "sums and epilogue tiles exceed the stages");
+    __syncthreads();
+    if (kh == 1) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < JN; ++j) {
+                red[(i * JN + j) * 64] = au[i][j];
+                if (HG) red[(MI * JN + i * JN + j) * 64] = ag[i][j];
+            }
+    }
+    __syncthreads();
+    if (kh == 1) return;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < JN; ++j) {
+            au[i][j] += red[(i * JN + j) * 64];
+            if (HG) ag[i][j] += red[(MI * JN + i * JN + j) * 64];
+        }
+    T *stg = reinterpret_cast<T *>(lds + 4 * kRed) + (size_t)wave * 16 * MI * (16 * JN + 8);
+    pf_store_hidden<T, HG, JN>(act, ag, au, stg, lane, 16 * MI * wm, j0 + 16 * JN * wn, M, n, n_pad, Hh, ldh, comb, ldc);
+}
+
+// ---------------------------------------------------------------------------
 // kernel 2: down projection
 // ---------------------------------------------------------------------------
 // Out[M,H] = Hh[M,n] Wd[n,H].  Wd's rows run along K, so its tile goes to LDS as it is ([k][column], whole
@@ -1096,6 +1247,143 @@ __global__ __launch_bounds__(kPwThreads) void prefill_down_wide_kernel(const T *
     ST_TL(4);
 }
 
+// ---------------------------------------------------------------------------
+// kernel 2 for up to 128 rows of x
+// ---------------------------------------------------------------------------
+// A block takes all rows (16 MT), 128 output columns and a K split; stages of 64 through a ring over the whole LDS as in
+// prefill_gateup_few_kernel (two K halves x two halves of the rows x two halves of the columns), Wd's rows as in the wide form.
+// H 2560, 6144 active rows, 77 rows: 14.2 us in 128 x 128 tiles with two
+// LDS buffers and sixteen splits of six stages, now 11.1 with twelve.
+template <typename T, int MT>
+__global__ __launch_bounds__(kPwThreads) void prefill_down_few_kernel(const T *__restrict__ Hh, const T *__restrict__ Wd,
+                                                                      const int *__restrict__ n_dev, long ldh, int M, int H,
+                                                                      int n_host, int split_k, int ct, T *__restrict__ Out,
+                                                                      float *__restrict__ partial)
+{
+    constexpr int MI = MT / 2;
+    constexpr int kDma = (2 * MT + 16 + 7) / 8;           // 1 KB loads per wave and stage: 2 MT of Hh, 16 of Wd, repeats of Hh
+    constexpr int kBuf = 8 * kDma * 64, kSlots = kPwLds / kBuf;   // 16-byte units of a stage
+    constexpr int kWdAt = 2 * MT * 64;                    // Wd's part of it
+    __shared__ uint4 lds[kSlots * kBuf];
+    const int n = device_count(n_host, n_dev);
+    const int tile = xcd_tile_id(blockIdx.x, ct * split_k);   // column tiles fastest: they share the rows of Hh
+    if (tile < 0) return;
+    const int z = tile / ct, c0 = (tile % ct) * kPfBN;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kh = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+    const int l16 = lane & 15, q = lane >> 4;
+    const int fsw = pf_swz(l16);
+    const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint4 *)lds;
+
+    // K range of this split, in stages of 64 (Hh is zero-padded to a multiple of 128 columns)
+    const int nst_all = (n + kPfBK - 1) / kPfBK * (kPfBK / kPfBK2);
+    const int per = (nst_all + split_k - 1) / split_k;
+    const int ks0 = z * per, ks1 = (ks0 + per < nst_all) ? ks0 + per : nst_all;
+    const int nst = ks1 - ks0;
+
+    // load L = kDma wave + j: L < 2 MT fills rows 8 L .. + 7 of the Hh tile, the next 16 four rows of Wd each, the rest repeat
+    // the last row of Hh.  Rows of Wd at or beyond n are replaced by the last valid one, as in prefill_down_wide_kernel.
+    auto dma = [&](int stage, int slot) __attribute__((always_inline)) {
+        const int k0 = (ks0 + stage) * kPfBK2;
+#pragma unroll
+        for (int j = 0; j < kDma; ++j) {
+            const int L = wave * kDma + j;                // uniform
+            const unsigned dst = (unsigned)(slot * kBuf + L * 64) * 16u + lds_base;
+            if (L < 2 * MT || L >= 2 * MT + 16) {
+                const int r = 8 * L + (lane >> 3), c = (lane & 7) ^ pf_swz(r), g = r < M ? r : M - 1;
+                load_to_lds(dst, (unsigned)((size_t)g * ldh * sizeof(T)) + (unsigned)c * 16u, reinterpret_cast<const char *>(Hh + k0));
+            } else {
+                const int kt = 4 * (L - 2 * MT) + (lane >> 4), c = (lane & 15) ^ pf_swz_b(kt);
+                const int last = n - 1 - k0;              // (below 0: the stage is all padding)
+                const int kc = kt < last ? kt : last;
+                const T *src = Wd + c0 + (last >= 0 ? (size_t)k0 * H : (size_t)(n - 1) * H);
+                load_to_lds(dst, (unsigned)(last >= 0 ? kc : 0) * (unsigned)H * (unsigned)sizeof(T) + (unsigned)c * 16u,
+                            reinterpret_cast<const char *>(src));
+            }
+        }
+    };
+
+    f32x4_t acc[MI][4];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    struct Frag { uint4 a[MI], b[4]; };
+    Frag F0, F1;
+    const int bsw = 2 * ((l16 >> 2) | ((q & 1) << 2));   // pf_swz_b of the rows this lane hands in
+    auto rd = [&](Frag &F, int slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+            F.a[i] = lds[slot * kBuf + (16 * (MI * wm + i) + l16) * kPfLd1 + ((4 * kh + q) ^ fsw)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            pf_v4i16_t h[2];
+#pragma unroll
+            for (int hh = 0; hh < 2; ++hh) {
+                const int k = 32 * kh + 8 * q + 4 * hh + (l16 >> 2);
+                const int col = 64 * wn + 16 * j + 4 * (l16 & 3);
+                const unsigned short *p16 =
+                    reinterpret_cast<const unsigned short *>(&lds[slot * kBuf + kWdAt + k * 16 + ((col >> 3) ^ bsw)]) + (col & 7);
+                h[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pf_v4i16_t *)p16);
+            }
+            typedef short v8i16_t __attribute__((ext_vector_type(8)));
+            F.b[j] = __builtin_bit_cast(uint4, (v8i16_t)__builtin_shufflevector(h[0], h[1], 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+    };
+    auto mm = [&](const Frag &F) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = Mfma<T>::run(F.a[i], F.b[j], acc[i][j]);
+    };
+    auto stage = [&](int s, int slot, const Frag &Fc, Frag &Fn) __attribute__((always_inline)) {
+        const int next = slot == kSlots - 1 ? 0 : slot + 1;
+        if (s + kSlots <= nst) ST_WAIT_VM_LGKM0((kSlots - 2) * kDma); else ST_WAIT_VM_LGKM0(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        rd(Fn, next);   // (past the last stage: a stale slot, not used)
+        __builtin_amdgcn_sched_barrier(0);
+        if (s + kSlots < nst) dma(s + kSlots, slot);   // (loads that wait to be accepted do not hold up the reads)
+        mm(Fc);
+        __builtin_amdgcn_sched_barrier(0);
+        return next;
+    };
+    if (nst > 0) {
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s)
+            if (s < nst) dma(s, s);
+        if (nst >= kSlots) ST_WAIT_VM_LGKM0((kSlots - 1) * kDma); else ST_WAIT_VM_LGKM0(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        rd(F0, 0);
+        int slot = 0;
+        for (int s = 0; s < nst; s += 2) {
+            slot = stage(s, slot, F0, F1);
+            if (s + 1 < nst) slot = stage(s + 1, slot, F1, F0);
+        }
+    }
+
+    f32x4_t *red = reinterpret_cast<f32x4_t *>(lds) + (wave & 3) * MI * 4 * 64 + lane;
+    static_assert(4 * MI * 4 * 64 + 4 * 16 * MI * kPfStgF / 4 <= kSlots * kBuf, "sums and epilogue tiles exceed the stages");
+    __syncthreads();
+    if (kh == 1) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) red[(i * 4 + j) * 64] = acc[i][j];
+    }
+    __syncthreads();
+    if (kh == 1) return;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] += red[(i * 4 + j) * 64];
+    float *stg = reinterpret_cast<float *>(lds + 4 * MI * 4 * 64) + (size_t)wave * 16 * MI * kPfStgF;
+    pf_store_out<T>(acc, stg, lane, 16 * MI * wm, c0 + 64 * wn, M, H, Out, split_k == 1 ? nullptr : partial + (size_t)z * M * H);
+}
+
 // out[m, c] = sum over splits of partial[z][m][c]
 template <typename T>
 __global__ __launch_bounds__(256) void prefill_reduce_kernel(const float *__restrict__ partial, int split_k, int M,
@@ -1157,6 +1445,17 @@ static int prefill_split_k_wide(int M, int H, int n)
     return s < 1 ? 1 : s;
 }
 
+// Up to 128 rows: one block per CU, at least eight stages of the capacity per split.
+constexpr int kFewRows = 128;
+static int prefill_split_k_few(int H, int n)
+{
+    const int nk = (n + kPfBK - 1) / kPfBK * (kPfBK / kPfBK2);
+    int s = device_cu_count() / (H / kPfBN);
+    if (s > nk / 8) s = nk / 8;
+    if (s > 16) s = 16;
+    return s < 1 ? 1 : s;
+}
+
 int64_t prefill_ldh(int64_t n) { return (n + kPfBK - 1) / kPfBK * kPfBK; }
 
 int64_t prefill_workspace_bytes(int64_t M, int64_t H, int64_t n)
@@ -1168,7 +1467,7 @@ int64_t prefill_workspace_bytes(int64_t M, int64_t H, int64_t n)
 
 template <typename T>
 static int launch_prefill_t(const void *x, int M, int H, const void *gate, const void *up, const void *down, int n,
-                            const int *n_dev, void *out, void *comb, long ldc, void *workspace, int act, int has_gate,
+                            const int *n_dev, int n_hint, void *out, void *comb, long ldc, void *workspace, int act, int has_gate,
                             hipStream_t stream)
 {
     // The intermediate Hh normally sits in the workspace, padded with zero columns to a multiple of 128.  When the
@@ -1181,9 +1480,34 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
     if (alias) comb = nullptr;
     const int64_t hh_bytes = (((int64_t)M * ldw * 2) + 255) & ~(int64_t)255;
     float *partial = reinterpret_cast<float *>(static_cast<unsigned char *>(workspace) + hh_bytes);
-    const bool wide_down = prefill_down_is_wide(M, H, n, ldh);
-    const int split_k = wide_down ? prefill_split_k_wide(M, H, n) : prefill_split_k(M, H, n);
-    {
+    const bool few = M <= kFewRows, wide_down = !few && prefill_down_is_wide(M, H, n, ldh);
+    const int split_k = few ? prefill_split_k_few(H, n) : wide_down ? prefill_split_k_wide(M, H, n) : prefill_split_k(M, H, n);
+    // (four K groups on 64-row tiles, below, are faster for two of them while those make no more blocks than CUs: H 2048, 2500 of
+    // 4096 active rows, 128 rows 27.2 us for the whole forward with the few-row kernel, 24.8 so; with one row tile the few-row kernel is: H 1024, 48 rows 20.9 / 18.0)
+    const bool two_quarters = M > 64 && H % 256 == 0 && 4 * (ldw / 64) <= device_cu_count();
+    if (few && !two_quarters) {
+        ProfScope ps(ST_K_MLP_PREFILL_GATEUP, stream);
+        const int guess = n_dev && n_hint > 0 && n_hint < n ? n_hint : n, cus = device_cu_count();
+        const int guess_pad = (guess + kPfBK - 1) / kPfBK * kPfBK;
+        auto go = [&](auto kern, int rows) {
+            ST_LAUNCH(ps, kern, dim3((int)((ldw + rows - 1) / rows)), dim3(kPwThreads), 0, stream, static_cast<const T *>(x),
+                      static_cast<const T *>(gate), static_cast<const T *>(up), n_dev, M, H, n, Hh, ldh, static_cast<T *>(comb), ldc, act);
+        };
+        // active rows per block: the fewest that make no more blocks than CUs (a block's loads of x are the same for any)
+        auto rows = [&](auto mt) {
+            constexpr int MT = decltype(mt)::value;
+            if (has_gate) {
+                if (guess_pad <= 32 * cus) go(prefill_gateup_few_kernel<T, true, MT, 1>, 32);
+                else go(prefill_gateup_few_kernel<T, true, MT, 2>, 64);
+            } else {
+                if (guess_pad <= 32 * cus) go(prefill_gateup_few_kernel<T, false, MT, 1>, 32);
+                else go(prefill_gateup_few_kernel<T, false, MT, 2>, 64);
+            }
+        };
+        if (M <= 64) rows(std::integral_constant<int, 4>{});
+        else if (M <= 96) rows(std::integral_constant<int, 6>{});
+        else rows(std::integral_constant<int, 8>{});
+    } else {
         ProfScope ps(ST_K_MLP_PREFILL_GATEUP, stream);
         const int cus = device_cu_count();
         const int jt64 = (int)(ldw / 64), mt128 = (M + 127) / 128;
@@ -1222,7 +1546,16 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
     ST_HIP(hipGetLastError());
     {
         ProfScope ps(ST_K_MLP_PREFILL_DOWN, stream);
-        if (wide_down) {
+        if (few) {
+            const int ct = H / kPfBN, grid = (ct * split_k + kXcds - 1) / kXcds * kXcds;
+            auto go = [&](auto kern) {
+                ST_LAUNCH(ps, kern, dim3(grid), dim3(kPwThreads), 0, stream, Hh, static_cast<const T *>(down), n_dev, ldh, M, H, n,
+                          split_k, ct, static_cast<T *>(out), partial);
+            };
+            if (M <= 64) go(prefill_down_few_kernel<T, 4>);
+            else if (M <= 96) go(prefill_down_few_kernel<T, 6>);
+            else go(prefill_down_few_kernel<T, 8>);
+        } else if (wide_down) {
             const int ct = (H + kPfBN - 1) / kPfBN, mt = (M + kPwBM - 1) / kPwBM;
             const int grid = (ct * mt * split_k + kXcds - 1) / kXcds * kXcds;
             ST_LAUNCH(ps, prefill_down_wide_kernel<T>, dim3(grid), dim3(kPwThreads), 0, stream, Hh,
@@ -1246,13 +1579,13 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
 }
 
 int launch_prefill(int dtype, const void *x, int M, int H, const void *gate, const void *up, const void *down, int n,
-                   const int *n_dev, void *out, void *comb, long ldc, void *workspace, int act, int has_gate,
+                   const int *n_dev, int n_hint, void *out, void *comb, long ldc, void *workspace, int act, int has_gate,
                    hipStream_t stream)
 {
     if (dtype == ST_F16)
-        return launch_prefill_t<f16_t>(x, M, H, gate, up, down, n, n_dev, out, comb, ldc, workspace, act, has_gate,
+        return launch_prefill_t<f16_t>(x, M, H, gate, up, down, n, n_dev, n_hint, out, comb, ldc, workspace, act, has_gate,
                                        stream);
-    return launch_prefill_t<bf16_t>(x, M, H, gate, up, down, n, n_dev, out, comb, ldc, workspace, act, has_gate,
+    return launch_prefill_t<bf16_t>(x, M, H, gate, up, down, n, n_dev, n_hint, out, comb, ldc, workspace, act, has_gate,
                                     stream);
 }
 

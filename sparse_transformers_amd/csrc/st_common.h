@@ -259,7 +259,7 @@ constexpr int kPrefillMinRows = 32;
 constexpr int kBatchMaxRows = 32;
 int64_t prefill_workspace_bytes(int64_t M, int64_t H, int64_t n);
 int launch_prefill(int dtype, const void *x, int M, int H, const void *gate, const void *up, const void *down, int n,
-                   const int *n_dev, void *out, void *comb, long ldc, void *workspace, int act, int has_gate,
+                   const int *n_dev, int n_hint, void *out, void *comb, long ldc, void *workspace, int act, int has_gate,
                    hipStream_t stream);
 
 // MFMA kernels for a small batch of rows (batch_min_rows() <= B <= 32, fp16 / bf16, supported hidden sizes only).

@@ -339,6 +339,38 @@ def test_prefill_big_tiles(M, H, I, n, gated):
     assert_close(comb[:, :n].float().cpu().numpy(), h.cpu().numpy(), "float16", f"intermediate, {M} rows, {n} active")
 
 
+@pytest.mark.parametrize("M,H,I,n,gated", [
+    (33, 128, 1000, 1, True), (64, 384, 9000, 8192, True), (65, 1152, 9000, 8193, True), (96, 640, 8448, 8447, True),
+    (97, 128, 4096, 4033, True), (128, 1024, 8200, 8200, True),
+    (48, 256, 9000, 8192, False), (64, 1152, 520, 33, False), (77, 2560, 9000, 6144, False), (97, 384, 8300, 8300, False),
+    (128, 128, 8320, 8257, False), (96, 768, 300, 300, False),
+])
+def test_prefill_few_rows(M, H, I, n, gated):
+    """Up to 128 rows of x: every form of the two kernels (64, 96, 128 rows; the fewer or the more active rows per block, which
+    the guess of the count chooses and which must not show in a bit), K loops shorter and longer than the ring, splits of the
+    down projection without stages, rows past the device's count NaN.  Bounds as in the tests above."""
+    g = torch.Generator().manual_seed(M + n)
+    gate, up, dn = ((torch.randn(I, H, generator=g) * 0.05).half().to(DEV) for _ in range(3))
+    x = torch.randn(M, H, generator=g).half().to(DEV)
+    h = torch.nn.functional.silu((x.float() @ (gate if gated else up)[:n].float().t()))
+    if gated:
+        h = h * (x.float() @ up[:n].float().t())
+    want = h @ dn[:n].float()
+    for t in (gate, up, dn):
+        t[n:] = float("nan")
+    n_dev = torch.tensor([n], dtype=torch.int32, device=DEV)
+    first = None
+    for hint in (0, 1, n, I):
+        out = torch.full((M, H), float("nan"), dtype=torch.float16, device=DEV)
+        comb = torch.full((M, (2 if gated else 1) * I), float("nan"), dtype=torch.float16, device=DEV)
+        mlp_forward_rows(x, gate if gated else None, up, dn, I, n_dev, out, comb, "silu", gated, n_hint=hint)
+        torch.cuda.synchronize()
+        assert_close(out.float().cpu().numpy(), want.cpu().numpy(), "float16", f"{M} rows, {n} active, guess {hint}")
+        assert_close(comb[:, :n].float().cpu().numpy(), h.cpu().numpy(), "float16", f"intermediate, {M} rows, {n} active")
+        first = out if first is None else first
+        assert torch.equal(first, out)
+
+
 def test_prefill_agrees_with_decode_kernel():
     """The MFMA path (B = 40) and the streaming path (the same rows, 4 at a time) agree to rounding."""
     x, cw, dn = _case(22, 40, 1024, 700, "float16", True)
