@@ -97,19 +97,20 @@ __global__ __launch_bounds__(TPB) void mlp_decode_kernel(
 
     // row of (batch, slot k) for this thread's group
     auto row_of = [&](int bat, int k) { return blk + G * (grp + ngrp * (bat * RB + k)); };
-    // Loads are issued unconditionally from a clamped row / chunk: a branch around every load costs far
-    // more than a few duplicate (cache-hit) loads.  What a clamped load returns is never used: x is zero
-    // on chunks past the row end, h is forced to zero for rows >= n, and the down row is replaced by
-    // zeros where it is consumed.  limit >= 1.
+    // Loads are issued unconditionally: a branch around every load costs far more than a few duplicate (cache-hit)
+    // loads.  A row past the limit reads the first 16 bytes of the buffer for the whole wave, a single request (the last row
+    // instead, whole, by every block that had slots to spare: 14.9 instead of 13.9 us, with the reduction, for 2200
+    // rows at H 3072, five for six slots).  What such a load returns is never used: x is
+    // zero on chunks past the row end, h is forced to zero for rows >= n, and the down row is replaced by zeros where it is
+    // consumed.
     auto load_batch = [&](RowBatch<RB, CPT> &w, int bat, int limit) __attribute__((always_inline)) {
         if (!wave_live) return;
 #pragma unroll
         for (int k = 0; k < RB; ++k) {
             const int row = row_of(bat, k);
-            const size_t ro = (size_t)(row < limit ? row : limit - 1) * H;
 #pragma unroll
             for (int q = 0; q < CPT; ++q) {
-                const size_t o = ro + coff[q];
+                const size_t o = row < limit ? (size_t)row * H + coff[q] : 0;
                 w.u[k][q] = ld16_stream(up + o);
                 w.d[k][q] = ld16_stream(down + o);
                 w.g[k][q] = has_gate ? ld16_stream(gate + o) : zero4;
@@ -402,13 +403,15 @@ template <typename T, int NB> static int launch_one(const MlpLaunch &a, int b0, 
         // (the rows in flight do not change which rows a group sums or in which order: when the expected count
         // gives a group seven rows, one batch of seven beats a batch of six followed by a batch of one; likewise
         // wherever sevens need fewer batches than sixes)
-        if constexpr (Elem<T>::kBytes == 2) {
-            int gs_log2 = 6;
-            while ((1 << gs_log2) < chunks && (1 << gs_log2) < 1024) ++gs_log2;
-            const int ngrp = 1024 >> gs_log2, expect = a.n_dev ? (a.n_hint < a.n ? a.n_hint : a.n) : a.n;
-            const int rpg = ((expect + a.G - 1) / a.G + ngrp - 1) / ngrp;
+        // (and three slots where three rows at most are expected.  With the reduction, six / three: 1100 rows ungated at H 4096
+        // 12.9 / 10.8 us, 1500 gated 15.5 / 13.3, 500 gated at H 1024 11.8 / 8.7)
+        int gs_log2 = 6;
+        while ((1 << gs_log2) < chunks && (1 << gs_log2) < 1024) ++gs_log2;
+        const int ngrp = 1024 >> gs_log2, expect = a.n_dev ? (a.n_hint < a.n ? a.n_hint : a.n) : a.n;
+        const int rpg = ((expect + a.G - 1) / a.G + ngrp - 1) / ngrp;
+        if (rpg >= 1 && rpg <= 3) return launch_inst<T, 1, 3, 1, 1024, false>(a, b0, bcount);
+        if constexpr (Elem<T>::kBytes == 2)
             if ((rpg + 6) / 7 < (rpg + 5) / 6) return launch_inst<T, 1, 7, 1, 1024, false>(a, b0, bcount);   // 7, 13, 14, ...
-        }
         return launch_inst<T, 1, DecodeRows<T>::value, 1, 1024, false>(a, b0, bcount);
     } else if constexpr (NB == 2) {
         return launch_inst<T, 2, 2, 1, 1024, true>(a, b0, bcount);
