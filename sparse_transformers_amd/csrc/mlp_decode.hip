@@ -387,6 +387,16 @@ static int env_int(const char *name)
     return v ? atoi(v) : 0;
 }
 
+// Rows a thread group of a 1024-thread block sums, on the expected count.
+template <typename T> static int rows_per_group(const MlpLaunch &a)
+{
+    const int chunks = a.H / Elem<T>::kVec;
+    int gs_log2 = 6;
+    while ((1 << gs_log2) < chunks && (1 << gs_log2) < 1024) ++gs_log2;
+    const int ngrp = 1024 >> gs_log2, expect = a.n_dev ? (a.n_hint < a.n ? a.n_hint : a.n) : a.n;
+    return ((expect + a.G - 1) / a.G + ngrp - 1) / ngrp;
+}
+
 // The launch shape trades registers for loads in flight: measured on MI355X,
 // about 12-18 outstanding 16-byte loads per thread with 16 waves per CU
 // streams fastest; many more per thread is slower.  RB is the depth of ONE of
@@ -405,15 +415,17 @@ template <typename T, int NB> static int launch_one(const MlpLaunch &a, int b0, 
         // wherever sevens need fewer batches than sixes)
         // (and three slots where three rows at most are expected.  With the reduction, six / three: 1100 rows ungated at H 4096
         // 12.9 / 10.8 us, 1500 gated 15.5 / 13.3, 500 gated at H 1024 11.8 / 8.7)
-        int gs_log2 = 6;
-        while ((1 << gs_log2) < chunks && (1 << gs_log2) < 1024) ++gs_log2;
-        const int ngrp = 1024 >> gs_log2, expect = a.n_dev ? (a.n_hint < a.n ? a.n_hint : a.n) : a.n;
-        const int rpg = ((expect + a.G - 1) / a.G + ngrp - 1) / ngrp;
+        const int rpg = rows_per_group<T>(a);
         if (rpg >= 1 && rpg <= 3) return launch_inst<T, 1, 3, 1, 1024, false>(a, b0, bcount);
         if constexpr (Elem<T>::kBytes == 2)
             if ((rpg + 6) / 7 < (rpg + 5) / 6) return launch_inst<T, 1, 7, 1, 1024, false>(a, b0, bcount);   // 7, 13, 14, ...
         return launch_inst<T, 1, DecodeRows<T>::value, 1, 1024, false>(a, b0, bcount);
     } else if constexpr (NB == 2) {
+        // (one batch where it holds what is expected: 2867 rows, six per group, at H 3072 19.5 us in double-buffered batches of
+        // two, 18.7 so; 1100 ungated at H 4096 15.4 / 14.4 with three)
+        const int rpg = rows_per_group<T>(a);
+        if (rpg >= 1 && rpg <= 3) return launch_inst<T, 2, 3, 1, 1024, false>(a, b0, bcount);
+        if (rpg >= 1 && rpg <= 6) return launch_inst<T, 2, 6, 1, 1024, false>(a, b0, bcount);
         return launch_inst<T, 2, 2, 1, 1024, true>(a, b0, bcount);
     } else if constexpr (NB == 4) {
         if (chunks > 512) return launch_inst<T, 4, 1, 2, 512, true>(a, b0, bcount);
