@@ -99,6 +99,25 @@ def lib() -> C.CDLL:
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The eager entry points' host side (csrc/host_ext.cpp), bound to the library; like the library it has no substitute."""
+    global _native
+    if _native is None:
+        L = lib()
+        try:
+            from . import _host
+        except ImportError as e:
+            raise NativeLibraryMissing(f"{HERE}/_host.so cannot be loaded ({e}): build it with "
+                                       "`python -m sparse_transformers_amd.build`") from e
+        _host.bind(*(C.cast(getattr(L, f), C.c_void_p).value
+                     for f in ("st_predictor_mask_ex", "st_cache_update_forward", "st_mlp_forward")))
+        _native = _host
+    return _native
+
+
 def last_error() -> str:
     return lib().st_last_error().decode("utf-8", "replace")
 

@@ -56,6 +56,26 @@ def build(verbose: bool = True) -> str:
     return LIB_PATH
 
 
+def build_host(verbose: bool = True) -> str:
+    """_host.so: the Python entry points' argument handling as a CPython extension against the installed torch (host code
+    only; it calls the library through addresses it is given)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    out = os.path.join(HERE, "_host.so")
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+                    f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+                    *[f for d in cpp_extension.include_paths() for f in ("-isystem", d)], "-I" + sysconfig.get_path("include"),
+                    os.path.join(CSRC, "host_ext.cpp"), "-o", out, "-L" + libs, "-ltorch_python", "-ltorch_cpu", "-lc10",
+                    "-Wl,-rpath," + libs], check=True)
+    if verbose:
+        print(f"[build] wrote {out}", flush=True)
+    return out
+
+
 def build_capi_client(verbose: bool = True) -> str:
     """tests/capi/capi_client: a C++ client of the C ABI that links nothing but the library and the HIP
     runtime (run by tests/test_gpu_capi_client.py on the GPU box)."""
@@ -71,5 +91,6 @@ def build_capi_client(verbose: bool = True) -> str:
 
 if __name__ == "__main__":
     build()
+    build_host()
     build_capi_client()
     sys.exit(0)

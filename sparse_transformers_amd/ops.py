@@ -189,6 +189,18 @@ def sparse_mlp_forward(x: torch.Tensor, concat_weight: torch.Tensor, active_down
     global _warned_layout
     from .weight_cache import ConcatWeightHandle
     handle = concat_weight if isinstance(concat_weight, ConcatWeightHandle) and concat_weight._real is None else None
+    if handle is not None and x.is_cuda and x.dim() == 2 and act in _lib.ACT_CODES and has_gate == handle._cache.has_gate \
+            and handle.fresh():
+        # the reference's call sequence natively: the cache's packed rows in place (None: something is not as usual)
+        c, n = handle._cache, handle._n
+        ws = _kept_workspace(c.device, mlp_workspace_bytes(x.size(0), c.hidden_size, n))
+        got = _lib.native().mlp_forward(x, c.gate_active if has_gate else None, c.up_active, active_down_weight, n, None,
+                                        down_proj_buffer, combined_proj_buffer, 0, ws, _lib.ACT_CODES[act],
+                                        current_stream_ptr(c.device), True)
+        if got is not None:
+            if type(got) is int:
+                _lib.check(got, "st_mlp_forward")
+            return got
     if isinstance(concat_weight, ConcatWeightHandle) and handle is None:
         concat_weight = concat_weight.materialize()
     dev = require_gpu(x, concat_weight, active_down_weight, down_proj_buffer, combined_proj_buffer)
@@ -254,6 +266,19 @@ def predictor_mask(x: torch.Tensor, down_weight: torch.Tensor, up_weight: torch.
     ``round_to_storage``: round the rank-r intermediate and the scores to x's dtype before they are used, as the
     reference's two half-precision modules do (by default both stay in fp32).
     """
+    if x.is_cuda and x.dim() == 2 and up_weight.dim() == 2:   # the common form natively (None: not one)
+        B, I = x.size(0), up_weight.size(0)
+        scores = scores_out
+        if scores is None and return_scores:
+            scores = torch.empty(B, I, dtype=torch.float32, device=x.device)
+        got = _lib.native().predictor_mask(x, down_weight, up_weight, thr, ge, out, t_ws, scores, 1 if round_to_storage else 0,
+                                           current_stream_ptr(x.device))
+        if got is not None:
+            if type(got) is int:
+                _lib.check(got, "st_predictor_mask_ex")
+            if scores is None:
+                return got
+            return got, scores if scores_out is None else scores_out.view(-1)[:B * I].view(B, I)
     dev = require_gpu(x, down_weight, up_weight, out)
     H = x.shape[-1]
     x2 = x if x.dim() == 2 else x.reshape(-1, H)

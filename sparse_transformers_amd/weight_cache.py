@@ -159,6 +159,7 @@ class WeightCache:
         self._pending_mask: Optional[torch.Tensor] = None
         self._concat_ref = None     # weak reference to the handle get_concat_weight() handed out last
         self._concat_serial = -1
+        self._ws_need: dict = {}    # workspace bytes by rows of x (at most 4096 of them)
         # weight_cache.h:226: the constructor ends with update_active_weights(init_mask); here in one pass over the weights
         mask = self._mask_arg(init_mask)
         rc = L.st_cache_load_weights_masked(self._h, gate_c.data_ptr() if self.has_gate else None, up_c.data_ptr(),
@@ -278,6 +279,28 @@ class WeightCache:
         x2 = x if x.dim() == 2 else x.reshape(-1, H)
         return x2 if x2.is_contiguous() else x2.contiguous()
 
+    def _native_call(self, x, act, out, workspace, call):
+        """The common form of a call through the native host path: rows of x as they are, a workspace that is large enough.
+        None: not that form (nothing has been done)."""
+        code = _lib.ACT_CODES.get(act)
+        if code is None or not x.is_cuda or x.dim() == 0:
+            return None
+        x2 = x
+        if x.dim() != 2:
+            if out is not None or x.shape[-1] != self.hidden_size or not x.is_contiguous():
+                return None
+            x2 = x.view(-1, self.hidden_size)
+        B = x2.size(0)
+        need = self._ws_need.get(B)
+        if need is None:
+            need = self._ws_need[B] = mlp_workspace_bytes(B, self.hidden_size, self.intermediate_size)
+        if workspace is None:
+            workspace = _kept_workspace(self.device, need)
+        elif workspace.numel() < need:
+            return None
+        got = call(x2, workspace, code, current_stream_ptr(self.device))
+        return got if got is None or type(got) is int or x.dim() == 2 else got.view(x.shape)
+
     def update_and_forward(self, mask: torch.Tensor, x: torch.Tensor, act: str = "silu",
                            out: Optional[torch.Tensor] = None, combined: Optional[torch.Tensor] = None,
                            n_hint: Optional[int] = None, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -288,6 +311,14 @@ class WeightCache:
         the last count an update told the host) only steers what the kernel requests before it knows the true count.
         ``workspace``: a caller-owned uint8 buffer of ``mlp_workspace_bytes(B, H, I)`` bytes (default: one
         kept per device and stream)."""
+        if combined is None and self._pending_mask is None and (self._concat_ref is None or self._concat_ref() is None):
+            got = self._native_call(x, act, out, workspace, lambda x2, ws, code, stream: _lib.native().update_forward(
+                self._h, self.up_pool, mask, x2, out, ws, self.intermediate_size, -1 if n_hint is None else n_hint, code, stream))
+            if got is not None:
+                if type(got) is int:
+                    _lib.check(got, "st_cache_update_forward")
+                self._dirty = True
+                return got
         m = self._mask_arg(mask)
         self._flush_pending()
         H, I = self.hidden_size, self.intermediate_size
@@ -322,6 +353,14 @@ class WeightCache:
             if combined is None or combined.size(-1) >= (2 if self.has_gate else 1) * self.intermediate_size:
                 return self.update_and_forward(m, x, act, out=out, combined=combined, workspace=workspace)
             self.update_active_weights_async(m)   # `combined` is sized for the current count only: two calls
+        if combined is None:
+            got = self._native_call(x, act, out, workspace, lambda x2, ws, code, stream: _lib.native().mlp_forward(
+                x2, self.gate_active, self.up_active, self.down_active, self.intermediate_size, self.n_active_dev, out, None,
+                self._seen.value, ws, code, stream, False))
+            if got is not None:
+                if type(got) is int:
+                    _lib.check(got, "st_mlp_forward")
+                return got
         x2 = self._x_rows(x)
         if out is None:
             out = torch.empty_like(x2)

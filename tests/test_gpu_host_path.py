@@ -1,0 +1,203 @@
+"""The native host path (csrc/host_ext.cpp) against the Python code that takes every form of a call: the same bits, or the same
+exception with the same words, for each form -- with the native functions answering None the general path runs alone."""
+import threading
+
+import pytest
+import torch
+
+import sparse_transformers_amd as st
+from sparse_transformers_amd import _lib
+
+DEV = "cuda:0"
+
+
+class _Nothing:
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+def test_native_functions_leave_everything_else_to_python():
+    """On the CPU: other devices, subclasses, transforms' wrappers, wrong counts and types of arguments."""
+    nat = _lib.native()
+    x, A, Bm = torch.zeros(1, 16), torch.zeros(8, 16), torch.zeros(32, 8)
+    assert nat.predictor_mask(x, A, Bm, 0.0, True, None, None, None, 0, 0) is None
+    assert nat.predictor_mask(x, A) is None and nat.update_forward() is None and nat.mlp_forward(1, 2, 3) is None
+    assert nat.predictor_mask(None, "a", 3, [], {}, 1.5, x, x, x, x) is None
+    assert nat.update_forward(*[x] * 10) is None and nat.mlp_forward(*[None] * 13) is None
+
+    class Sub(torch.Tensor):
+        pass
+    assert nat.predictor_mask(x.as_subclass(Sub), A, Bm, 0.0, True, None, None, None, 0, 0) is None
+    seen = []
+    torch.func.vmap(lambda v: (seen.append(nat.mlp_forward(v, None, v, v, 1, None, None, None, 0, v, 0, 0, False)), v)[1])(torch.zeros(2, 3, 4))
+    torch.func.grad(lambda v: (seen.append(nat.mlp_forward(v, None, v, v, 1, None, None, None, 0, v, 0, 0, False)), v.sum())[1])(torch.zeros(3, 4))
+    assert seen == [None, None]
+    with pytest.raises(TypeError):
+        nat.bind(1)
+
+
+def _both(monkeypatch, f):
+    """f() with and without the native path: (kind, payload) of each."""
+    got = []
+    for native in (None, _Nothing()):
+        with monkeypatch.context() as m:
+            if native is not None:
+                m.setattr(_lib, "native", lambda: native)
+            try:
+                r = f()
+                r = r if isinstance(r, (tuple, list)) else (r,)
+                torch.cuda.synchronize()
+                got.append(("value", [(t.clone(), tuple(t.shape), t.stride(), t.dtype) for t in r]))
+            except Exception as e:
+                got.append((type(e).__name__, str(e)))
+    return got
+
+
+def _same(a, b):
+    if a[0] != "value" or b[0] != "value":
+        assert a == b
+        return
+    for x, y in zip(a[1], b[1]):
+        assert x[1:] == y[1:] and torch.equal(x[0], y[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16, torch.float64, torch.int32])
+def test_predictor_mask_forms(monkeypatch, dtype):
+    H, r, I, B = 64, 16, 200, 3
+    g = torch.Generator().manual_seed(1)
+    x, A, Bm = ((torch.randn(s, generator=g) * 2).to(dtype).to(DEV) for s in ((B, H), (r, H), (I, r)))
+    f32 = dict(dtype=torch.float32, device=DEV)
+    forms = [
+        lambda: st.predictor_mask(x, A, Bm, 0.5), lambda: st.predictor_mask(x, A, Bm, 0.5, False, True),
+        lambda: st.predictor_mask(x[:1], A, Bm, 0.5, round_to_storage=True), lambda: st.predictor_mask(x[0], A, Bm),
+        lambda: st.predictor_mask(x.view(1, B, H), A, Bm), lambda: st.predictor_mask(x.t().contiguous().t(), A, Bm),
+        lambda: st.predictor_mask(x, A.t().contiguous().t(), Bm), lambda: st.predictor_mask(x, A, Bm[::2]),
+        lambda: st.predictor_mask(x, torch.nn.Parameter(A) if dtype.is_floating_point else A, Bm),
+        lambda: st.predictor_mask(x, A[:, :32], Bm), lambda: st.predictor_mask(x, A, Bm[:, :8]), lambda: st.predictor_mask(x, A[0], Bm),
+        lambda: st.predictor_mask(x, A.to(torch.float16), Bm), lambda: st.predictor_mask(x, A.cpu(), Bm), lambda: st.predictor_mask(x.cpu(), A, Bm),
+        lambda: st.predictor_mask(x, A, Bm, out=torch.zeros(I, dtype=torch.bool, device=DEV)),
+        lambda: st.predictor_mask(x, A, Bm, out=torch.zeros(I - 1, dtype=torch.bool, device=DEV)),
+        lambda: st.predictor_mask(x, A, Bm, out=torch.zeros(I, dtype=torch.uint8, device=DEV)),
+        lambda: st.predictor_mask(x, A, Bm, out=torch.zeros(2 * I, dtype=torch.bool, device=DEV)[::2]),
+        lambda: st.predictor_mask(x, A, Bm, t_ws=torch.zeros(B * r, **f32)), lambda: st.predictor_mask(x, A, Bm, t_ws=torch.zeros(3, **f32)),
+        lambda: st.predictor_mask(x, A, Bm, t_ws=torch.zeros(B * r)),
+        lambda: st.predictor_mask(x, A, Bm, scores_out=torch.zeros(2 * B * I, **f32)),
+        lambda: st.predictor_mask(x, A, Bm, scores_out=torch.zeros(3, **f32)), lambda: st.predictor_mask(x, A, Bm, "a"),
+        lambda: st.predictor_scores(x[:0], A, Bm), lambda: st.predictor_scores(x, A, Bm),
+    ]
+    for f in forms:
+        _same(*_both(monkeypatch, f))
+
+
+def _cache(dtype=torch.float16, H=256, I=512, gated=True, seed=2):
+    g = torch.Generator().manual_seed(seed)
+    gate, up, down = ((torch.randn(s, generator=g) * 0.1).to(dtype).to(DEV) for s in ((I, H), (I, H), (H, I)))
+    ones = torch.ones(I, dtype=torch.bool, device=DEV)
+    return st.WeightCache(ones, H, gate if gated else None, up, down, gated), g
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("gated", [True, False])
+def test_cache_call_forms(monkeypatch, gated):
+    H, I, B = 256, 512, 4
+    x = torch.randn(B, H, generator=torch.Generator().manual_seed(5)).half().to(DEV)
+    mask = (torch.rand(I, generator=torch.Generator().manual_seed(6)) < 0.4).to(DEV)
+
+    def fresh(f):
+        def run():
+            c, _ = _cache(gated=gated)
+            r = f(c)
+            return (r, c.get_active_indices()) if isinstance(r, torch.Tensor) else (*r, c.get_active_indices())
+        return run
+
+    def lazy(c):
+        c.lazy_updates = True
+        c.update_active_weights(mask)
+        return c.update_and_forward(~mask, x)
+
+    def held(c):
+        w = c.get_concat_weight()           # alive across the update: filled first
+        return c.update_and_forward(mask, x), w + 0
+    half = lambda *s: torch.zeros(*s, dtype=torch.float16, device=DEV)
+    forms = [
+        lambda c: c.update_and_forward(mask, x), lambda c: c.update_and_forward(mask, x[:1], "relu"), lambda c: c.update_and_forward(mask, x[0]),
+        lambda c: c.update_and_forward(mask, x.view(2, 2, H)), lambda c: c.update_and_forward(mask.to(torch.uint8) * 3, x),
+        lambda c: c.update_and_forward(mask.int(), x), lambda c: c.update_and_forward(mask.cpu(), x), lambda c: c.update_and_forward(mask[:-1], x),
+        lambda c: c.update_and_forward(torch.stack([mask, mask], 1)[:, 0], x), lambda c: c.update_and_forward(mask, x.float()),
+        lambda c: c.update_and_forward(mask, x[:, :-8]), lambda c: c.update_and_forward(mask, x.t().contiguous().t()),
+        lambda c: c.update_and_forward(mask, x, "tanh"), lambda c: c.update_and_forward(mask, x.cpu()), lambda c: c.update_and_forward(mask, x[:0]),
+        lambda c: c.update_and_forward(mask, x, out=half(B, H)), lambda c: c.update_and_forward(mask, x, out=half(B, H + 1)),
+        lambda c: c.update_and_forward(mask, x, out=half(B, H).float()), lambda c: c.update_and_forward(mask, x, out=half(H, B).t()),
+        lambda c: c.update_and_forward(mask, x, workspace=torch.zeros(1 << 24, dtype=torch.uint8, device=DEV)),
+        lambda c: c.update_and_forward(mask, x, workspace=torch.zeros(64, dtype=torch.uint8, device=DEV)),
+        lambda c: c.update_and_forward(mask, x, workspace=torch.zeros(1 << 24, dtype=torch.int8, device=DEV)),
+        lambda c: c.update_and_forward(mask, x, combined=half(B, 2 * I)), lambda c: c.update_and_forward(mask, x, n_hint=7),
+        lazy, held,
+        lambda c: c.forward(x), lambda c: c.forward(x.view(1, B, H), "relu"), lambda c: c.forward(x[:1], out=half(1, H)),
+        lambda c: c.forward(x, out=half(B + 1, H)), lambda c: c.forward(x.float()), lambda c: c.forward(x, "swish"),
+        lambda c: c.forward(x, workspace=torch.zeros(8, dtype=torch.uint8, device=DEV)), lambda c: c.forward(x[:, ::1], "gelu_pytorch_tanh"),
+    ]
+    for f in forms:
+        _same(*_both(monkeypatch, fresh(f)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("gated", [True, False])
+def test_operator_forms(monkeypatch, gated):
+    H, I, B = 256, 512, 2
+    x = torch.randn(B, H, generator=torch.Generator().manual_seed(7)).half().to(DEV)
+    mask = (torch.rand(I, generator=torch.Generator().manual_seed(8)) < 0.3).to(DEV)
+    half = lambda *s: torch.zeros(*s, dtype=torch.float16, device=DEV)
+
+    def call(f):
+        def run():
+            c, _ = _cache(gated=gated)
+            c.update_active_weights(mask)
+            n = c.get_num_active()
+            bufs = [half(B, H), half(B, (2 if gated else 1) * n)]
+            return (f(c, bufs, n), *bufs)
+        return run
+    F = st.sparse_mlp_forward
+    forms = [
+        lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), *b, "silu", gated),
+        lambda c, b, n: F(x, c.get_concat_weight() + 0, c.get_active_down_weight(), *b, "silu", gated),
+        lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight().contiguous(), *b, "relu", gated),
+        lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight()[:, :-1], *b, "silu", gated),
+        lambda c, b, n: F(x[:1], c.get_concat_weight(), c.get_active_down_weight(), *b, "silu", gated),        # resized
+        lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), b[0].resize_(1, 8), b[1].resize_(3), "silu", gated),
+        lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), half(H, B).t(), b[1], "silu", gated),
+        lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), b[0], b[1].float(), "silu", gated),
+        lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), b[0].cpu(), b[1], "silu", gated),
+        lambda c, b, n: F(x.view(B, 1, H), c.get_concat_weight(), c.get_active_down_weight(), *b, "silu", gated),
+        lambda c, b, n: F(x.float(), c.get_concat_weight(), c.get_active_down_weight(), *b, "silu", gated),
+        lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), *b, "silu", not gated),
+        lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), *b, "cube", gated),
+        lambda c, b, n: (lambda w, d: (c.update_active_weights(~mask), F(x, w, d, *b, "silu", gated))[1])(c.get_concat_weight(), c.get_active_down_weight()),
+    ]
+    for f in forms:
+        _same(*_both(monkeypatch, call(f)))
+
+
+@pytest.mark.gpu
+def test_threads_and_streams():
+    """Several threads, each with a cache and a stream of its own, through the native path: the results of one thread alone."""
+    c0, _ = _cache()
+    x = torch.randn(1, 256, generator=torch.Generator().manual_seed(9)).half().to(DEV)
+    masks = [(torch.rand(512, generator=torch.Generator().manual_seed(i)) < 0.3).to(DEV) for i in range(6)]
+    sequence = lambda c: [c.update_and_forward(m, x).clone() for _ in range(20) for m in masks]   # (the list's order has a history)
+    want = sequence(c0)
+    caches = [_cache()[0] for _ in range(4)]
+    torch.cuda.synchronize()
+    got = [None] * 4
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            got[i] = sequence(caches[i])
+            torch.cuda.current_stream().synchronize()
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join(60)
+    assert all(torch.equal(a, b) for g in got for a, b in zip(g, want))
