@@ -22,10 +22,12 @@ constexpr int kPredDownUnroll = 2;  // chunks per thread issued together
 template <typename T, int BT, typename Tab>
 __global__ __launch_bounds__(kPredDownThreads) void predictor_down_kernel(const T *__restrict__ x, int B, int H,
                                                                           const T *__restrict__ A, int r,
-                                                                          float *__restrict__ t, int round_storage, Tab tab)
+                                                                          float *__restrict__ t, int round_storage,
+                                                                          uint8_t *__restrict__ mask, int I, Tab tab)
 {
     if constexpr (Tab::kLayers) {
         A = static_cast<const T *>(tab.l[blockIdx.y].A);
+        if (I > 0) mask = tab.l[blockIdx.y].mask;
         x += (size_t)blockIdx.y * B * H;
         t += (size_t)blockIdx.y * B * r;
     }
@@ -35,6 +37,9 @@ __global__ __launch_bounds__(kPredDownThreads) void predictor_down_kernel(const 
     const int chunks = H / VEC;
     const T *row = A + (size_t)k * H;
     const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
+    // (I > 0: the kernel behind this one only switches bytes of the mask on; r blocks)
+    if constexpr (BT == kPredBTile)
+        for (int i = k * kPredDownThreads + tid; i < I; i += r * kPredDownThreads) mask[i] = 0;
     for (int b0 = 0; b0 < B; b0 += BT) {
         float acc[BT];
 #pragma unroll
@@ -328,17 +333,23 @@ static void launch_up(ProfScope &ps, const PredLaunch &a, const Tab &tab)
 template <typename T, typename Tab>
 static int launch_predictor(const PredLaunch &a, const Tab &tab)
 {
+    constexpr int dtype = Elem<T>::kBytes == 4 ? ST_F32 : __is_same(T, f16_t) ? ST_F16 : ST_BF16;
+    // (not a later pass over more rows of x, which must not clear what an earlier one switched on: those have up to 64 rows each)
+    const bool up_mfma = (a.flags & 4) == 0 && predictor_up_mfma_supported(dtype, a.B, a.r, a.I);
     {
         ProfScope ps(ST_K_PRED_DOWN, a.stream);
         auto go = [&](auto kern) {
             ST_LAUNCH(ps, kern, dim3(a.r, a.layers), dim3(kPredDownThreads), 0, a.stream, static_cast<const T *>(a.x), a.B,
-                      a.H, static_cast<const T *>(a.A), a.r, a.t_ws, (a.flags >> 1) & 1, tab);
+                      a.H, static_cast<const T *>(a.A), a.r, a.t_ws, (a.flags >> 1) & 1, a.mask, up_mfma ? a.I : 0, tab);
         };
         if (a.B == 1) go(predictor_down_kernel<T, 1, Tab>);
         else if (a.B <= kPredBTile) go(predictor_down_kernel<T, kPredBTile, Tab>);
         else go(predictor_down_kernel<T, 2 * kPredBTile, Tab>);   // 9 to 16 rows of x in one pass (one memory round trip instead of two)
     }
     ST_HIP(hipGetLastError());
+    if (up_mfma)
+        return launch_predictor_up_mfma(dtype, tab, a.layers, a.B, a.r, a.Bm, a.I, a.thr, a.flags & 1, a.t_ws, a.scores, a.mask,
+                                        (a.flags >> 1) & 1, a.stream);
     const int chunks = a.r / Elem<T>::kVec;
     {
         ProfScope ps(ST_K_PRED_UP_MASK, a.stream);

@@ -439,38 +439,13 @@ bool predictor_mfma_supported(int dtype, int B, int H, int r)
     return dtype != ST_F32 && B > 8 && r <= 512 && H < (1 << 26);
 }
 
+// The second kernel alone.  What it switches on has to be off.
 template <typename T, typename Tab>
-static int launch_t(const Tab &tab, int layers, const void *x, int B, int H, const void *A, int r, const void *Bm, int I,
-                    float thr, int cmp_ge, float *t_ws, float *scores, uint8_t *mask, int round_storage, hipStream_t stream)
+static int launch_up_t(const Tab &tab, int layers, int B, int r, const void *Bm, int I, float thr, int cmp_ge, float *t_ws,
+                       float *scores, uint8_t *mask, int round_storage, hipStream_t stream)
 {
     // (the CUs a layer can count on when several share the launch)
     const int cus = (device_cu_count() + layers - 1) / layers;
-    {
-        ProfScope ps(ST_K_PRED_DOWN, stream);
-        auto go = [&](auto kern, int mi, int ni, int waves, int row_chunks) -> int {
-            int mt = (B + 16 * mi - 1) / (16 * mi);
-            const int nt = (r + 16 * ni - 1) / (16 * ni);
-            if (mt > kXcds) mt = (mt + kXcds - 1) / kXcds * kXcds;
-            const int lds = waves * 16 * (mi + ni) * row_chunks * 16;
-            const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
-            if (rc != ST_OK) return rc;
-            ST_LAUNCH(ps, kern, dim3(mt, nt, layers), dim3(waves * kWave), lds, stream, static_cast<const T *>(x),
-                      static_cast<const T *>(A), B, H, r, t_ws, mask, I, mt << 1 | (round_storage ? 1 : 0), mt * nt, tab);
-            return ST_OK;
-        };
-        auto blocks = [&](int mi, int ni) { return ((B + 16 * mi - 1) / (16 * mi)) * ((r + 16 * ni - 1) / (16 * ni)); };
-        // The largest tile of which there is one for three quarters of the CUs (by the shape alone: how many layers share the
-        // launch must not change how the sums are split).  32 x 32 tiles have half the traffic from L2: 6.7 (16 x 16) against
-        // 8.6 us with 64 of them (512 rows, H 3072, rank 128), 17.8 against 11.8 us with 224, 40 against 26 us with 512.  64 x
-        // 32 tiles a quarter less again and 96 KB of loads in flight instead of 64, both kernels, 32 x 32 / 64 x 32: 33.7 / 35.0
-        // us with 128 of them (1024 rows, H 4096, rank 256), 57.4 / 52.0 with 192, 54.9 / 48.4 with 256 (2048 rows).
-        const int want = 3 * device_cu_count();
-        const int rc = 4 * blocks(4, 2) >= want   ? go(predictor_down_mfma_kernel<T, 4, 2, 4, 8, 3, Tab>, 4, 2, 4, 24)
-                       : 4 * blocks(2, 2) >= want ? go(predictor_down_mfma_kernel<T, 2, 2, 4, 16, 2, Tab>, 2, 2, 4, 32)
-                                                  : go(predictor_down_mfma_kernel<T, 1, 1, 8, 16, 2, Tab>, 1, 1, 8, 32);
-        if (rc != ST_OK) return rc;
-    }
-    ST_HIP(hipGetLastError());
     {
         ProfScope ps(ST_K_PRED_UP_MASK, stream);
         // resident: blocks a CU holds at once (registers, LDS).  One round of blocks: every further one would split its
@@ -514,6 +489,39 @@ static int launch_t(const Tab &tab, int layers, const void *x, int B, int H, con
     return ST_OK;
 }
 
+template <typename T, typename Tab>
+static int launch_t(const Tab &tab, int layers, const void *x, int B, int H, const void *A, int r, const void *Bm, int I,
+                    float thr, int cmp_ge, float *t_ws, float *scores, uint8_t *mask, int round_storage, hipStream_t stream)
+{
+    {
+        ProfScope ps(ST_K_PRED_DOWN, stream);
+        auto go = [&](auto kern, int mi, int ni, int waves, int row_chunks) -> int {
+            int mt = (B + 16 * mi - 1) / (16 * mi);
+            const int nt = (r + 16 * ni - 1) / (16 * ni);
+            if (mt > kXcds) mt = (mt + kXcds - 1) / kXcds * kXcds;
+            const int lds = waves * 16 * (mi + ni) * row_chunks * 16;
+            const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
+            if (rc != ST_OK) return rc;
+            ST_LAUNCH(ps, kern, dim3(mt, nt, layers), dim3(waves * kWave), lds, stream, static_cast<const T *>(x),
+                      static_cast<const T *>(A), B, H, r, t_ws, mask, I, mt << 1 | (round_storage ? 1 : 0), mt * nt, tab);
+            return ST_OK;
+        };
+        auto blocks = [&](int mi, int ni) { return ((B + 16 * mi - 1) / (16 * mi)) * ((r + 16 * ni - 1) / (16 * ni)); };
+        // The largest tile of which there is one for three quarters of the CUs (by the shape alone: how many layers share the
+        // launch must not change how the sums are split).  32 x 32 tiles have half the traffic from L2: 6.7 (16 x 16) against
+        // 8.6 us with 64 of them (512 rows, H 3072, rank 128), 17.8 against 11.8 us with 224, 40 against 26 us with 512.  64 x
+        // 32 tiles a quarter less again and 96 KB of loads in flight instead of 64, both kernels, 32 x 32 / 64 x 32: 33.7 / 35.0
+        // us with 128 of them (1024 rows, H 4096, rank 256), 57.4 / 52.0 with 192, 54.9 / 48.4 with 256 (2048 rows).
+        const int want = 3 * device_cu_count();
+        const int rc = 4 * blocks(4, 2) >= want   ? go(predictor_down_mfma_kernel<T, 4, 2, 4, 8, 3, Tab>, 4, 2, 4, 24)
+                       : 4 * blocks(2, 2) >= want ? go(predictor_down_mfma_kernel<T, 2, 2, 4, 16, 2, Tab>, 2, 2, 4, 32)
+                                                  : go(predictor_down_mfma_kernel<T, 1, 1, 8, 16, 2, Tab>, 1, 1, 8, 32);
+        if (rc != ST_OK) return rc;
+    }
+    ST_HIP(hipGetLastError());
+    return launch_up_t<T>(tab, layers, B, r, Bm, I, thr, cmp_ge, t_ws, scores, mask, round_storage, stream);
+}
+
 int launch_predictor_mfma(int dtype, const void *x, int B, int H, const void *A, int r, const void *Bm, int I, float thr,
                           int cmp_ge, float *t_ws, float *scores, uint8_t *mask, int round_storage, hipStream_t stream)
 {
@@ -527,5 +535,27 @@ int launch_predictor_mfma_layers(int dtype, const PredLayers &tab, int layers, c
     auto go = dtype == ST_F16 ? launch_t<f16_t, PredLayers> : launch_t<bf16_t, PredLayers>;
     return go(tab, layers, x, B, H, nullptr, r, nullptr, I, 0.f, 0, t_ws, nullptr, nullptr, round_storage, stream);
 }
+
+// Five to eight rows at ranks of 129 to 256: the first map as for fewer rows (one wave of loads per rank row on the whole chip;
+// 16-row tiles of x would be half empty), the second on the matrix cores once its multiplications outweigh splitting the rows
+// of t into parts (by the shape alone, as above).  Both kernels, on the vector ALUs / so, us: 18.3 million of them (H 4096, rank
+// 256, I 14336, 5 rows, bf16) 9.64 / 9.53, four layers together 23.2 / 19.2; 29.4 million (8 rows) 10.8 / 10.1, four 26.8 / 19.6,
+// eight 40.9 / 26.8; 13.1 million (rank 160, I 10240, 8 rows, fp16) 9.2 / 10.3.
+bool predictor_up_mfma_supported(int dtype, int B, int r, int I)
+{
+    return dtype != ST_F32 && B >= 5 && B <= 8 && r > 128 && r <= 256 && (int64_t)B * r * I >= 18000000;
+}
+
+template <typename Tab>
+int launch_predictor_up_mfma(int dtype, const Tab &tab, int layers, int B, int r, const void *Bm, int I, float thr, int cmp_ge,
+                             float *t_ws, float *scores, uint8_t *mask, int round_storage, hipStream_t stream)
+{
+    auto go = dtype == ST_F16 ? launch_up_t<f16_t, Tab> : launch_up_t<bf16_t, Tab>;
+    return go(tab, layers, B, r, Bm, I, thr, cmp_ge, t_ws, scores, mask, round_storage, stream);
+}
+template int launch_predictor_up_mfma<NoLayers>(int, const NoLayers &, int, int, int, const void *, int, float, int, float *, float *,
+                                                uint8_t *, int, hipStream_t);
+template int launch_predictor_up_mfma<PredLayers>(int, const PredLayers &, int, int, int, const void *, int, float, int, float *,
+                                                  float *, uint8_t *, int, hipStream_t);
 
 }  // namespace st

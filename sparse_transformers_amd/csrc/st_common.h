@@ -286,6 +286,12 @@ int launch_predictor_mfma(int dtype, const void *x, int B, int H, const void *A,
 int launch_predictor_mfma_layers(int dtype, const PredLayers &tab, int layers, const void *x, int B, int H, int r, int I,
                                  float *t_ws, int round_storage, hipStream_t stream);
 
+// Its second kernel behind the first of predictor.hip (which then clears the mask).
+bool predictor_up_mfma_supported(int dtype, int B, int r, int I);
+template <typename Tab>
+int launch_predictor_up_mfma(int dtype, const Tab &tab, int layers, int B, int r, const void *Bm, int I, float thr, int cmp_ge,
+                             float *t_ws, float *scores, uint8_t *mask, int round_storage, hipStream_t stream);
+
 // Double precision forward (plain kernels, for checking a model in fp64).
 int64_t f64_workspace_bytes(int64_t B, int64_t H, int64_t n);
 int launch_f64(const void *x, int B, int H, const void *gate, const void *up, const void *down, int n, const int *n_dev,

@@ -182,6 +182,7 @@ def test_infinite_intermediate_decides_by_sign(dtype, r, B):
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("B,H,r,I", [
+    (5, 520, 136, 26600), (8, 1000, 256, 14336),                                              # the second map alone
     (9, 64, 16, 200), (20, 1000, 128, 8192), (33, 520, 200, 5001), (64, 256, 256, 1000),      # four waves, 4 / 2 / 1 groups
     (77, 520, 104, 5001), (130, 128, 384, 777), (300, 264, 440, 8191), (257, 64, 512, 640),   # eight (four above rank 384)
     (2100, 200, 200, 5001), (2100, 1000, 224, 1000),                                         # 64 x 32 tiles of the intermediate
@@ -324,3 +325,21 @@ def test_scores_rounded_to_the_storage_type(dtype, B, H, r, I):
     a = st.predictor_scores(x32.to(DEV), A32.to(DEV), B32.to(DEV), round_to_storage=True)
     b = st.predictor_scores(x32.to(DEV), A32.to(DEV), B32.to(DEV))
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,H,r,I,dtype", [(8, 1000, 256, 14336, "bfloat16"), (5, 520, 136, 26600, "float16"), (3, 512, 128, 4096, "float16"),
+                                           (20, 512, 200, 5001, "bfloat16")])
+def test_layers_together_give_the_masks_of_one(B, H, r, I, dtype):
+    """What a stack's layers share is the launch: masks and intermediate equal the single-layer calls', bit for bit."""
+    L = 3
+    ws = [tuple(t.to(DEV) for t in _weights(10 * l + B, B, H, r, I, dtype)) for l in range(L)]
+    x = torch.stack([w[0] for w in ws])
+    t_all, masks = torch.empty(L * B * r, dtype=torch.float32, device=DEV), [torch.ones(I, dtype=torch.bool, device=DEV) for _ in range(L)]
+    thrs = []
+    for _, A, Bm in ws:
+        thrs.append(float(st.predictor_scores(x[len(thrs)], A, Bm).amax(0).sort().values[I // 2]))   # a score: a tie
+    st.ops.predictor_mask_layers(x, [(A, Bm, m, thr, l % 2 == 0) for l, ((_, A, Bm), m, thr) in enumerate(zip(ws, masks, thrs))], t_all)
+    for l, (_, A, Bm) in enumerate(ws):
+        t = torch.empty(B * r, dtype=torch.float32, device=DEV)
+        assert torch.equal(masks[l], st.predictor_mask(x[l], A, Bm, thrs[l], l % 2 == 0, t_ws=t))
+        assert torch.equal(t_all[l * B * r:(l + 1) * B * r], t)
