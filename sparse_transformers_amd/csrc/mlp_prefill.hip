@@ -10,11 +10,13 @@
 //             down columns, i.e. K runs down the rows: the tile sits in LDS
 //             as [k][column] and the fragments are read with the
 //             transposing LDS load (ds_read_b64_tr_b16)
-// Each kernel has two forms.  The first (kernel 1: 64 or 128 rows of x by 32 or 64 active rows of gate and of up
-// per block; kernel 2: block tile 128 x 128 with split-K) has waves of 64 x 64 and K stages of 64 through two LDS
-// buffers with the following stages' global loads held in registers, one barrier per stage; it serves the shapes
-// whose tiles do not fill the chip.  The wide form (256 x 128 block tiles, waves of 128 x 64 whose K the two waves
-// of a SIMD share, operands loaded global -> LDS directly through three buffers) takes over when they do.
+// Forms, by the number of rows of x and of tiles:
+//   few    up to 128 rows: one row of tiles, the whole LDS a ring of K stages (two row tiles of 64 on four K groups of the plain
+//          form instead where the capacity is small)
+//   plain  kernel 1: 64 or 128 rows of x by 32 or 64 active rows of gate and of up per block; kernel 2: block tile 128 x 128
+//          with split-K; waves of 64 x 64, K stages of 64 through two LDS buffers with the following stages' global loads held
+//          in registers, one barrier per stage: the shapes whose tiles do not fill the chip
+//   wide, big   256-row tiles, waves of 128 x 64, operands loaded global -> LDS directly
 //
 // The reference only runs the sparse path for decode (src/modeling_skip.py:236);
 // this is the same contraction as sparse_mlp_forward_cpu
@@ -1511,12 +1513,11 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
         ProfScope ps(ST_K_MLP_PREFILL_GATEUP, stream);
         const int cus = device_cu_count();
         const int jt64 = (int)(ldw / 64), mt128 = (M + 127) / 128;
-        // 256-row blocks with 64 + 64 weight rows (one per CU, 25 % less operand traffic; the wide kernel) once
-        // 128-row tiles outnumber the CUs.  Below that the K loop of a block, not the chip, is what takes the time: two thread
-        // groups per tile with half of K each, on 128 x (64 + 64) tiles while those number more than half the
-        // CUs and on 128 x (32 + 32) tiles (twice the blocks) when there are fewer -- four groups with a quarter
-        // of K each on 64 x (32 + 32) tiles while those fit one per CU.  What is left (one row tile and more
-        // than 16384 active rows) takes 128 x (32 + 32) tiles without K groups.
+        // 256-row tiles (one per CU; the wide kernel) once 128-row tiles outnumber the CUs.  Below that the K loop of a block,
+        // not the chip, is what takes the time: two thread groups per tile with half of K each, on 128 x (64 + 64) tiles while
+        // those number more than half the CUs and on 128 x (32 + 32) tiles (twice the blocks) when there are fewer -- four groups
+        // with a quarter of K each on 64 x (32 + 32) tiles while those fit one per CU.  What is left (operands beyond the wide
+        // kernel's offsets) takes 128 x (32 + 32) tiles without K groups.
         // (32-bit byte offsets into x and the weight rows in the wide kernel)
         const bool big = M > 128 && jt64 * mt128 > cus && (int64_t)(M > n ? M : n) * H * 2 < ((int64_t)1 << 32);
         const bool halves = !big && 2 * jt64 * mt128 <= cus;

@@ -145,6 +145,7 @@ def test_cache_call_forms(monkeypatch, gated):
 @pytest.mark.gpu
 @pytest.mark.parametrize("gated", [True, False])
 def test_operator_forms(monkeypatch, gated):
+    monkeypatch.setattr(st.ops, "_warned_layout", True)    # (warns once per process; restored for the test of that)
     H, I, B = 256, 512, 2
     x = torch.randn(B, H, generator=torch.Generator().manual_seed(7)).half().to(DEV)
     mask = (torch.rand(I, generator=torch.Generator().manual_seed(8)) < 0.3).to(DEV)
