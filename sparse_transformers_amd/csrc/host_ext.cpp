@@ -160,9 +160,10 @@ PyObject *update_forward(PyObject *, PyObject *const *a, Py_ssize_t n)
     });
 }
 
-// mlp_forward(x, gate | None, up, down, n, n_dev | None, out | None, combined | None, hint, workspace, act, stream, resize) ->
-// out | status | None.  `out` and `combined` are contiguous [B, H] and [B, (gate and up: 2) n]; `resize`: made so as the last
-// thing before the launch.
+// mlp_forward(x, gate | None, up, down, n, n_dev | None, out | None, combined | None, hint, workspace, act, stream, operator) ->
+// out | status | None.  `out` and `combined` are contiguous [B, H] and [B, (gate and up: 2) n].  The operator's form makes them
+// so as the last thing before the launch, and its `down` is the matrix [H, n]: only as the transposed view of packed rows is it
+// read in place (n = H does not make a row-major one packed rows).  The cache's form hands over packed rows [>= n, H].
 PyObject *mlp_forward(PyObject *, PyObject *const *a, Py_ssize_t n_args)
 {
     if (n_args != 13 || !f_mlp_forward) return none();
@@ -173,15 +174,15 @@ PyObject *mlp_forward(PyObject *, PyObject *const *a, Py_ssize_t n_args)
         const int64_t B = x->size(0), H = x->size(1), n = PyLong_AsLongLong(a[4]), hint = PyLong_AsLongLong(a[8]);
         const long act = PyLong_AsLong(a[10]);
         void *stream = PyLong_AsVoidPtr(a[11]);
-        const int resize = PyObject_IsTrue(a[12]);
+        const int as_operator = PyObject_IsTrue(a[12]);
         if (PyErr_Occurred()) { PyErr_Clear(); return none(); }
         const int code = code_of(*x);
         if (code < 0 || n < 0 || !workspace_of(*ws, *x)) return none();
         auto packed = [&](const at::Tensor &t) { return rows_of(t, H) && t.size(0) >= n && same_kind(t, *x); };
-        // (the transposed view [H, n] with strides (1, H) of packed rows stands for them)
+        // (strides (1, H): packed rows [n, H], transposed)
         const bool view = down->dim() == 2 && down->size(0) == H && down->size(1) == n && n > 0 && down->stride(0) == 1 &&
                           down->stride(1) == H && same_kind(*down, *x);
-        if (!packed(*up) || (gate && !packed(*gate)) || !(packed(*down) || view)) return none();
+        if (!packed(*up) || (gate && !packed(*gate)) || !(as_operator ? view : packed(*down))) return none();
         const int32_t *n_dev = nullptr;
         if (a[5] != Py_None) {
             const at::Tensor *t = gpu_tensor(a[5]);
@@ -192,7 +193,7 @@ PyObject *mlp_forward(PyObject *, PyObject *const *a, Py_ssize_t n_args)
         auto buffer = [&](const at::Tensor *t, int64_t width) {   // usable as it is, or once resized
             if (!t || !same_kind(*t, *x)) return false;
             const bool fits = t->dim() == 2 && t->size(0) == B && t->size(1) == width;
-            return fits ? t->is_contiguous() : resize != 0;
+            return fits ? t->is_contiguous() : as_operator != 0;
         };
         const at::Tensor *comb = a[7] == Py_None ? nullptr : gpu_tensor(a[7]), *o = a[6] == Py_None ? nullptr : gpu_tensor(a[6]);
         if ((a[7] != Py_None && !buffer(comb, cols)) || (a[6] != Py_None && !buffer(o, H))) return none();

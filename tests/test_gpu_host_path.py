@@ -165,6 +165,9 @@ def test_operator_forms(monkeypatch, gated):
         lambda c, b, n: F(x, c.get_concat_weight() + 0, c.get_active_down_weight(), *b, "silu", gated),
         lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight().contiguous(), *b, "relu", gated),
         lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight()[:, :-1], *b, "silu", gated),
+        lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight().t(), *b, "silu", gated),        # packed rows are not the
+        lambda c, b, n: F(x, c.get_concat_weight(), c.down_active, *b, "silu", gated),                         # operator's [H, n]
+        lambda c, b, n: F(x, c.get_concat_weight(), c.down_active[:n], *b, "silu", gated),
         lambda c, b, n: F(x[:1], c.get_concat_weight(), c.get_active_down_weight(), *b, "silu", gated),        # resized
         lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), b[0].resize_(1, 8), b[1].resize_(3), "silu", gated),
         lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), half(H, B).t(), b[1], "silu", gated),
@@ -178,6 +181,31 @@ def test_operator_forms(monkeypatch, gated):
     ]
     for f in forms:
         _same(*_both(monkeypatch, call(f)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("gated", [True, False])
+def test_operator_with_as_many_active_rows_as_columns(monkeypatch, gated):
+    """n = H: the shape does not tell [H, n] from packed [n, H] rows.  A row-major down weight is the matrix it says it is."""
+    monkeypatch.setattr(st.ops, "_warned_layout", True)
+    H, I, B = 256, 1024, 3
+    c, g = _cache(H=H, I=I, gated=gated)
+    c.update_active_weights((torch.randperm(I, generator=g) < H).to(DEV))
+    x = torch.randn(B, H, generator=g).half().to(DEV)
+    view = c.get_active_down_weight()
+    assert tuple(view.shape) == (H, H)
+    h = torch.nn.functional.silu(x.float() @ (c.gate_active if gated else c.up_active)[:H].float().t())
+    if gated:
+        h = h * (x.float() @ c.up_active[:H].float().t())
+    for down in (view, view.contiguous(), view.t(), c.down_active[:H]):
+        def call():
+            bufs = [torch.zeros(B, k, dtype=torch.float16, device=DEV) for k in (H, (2 if gated else 1) * H)]
+            return (st.sparse_mlp_forward(x, c.get_concat_weight(), down, *bufs, "silu", gated), *bufs)
+        a, b = _both(monkeypatch, call)
+        _same(a, b)
+        # (fp32 sums of fp16 operands, the intermediate in fp32 or rounded once, one rounding of the output: 2^-11 each)
+        want = h @ down.float().t()
+        assert (a[1][0][0].float() - want).abs().max() <= 2 * 2.0 ** -11 * (h.abs() @ down.float().abs().t()).max()
 
 
 @pytest.mark.gpu
