@@ -395,6 +395,41 @@ def test_prefill_few_rows(M, H, I, n, gated):
         assert torch.equal(first, out)
 
 
+@pytest.mark.parametrize("M,H,I,n,gated", [
+    (33, 128, 1000, 1, True), (48, 256, 9000, 8191, False), (64, 1152, 520, 63, False), (65, 1152, 9000, 8129, True),
+    (77, 2560, 9000, 6081, False), (96, 640, 8448, 8384, True), (128, 512, 4096, 2500, True), (128, 1024, 8200, 8199, True),
+])
+def test_prefill_few_rows_infinite_last_row(M, H, I, n, gated):
+    """An infinity and a NaN in the last active row of the down weights, 33 to 128 rows of x and a count that is not a multiple
+    of the padding: the padding's zeros must not meet them, so that an infinite element is infinite with the intermediate's
+    sign and the other columns are finite.  Bounds as in the tests above."""
+    g = torch.Generator().manual_seed(M * n)
+    gate, up, dn = ((torch.randn(I, H, generator=g) * 0.05).half().to(DEV) for _ in range(3))
+    x = torch.randn(M, H, generator=g).half().to(DEV)
+    x[:, 0], x[:, 1] = 8.0, torch.where(torch.arange(M, device=DEV) % 3 > 0, 1.0, -1.0).half()
+    gate[n - 1], up[n - 1] = 0.0, 0.0
+    (gate if gated else up)[n - 1, 0] = 1.0                  # the last intermediate: silu(8), times 1 or -1 with a gate
+    if gated:
+        up[n - 1, 1] = 1.0
+    h = torch.nn.functional.silu(x.float() @ (gate if gated else up)[:n].float().t())
+    if gated:
+        h = h * (x.float() @ up[:n].float().t())
+    dn[n - 1, 1], dn[n - 1, H // 2], dn[n - 1, H - 1] = float("inf"), float("-inf"), float("nan")
+    finite = torch.ones(H, dtype=torch.bool, device=DEV)
+    finite[[1, H // 2, H - 1]] = False
+    want = h @ torch.where(torch.isfinite(dn[:n]), dn[:n], 0).float()
+    for t in (gate, up, dn):
+        t[n:] = float("nan")
+    out = torch.full((M, H), float("nan"), dtype=torch.float16, device=DEV)
+    mlp_forward_rows(x, gate if gated else None, up, dn, I, torch.tensor([n], dtype=torch.int32, device=DEV), out, None, "silu",
+                     gated)
+    torch.cuda.synchronize()
+    sign = x[:, 1].float() if gated else torch.ones(M, device=DEV)
+    assert torch.equal(out[:, 1].float(), sign * float("inf")) and torch.equal(out[:, H // 2].float(), -sign * float("inf"))
+    assert bool(torch.isnan(out[:, H - 1]).all())
+    assert_close(out[:, finite].float().cpu().numpy(), want[:, finite].cpu().numpy(), "float16", f"{M} rows, {n} active")
+
+
 def test_prefill_agrees_with_decode_kernel():
     """The MFMA path (B = 40) and the streaming path (the same rows, 4 at a time) agree to rounding."""
     x, cw, dn = _case(22, 40, 1024, 700, "float16", True)
