@@ -432,8 +432,8 @@ __global__ __launch_bounds__(W * kWave) void predictor_up_mfma_kernel(const floa
 // row at rank 256) and take x in passes of eight, sixteen and at last 64 rows; these take 7-14 us for any number up to 64.
 // Both kernels, replayed from a graph, there / here, at H 3072, rank 128, I 8192 (bf16): 7.5 / 8.4 us for 8 rows, 9.9 / 8.7
 // for 12, 17.0 / 9.6 for 32, 29.5 / 10.6 for 64, 233 / 15.6 for 512, 929 / 31 for 2048; at H 4096, rank 256, I 14336:
-// 10.6 / 10.6, 14.3 / 11.0, 25.0 / 12.1, 68.9 / 13.2, 538 / 29, 2236 / 78.  Ranks above 512 do not fit the registers, and a
-// tile's 32 rows of x have to stay within 32-bit offsets.
+// 10.6 / 10.6, 14.3 / 11.0, 25.0 / 12.1, 68.9 / 13.2, 538 / 29, 2236 / 78.  Ranks above 512 do not fit the registers, and
+// the 32 rows of x of a tile (64 where H allows it, launch_t) have to stay within 32-bit offsets.
 bool predictor_mfma_supported(int dtype, int B, int H, int r)
 {
     return dtype != ST_F32 && B > 8 && r <= 512 && H < (1 << 26);
@@ -512,10 +512,12 @@ static int launch_t(const Tab &tab, int layers, const void *x, int B, int H, con
         // 8.6 us with 64 of them (512 rows, H 3072, rank 128), 17.8 against 11.8 us with 224, 40 against 26 us with 512.  64 x
         // 32 tiles a quarter less again and 96 KB of loads in flight instead of 64, both kernels, 32 x 32 / 64 x 32: 33.7 / 35.0
         // us with 128 of them (1024 rows, H 4096, rank 256), 57.4 / 52.0 with 192, 54.9 / 48.4 with 256 (2048 rows).
+        // (a tile's rows of x have to stay within 32-bit offsets: 64 of them up to H = 2^25, 32 for every H that is taken at all)
+        const bool reach = (int64_t)64 * H * (int64_t)sizeof(T) <= (int64_t)1 << 32;
         const int want = 3 * device_cu_count();
-        const int rc = 4 * blocks(4, 2) >= want   ? go(predictor_down_mfma_kernel<T, 4, 2, 4, 8, 3, Tab>, 4, 2, 4, 24)
-                       : 4 * blocks(2, 2) >= want ? go(predictor_down_mfma_kernel<T, 2, 2, 4, 16, 2, Tab>, 2, 2, 4, 32)
-                                                  : go(predictor_down_mfma_kernel<T, 1, 1, 8, 16, 2, Tab>, 1, 1, 8, 32);
+        const int rc = reach && 4 * blocks(4, 2) >= want ? go(predictor_down_mfma_kernel<T, 4, 2, 4, 8, 3, Tab>, 4, 2, 4, 24)
+                       : 4 * blocks(2, 2) >= want        ? go(predictor_down_mfma_kernel<T, 2, 2, 4, 16, 2, Tab>, 2, 2, 4, 32)
+                                                         : go(predictor_down_mfma_kernel<T, 1, 1, 8, 16, 2, Tab>, 1, 1, 8, 32);
         if (rc != ST_OK) return rc;
     }
     ST_HIP(hipGetLastError());

@@ -122,6 +122,27 @@ def test_matrix_core_predictor_reads_beyond_4_gib():
     assert st.predictor_mask(x, A, Bm, 1.0, True).nonzero().flatten().tolist() == [I - 1]
 
 
+def test_matrix_core_predictor_rows_beyond_32_bit_offsets():
+    """Enough rows of x for tiles of 64, so wide that 64 of them are more than 4 GiB (H a little above 2^25): products of the
+    first and last columns only, so that a row read for another would show.  fp32 sums of 32 products: 1e-6 of the largest."""
+    H, r, I, B = (1 << 25) + 8, 512, 64, 705
+    if torch.cuda.mem_get_info()[0] < 100 << 30:
+        pytest.skip("needs 100 GB of device memory")
+    g = torch.Generator(device=DEV).manual_seed(5)
+    x = torch.zeros(B, H, dtype=torch.float16, device=DEV)          # 47 GB
+    A = torch.zeros(r, H, dtype=torch.float16, device=DEV)          # 34 GB
+    for t in (x, A):
+        for cols in (slice(0, 16), slice(H - 16, H)):
+            t[:, cols] = torch.randn(t.size(0), 16, generator=g, device=DEV).half()
+    edge = lambda t: torch.cat([t[:, :16], t[:, -16:]], 1).double()
+    t_ws = torch.empty(B, r, dtype=torch.float32, device=DEV)
+    st.predictor_mask(x, A, torch.zeros(I, r, dtype=torch.float16, device=DEV), t_ws=t_ws)
+    want = edge(x) @ edge(A).t()
+    assert (t_ws - want).abs().max() <= 1e-6 * want.abs().max()
+    del x, A
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("where", ["x", "A", "Bm"])
 @pytest.mark.parametrize("round_to_storage", [False, True])
