@@ -197,6 +197,7 @@ PyObject *mlp_forward(PyObject *, PyObject *const *a, Py_ssize_t n_args)
         };
         const at::Tensor *comb = a[7] == Py_None ? nullptr : gpu_tensor(a[7]), *o = a[6] == Py_None ? nullptr : gpu_tensor(a[6]);
         if ((a[7] != Py_None && !buffer(comb, cols)) || (a[6] != Py_None && !buffer(o, H))) return none();
+        if (o && comb && o->is_same(*comb) && cols != H) return none();   // (one tensor cannot become both)
         auto fit = [&](const at::Tensor *t, int64_t width) {
             if (t->dim() != 2 || t->size(0) != B || t->size(1) != width) t->resize_({B, width});
         };

@@ -173,6 +173,7 @@ def test_operator_forms(monkeypatch, gated):
         lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), half(H, B).t(), b[1], "silu", gated),
         lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), b[0], b[1].float(), "silu", gated),
         lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), b[0].cpu(), b[1], "silu", gated),
+        lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), b[0], b[0], "silu", gated),   # one buffer for both
         lambda c, b, n: F(x.view(B, 1, H), c.get_concat_weight(), c.get_active_down_weight(), *b, "silu", gated),
         lambda c, b, n: F(x.float(), c.get_concat_weight(), c.get_active_down_weight(), *b, "silu", gated),
         lambda c, b, n: F(x, c.get_concat_weight(), c.get_active_down_weight(), *b, "silu", not gated),
