@@ -193,14 +193,15 @@ def sparse_mlp_forward(x: torch.Tensor, concat_weight: torch.Tensor, active_down
             and handle.fresh():
         # the reference's call sequence natively: the cache's packed rows in place (None: something is not as usual)
         c, n = handle._cache, handle._n
-        ws = _kept_workspace(c.device, mlp_workspace_bytes(x.size(0), c.hidden_size, n))
-        got = _lib.native().mlp_forward(x, c.gate_active if has_gate else None, c.up_active, active_down_weight, n, None,
-                                        down_proj_buffer, combined_proj_buffer, 0, ws, _lib.ACT_CODES[act],
-                                        current_stream_ptr(c.device), True)
-        if got is not None:
-            if type(got) is int:
-                _lib.check(got, "st_mlp_forward")
-            return got
+        need = c._workspace_need(x)
+        if need is not None:
+            got = _lib.native().mlp_forward(x, c.gate_active if has_gate else None, c.up_active, active_down_weight, n, None,
+                                            down_proj_buffer, combined_proj_buffer, 0, _kept_workspace(c.device, need),
+                                            _lib.ACT_CODES[act], current_stream_ptr(c.device), True)
+            if got is not None:
+                if type(got) is int:
+                    _lib.check(got, "st_mlp_forward")
+                return got
     if isinstance(concat_weight, ConcatWeightHandle) and handle is None:
         concat_weight = concat_weight.materialize()
     dev = require_gpu(x, concat_weight, active_down_weight, down_proj_buffer, combined_proj_buffer)

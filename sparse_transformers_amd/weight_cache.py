@@ -159,7 +159,7 @@ class WeightCache:
         self._pending_mask: Optional[torch.Tensor] = None
         self._concat_ref = None     # weak reference to the handle get_concat_weight() handed out last
         self._concat_serial = -1
-        self._ws_need: dict = {}    # workspace bytes by rows of x (at most 4096 of them)
+        self._ws_need: dict = {}    # workspace bytes by rows of x (1 to 4096)
         # weight_cache.h:226: the constructor ends with update_active_weights(init_mask); here in one pass over the weights
         mask = self._mask_arg(init_mask)
         rc = L.st_cache_load_weights_masked(self._h, gate_c.data_ptr() if self.has_gate else None, up_c.data_ptr(),
@@ -279,6 +279,15 @@ class WeightCache:
         x2 = x if x.dim() == 2 else x.reshape(-1, H)
         return x2 if x2.is_contiguous() else x2.contiguous()
 
+    def _workspace_need(self, x2):
+        """Workspace bytes for the rows of x [B,H] at any count.  None for an x that the general path refuses (so that none of
+        those sizes the workspace, which is kept), looked at once per number of rows."""
+        B = x2.size(0)
+        need = self._ws_need.get(B)
+        if need is None and 1 <= B <= 4096 and x2.size(1) == self.hidden_size and x2.dtype == self.dtype and x2.device == self.device:
+            need = self._ws_need[B] = mlp_workspace_bytes(B, self.hidden_size, self.intermediate_size)
+        return need
+
     def _native_call(self, x, act, out, workspace, call):
         """The common form of a call through the native host path: rows of x as they are, a workspace that is large enough.
         None: not that form (nothing has been done)."""
@@ -290,10 +299,9 @@ class WeightCache:
             if out is not None or x.shape[-1] != self.hidden_size or not x.is_contiguous():
                 return None
             x2 = x.view(-1, self.hidden_size)
-        B = x2.size(0)
-        need = self._ws_need.get(B)
+        need = self._workspace_need(x2)
         if need is None:
-            need = self._ws_need[B] = mlp_workspace_bytes(B, self.hidden_size, self.intermediate_size)
+            return None
         if workspace is None:
             workspace = _kept_workspace(self.device, need)
         elif workspace.numel() < need:

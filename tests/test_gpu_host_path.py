@@ -210,6 +210,28 @@ def test_operator_with_as_many_active_rows_as_columns(monkeypatch, gated):
 
 
 @pytest.mark.gpu
+def test_refused_calls_leave_the_workspace_alone(monkeypatch):
+    """Calls whose x the general path refuses must not have grown the scratch that is kept for the process."""
+    c, _ = _cache()
+    mask = torch.ones(512, dtype=torch.bool, device=DEV)
+    w, d = c.get_concat_weight(), c.get_active_down_weight()
+    asked = []
+    kept = st.ops._kept_workspace
+    for module in (st.ops, st.weight_cache):
+        monkeypatch.setattr(module, "_kept_workspace", lambda dev, need: (asked.append(need), kept(dev, need))[1])
+    half = lambda *s: torch.zeros(*s, dtype=torch.float16, device=DEV)
+    for x in (half(4000, 248), torch.zeros(4000, 256, device=DEV), half(30, 100, 248), torch.zeros(30, 100, 256, dtype=torch.bfloat16, device=DEV)):
+        for call in (lambda: c.forward(x), lambda: c.update_and_forward(mask, x), lambda: st.sparse_mlp_forward(x, w, d, half(1, 256), half(1, 8))):
+            with pytest.raises((ValueError, TypeError)):
+                call()
+    assert asked == []
+    for rows in (0, 5000):
+        with pytest.raises(ValueError):
+            c.forward(half(rows, 256))
+    assert not {0, 5000} & set(c._ws_need)
+
+
+@pytest.mark.gpu
 def test_threads_and_streams():
     """Several threads, each with a cache and a stream of its own, through the native path: the results of one thread alone."""
     c0, _ = _cache()
