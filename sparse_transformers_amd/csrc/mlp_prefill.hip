@@ -219,17 +219,17 @@ __global__ __launch_bounds__(2 * BM * KS) void prefill_gateup_kernel(const T *__
         }
 
     // Loads are unconditional (rows clamped into range): rows of x beyond M only feed outputs that are
-    // never stored, weight rows beyond n only feed columns that are written as zeros below.
-    int xoff[kXL], woff[kWL];
+    // never stored, weight rows beyond n only feed columns that are written as zeros below.  (Either may be larger than 4 GiB.)
+    size_t xoff[kXL], woff[kWL];
 #pragma unroll
     for (int i = 0; i < kXL; ++i) {
         const int r = m0 + r0 + kRowStep * i;
-        xoff[i] = (r < M ? r : M - 1) * H + ch * 8;
+        xoff[i] = (size_t)(r < M ? r : M - 1) * H + ch * 8;
     }
 #pragma unroll
     for (int i = 0; i < kWL; ++i) {
         const int r = j0 + r0 + kRowStep * i;
-        woff[i] = (r < n ? r : (n > 0 ? n - 1 : 0)) * H + ch * 8;
+        woff[i] = (size_t)(r < n ? r : (n > 0 ? n - 1 : 0)) * H + ch * 8;
     }
     struct Stage { uint4 x[kXL], g[kWL], u[kWL]; };
     Stage R[NS];
@@ -939,11 +939,12 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_down_kernel(const T *__
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
+    const T *const h_tile = Hh + (size_t)m0 * ldh;    // (Hh may be larger than 4 GiB, a tile's rows of it are not)
     int aoff[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int r = m0 + ar0 + 32 * i;
-        aoff[i] = (int)((r < M ? r : M - 1) * ldh) + ach * 8;
+        aoff[i] = (int)(((r < M ? r : M - 1) - m0) * ldh) + ach * 8;
     }
     const T *wcol = Wd + c0 + 8 * bch;
     const int nlast = n > 0 ? n - 1 : 0;
@@ -954,7 +955,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_down_kernel(const T *__
     auto gload = [&](Stage &st, int s) __attribute__((always_inline)) {
         const int k0 = (s < ks1 ? s : ks1 - 1) * kPfBK2;   // past the end: a harmless repeat
 #pragma unroll
-        for (int i = 0; i < 4; ++i) st.a[i] = ld16(Hh + aoff[i] + k0);
+        for (int i = 0; i < 4; ++i) st.a[i] = ld16(h_tile + aoff[i] + k0);
         if (k0 + kPfBK2 <= n) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) st.b[i] = ld16(wcol + (size_t)(k0 + br0 + 16 * i) * H);
@@ -1471,6 +1472,12 @@ static int prefill_split_k_wide(int M, int H, int n)
 
 // Up to 128 rows: one block per CU, at least eight stages of the capacity per split.
 constexpr int kFewRows = 128;
+// (32-bit byte offsets reach over the rows of x and over 64 weight rows; the plain forms' of 64 bits over anything)
+static bool prefill_few(int M, int H, int n)
+{
+    const int wrows = n < 64 ? n : 64, rows = M > wrows ? M : wrows;
+    return M <= kFewRows && (int64_t)rows * H <= (int64_t)1 << 31;
+}
 static int prefill_split_k_few(int H, int n)
 {
     const int nk = (n + kPfBK - 1) / kPfBK * (kPfBK / kPfBK2);
@@ -1496,15 +1503,16 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
 {
     // The intermediate Hh normally sits in the workspace, padded with zero columns to a multiple of 128.  When the
     // caller's combined buffer can take that padding (16-byte aligned rows with room up to the padded width) the
-    // gate/up kernel writes there only and the down kernel reads it back from there: one store of M x n less.
+    // gate/up kernel writes there only and the down kernel reads it back from there: one store of M x n less.  (A tile's
+    // 128 rows of Hh have to stay within 32-bit byte offsets; in the workspace they do for every n that is taken.)
     const long ldw = (long)prefill_ldh(n);
-    const bool alias = comb && ldc % 8 == 0 && ldc >= ldw && (reinterpret_cast<uintptr_t>(comb) & 15) == 0;
+    const bool alias = comb && ldc % 8 == 0 && ldc >= ldw && ldc <= (1L << 24) && (reinterpret_cast<uintptr_t>(comb) & 15) == 0;
     const long ldh = alias ? ldc : ldw;
     T *Hh = alias ? static_cast<T *>(comb) : static_cast<T *>(workspace);
     if (alias) comb = nullptr;
     const int64_t hh_bytes = (((int64_t)M * ldw * 2) + 255) & ~(int64_t)255;
     float *partial = reinterpret_cast<float *>(static_cast<unsigned char *>(workspace) + hh_bytes);
-    const bool few = M <= kFewRows, wide_down = !few && prefill_down_is_wide(M, H, n, ldh);
+    const bool few = prefill_few(M, H, n), wide_down = !few && prefill_down_is_wide(M, H, n, ldh);
     const int split_k = few ? prefill_split_k_few(H, n) : wide_down ? prefill_split_k_wide(M, H, n) : prefill_split_k(M, H, n);
     // (four K groups on 64-row tiles, below, are faster for two of them while those make no more blocks than CUs: H 2048, 2500 of
     // 4096 active rows, 128 rows 27.2 us for the whole forward with the few-row kernel, 24.8 so; with one row tile the few-row kernel is: H 1024, 48 rows 20.9 / 18.0)

@@ -430,6 +430,45 @@ def test_prefill_few_rows_infinite_last_row(M, H, I, n, gated):
     assert_close(out[:, finite].float().cpu().numpy(), want[:, finite].cpu().numpy(), "float16", f"{M} rows, {n} active")
 
 
+@pytest.mark.parametrize("M,H,n,gated,stride", [
+    (200, 65536, 33000, False, 0),                # weights of 4.3 GB
+    (4096, 128, 524416, False, 0),                # an intermediate of 4.3 GB
+    (128, 128, 520, True, (1 << 24) + 8),         # rows of the combined buffer 2^24 + 8 elements apart, 4.3 GB
+    (300, 128, 520, True, (1 << 24) + 8),
+    (128, (1 << 24) + 128, 3, False, 0),          # 128 rows of x of 33.6 MB
+])
+def test_prefill_beyond_4_gib(M, H, n, gated, stride):
+    """Operands whose offsets from their own start do not fit 32 bits.  Bounds as in the tests above (the down weights are
+    scaled so that the roundings of the intermediate, at random, add up to about 1e-3 of an output of about 2)."""
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, H, generator=g, device=DEV).half()
+    gate, up, dn = (torch.empty(n if i or gated else 1, H, dtype=torch.float16, device=DEV).normal_(0, s, generator=g)
+                    for i, s in enumerate((H ** -0.5, H ** -0.5, 4 * n ** -0.5)))
+    comb = torch.empty(M, stride, dtype=torch.float16, device=DEV)[:, :2 * n] if stride else None
+    out = torch.full((M, H), float("nan"), dtype=torch.float16, device=DEV)
+    need = st.ops.mlp_workspace_bytes(M, H, n)               # (140 GB for the widest x; kept by the test, not by the process)
+    if torch.cuda.mem_get_info()[0] < need + (40 << 30):
+        pytest.skip(f"needs {need >> 30} GB of scratch")
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    mlp_forward_rows(x, gate if gated else None, up, dn, n, None, out, comb, "silu", gated, workspace=ws)
+    for rows in torch.arange(M, device=DEV).split(512):
+        h = torch.nn.functional.silu(x[rows].float() @ (gate if gated else up).float().t())
+        if gated:
+            h = h * (x[rows].float() @ up.float().t())
+        # (with few active rows and many columns some sums cancel: the intermediate is off by its rounding, at most 2^-11 of it,
+        # and by its fp32 sum, 2^-12 for 2^24 products in 2^18 steps of a wave; three such errors add up to less than 1.8 times
+        # their root of squares, many at random to less.  Reference products of no more than 2^31 elements.)
+        for cols in range(0, H, 1 << 20):
+            d = dn[:, cols:cols + (1 << 20)].float()
+            want, got = h @ d, out[rows, cols:cols + (1 << 20)].float()
+            bound = 2e-2 + 1e-2 * want.abs() + 2.0 ** -9 * ((h * h) @ (d * d)).sqrt()
+            assert bool(((got - want).abs() <= bound).all()) and float(want.abs().max()) > 0.5
+        if comb is not None:
+            assert_close(comb[rows, :n].float().cpu().numpy(), h.cpu().numpy(), "float16", f"intermediate, {M} rows")
+    del x, gate, up, dn, comb, out, ws, h, d, want, got, bound
+    torch.cuda.empty_cache()
+
+
 def test_prefill_agrees_with_decode_kernel():
     """The MFMA path (B = 40) and the streaming path (the same rows, 4 at a time) agree to rounding."""
     x, cw, dn = _case(22, 40, 1024, 700, "float16", True)
