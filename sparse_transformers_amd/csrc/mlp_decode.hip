@@ -421,11 +421,15 @@ template <typename T, int NB> static int launch_one(const MlpLaunch &a, int b0, 
             if ((rpg + 6) / 7 < (rpg + 5) / 6) return launch_inst<T, 1, 7, 1, 1024, false>(a, b0, bcount);   // 7, 13, 14, ...
         return launch_inst<T, 1, DecodeRows<T>::value, 1, 1024, false>(a, b0, bcount);
     } else if constexpr (NB == 2) {
-        // (one batch where it holds what is expected: 2867 rows, six per group, at H 3072 19.5 us in double-buffered batches of
-        // two, 18.7 so; 1100 ungated at H 4096 15.4 / 14.4 with three)
+        // (one batch where it holds what is expected.  H 3072, fp16 / bf16, double-buffered batches of two then one batch:
+        // 2867 rows, six per group, 19.6 -> 18.6 / 19.6 -> 19.3 us; 2300, five, 19.3 -> 17.6 / 19.3 -> 18.5; 1400, three,
+        // 16.5 -> 13.9 / 16.4 -> 14.1.  Four per group are two whole batches and leave two of six slots empty: 2000 rows 16.9 ->
+        // 17.0 / 16.9 -> 17.8; bf16, whose six slots also spill five registers, keeps the two batches, except where one group
+        // is the whole block: H 8192, 1000 rows, 24.3 -> 23.7)
         const int rpg = rows_per_group<T>(a);
+        const bool two_whole = std::is_same<T, bf16_t>::value && rpg == 4 && chunks <= 512;
         if (rpg >= 1 && rpg <= 3) return launch_inst<T, 2, 3, 1, 1024, false>(a, b0, bcount);
-        if (rpg >= 1 && rpg <= 6) return launch_inst<T, 2, 6, 1, 1024, false>(a, b0, bcount);
+        if (rpg >= 1 && rpg <= 6 && !two_whole) return launch_inst<T, 2, 6, 1, 1024, false>(a, b0, bcount);
         return launch_inst<T, 2, 2, 1, 1024, true>(a, b0, bcount);
     } else if constexpr (NB == 4) {
         if (chunks > 512) return launch_inst<T, 4, 1, 2, 512, true>(a, b0, bcount);

@@ -168,25 +168,26 @@ def test_batch_device_count_and_hint_paths(B, H, dt):
 
 
 @pytest.mark.parametrize("B", [1, 2])
-@pytest.mark.parametrize("n", [1, 2049, 6144, 6145, 12288, 12289, 14337])
-def test_streaming_kernel_slots(B, n):
+@pytest.mark.parametrize("n", [1, 2049, 6144, 6145, 8192, 12288, 12289, 14337])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_streaming_kernel_slots(B, n, dtype):
     """The forms of the streaming kernel by rows per thread group (three, six, seven, double-buffered twos: the guess of the
     count chooses) sum the same rows in the same order: the same bits for every guess, rows past the count NaN."""
     H, I = 1024, 16000                    # eight thread groups per block: n / 2048 rows per group
     g = torch.Generator().manual_seed(n)
-    gate, up, dn = ((torch.randn(I, H, generator=g) * 0.03).half().to(DEV) for _ in range(3))
-    x = torch.randn(B, H, generator=g).half().to(DEV)
+    gate, up, dn = ((torch.randn(I, H, generator=g) * 0.03).to(getattr(torch, dtype)).to(DEV) for _ in range(3))
+    x = torch.randn(B, H, generator=g).to(gate.dtype).to(DEV)
     h = torch.nn.functional.silu(x.float() @ gate[:n].float().t()) * (x.float() @ up[:n].float().t())
     want = (h @ dn[:n].float()).cpu().numpy()
     for t in (gate, up, dn):
         t[n:] = float("nan")
     n_dev = torch.tensor([n], dtype=torch.int32, device=DEV)
     first = None
-    for hint in (0, 1, n - 1, n, 6144, 12288, I):
-        out = torch.full((B, H), float("nan"), dtype=torch.float16, device=DEV)
+    for hint in (0, 1, n - 1, n, 6144, 8192, 12288, I):
+        out = torch.full((B, H), float("nan"), dtype=gate.dtype, device=DEV)
         mlp_forward_rows(x, gate, up, dn, I, n_dev, out, None, "silu", True, n_hint=hint)
         torch.cuda.synchronize()
-        assert_close(out.float().cpu().numpy(), want, "float16", f"{n} active, guess {hint}")
+        assert_close(out.float().cpu().numpy(), want, dtype, f"{n} active, guess {hint}")
         first = out if first is None else first
         assert torch.equal(first, out), hint
 
