@@ -44,7 +44,7 @@ __global__ __launch_bounds__(W * kWave) void predictor_down_mfma_kernel(const T 
         t += (size_t)blockIdx.z * B * r;
     }
     // (14 dwords of arguments, all in scalar registers when the wave starts; the grid's size would arrive by a load)
-    const int gx = launch_word >> 1, round_storage = launch_word & 1;
+    const int gx = launch_word >> 2, rank_first = launch_word & 2, round_storage = launch_word & 1;
     constexpr int kThreads = W * kWave, kPiece = 8 * PC;
     constexpr int kRows = 16 * (MI + NI), kBuf = kRows * PC, kDma = kBuf / 64;   // a wave's buffer in chunks, its 1 KB loads
     static_assert((PC == 16 || PC == 8) && (NB - 1) * kDma < 64, "swizzle; waits count to 63");
@@ -52,9 +52,9 @@ __global__ __launch_bounds__(W * kWave) void predictor_down_mfma_kernel(const T 
     auto swz = [](int row) __attribute__((always_inline)) { return PC == 16 ? row & 15 : (row >> 1) & 7; };
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, q = lane >> 4;
-    // (tiles of x fastest, their number padded to a multiple of the XCDs: a tile's rows come through one L2 only; no division,
-    // which takes a launch of this size 0.3 us)
-    const int m0 = blockIdx.x * 16 * MI, k0 = blockIdx.y * 16 * NI;
+    // (tiles of x fastest, their number padded to a multiple of the XCDs: a tile's rows come through one L2 only.  Or tiles of
+    // the rank, launch_t.  No division, which takes a launch of this size 0.3 us)
+    const int m0 = (rank_first ? blockIdx.y : blockIdx.x) * 16 * MI, k0 = (rank_first ? blockIdx.x : blockIdx.y) * 16 * NI;
     const bool live = m0 < B;
     const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
     const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint4 *)lds;
@@ -498,12 +498,21 @@ static int launch_t(const Tab &tab, int layers, const void *x, int B, int H, con
         auto go = [&](auto kern, int mi, int ni, int waves, int row_chunks) -> int {
             int mt = (B + 16 * mi - 1) / (16 * mi);
             const int nt = (r + 16 * ni - 1) / (16 * ni);
-            if (mt > kXcds) mt = (mt + kXcds - 1) / kXcds * kXcds;
+            // Tiles of x by XCD where x is the larger operand, unless their padded number takes the CUs of an XCD more rounds
+            // than tiles dealt out evenly.  (Order only: the sums are the same.)  Both kernels, bf16, H 4096, tiles of x first
+            // / of the rank first: 100 rows, rank 384, 21.3 / 19.6 us; 160 rows, rank 320, 27.2 / 23.3 (ten tiles: two rounds on
+            // two XCDs); 400 rows, rank 320, 33.7 / 30.4; 1024 rows, rank 256, 32.8 / 37.4
+            const int cus = device_cu_count(), xcd_cus = cus >= kXcds ? cus / kXcds : 1;
+            const bool rank_first = B < r || (layers * ((mt + kXcds - 1) / kXcds) * nt + xcd_cus - 1) / xcd_cus >
+                                                 (layers * mt * nt + cus - 1) / cus;
+            if (!rank_first && mt > kXcds) mt = (mt + kXcds - 1) / kXcds * kXcds;
+            const int gx = rank_first ? nt : mt, gy = rank_first ? mt : nt;
             const int lds = waves * 16 * (mi + ni) * row_chunks * 16;
             const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
             if (rc != ST_OK) return rc;
-            ST_LAUNCH(ps, kern, dim3(mt, nt, layers), dim3(waves * kWave), lds, stream, static_cast<const T *>(x),
-                      static_cast<const T *>(A), B, H, r, t_ws, mask, I, mt << 1 | (round_storage ? 1 : 0), mt * nt, tab);
+            ST_LAUNCH(ps, kern, dim3(gx, gy, layers), dim3(waves * kWave), lds, stream, static_cast<const T *>(x),
+                      static_cast<const T *>(A), B, H, r, t_ws, mask, I, gx << 2 | (rank_first ? 2 : 0) | (round_storage ? 1 : 0),
+                      mt * nt, tab);
             return ST_OK;
         };
         auto blocks = [&](int mi, int ni) { return ((B + 16 * mi - 1) / (16 * mi)) * ((r + 16 * ni - 1) / (16 * ni)); };

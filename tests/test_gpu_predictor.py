@@ -207,6 +207,7 @@ def test_infinite_intermediate_decides_by_sign(dtype, r, B):
     (9, 64, 16, 200), (20, 1000, 128, 8192), (33, 520, 200, 5001), (64, 256, 256, 1000),      # four waves, 4 / 2 / 1 groups
     (77, 520, 104, 5001), (130, 128, 384, 777), (300, 264, 440, 8191), (257, 64, 512, 640),   # eight (four above rank 384)
     (2100, 200, 200, 5001), (2100, 1000, 224, 1000),                                         # 64 x 32 tiles of the intermediate
+    (200, 520, 48, 1000), (160, 264, 320, 1000), (400, 264, 320, 1000), (530, 136, 512, 640),   # tiles of x first; of the rank: x smaller, an uneven number
 ])
 def test_matrix_core_mask_without_scores(dtype, B, H, r, I):
     """Masks decided in registers against the scores the same kernels write: every rank and group form, thresholds that are a
