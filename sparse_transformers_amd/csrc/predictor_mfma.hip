@@ -547,14 +547,19 @@ int launch_predictor_mfma_layers(int dtype, const PredLayers &tab, int layers, c
     return go(tab, layers, x, B, H, nullptr, r, nullptr, I, 0.f, 0, t_ws, nullptr, nullptr, round_storage, stream);
 }
 
-// Five to eight rows at ranks of 129 to 256: the first map as for fewer rows (one wave of loads per rank row on the whole chip;
-// 16-row tiles of x would be half empty), the second on the matrix cores once its multiplications outweigh splitting the rows
-// of t into parts (by the shape alone, as above).  Both kernels, on the vector ALUs / so, us: 18.3 million of them (H 4096, rank
-// 256, I 14336, 5 rows, bf16) 9.64 / 9.53, four layers together 23.2 / 19.2; 29.4 million (8 rows) 10.8 / 10.1, four 26.8 / 19.6,
-// eight 40.9 / 26.8; 13.1 million (rank 160, I 10240, 8 rows, fp16) 9.2 / 10.3.
+// Five to eight rows of bf16 at ranks of 129 to 256: the first map as for fewer rows (one wave of loads per rank row on the
+// whole chip; 16-row tiles of x would be half empty), the second on the matrix cores once its multiplications outweigh
+// splitting the rows of t into parts (by the shape alone, as above).  Both kernels, on the vector ALUs / so, us, H 3072, one
+// layer | eight together, by millions of multiplications (rows, rank, I):
+//    6.6 (5, 160, 8192)   8.29 / 8.71 | 25.2 / 19.5       14.1 (5, 256, 11008)  9.27 / 9.16 | 32.3 / 24.1
+//    9.2 (5, 224, 8192)   8.81 / 8.90 | 28.4 / 22.3       18.4 (8, 160, 14336) 10.21 / 9.53 | 38.3 / 22.9
+//   10.5 (8, 160, 8192)   9.25 / 9.02 | 28.6 / 20.0       25.7 (8, 224, 14336) 10.82 / 9.85 | 40.4 / 25.0
+// fp16 also scales the rows of t, which a single layer does not earn back (18.4 million, 5 rows of rank 256: 9.36 / 10.69; 29.4
+// million, 8 rows: 10.20 / 10.94; eight layers together 33.4 / 26.7, 38.0 / 27.3).  Ranks of 320 to 512 (H 4096, single layers
+// of bf16): 22.9 million, rank 320, 12.7 / 11.6; 15.7, rank 384, 11.5 / 11.3; 21.0, rank 512, 12.0 / 12.4.
 bool predictor_up_mfma_supported(int dtype, int B, int r, int I)
 {
-    return dtype != ST_F32 && B >= 5 && B <= 8 && r > 128 && r <= 256 && (int64_t)B * r * I >= 18000000;
+    return dtype == ST_BF16 && B >= 5 && B <= 8 && r > 128 && r <= 256 && (int64_t)B * r * I >= 10000000;
 }
 
 template <typename Tab>
