@@ -19,7 +19,9 @@ constexpr int kPredDownUnroll = 2;  // chunks per thread issued together
 // any arithmetic, so the kernel costs one memory round trip.
 // BT = rows of x per pass (1 for single-row decode, so that nothing is requested twice).
 // (tab: several layers of equal shape at once, grid dimension y; x [layers,B,H], t [layers,B,r])
-template <typename T, int BT, typename Tab>
+// CLEAR: the mask too, for a second kernel that only switches bytes of it on.  A form of its own: as a run-time case in the
+// eight-row form this kernel took 4.4 and 3.8 us on two machines (H 3072, rank 128, four rows), without it 3.8 and 3.6.
+template <typename T, int BT, bool CLEAR, typename Tab>
 __global__ __launch_bounds__(kPredDownThreads) void predictor_down_kernel(const T *__restrict__ x, int B, int H,
                                                                           const T *__restrict__ A, int r,
                                                                           float *__restrict__ t, int round_storage,
@@ -27,7 +29,7 @@ __global__ __launch_bounds__(kPredDownThreads) void predictor_down_kernel(const 
 {
     if constexpr (Tab::kLayers) {
         A = static_cast<const T *>(tab.l[blockIdx.y].A);
-        if (I > 0) mask = tab.l[blockIdx.y].mask;
+        if (CLEAR) mask = tab.l[blockIdx.y].mask;
         x += (size_t)blockIdx.y * B * H;
         t += (size_t)blockIdx.y * B * r;
     }
@@ -37,8 +39,7 @@ __global__ __launch_bounds__(kPredDownThreads) void predictor_down_kernel(const 
     const int chunks = H / VEC;
     const T *row = A + (size_t)k * H;
     const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
-    // (I > 0: the kernel behind this one only switches bytes of the mask on; r blocks)
-    if constexpr (BT == kPredBTile)
+    if constexpr (CLEAR)   // (r blocks)
         for (int i = k * kPredDownThreads + tid; i < I; i += r * kPredDownThreads) mask[i] = 0;
     for (int b0 = 0; b0 < B; b0 += BT) {
         float acc[BT];
@@ -340,11 +341,12 @@ static int launch_predictor(const PredLaunch &a, const Tab &tab)
         ProfScope ps(ST_K_PRED_DOWN, a.stream);
         auto go = [&](auto kern) {
             ST_LAUNCH(ps, kern, dim3(a.r, a.layers), dim3(kPredDownThreads), 0, a.stream, static_cast<const T *>(a.x), a.B,
-                      a.H, static_cast<const T *>(a.A), a.r, a.t_ws, (a.flags >> 1) & 1, a.mask, up_mfma ? a.I : 0, tab);
+                      a.H, static_cast<const T *>(a.A), a.r, a.t_ws, (a.flags >> 1) & 1, a.mask, a.I, tab);
         };
-        if (a.B == 1) go(predictor_down_kernel<T, 1, Tab>);
-        else if (a.B <= kPredBTile) go(predictor_down_kernel<T, kPredBTile, Tab>);
-        else go(predictor_down_kernel<T, 2 * kPredBTile, Tab>);   // 9 to 16 rows of x in one pass (one memory round trip instead of two)
+        if (a.B == 1) go(predictor_down_kernel<T, 1, false, Tab>);
+        else if (up_mfma) go(predictor_down_kernel<T, kPredBTile, dtype == ST_BF16, Tab>);   // (up_mfma: bf16 only)
+        else if (a.B <= kPredBTile) go(predictor_down_kernel<T, kPredBTile, false, Tab>);
+        else go(predictor_down_kernel<T, 2 * kPredBTile, false, Tab>);   // 9 to 16 rows of x in one pass (one memory round trip instead of two)
     }
     ST_HIP(hipGetLastError());
     if (up_mfma)
