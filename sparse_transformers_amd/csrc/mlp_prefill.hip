@@ -370,21 +370,21 @@ __global__ __launch_bounds__(2 * BM * KS) void prefill_gateup_kernel(const T *__
 // per clock, whatever the number of loads in flight):
 //   wide  256 rows of x by 128 weight rows (64 + 64): 48 KB for 2 x 256 x 128 x 64 flops, about even; the two waves of a SIMD
 //         share a tile (wave kh takes the kh-th 32 of K into accumulators of its own; the pair is summed through LDS once at
-//         the end), three LDS buffers
+//         the end), three LDS buffers; ungated also by 64 weight rows
 //   big   256 by 256 (128 + 128): 64 KB for twice the flops, MFMA bound; x in two LDS buffers, one stage ahead (L2 hits),
 //         the weights, which come from HBM, in three, two stages ahead: the whole 160 KB.  2048 rows, H 4096, 12902 of 14336
 //         active, bf16: 342-355 us against 400 in wide tiles alone (433 GFLOP; 270 without the loads)
 constexpr int kPwBM = 256, kPwThreads = 512, kPwBufs = 3;
 constexpr int kPwLds = 5 * 256 * kPfLd1;   // 16-byte units: the big tile's five buffers, 160 KB (the wide tile's three take 144)
 
-template <typename T, bool HG>
+// kJ: 16-row tiles of up (and of gate) per wave
+template <typename T, bool HG, int kJ>
 __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict__ X, const T *__restrict__ gate,
                                                  const T *__restrict__ up, int M, int H, int n, int n_pad, int j0, int m0,
                                                  T *__restrict__ Hh, long ldh, T *__restrict__ comb, long ldc, int act)
 {
-    constexpr int kWR = HG ? 64 : 128;                    // active rows of the tile
-    constexpr int kJ = HG ? 2 : 4;                        // 16-row tiles of up (and of gate) per wave
-    constexpr int kRows = kPwBM + 128;                    // LDS rows of one buffer: x, gate, up
+    constexpr int kWR = 32 * kJ;                          // active rows of the tile
+    constexpr int kRows = kPwBM + (HG ? 2 : 1) * kWR;     // LDS rows of one buffer: x, gate, up
     constexpr int kBuf = kRows * kPfLd1;                  // 16-byte units per buffer
     constexpr int kDma = kRows / 64;                      // 1 KB loads per wave and stage
     constexpr int kGRow = kPwBM, kURow = kPwBM + (HG ? kWR : 0);
@@ -438,7 +438,7 @@ __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict
             au[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
     // fragments: the wave's k step of a stage is the kh-th 32 of its 64.  The 128 rows of x go through the MFMAs
-    // as four pairs of 16-row fragments, each pair against the wave's four weight fragments.
+    // as four pairs of 16-row fragments, each pair against the wave's weight fragments.
     struct FragB { uint4 g[kJ], u[kJ]; };
     uint4 A[3][2];
     FragB Bc, Bn;
@@ -522,7 +522,7 @@ __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict
     // The pair's sums: the wave with kh = 0 finishes the first 64 rows of the tile, the other the last 64; each
     // hands the other half of its accumulators over through LDS (all stage buffers are free: the last stage ends
     // behind its barrier with no fragment read outstanding).
-    constexpr int kQuads = 16;   // accumulator quads per lane handed over
+    constexpr int kQuads = (HG ? 8 : 4) * kJ;   // accumulator quads per lane handed over
     f32x4_t *red = reinterpret_cast<f32x4_t *>(lds);
     f32x4_t fg[4][kJ], fu[4][kJ];
     {
@@ -533,7 +533,7 @@ __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict
 #pragma unroll
                 for (int j = 0; j < kJ; ++j) {
                     mine[(i * kJ + j) * 64] = au[4 * h + i][j];
-                    if (HG) mine[(8 + i * kJ + j) * 64] = ag[4 * h + i][j];
+                    if (HG) mine[(4 * kJ + i * kJ + j) * 64] = ag[4 * h + i][j];
                     fu[i][j] = au[4 * (1 - h) + i][j];
                     if (HG) fg[i][j] = ag[4 * (1 - h) + i][j];
                 }
@@ -548,7 +548,7 @@ __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict
 #pragma unroll
             for (int j = 0; j < kJ; ++j) {
                 fu[i][j] += other[(i * kJ + j) * 64];
-                if (HG) fg[i][j] += other[(8 + i * kJ + j) * 64];
+                if (HG) fg[i][j] += other[(4 * kJ + i * kJ + j) * 64];
             }
     }
     __syncthreads();
@@ -699,14 +699,23 @@ __device__ __forceinline__ void gateup_big_tile(uint4 *lds, const T *__restrict_
 
 // How the active rows are dealt into tiles: big ones as long as they come in whole rounds over the CUs; what is left over
 // stays big when it keeps more than half of the CUs busy, and is halved into wide tiles (which take about 0.65 of the time)
-// when it does not.  Whole forward, 2048 rows, H 3072, us, the rest big / halved: rest 112 of 256 CUs 217 / 203, 128 220 / 209,
-// 144 225 / 243; no whole round, 128 tiles 94 / 79, 136 95 / 113.
-struct GateupTiles { int big, wide; };
-__host__ __device__ __forceinline__ GateupTiles gateup_tiles(int n_pad, int rows, int mt, int cus)
+// when it does not; ungated, whose halves have no gate rows to split off, into quarters while those fit the CUs too.  Whole
+// forward, 2048 rows, H 3072, us, the rest big / halved: rest 112 of 256 CUs 217 / 203, 128 220 / 209, 144 225 / 243; no whole
+// round, 128 tiles 94 / 79, 136 95 / 113.  Ungated,
+// H 3072, 300 rows, halved / quartered: 48 tiles 68.8 / 58.7, 68 (two rounds of quarters) 75.8 / 92.0; 400 rows, H 4096, 64 99.9 / 91.4.
+struct GateupTiles { int big, small, parts; };   // big tiles, smaller ones, smaller ones per big one
+template <bool HG> __host__ __device__ __forceinline__ GateupTiles gateup_tiles(int n_pad, int rows, int mt, int cus)
 {
     const int t = (n_pad + rows - 1) / rows * mt, rest = t % cus;
-    const int halved = 2 * rest <= cus ? rest : 0;
-    return {t - halved, 2 * halved};
+    const int parts = !HG && 4 * rest <= cus ? 4 : 2 * rest <= cus ? 2 : 1;
+    return parts == 1 ? GateupTiles{t, 0, 1} : GateupTiles{t - rest, parts * rest, parts};
+}
+// The most blocks that any count up to the capacity's `t` big tiles asks for (both kinds in whole eights): the rest of the last
+// round, or any of a whole one before, in the parts that make most of it.
+template <bool HG> static int gateup_blocks(int t, int cus)
+{
+    const int rest = t % cus, in4 = HG ? 0 : 4 * (rest < cus / 4 ? rest : cus / 4), in2 = 2 * (rest < cus / 2 ? rest : cus / 2);
+    return t - rest + (in4 > in2 ? in4 : in2 > rest ? in2 : rest) + kXcds;
 }
 
 template <typename T, bool HG>
@@ -722,7 +731,7 @@ __global__ __launch_bounds__(kPwThreads) void prefill_gateup_wide_kernel(const T
     __shared__ uint4 lds[kPwLds];
     const int n = device_count(n_host, n_dev);
     const int n_pad = (n + kPfBK - 1) / kPfBK * kPfBK;
-    const GateupTiles tiles = gateup_tiles(n_pad, kBigRows, mt, cus);
+    const GateupTiles tiles = gateup_tiles<HG>(n_pad, kBigRows, mt, cus);
     const int big_blocks = (tiles.big + kXcds - 1) / kXcds * kXcds;
     ST_TL(0);
     if ((int)blockIdx.x < big_blocks) {
@@ -730,10 +739,13 @@ __global__ __launch_bounds__(kPwThreads) void prefill_gateup_wide_kernel(const T
         if (tile >= 0)
             gateup_big_tile<T, HG>(lds, X, gate, up, M, H, n, n_pad, tile / mt * kBigRows, tile % mt * kPwBM, Hh, ldh, comb, ldc, act);
     } else {
-        const int half = xcd_tile_id(blockIdx.x - big_blocks, tiles.wide);
-        if (half < 0) return;
-        const int tile = tiles.big + (half >> 1), j0 = tile / mt * kBigRows + (half & 1) * (kBigRows / 2);
-        if (j0 < n_pad) gateup_wide_tile<T, HG>(lds, X, gate, up, M, H, n, n_pad, j0, tile % mt * kPwBM, Hh, ldh, comb, ldc, act);
+        const int part = xcd_tile_id(blockIdx.x - big_blocks, tiles.small);
+        if (part < 0) return;
+        const int shift = tiles.parts == 4 ? 2 : 1, tile = tiles.big + (part >> shift);
+        const int j0 = tile / mt * kBigRows + (part & (tiles.parts - 1)) * (kBigRows >> shift), m0 = tile % mt * kPwBM;
+        if (j0 >= n_pad) return;
+        if (HG || tiles.parts == 4) gateup_wide_tile<T, HG, 2>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
+        else gateup_wide_tile<T, HG, HG ? 2 : 4>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
     }
 }
 
@@ -1556,9 +1568,9 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
         const bool wide_halves = !big && !halves && jt64 * mt128 <= cus;   // K groups on 64 + 64 rows: one block per CU
         const int jt = wide_halves && !quarters ? jt64 : 2 * jt64;
         const int mt = big ? (M + 255) / 256 : quarters ? (M + 63) / 64 : mt128;
-        // (the tiles are dealt out over the device's count: `rest` of gateup_tiles is at most half the CUs for any count)
+        // (the tiles are dealt out over the device's count)
         const int big_tiles = (int)((ldw + (has_gate ? 127 : 255)) / (has_gate ? 128 : 256)) * mt;
-        const int blocks = big ? big_tiles + (big_tiles < cus / 2 ? big_tiles : cus / 2) + kXcds : jt * mt;
+        const int blocks = !big ? jt * mt : has_gate ? gateup_blocks<true>(big_tiles, cus) : gateup_blocks<false>(big_tiles, cus);
         const int grid = (blocks + kXcds - 1) / kXcds * kXcds;
         auto go = [&](auto kern, int threads) -> int {
             ST_LAUNCH(ps, kern, dim3(grid), dim3(threads), 0, stream, static_cast<const T *>(x),

@@ -337,8 +337,12 @@ def test_prefill_tiles_follow_the_device_count(M, n):
     (1030, 128, 8192, 6527, True),     # t = 255; two K stages
     (1030, 256, 8192, 6529, True),     # t = 260: 256 big, 4 halved
     (1030, 256, 8192, 8192, True),     # t = 320: 256 big, 64 halved
-    (2030, 256, 8448, 8200, False),    # t = 264: 256 big, 8 halved, of which the second halves are past the padded count
-    (2030, 384, 8448, 8447, False),    # the same with both halves
+    (2030, 256, 8448, 8200, False),    # t = 264: 256 big, 8 quartered, of which the last two quarters are past the padded count
+    (2030, 384, 8448, 8447, False),    # the same with all quarters
+    (150, 256, 8448, 8447, False),     # t = 33: all quartered, one row tile
+    (1030, 384, 8448, 3001, False),    # t = 60: all quartered
+    (2030, 128, 8448, 2048, False),    # t = 64: the last that is quartered
+    (1030, 640, 8448, 3210, False),    # t = 65: all halved
     (2030, 128, 8448, 4000, False),    # t = 128: all halved
     (2030, 640, 8448, 4200, False),    # t = 136: all big
 ])
