@@ -1524,8 +1524,12 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
     if (alias) comb = nullptr;
     const int64_t hh_bytes = (((int64_t)M * ldw * 2) + 255) & ~(int64_t)255;
     float *partial = reinterpret_cast<float *>(static_cast<unsigned char *>(workspace) + hh_bytes);
-    const bool few = prefill_few(M, H, n), wide_down = !few && prefill_down_is_wide(M, H, n, ldh);
-    const int split_k = few ? prefill_split_k_few(H, n) : wide_down ? prefill_split_k_wide(M, H, n) : prefill_split_k(M, H, n);
+    // (97 to 128 rows fill the plain form's 128-row tile, and up to H = 2048 its splits fill the CUs.  Whole forward, us, few-row
+    // down kernel / plain: 128 rows, H 2048, I 8192, 7372 active, ungated 35.8 / 34.3; H 1024, I 2816, 2534, gated 22.0 / 21.5; H
+    // 2560, I 7040, 4224, gated 43.5 / 48.2)
+    const bool few = prefill_few(M, H, n), few_down = few && (M <= 96 || H > 2048);
+    const bool wide_down = !few && prefill_down_is_wide(M, H, n, ldh);
+    const int split_k = few_down ? prefill_split_k_few(H, n) : wide_down ? prefill_split_k_wide(M, H, n) : prefill_split_k(M, H, n);
     // (four K groups on 64-row tiles, below, are faster for two of them while those make no more blocks than CUs: H 2048, 2500 of
     // 4096 active rows, 128 rows 27.2 us for the whole forward with the few-row kernel, 24.8 so; with one row tile the few-row kernel is: H 1024, 48 rows 20.9 / 18.0)
     const bool two_quarters = M > 64 && H % 256 == 0 && 4 * (ldw / 64) <= device_cu_count();
@@ -1589,7 +1593,7 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
     ST_HIP(hipGetLastError());
     {
         ProfScope ps(ST_K_MLP_PREFILL_DOWN, stream);
-        if (few) {
+        if (few_down) {
             const int ct = H / kPfBN, grid = (ct * split_k + kXcds - 1) / kXcds * kXcds;
             auto go = [&](auto kern) {
                 ST_LAUNCH(ps, kern, dim3(grid), dim3(kPwThreads), 0, stream, Hh, static_cast<const T *>(down), n_dev, ldh, M, H, n,
