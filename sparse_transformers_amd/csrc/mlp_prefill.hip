@@ -1270,7 +1270,7 @@ __global__ __launch_bounds__(kPwThreads) void prefill_down_wide_kernel(const T *
 // A block takes all rows (16 MT), 128 output columns and a K split; stages of 64 through a ring over the whole LDS as in
 // prefill_gateup_few_kernel (two K halves x two halves of the rows x two halves of the columns), Wd's rows as in the wide form.
 // H 2560, 6144 active rows, 77 rows: 14.2 us in 128 x 128 tiles with two
-// LDS buffers and sixteen splits of six stages, now 11.1 with twelve.
+// LDS buffers and sixteen splits of six stages, now 11.2 with twelve.
 template <typename T, int MT>
 __global__ __launch_bounds__(kPwThreads) void prefill_down_few_kernel(const T *__restrict__ Hh, const T *__restrict__ Wd,
                                                                       const int *__restrict__ n_dev, long ldh, int M, int H,

@@ -471,7 +471,9 @@ static int launch_up_t(const Tab &tab, int layers, int B, int r, const void *Bm,
 #define ST_PM_UP(KS, W, IG, RES) go(predictor_up_mfma_kernel<T, KS, W, IG, Tab>, KS, W / IG, W, RES)
 #define ST_PM_UP4(KS, RES) (B <= 16 ? ST_PM_UP(KS, 4, 4, RES) : B <= 32 ? ST_PM_UP(KS, 4, 2, RES) : ST_PM_UP(KS, 4, 1, RES))
         int rc;
-        // (eight waves share a stage once there are rows of x for them: 16 rows in blocks of eight waves 5.2 us, of four 4.4)
+        // (eight waves share a stage once there are rows of x for them: 16 rows in blocks of eight waves 5.2 us, of four 4.4.
+        // At ranks 257 to 384 their fp16 form spills 46 registers, most of them outside the loop: both kernels, 128 rows, rank
+        // 384, fp16 / bf16 26.0 / 20.6 us)
         if (B <= 64) {
             if (r <= 128) rc = ST_PM_UP4(4, 4);
             else if (r <= 256) rc = ST_PM_UP4(8, 2);
