@@ -1524,10 +1524,12 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
     if (alias) comb = nullptr;
     const int64_t hh_bytes = (((int64_t)M * ldw * 2) + 255) & ~(int64_t)255;
     float *partial = reinterpret_cast<float *>(static_cast<unsigned char *>(workspace) + hh_bytes);
-    // (97 to 128 rows fill the plain form's 128-row tile, and up to H = 2048 its splits fill the CUs.  Whole forward, us, few-row
-    // down kernel / plain: 128 rows, H 2048, I 8192, 7372 active, ungated 35.8 / 34.3; H 1024, I 2816, 2534, gated 22.0 / 21.5; H
-    // 2560, I 7040, 4224, gated 43.5 / 48.2)
-    const bool few = prefill_few(M, H, n), few_down = few && (M <= 96 || H > 2048);
+    // (97 to 128 rows fill the plain form's 128-row tile.  Where its sixteen splits at most make one block per CU it is faster for
+    // every count: 128 rows, H 2048, whole forward, us, few-row down kernel / plain, I 8192 ungated 7372 active 35.8 / 34.3, 4915
+    // 32.7 / 31.8; I 5632 gated 3379 33.7 / 32.6.  Narrower than that it depends on the stages of a split -- one more than a
+    // multiple of four costs the plain form 2 to 7 %, others gain 0 to 4: H 768, I 3072, ungated 1843 17.6 / 18.6, 2764 19.5 /
+    // 18.9 -- and wider the few-row kernel is faster: H 2560, I 7040, gated 4224 43.5 / 48.2)
+    const bool few = prefill_few(M, H, n), few_down = few && (M <= 96 || 16 * (H / kPfBN) != device_cu_count());
     const bool wide_down = !few && prefill_down_is_wide(M, H, n, ldh);
     const int split_k = few_down ? prefill_split_k_few(H, n) : wide_down ? prefill_split_k_wide(M, H, n) : prefill_split_k(M, H, n);
     // (four K groups on 64-row tiles, below, are faster for two of them while those make no more blocks than CUs: H 2048, 2500 of
