@@ -193,7 +193,7 @@ def sparse_mlp_forward(x: torch.Tensor, concat_weight: torch.Tensor, active_down
             and handle.fresh():
         # the reference's call sequence natively: the cache's packed rows in place (None: something is not as usual)
         c, n = handle._cache, handle._n
-        need = c._workspace_need(x)
+        need = c._ws_need.get(x.size(0)) or c._size_workspace(x)
         if need is not None:
             got = _lib.native().mlp_forward(x, c.gate_active if has_gate else None, c.up_active, active_down_weight, n, None,
                                             down_proj_buffer, combined_proj_buffer, 0, _kept_workspace(c.device, need),

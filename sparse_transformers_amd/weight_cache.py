@@ -279,13 +279,13 @@ class WeightCache:
         x2 = x if x.dim() == 2 else x.reshape(-1, H)
         return x2 if x2.is_contiguous() else x2.contiguous()
 
-    def _workspace_need(self, x2):
-        """Workspace bytes for the rows of x [B,H] at any count.  None for an x that the general path refuses (so that none of
-        those sizes the workspace, which is kept), looked at once per number of rows."""
+    def _size_workspace(self, x2):
+        """Workspace bytes for the rows of x [B,H] at any count, entered in ``_ws_need``.  None for an x that the general path
+        refuses, so that none of those sizes the workspace, which is kept."""
         B = x2.size(0)
-        need = self._ws_need.get(B)
-        if need is None and 1 <= B <= 4096 and x2.size(1) == self.hidden_size and x2.dtype == self.dtype and x2.device == self.device:
-            need = self._ws_need[B] = mlp_workspace_bytes(B, self.hidden_size, self.intermediate_size)
+        if not 1 <= B <= 4096 or x2.size(1) != self.hidden_size or x2.dtype != self.dtype or x2.device != self.device:
+            return None
+        need = self._ws_need[B] = mlp_workspace_bytes(B, self.hidden_size, self.intermediate_size)
         return need
 
     def _native_call(self, x, act, out, workspace, call):
@@ -299,7 +299,7 @@ class WeightCache:
             if out is not None or x.shape[-1] != self.hidden_size or not x.is_contiguous():
                 return None
             x2 = x.view(-1, self.hidden_size)
-        need = self._workspace_need(x2)
+        need = self._ws_need.get(x2.size(0)) or self._size_workspace(x2)
         if need is None:
             return None
         if workspace is None:
