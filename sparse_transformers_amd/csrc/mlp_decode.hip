@@ -479,6 +479,19 @@ int batch_min_rows()
     return v;
 }
 
+// Rows of x that take the GEMM kernels (mlp_prefill.hip) rather than the batch kernels: all beyond two MFMA tiles; of 17 to 32
+// those whose intermediate is held in the storage type either way, where the matrices are large (by their capacity, so that
+// the form does not change with the count).  Whole forward, us, batch / GEMM kernels: 32 rows, H 3840, 5000 of 10240 45.2 /
+// 39.1; 24 rows, H 4864, 6000 of 16384 56.3 / 45.1; 20 rows, H 4096, 2000 of 14336 26.3 / 27.7; 32 rows, H 2560, 3000 of 10240
+// 27.3 / 26.8, 20 rows 24.1 / 24.8; 24 rows, H 3072, 2867 of 8192 26.4 / 27.4.  32 rows where H is no multiple of 256: H 3200,
+// 5000 of 11200 48.4 / 34.3.  (17 to 31 rows there keep fp32 between the batch kernels.)
+static bool gemm_rows(int dtype, int64_t B, int64_t H, int64_t n)
+{
+    if (dtype == ST_F32 || H % 128 != 0 || n < 1) return false;
+    if (B > kBatchMaxRows) return true;
+    return H % 256 != 0 ? B == kBatchMaxRows : B > 16 && n * H >= (int64_t)32 << 20;
+}
+
 // Blocks per launch: one per CU by default; ST_MLP_GMULT (1..4) multiplies it.
 int mlp_grid()
 {
@@ -606,11 +619,11 @@ extern "C" int64_t st_mlp_workspace_bytes(int64_t B, int64_t H, int64_t n)
 {
     const int64_t G = st::mlp_grid();
     int64_t decode = G * st::kMlpMaxBatchPerLaunch * H * 4;
-    if (B >= st::batch_min_rows() && B <= st::kBatchMaxRows) {   // dtype is not known here: size for both paths
+    if (B >= st::batch_min_rows()) {   // dtype is not known here: size for both paths
         const int64_t batch = st::batch_workspace_bytes(H, n);
         decode = batch > decode ? batch : decode;
     }
-    if (B < st::kPrefillMinRows) return decode;
+    if (B <= 16) return decode;   // (gemm_rows)
     const int64_t prefill = st::prefill_workspace_bytes(B, H, n);
     return prefill > decode ? prefill : decode;
 }
@@ -634,8 +647,9 @@ extern "C" int st_mlp_forward(const void *x, int64_t B, int64_t H, const void *g
     ST_REQUIRE(workspace_bytes >= st_mlp_workspace_bytes(B, H, n), "st_mlp_forward: workspace too small (%lld < %lld)",
                (long long)workspace_bytes, (long long)st_mlp_workspace_bytes(B, H, n));
 
-    const bool batch = B >= batch_min_rows() && B <= kBatchMaxRows && batch_supported(dtype, (int)H);
-    if (B >= kPrefillMinRows && !batch && dtype != ST_F32 && H % 128 == 0 && n >= 1)
+    const bool gemm = gemm_rows(dtype, B, H, n);
+    const bool batch = !gemm && B >= batch_min_rows() && batch_supported(dtype, (int)B, (int)H);
+    if (gemm || (!batch && B >= kPrefillMinRows && gemm_rows(dtype, kBatchMaxRows + 1, H, n)))
         return launch_prefill(dtype, x, (int)B, (int)H, gate_rows, up_rows, down_rows, (int)n, n_dev,
                               (int)(n_hint < 0 ? 0 : n_hint > n ? n : n_hint), out, combined,
                               (long)ldc, workspace, act, has_gate ? 1 : 0, static_cast<hipStream_t>(stream));

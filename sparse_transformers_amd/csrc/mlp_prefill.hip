@@ -1554,7 +1554,8 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
                 else go(prefill_gateup_few_kernel<T, false, MT, 2>, 64);
             }
         };
-        if (M <= 64) rows(std::integral_constant<int, 4>{});
+        if (M <= 32) rows(std::integral_constant<int, 2>{});
+        else if (M <= 64) rows(std::integral_constant<int, 4>{});
         else if (M <= 96) rows(std::integral_constant<int, 6>{});
         else rows(std::integral_constant<int, 8>{});
     } else {
@@ -1601,7 +1602,8 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
                 ST_LAUNCH(ps, kern, dim3(grid), dim3(kPwThreads), 0, stream, Hh, static_cast<const T *>(down), n_dev, ldh, M, H, n,
                           split_k, ct, static_cast<T *>(out), partial);
             };
-            if (M <= 64) go(prefill_down_few_kernel<T, 4>);
+            if (M <= 32) go(prefill_down_few_kernel<T, 2>);
+            else if (M <= 64) go(prefill_down_few_kernel<T, 4>);
             else if (M <= 96) go(prefill_down_few_kernel<T, 6>);
             else go(prefill_down_few_kernel<T, 8>);
         } else if (wide_down) {

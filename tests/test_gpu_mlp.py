@@ -435,6 +435,18 @@ def test_prefill_few_rows_infinite_last_row(M, H, I, n, gated):
     assert_close(out[:, finite].float().cpu().numpy(), want[:, finite].cpu().numpy(), "float16", f"{M} rows, {n} active")
 
 
+@pytest.mark.parametrize("M,H,I,n,gated", [
+    (17, 1024, 33000, 8129, True), (31, 2048, 16500, 63, False), (32, 640, 9000, 8191, True), (32, 128, 40, 1, True),
+    (24, 768, 44000, 6143, False),
+])
+def test_prefill_of_17_to_32_rows(M, H, I, n, gated):
+    """The few-row form of one pair of tiles, where it takes rows that the batch kernels could: the checks of the two tests above.
+    (At most 2048 wide: rounding the intermediate to fp16 puts sqrt(n) * 0.05 * rms(h) * 1e-4 on a result, 0.0016 at rms(h) = 3.6 and
+    8129 rows, against a bound of 0.02; at 4096, rms(h) near 10, two of 69632 results pass it.)"""
+    test_prefill_few_rows(M, H, I, n, gated)
+    test_prefill_few_rows_infinite_last_row(M, H, I, n, gated)
+
+
 @pytest.mark.parametrize("M,H,n,gated,stride", [
     (200, 65536, 33000, False, 0),                # weights of 4.3 GB
     (4096, 128, 524416, False, 0),                # an intermediate of 4.3 GB
@@ -558,6 +570,49 @@ def test_batch_mfma_vs_oracle(name, B, H, n, dtype, act, has_gate):
     assert tuple(out.shape) == (B, H) and tuple(cb.shape) == (B, cw.shape[0])
     assert_close(out.float().cpu().numpy(), want, dtype, name)
     assert_close(cb.float().cpu().numpy(), wantc, dtype, name + " combined")
+
+
+@pytest.mark.parametrize("B,H,I,n,dtype,gated", [
+    (3, 64, 40, 1, "float32", True), (8, 128, 300, 257, "float32", False), (17, 1424, 700, 511, "float32", True),
+    (5, 2816, 5000, 4113, "float32", True), (33, 912, 4500, 4097, "float32", True), (70, 8192, 300, 299, "float32", False),
+    (3, 64, 40, 16, "float16", True), (16, 192, 17000, 16385, "bfloat16", False), (17, 128, 33, 17, "float16", True),
+    (9, 1664, 6144, 1230, "bfloat16", True), (32, 896, 4500, 4096, "float16", True), (25, 1152, 9000, 8200, "bfloat16", True),
+    (32, 1600, 5000, 4095, "float16", False), (31, 3200, 2000, 1999, "bfloat16", True), (12, 4736, 700, 333, "float16", True),
+    (22, 16384, 100, 97, "bfloat16", False), (40, 1216, 3000, 2900, "float16", True),
+])
+def test_batch_any_width(B, H, I, n, dtype, gated):
+    """The batch kernels for any width whose rows are multiples of 64 bytes, and fp32: remainders of the steps per wave, both
+    forms of x (LDS, registers), one and two subtiles per tile, several passes of 32 rows; the count comes from the device, rows
+    past it are NaN and the last active row of the down weights holds an infinity, which must meet nothing but its own
+    intermediate.  Against float64; fp32 sums of at most 16384 products in another order: within 1e-5 of the largest value."""
+    td = getattr(torch, dtype)
+    g = torch.Generator().manual_seed(B * H + n)
+    gate, up, dn = ((torch.randn(I, H, generator=g) * H ** -0.5).to(td).to(DEV) for _ in range(3))
+    x = torch.randn(B, H, generator=g).to(td).to(DEV)
+    dn[n - 1, H // 2] = float("inf")
+    hu = x.double() @ up[:n].double().t()
+    hh = (x.double() @ gate[:n].double().t()) if gated else hu
+    h = torch.nn.functional.silu(hh) * (hu if gated else 1.0)
+    fin = dn[:n].double()
+    fin[n - 1, H // 2] = 0.0
+    want = h @ fin
+    for t in (gate, up, dn):
+        t[n:] = float("nan")
+    comb = torch.full((B, 2 * n if gated else n), float("nan"), dtype=td, device=DEV)
+    outs = []
+    for cap, n_dev, c in ((I, torch.tensor([n], dtype=torch.int32, device=DEV), None), (n, None, comb)):
+        out = torch.full((B, H), float("nan"), dtype=td, device=DEV)
+        mlp_forward_rows(x, gate if gated else None, up, dn, cap, n_dev, out, c, "silu", gated)
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])                       # the form does not depend on where the count comes from
+    inf_col = outs[0][:, H // 2].double()
+    assert torch.equal(inf_col, h[:, n - 1].sign() * float("inf"))
+    outs[0][:, H // 2], want[:, H // 2] = 0, 0
+    assert_close(outs[0].float().cpu().numpy(), want.cpu().numpy(), dtype, "out")
+    assert_close(comb[:, :n].float().cpu().numpy(), h.cpu().numpy(), dtype, "combined, h")
+    if gated:
+        assert_close(comb[:, n:].float().cpu().numpy(), hu.cpu().numpy(), dtype, "combined, up")
 
 
 def test_batch_mfma_device_count_and_determinism():
