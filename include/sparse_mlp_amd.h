@@ -7,7 +7,7 @@
  * ST_OK (0) or a negative st_status; st_last_error() gives a message for the
  * calling thread.  No entry point except st_cache_create/st_cache_destroy
  * (host memory only) and st_cache_sync_state, st_cache_update_sync and
- * st_cache_load_weights_masked (which wait for `stream`) allocates or
+ * st_cache_load_weights_masked / _end (which wait for `stream`) allocates or
  * synchronises: work is enqueued on `stream` and ordered with whatever else
  * the caller enqueues there.
  *
@@ -242,6 +242,12 @@ int st_cache_load_weights(st_cache *c, const void *gate, const void *up, const v
  * st_cache_update_sync. */
 int st_cache_load_weights_masked(st_cache *c, const void *gate, const void *up, const void *down, const uint8_t *mask,
                                  int32_t *state_out, void *stream);
+
+/* The same in two halves: _begin enqueues on `stream` and returns (the weights and the mask are read after it returns),
+ * _end waits for what _begin enqueued on that stream and gives the outcome.  Nothing else is called on the cache in between. */
+int st_cache_load_weights_begin(st_cache *c, const void *gate, const void *up, const void *down, const uint8_t *mask,
+                                void *stream);
+int st_cache_load_weights_end(st_cache *c, int32_t *state_out, void *stream);
 
 /* update_active_weights(mask): weight_cache.h:229-359 (diff :84-110, pairing
  * :248-277, append :280-307, swap-with-last :310-353).  mask: uint8/bool [I]

@@ -59,6 +59,8 @@ SIGNATURES = {
     "st_cache_destroy": (None, [_vp]),
     "st_cache_load_weights": (_ci, [_vp, _vp, _vp, _vp, _vp]),
     "st_cache_load_weights_masked": (_ci, [_vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "st_cache_load_weights_begin": (_ci, [_vp, _vp, _vp, _vp, _vp, _vp]),
+    "st_cache_load_weights_end": (_ci, [_vp, _vp, _vp]),
     "st_cache_update_async": (_ci, [_vp, _vp, _vp]),
     "st_cache_update_layers": (_ci, [C.POINTER(_vp), C.POINTER(_vp), _i64, _vp]),
     "st_cache_update_sync": (_ci, [_vp, _vp, _vp, _vp]),
@@ -113,7 +115,8 @@ def native():
             raise NativeLibraryMissing(f"{HERE}/_host.so cannot be loaded ({e}): build it with "
                                        "`python -m sparse_transformers_amd.build`") from e
         _host.bind(*(C.cast(getattr(L, f), C.c_void_p).value
-                     for f in ("st_predictor_mask_ex", "st_cache_update_forward", "st_mlp_forward")))
+                     for f in ("st_predictor_mask_ex", "st_cache_update_forward", "st_mlp_forward", "st_cache_create",
+                               "st_cache_destroy", "st_cache_load_weights_begin", "st_cache_max_intermediate")))
         _native = _host
     return _native
 

@@ -19,6 +19,10 @@ namespace {
 decltype(&st_predictor_mask_ex) f_predictor;
 decltype(&st_cache_update_forward) f_update_forward;
 decltype(&st_mlp_forward) f_mlp_forward;
+decltype(&st_cache_create) f_cache_create;
+decltype(&st_cache_destroy) f_cache_destroy;
+decltype(&st_cache_load_weights_begin) f_load_begin;
+decltype(&st_cache_max_intermediate) f_max_intermediate;
 
 // A plain tensor with memory of its own on a GPU (no subclass, no wrapper of a transform); nullptr: not one.
 const at::Tensor *gpu_tensor(PyObject *o)
@@ -217,21 +221,78 @@ PyObject *mlp_forward(PyObject *, PyObject *const *a, Py_ssize_t n_args)
     });
 }
 
-// bind(st_predictor_mask_ex, st_cache_update_forward, st_mlp_forward): their addresses in the loaded library
+// cache_build(gate | None, up, down, mask, H, state_words, stream) -> (handle, gate_pool | None, up_pool, downT_pool, gate_active |
+// None, up_active, down_active, book) | status | None: a new cache's buffers and handle, its kernel launched.  The caller
+// waits for it (st_cache_load_weights_end) and keeps the weights and the mask until then.  `book` (int32) holds the index list
+// [2, I], the remembered mask (2 I bytes) and the state words, each at a multiple of 64 words.
+PyObject *cache_build(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    if (n != 7 || !f_load_begin) return none();
+    return guarded([&]() -> PyObject * {
+        const at::Tensor *gate = a[0] == Py_None ? nullptr : gpu_tensor(a[0]), *up = gpu_tensor(a[1]), *down = gpu_tensor(a[2]),
+                         *mask = gpu_tensor(a[3]);
+        if (!up || !down || !mask || (a[0] != Py_None && !gate) || up->dim() != 2) return none();
+        const int64_t I = up->size(0), H = up->size(1), hidden = PyLong_AsLongLong(a[4]), words = PyLong_AsLongLong(a[5]);
+        void *stream = PyLong_AsVoidPtr(a[6]);
+        if (PyErr_Occurred()) { PyErr_Clear(); return none(); }
+        const int code = code_of(*up);
+        if (code < 0 || I < 1 || I > f_max_intermediate() || H < 1 || H != hidden || words < 1) return none();
+        if (!rows_of(*up, H) || !rows_of(*down, I) || down->size(0) != H || !same_kind(*down, *up)) return none();
+        if (gate && (!rows_of(*gate, H) || gate->size(0) != I || !same_kind(*gate, *up))) return none();
+        if (!bytes_of(*mask, *up, I)) return none();
+        at::Tensor t[6];   // pools, packed rows
+        for (int k = 0; k < 6; ++k)
+            if (gate || k % 3 != 0) t[k] = at::empty({I, H}, up->options());
+        auto whole = [](int64_t v) { return (v + 63) / 64 * 64; };
+        const int64_t at_mask = whole(2 * I), at_state = at_mask + whole((2 * I + 3) / 4);
+        at::Tensor book = at::empty({at_state + words}, up->options().dtype(at::kInt));
+        int32_t *pb = static_cast<int32_t *>(book.data_ptr());
+        auto ptr = [&](int k) { return t[k].defined() ? t[k].data_ptr() : nullptr; };
+        const st_cache_buffers bufs = {ptr(0), ptr(1), ptr(2), ptr(3), ptr(4), ptr(5), pb, reinterpret_cast<uint8_t *>(pb + at_mask), pb + at_state};
+        st_cache *c = f_cache_create(&bufs, I, H, code, gate ? 1 : 0);
+        if (!c) return none();   // (the general path raises what it says)
+        const void *pg = gate ? gate->data_ptr() : nullptr, *pu = up->data_ptr(), *pd = down->data_ptr();
+        const uint8_t *pm = static_cast<const uint8_t *>(mask->data_ptr());
+        const int rc = launched([&] { return f_load_begin(c, pg, pu, pd, pm, stream); });
+        if (rc != ST_OK) {
+            f_cache_destroy(c);
+            return PyLong_FromLong(rc);
+        }
+        // from here on nothing throws: the kernel writes to these buffers
+        auto wrap = [](const at::Tensor &v) -> PyObject * {
+            if (!v.defined()) { Py_RETURN_NONE; }
+            return THPVariable_Wrap(v);
+        };
+        PyObject *r = PyTuple_New(8);
+        if (!r) return nullptr;
+        PyTuple_SET_ITEM(r, 0, PyLong_FromVoidPtr(c));
+        for (int k = 0; k < 6; ++k) PyTuple_SET_ITEM(r, 1 + k, wrap(t[k]));
+        PyTuple_SET_ITEM(r, 7, wrap(book));
+        return r;
+    });
+}
+
+// bind(st_predictor_mask_ex, st_cache_update_forward, st_mlp_forward, st_cache_create, st_cache_destroy,
+// st_cache_load_weights_begin, st_cache_max_intermediate): their addresses in the loaded library
 PyObject *bind(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
-    if (n != 3) {
-        PyErr_SetString(PyExc_TypeError, "bind takes three addresses");
+    constexpr int kFunctions = 7;
+    if (n != kFunctions) {
+        PyErr_SetString(PyExc_TypeError, "bind takes seven addresses");
         return nullptr;
     }
-    void *p[3];
-    for (int i = 0; i < 3; ++i) {
+    void *p[kFunctions];
+    for (int i = 0; i < kFunctions; ++i) {
         p[i] = PyLong_AsVoidPtr(a[i]);
         if (PyErr_Occurred()) return nullptr;
     }
     f_predictor = reinterpret_cast<decltype(f_predictor)>(p[0]);
     f_update_forward = reinterpret_cast<decltype(f_update_forward)>(p[1]);
     f_mlp_forward = reinterpret_cast<decltype(f_mlp_forward)>(p[2]);
+    f_cache_create = reinterpret_cast<decltype(f_cache_create)>(p[3]);
+    f_cache_destroy = reinterpret_cast<decltype(f_cache_destroy)>(p[4]);
+    f_load_begin = reinterpret_cast<decltype(f_load_begin)>(p[5]);
+    f_max_intermediate = reinterpret_cast<decltype(f_max_intermediate)>(p[6]);
     Py_RETURN_NONE;
 }
 
@@ -240,6 +301,7 @@ PyMethodDef methods[] = {
     {"predictor_mask", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(predictor_mask)), METH_FASTCALL, nullptr},
     {"update_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(update_forward)), METH_FASTCALL, nullptr},
     {"mlp_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(mlp_forward)), METH_FASTCALL, nullptr},
+    {"cache_build", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(cache_build)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -107,65 +107,86 @@ class WeightCache:
         self.has_gate = bool(has_gate)
         if self.has_gate and gate_weight is None:
             raise ValueError("has_gate=True needs gate_weight")
-        dev = require_gpu(up_weight, down_weight, gate_weight if self.has_gate else None)
-        self.device = dev
-        self.dtype = up_weight.dtype
-        self.hidden_size = int(hidden_size)
-        self.intermediate_size = int(up_weight.size(0))
-        I, H = self.intermediate_size, self.hidden_size
-        if tuple(up_weight.shape) != (I, H) or tuple(down_weight.shape) != (H, I):
-            raise ValueError(f"up must be [I,H] and down [H,I]; got {tuple(up_weight.shape)}, {tuple(down_weight.shape)}")
-        if self.has_gate and tuple(gate_weight.shape) != (I, H):
-            raise ValueError(f"gate must be [{I},{H}], got {tuple(gate_weight.shape)}")
-        if down_weight.dtype != self.dtype or (self.has_gate and gate_weight.dtype != self.dtype):
-            raise TypeError("gate, up and down weights must share one dtype")
-        if self.dtype == torch.float64:
-            raise TypeError("the weight cache holds float32, float16 or bfloat16 rows (float64 is served by "
-                            "sparse_mlp_forward on caller-owned rows only)")
-        code = dtype_code(up_weight)
         L = _lib.lib()
-        if I > L.st_cache_max_intermediate():
-            raise ValueError(f"intermediate size {I} exceeds the supported maximum {L.st_cache_max_intermediate()}")
-
-        def wbuf():
-            return torch.empty(I, H, dtype=self.dtype, device=dev)
-
-        self.gate_pool = wbuf() if self.has_gate else None
-        self.up_pool = wbuf()
-        self.downT_pool = wbuf()
-        self.gate_active = wbuf() if self.has_gate else None
-        self.up_active = wbuf()
-        self.down_active = wbuf()
-        # bookkeeping is double-buffered on the device; state[STATE_EPOCH] says which half is current
-        self.indices = torch.empty(2, I, dtype=torch.int32, device=dev)
-        self.cur_mask = torch.empty(2, I, dtype=torch.uint8, device=dev)
-        self.state = torch.empty(_lib.STATE_WORDS, dtype=torch.int32, device=dev)
-        self.n_active_dev = self.state[_lib.STATE_N_ACTIVE:_lib.STATE_N_ACTIVE + 1]
-
-        bufs = _lib.CacheBuffers(
-            self.gate_pool.data_ptr() if self.has_gate else None, self.up_pool.data_ptr(), self.downT_pool.data_ptr(),
-            self.gate_active.data_ptr() if self.has_gate else None, self.up_active.data_ptr(),
-            self.down_active.data_ptr(), self.indices.data_ptr(), self.cur_mask.data_ptr(), self.state.data_ptr())
-        self._h = L.st_cache_create(C.byref(bufs), I, H, code, int(self.has_gate))
-        if not self._h:
-            raise ValueError(_lib.last_error())
-
-        up_c = up_weight.detach().contiguous()
-        down_c = down_weight.detach().contiguous()
-        gate_c = gate_weight.detach().contiguous() if self.has_gate else None
+        # weight_cache.h:226: the constructor ends with update_active_weights(init_mask); here in one pass over the weights,
+        # whose kernel runs while the object is put together
+        dev = up_weight.device
+        stream = current_stream_ptr(dev) if dev.type == "cuda" else None
+        built = None if stream is None else _lib.native().cache_build(
+            gate_weight if self.has_gate else None, up_weight, down_weight, init_mask, int(hidden_size), _lib.STATE_WORDS, stream)
+        if type(built) is int:
+            _lib.check(built, "st_cache_load_weights_masked")
+        keep = None
+        if built is None:
+            built, keep = self._build(init_mask, int(hidden_size), gate_weight, up_weight, down_weight)
+            stream = current_stream_ptr(built[2].device)
+        (self._h, self.gate_pool, self.up_pool, self.downT_pool, self.gate_active, self.up_active, self.down_active,
+         book) = built
+        self._dirty = True          # updates enqueued since the last read-back
         self._host_state = (C.c_int32 * _lib.STATE_WORDS)()
+        self.device = self.up_pool.device
+        self.dtype = self.up_pool.dtype
+        self.intermediate_size, self.hidden_size = I, _ = self.up_pool.shape
+        # bookkeeping is double-buffered on the device; state[STATE_EPOCH] says which half is current
+        at_mask, at_state = self._book_layout(I)
+        self.indices = book[:2 * I].view(2, I)
+        self.cur_mask = book[at_mask:at_state].view(torch.uint8)[:2 * I].view(2, I)
+        self.state = book[at_state:]
+        self.n_active_dev = self.state[_lib.STATE_N_ACTIVE:_lib.STATE_N_ACTIVE + 1]
         self._seen = C.c_int32.from_address(L.st_cache_seen_count(self._h))   # the count the last finished update told the host
         self.lazy_updates = False
         self._pending_mask: Optional[torch.Tensor] = None
         self._concat_ref = None     # weak reference to the handle get_concat_weight() handed out last
         self._concat_serial = -1
         self._ws_need: dict = {}    # workspace bytes by rows of x (1 to 4096)
-        # weight_cache.h:226: the constructor ends with update_active_weights(init_mask); here in one pass over the weights
-        mask = self._mask_arg(init_mask)
-        rc = L.st_cache_load_weights_masked(self._h, gate_c.data_ptr() if self.has_gate else None, up_c.data_ptr(),
-                                            down_c.data_ptr(), mask.data_ptr(), self._host_state, current_stream_ptr(dev))
-        self._dirty = rc != _lib.ST_OK   # updates enqueued since the last read-back
+        rc = L.st_cache_load_weights_end(self._h, self._host_state, stream)
+        del keep
+        self._dirty = rc != _lib.ST_OK
         _lib.check(rc, "st_cache_load_weights_masked")
+
+    @staticmethod
+    def _book_layout(I: int):
+        """Words of the bookkeeping buffer in front of the remembered mask and of the state words (csrc/host_ext.cpp)."""
+        at_mask = (2 * I + 63) // 64 * 64
+        return at_mask, at_mask + ((2 * I + 3) // 4 + 63) // 64 * 64
+
+    def _build(self, init_mask: torch.Tensor, H: int, gate_weight: Optional[torch.Tensor], up_weight: torch.Tensor,
+               down_weight: torch.Tensor):
+        """What ``cache_build`` does, for every form of the arguments, and what has to outlive the kernel."""
+        dev = self.device = require_gpu(up_weight, down_weight, gate_weight if self.has_gate else None)
+        dtype = up_weight.dtype
+        I = self.intermediate_size = int(up_weight.size(0))
+        if tuple(up_weight.shape) != (I, H) or tuple(down_weight.shape) != (H, I):
+            raise ValueError(f"up must be [I,H] and down [H,I]; got {tuple(up_weight.shape)}, {tuple(down_weight.shape)}")
+        if self.has_gate and tuple(gate_weight.shape) != (I, H):
+            raise ValueError(f"gate must be [{I},{H}], got {tuple(gate_weight.shape)}")
+        if down_weight.dtype != dtype or (self.has_gate and gate_weight.dtype != dtype):
+            raise TypeError("gate, up and down weights must share one dtype")
+        if dtype == torch.float64:
+            raise TypeError("the weight cache holds float32, float16 or bfloat16 rows (float64 is served by "
+                            "sparse_mlp_forward on caller-owned rows only)")
+        code = dtype_code(up_weight)
+        L = _lib.lib()
+        if I > L.st_cache_max_intermediate():
+            raise ValueError(f"intermediate size {I} exceeds the supported maximum {L.st_cache_max_intermediate()}")
+        bufs = [torch.empty(I, H, dtype=dtype, device=dev) if self.has_gate or k % 3 else None for k in range(6)]
+        at_mask, at_state = self._book_layout(I)
+        book = torch.empty(at_state + _lib.STATE_WORDS, dtype=torch.int32, device=dev)
+        ptrs = [t.data_ptr() if t is not None else None for t in bufs]
+        base = book.data_ptr()
+        h = L.st_cache_create(C.byref(_lib.CacheBuffers(*ptrs, base, base + 4 * at_mask, base + 4 * at_state)), I, H, code,
+                              int(self.has_gate))
+        if not h:
+            raise ValueError(_lib.last_error())
+        self._h = h
+        up_c = up_weight.detach().contiguous()
+        down_c = down_weight.detach().contiguous()
+        gate_c = gate_weight.detach().contiguous() if self.has_gate else None
+        mask = self._mask_arg(init_mask)
+        rc = L.st_cache_load_weights_begin(h, gate_c.data_ptr() if self.has_gate else None, up_c.data_ptr(), down_c.data_ptr(),
+                                           mask.data_ptr(), current_stream_ptr(dev))
+        _lib.check(rc, "st_cache_load_weights_masked")
+        return (h, *bufs, book), (up_c, down_c, gate_c, mask)
 
     def __del__(self):
         h, self._h = getattr(self, "_h", None), None

@@ -253,3 +253,38 @@ def test_threads_and_streams():
     for t in ts:
         t.join(60)
     assert all(torch.equal(a, b) for g in got for a, b in zip(g, want))
+
+
+@pytest.mark.parametrize("I,H,gated,dtype", [(1, 64, True, torch.float32), (203, 72, False, torch.float16), (2048, 256, True, torch.bfloat16)])
+def test_cache_construction_forms(I, H, gated, dtype):
+    """A cache built by the native path and by the general one, which takes every other form of the arguments (strided weights, a
+    mask of numbers or on the host), hold the same; sizes and types that do not fit are refused by either."""
+    g = torch.Generator(device=DEV).manual_seed(I)
+    gate, up, down = (torch.randn(*s, generator=g, device=DEV).to(dtype) for s in ((I, H), (I, H), (H, I)))
+    mask = torch.rand(I, generator=g, device=DEV) < 0.7
+    mask[0] = True
+    native = st._lib.native()
+    fast = st.WeightCache(mask, H, gate if gated else None, up, down, gated)
+    strided = down.t().contiguous().t()
+    for args in ((mask.float(), H, gate, up, down), (mask.cpu(), H, gate, up, down), (mask, H, gate, up, strided)):
+        if args[4] is strided and I == 1:
+            continue                                       # (one column: contiguous either way)
+        assert native.cache_build(args[2] if gated else None, args[3], args[4], args[0], H, st._lib.STATE_WORDS,
+                                  torch.cuda.current_stream().cuda_stream) is None
+        slow = st.WeightCache(args[0], args[1], args[2] if gated else None, *args[3:], gated)
+        assert fast.sync_state() == slow.sync_state() and (fast.intermediate_size, fast.hidden_size) == (I, H)
+        n = fast.get_num_active()
+        for name in ("gate_pool", "up_pool", "downT_pool", "gate_active", "up_active", "down_active", "indices", "cur_mask", "state"):
+            a, b = getattr(fast, name), getattr(slow, name)
+            assert (a is None) == (b is None) == (name.startswith("gate") and not gated)
+            if a is not None:
+                assert a.shape == b.shape and a.dtype == b.dtype
+                e = int(fast.sync_state()["epoch"])
+                rows = slice(0, n) if name.endswith("active") else e if name == "cur_mask" else slice(None)
+                assert torch.equal(a[e, :n], b[e, :n]) if name == "indices" else torch.equal(a[rows], b[rows]), name
+    for bad in ((mask, H + 8, gate, up, down), (mask, H, gate, up, down[:, :-1] if I > 1 else down[:-1]), (mask[:-1], H, gate, up, down),
+                (mask, H, gate.double(), up.double(), down.double())):
+        with pytest.raises((ValueError, TypeError)):
+            st.WeightCache(bad[0], bad[1], bad[2] if gated else None, *bad[3:], gated)
+    with pytest.raises(RuntimeError):
+        st.WeightCache(torch.zeros_like(mask), H, gate if gated else None, up, down, gated)
