@@ -137,6 +137,48 @@ __device__ __forceinline__ uint32_t pack_bits8(uint64_t ones)
     return (uint32_t)((ones * 0x0102040810204080ull) >> 56);
 }
 
+// Eight bytes of a mask and four entries of an index list at any alignment: sizes that are no multiples of eight put the second
+// half of the double buffers, and the masks of a stack's layers, anywhere.  (The loads are the same instructions.)  The last
+// word of such a mask, or the last vector of a list, is the one that ends with it; mask_tail and list_tail shift its first
+// elements down, at the place of use: shifted where it is loaded, the load would be waited for there.  I >= 8; what lies
+// past I reads as zero in a mask and as anything in a list.  I 3405, H 896, bf16, eight rows, a stack of four layers: 86 us with
+// the updates byte by byte, layer by layer; 70 so, in one launch.  One or two rows of x also get the fused kernel.
+__device__ __forceinline__ uint64_t load_mask(const uint8_t *m, int e, int I)
+{
+    uint64_t v;
+    __builtin_memcpy(&v, m + (e < I - 8 ? e : I - 8), 8);
+    return v;
+}
+__device__ __forceinline__ uint64_t mask_tail(uint64_t v, int e, int I)
+{
+    const int over = e + 8 - I;   // (words past the end, all of whose elements are, come out as anything)
+    return v >> (8 * (over > 0 ? over : 0) & 63);
+}
+__device__ __forceinline__ void store_mask(uint8_t *m, int e, int I, uint64_t v)
+{
+    if (e + 8 <= I) {
+        __builtin_memcpy(m + e, &v, 8);
+    } else {
+        for (int k = 0; k < I - e; ++k) m[e + k] = (uint8_t)(v >> (8 * k));
+    }
+}
+typedef int list4_t __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ int4 load_list(const int32_t *l, int p, int I)
+{
+    const list4_t v = *reinterpret_cast<const list4_t *>(l + (p < I - 4 ? p : I - 4));
+    return make_int4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ int4 list_tail(int4 c, int p, int I)
+{
+    if (I & 3) {   // uniform
+        const int over = p + 4 - I;
+        const bool one = over > 0 && (over & 1), two = over > 0 && (over & 2);
+        c.x = one ? c.y : c.x; c.y = one ? c.z : c.y; c.z = one ? c.w : c.z;
+        c.x = two ? c.z : c.x; c.y = two ? c.w : c.y;
+    }
+    return c;
+}
+
 // The plan as every block computes it, and the LDS arrays that hold it.
 struct PlanView {
     uint16_t *pos_l;    // index -> position (kNone when absent)
@@ -155,7 +197,7 @@ struct PlanView {
 
 constexpr size_t plan_lds_bytes(int I)
 {
-    return (size_t)I * 6 + (size_t)(I & 1) * 2 + (size_t)((((I + 31) >> 5) + 1) & ~1) * 4 + (size_t)I + 16;
+    return (size_t)((I + 7) & ~7) * 4 + (size_t)I * 2 + (size_t)(I & 1) * 2 + (size_t)((((I + 31) >> 5) + 1) & ~1) * 4 + (size_t)I + 16;
 }
 
 // Small block-wide scalars of the plan (static LDS, declared by the kernel so that waves which do not take
@@ -221,8 +263,7 @@ __device__ __forceinline__ void surplus_ends(P place, Q stays, int base, int n, 
 
 // Replays the bookkeeping of one update in LDS and publishes it (block 0 writes the other bookkeeping
 // buffer, the last block to arrive flips the epoch).  Called by all PT threads of the block (tid = 0..PT-1);
-// contains block barriers.  VEC: I % 8 == 0 and the mask is
-// 8-byte aligned, so masks are read as 8-byte words and indices as 16-byte vectors; both bookkeeping
+// contains block barriers.  VEC (I >= 8): masks are read as 8-byte words and indices as 16-byte vectors; both bookkeeping
 // buffers are requested together with the ticket, so the front costs one memory round trip.  MARK: the
 // dirty bitmap is kept on the fast path too.
 // NW: 8-element words per thread of the vector path (I <= 8 NW threads); the registers of the front loads follow from it.
@@ -238,11 +279,11 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
 {
     constexpr int TPB = PT;
     uint16_t *pos_l = reinterpret_cast<uint16_t *>(smem);  // index -> position
-    uint16_t *idx_l = pos_l + I;                           // position -> index
+    uint16_t *idx_l = pos_l + ((I + 7) & ~7);              // position -> index
     // added indices ascending from the front, removed indices ascending from the
     // back (k-th removed at lists[I-1-k]); the two never meet: na + nr <= I.
     // After the plan the same array holds the positions to rewrite.
-    uint16_t *lists = idx_l + I;
+    uint16_t *lists = idx_l + ((I + 7) & ~7);
     uint32_t *dirty = reinterpret_cast<uint32_t *>(lists + I + (I & 1));  // bit per position
     const int dirty_words = (I + 31) >> 5;
     uint8_t *flag_l = reinterpret_cast<uint8_t *>(dirty + ((dirty_words + 1) & ~1));  // bit0 new, bit1 old; 8-byte aligned
@@ -274,13 +315,13 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
         for (int w = 0; w < NW; ++w) {
             const int e = e0 + 8 * w;
             if (e < e1) {
-                v_new[w] = *reinterpret_cast<const uint64_t *>(new_mask + e);
-                v_cur0[w] = *reinterpret_cast<const uint64_t *>(cur_mask2 + e);
-                v_cur1[w] = *reinterpret_cast<const uint64_t *>(cur_mask2 + (size_t)I + e);
-                v_i0a[w] = *reinterpret_cast<const int4 *>(indices2 + e);
-                v_i0b[w] = *reinterpret_cast<const int4 *>(indices2 + e + 4);
-                v_i1a[w] = *reinterpret_cast<const int4 *>(indices2 + (size_t)I + e);
-                v_i1b[w] = *reinterpret_cast<const int4 *>(indices2 + (size_t)I + e + 4);
+                v_new[w] = load_mask(new_mask, e, I);
+                v_cur0[w] = load_mask(cur_mask2, e, I);
+                v_cur1[w] = load_mask(cur_mask2 + I, e, I);
+                v_i0a[w] = load_list(indices2, e, I);
+                v_i0b[w] = load_list(indices2, e + 4, I);
+                v_i1a[w] = load_list(indices2 + I, e, I);
+                v_i1b[w] = load_list(indices2 + I, e + 4, I);
             }
         }
         n_both[0] = state[ST_STATE_N_BUF0];
@@ -301,9 +342,9 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
             const int e = e0 + 8 * w;
             w_new[w] = w_cur[w] = 0;
             if (e < e1) {
-                w_new[w] = nonzero_bytes(v_new[w]);
-                w_cur[w] = nonzero_bytes(ep ? v_cur1[w] : v_cur0[w]);
-                const int4 a = ep ? v_i1a[w] : v_i0a[w], b4 = ep ? v_i1b[w] : v_i0b[w];
+                w_new[w] = nonzero_bytes(mask_tail(v_new[w], e, I));
+                w_cur[w] = nonzero_bytes(mask_tail(ep ? v_cur1[w] : v_cur0[w], e, I));
+                const int4 a = list_tail(ep ? v_i1a[w] : v_i0a[w], e, I), b4 = list_tail(ep ? v_i1b[w] : v_i0b[w], e + 4, I);
                 uint4 packed;
                 packed.x = (uint32_t)(a.x & 0xffff) | ((uint32_t)a.y << 16);
                 packed.y = (uint32_t)(a.z & 0xffff) | ((uint32_t)a.w << 16);
@@ -469,7 +510,7 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
 #pragma unroll
             for (int w = 0; w < NW; ++w) {
                 const int e = e0 + 8 * w;
-                if (e < e1) *reinterpret_cast<uint64_t *>(mask_out + e) = n_new > 0 ? w_new[w] : w_cur[w];
+                if (e < e1) store_mask(mask_out, e, I, n_new > 0 ? w_new[w] : w_cur[w]);
             }
         } else {
             for (int i = tid; i < I; i += TPB) mask_out[i] = n_new > 0 ? (flag_l[i] & 1) : (flag_l[i] >> 1);
@@ -608,7 +649,7 @@ constexpr size_t update_lds_bytes(int I)
 // the plan is one scan, one pass over the list -- every thread keeps the positions it loaded in registers -- and two
 // barriers when removals do not outnumber additions.  Every block plans for itself (as a launch of its own the plan would
 // cost a kernel boundary) and copies its share of the items.
-// Masks in 8-byte words, lists in 16-byte vectors (I % 8 == 0, aligned buffers); I <= 8 NW TPB.
+// Masks in 8-byte words, lists in 16-byte vectors, at any alignment (I >= 8); I <= 8 NW TPB.
 template <int TPB, int NW, typename Tab>
 __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__restrict__ new_mask,
                                                            uint8_t *__restrict__ cur_mask2,
@@ -648,17 +689,17 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
     uint64_t v_new[NW], v_cur0[NW], v_cur1[NW];
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-        const int e = 8 * (tid * words + w), ec = w < words && e < I ? e : 0;
-        v_new[w] = *reinterpret_cast<const uint64_t *>(new_mask + ec);
-        v_cur0[w] = *reinterpret_cast<const uint64_t *>(cur_mask2 + ec);
-        v_cur1[w] = *reinterpret_cast<const uint64_t *>(cur_mask2 + (size_t)I + ec);
+        const int e = 8 * (tid * words + w);
+        v_new[w] = load_mask(new_mask, e, I);
+        v_cur0[w] = load_mask(cur_mask2, e, I);
+        v_cur1[w] = load_mask(cur_mask2 + I, e, I);
     }
     int4 v_i0[NV], v_i1[NV];
 #pragma unroll
     for (int q = 0; q < NV; ++q) {
         const int p = 4 * (tid + TPB * q), pc = p < idx_cap ? p : 0;   // (idx_cap: a multiple of 8, or I)
-        v_i0[q] = *reinterpret_cast<const int4 *>(indices2 + pc);
-        v_i1[q] = *reinterpret_cast<const int4 *>(indices2 + (size_t)I + pc);
+        v_i0[q] = load_list(indices2, pc, I);
+        v_i1[q] = load_list(indices2 + I, pc, I);
     }
     const int n_buf0 = state[ST_STATE_N_BUF0], n_buf1 = state[ST_STATE_N_BUF1];
     const int serial_old = state[ST_STATE_SERIAL], valid_old = state[ST_STATE_VALID];
@@ -671,9 +712,10 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
     uint32_t cnt = 0;   // added in the low half, removed in the high half
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-        const bool in = w < words && 8 * (tid * words + w) < I;
-        w_new[w] = in ? nonzero_bytes(v_new[w]) : 0ull;
-        w_cur[w] = in ? nonzero_bytes(ep ? v_cur1[w] : v_cur0[w]) : 0ull;
+        const int e = 8 * (tid * words + w);
+        const bool in = w < words && e < I;
+        w_new[w] = in ? nonzero_bytes(mask_tail(v_new[w], e, I)) : 0ull;
+        w_cur[w] = in ? nonzero_bytes(mask_tail(ep ? v_cur1[w] : v_cur0[w], e, I)) : 0ull;
         cnt += (uint32_t)__popcll(w_new[w] & ~w_cur[w]) + ((uint32_t)__popcll(w_cur[w] & ~w_new[w]) << 16);
     }
     ST_TL(1);
@@ -739,7 +781,8 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
             const int p0 = 4 * (tid + TPB * q);
             int4 c = ep ? v_i1[q] : v_i0[q];
             if (n > idx_cap && p0 >= idx_cap && p0 < n)   // more positions in use than the caller expected (one more round trip)
-                c = *reinterpret_cast<const int4 *>(indices2 + (size_t)ep * I + p0);
+                c = load_list(indices2 + (size_t)ep * I, p0, I);
+            c = list_tail(c, p0, I);
             const int e4[4] = {c.x, c.y, c.z, c.w};
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
@@ -805,7 +848,7 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
 #pragma unroll
             for (int w = 0; w < NW; ++w) {
                 const int e = 8 * (tid * words + w);
-                if (w < words && e < I) *reinterpret_cast<uint64_t *>(mask_out + e) = n_new > 0 ? w_new[w] : w_cur[w];
+                if (w < words && e < I) store_mask(mask_out, e, I, n_new > 0 ? w_new[w] : w_cur[w]);
             }
             uint32_t mine = 0;
             if (S_all > 0)
@@ -843,7 +886,7 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
     ST_TL(6);
 }
 
-// The same for masks that cannot be read in 8-byte words: cache_plan above, then the copies.
+// The same for masks of less than one 8-byte word: cache_plan above, then the copies.
 template <int TPB>
 __global__ __launch_bounds__(TPB) void cache_update_bytes_kernel(const uint8_t *__restrict__ new_mask,
                                                                  uint8_t *__restrict__ cur_mask2,
@@ -960,10 +1003,9 @@ __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
         const int e = (tid * nw_rt + w) * 8;
-        const int ec = e + 8 <= I ? e : I - 8;
-        v_new[w] = *reinterpret_cast<const uint64_t *>(new_mask + ec);
-        v_c0[w] = *reinterpret_cast<const uint64_t *>(cur_mask2 + ec);
-        v_c1[w] = *reinterpret_cast<const uint64_t *>(cur_mask2 + (size_t)I + ec);
+        v_new[w] = load_mask(new_mask, e, I);
+        v_c0[w] = load_mask(cur_mask2, e, I);
+        v_c1[w] = load_mask(cur_mask2 + I, e, I);
     }
     // The plan is worked out by ONE wave, the last of the block (with 6 KB rows a wave that owns no columns), while
     // the others already request rows; its lanes own the block's positions.
@@ -983,8 +1025,8 @@ __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
     const bool scan_in = scan_p + kSparseScan <= scan_cap;
     const int scan_pc = scan_in ? scan_p : 0;
     static_assert(kSparseScan == 4, "one 16-byte load per bookkeeping buffer");
-    const int4 sc0 = *reinterpret_cast<const int4 *>(indices2 + scan_pc);
-    const int4 sc1 = *reinterpret_cast<const int4 *>(indices2 + (size_t)I + scan_pc);
+    const int4 sc0 = load_list(indices2, scan_pc, I);
+    const int4 sc1 = load_list(indices2 + I, scan_pc, I);
     uint4 xr[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b)
@@ -1034,8 +1076,8 @@ __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
     for (int w = 0; w < NW; ++w) {
         const int bi = tid * nw_rt + w;            // byte of the bitmaps = elements [8 bi, 8 bi + 8)
         const bool in = w < nw_rt && bi * 8 < I;
-        w_new[w] = in ? nonzero_bytes(v_new[w]) : 0ull;
-        w_cur[w] = in ? nonzero_bytes(ep ? v_c1[w] : v_c0[w]) : 0ull;
+        w_new[w] = in ? nonzero_bytes(mask_tail(v_new[w], bi * 8, I)) : 0ull;
+        w_cur[w] = in ? nonzero_bytes(mask_tail(ep ? v_c1[w] : v_c0[w], bi * 8, I)) : 0ull;
         if (w < nw_rt && bi < W32 * 4) {
             reinterpret_cast<uint8_t *>(sh.newbits)[bi] = (uint8_t)pack_bits8(w_new[w]);
             reinterpret_cast<uint8_t *>(sh.oldbits)[bi] = (uint8_t)pack_bits8(w_cur[w]);
@@ -1449,7 +1491,7 @@ __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
             for (int w = 0; w < NW; ++w) {
                 const int bi = tid * nw_rt + w;
                 if (w < nw_rt && bi * 8 < I && (bi % G) == blk)
-                    *reinterpret_cast<uint64_t *>(mask_out + (size_t)bi * 8) = n > 0 ? w_new[w] : w_cur[w];
+                    store_mask(mask_out, bi * 8, I, n > 0 ? w_new[w] : w_cur[w]);
             }
             if (blk == 0 && arriver) {
                 state[ST_STATE_N_BUF0 + (ep ^ 1)] = n;
@@ -2264,12 +2306,6 @@ static st::UpdateLayer update_layer(const st_cache *c, const uint8_t *mask)
     return y;
 }
 
-// Masks as 8-byte words, index lists as 16-byte vectors?
-static bool update_is_aligned(const st_cache *c, const uint8_t *mask)
-{
-    return c->I % 8 == 0 && (uintptr_t)mask % 8 == 0 && (uintptr_t)c->b.cur_mask % 8 == 0 && (uintptr_t)c->b.indices % 16 == 0;
-}
-
 // The count an update last told the host, 0 if none has yet.  A guess: later updates may be on their way.
 static int seen_count(const st_cache *c) { return *const_cast<const volatile int32_t *>(&c->host->count); }
 
@@ -2281,7 +2317,7 @@ static int update_idx_cap(const st_cache *c)
     return seen > 0 && seen + seen / 4 + 64 < I ? (seen + seen / 4 + 64 + 7) & ~7 : I;
 }
 
-// One update, or those of L > 1 caches of equal shape in one launch (I <= kPlanMaxI; 8-byte masks only).
+// One update, or those of L > 1 caches of equal shape in one launch (I <= kPlanMaxI; L > 1: I >= 8).
 static int launch_update(st_cache *const *caches, const uint8_t *const *masks, int L, hipStream_t s)
 {
     using namespace st;
@@ -2296,10 +2332,10 @@ static int launch_update(st_cache *const *caches, const uint8_t *const *masks, i
         const char *v = getenv("ST_CACHE_TPB");
         return v ? atoi(v) : 0;
     }();
-    const bool aligned = update_is_aligned(c, masks[0]);
+    const bool words_fit = I >= 8;
     // 512-thread blocks (ST_CACHE_TPB=512) leave room on the CU for a kernel of another stream, but
     // measure slower on their own; they cover I <= 12288.
-    const bool small = L == 1 && want_tpb == 512 && aligned && I <= 8 * 512 * 3;
+    const bool small = L == 1 && want_tpb == 512 && words_fit && I <= 8 * 512 * 3;
     const int tpb = small ? 512 : kPlanThreads, words = (I + 8 * tpb - 1) / (8 * tpb);
     const UpdateLayer y = update_layer(c, masks[0]);
     CopyPlan cp;
@@ -2338,7 +2374,7 @@ static int launch_update(st_cache *const *caches, const uint8_t *const *masks, i
         const int grid = blocks ? blocks : device_cu_count() * 3 / 4;   // (measured against 1/4, 3/8, 1/2 and all of the CUs)
         const size_t lds = update_lds_bytes(I);
         const int idx_cap = update_idx_cap(c);
-        rc = !aligned     ? launch(cache_update_bytes_kernel<1024>, grid, plan_lds_bytes(I), cp, c->host)
+        rc = !words_fit   ? launch(cache_update_bytes_kernel<1024>, grid, plan_lds_bytes(I), cp, c->host)
              : small      ? launch(cache_update_kernel<512, 3, NoLayers>, grid, lds, idx_cap, cp, c->host, NoLayers{})
              : words == 1 ? launch(cache_update_kernel<1024, 1, NoLayers>, grid, lds, idx_cap, cp, c->host, NoLayers{})
              : words == 2 ? launch(cache_update_kernel<1024, 2, NoLayers>, grid, lds, idx_cap, cp, c->host, NoLayers{})
@@ -2399,9 +2435,7 @@ extern "C" int st_cache_update_layers(st_cache *const *caches, const uint8_t *co
         while (nl < kMaxLayers && l0 + nl < L && caches[l0 + nl]->I == c->I && caches[l0 + nl]->H == c->H &&
                caches[l0 + nl]->dtype == c->dtype && caches[l0 + nl]->has_gate == c->has_gate)
             ++nl;
-        bool aligned = c->I <= kPlanMaxI;
-        for (int l = 0; l < nl; ++l) aligned = aligned && update_is_aligned(caches[l0 + l], masks[l0 + l]);
-        if (nl == 1 || !aligned) {
+        if (nl == 1 || c->I < 8 || c->I > kPlanMaxI) {
             const int rc = st_cache_update_async(caches[l0], masks[l0], stream);
             if (rc != ST_OK) return rc;
             l0 += 1;
@@ -2440,12 +2474,10 @@ extern "C" int st_cache_update_forward(st_cache *c, const uint8_t *mask, const v
     const int NBF = B == 2 ? 2 : 1;   // rows of x the fused kernel takes in one pass
     const size_t lds = plan_bytes + (size_t)(ngrp - 1) * NBF * H * 4;
     const int G = mlp_grid();
-    const bool aligned = (I % 8 == 0) && ((uintptr_t)mask % 8 == 0) && ((uintptr_t)c->b.cur_mask % 8 == 0) &&
-                         ((uintptr_t)c->b.indices % 16 == 0);
     static const bool fused_off = [] { const char *v = getenv("ST_CACHE_FUSED"); return v && atoi(v) == 0; }();
     // One kernel for one or two rows of x when a block owns at most kSparseMaxQ positions, the masks fit the
     // kernel's bitmaps and a row fits one pass of a thread group; everything else runs as two calls.
-    const bool fused = !fused_off && B <= 2 && aligned && I >= 8 && G <= 0xffff && (I + G - 1) / G <= kSparseMaxQ &&
+    const bool fused = !fused_off && B <= 2 && I >= 8 && G <= 0xffff && (I + G - 1) / G <= kSparseMaxQ &&
                        I <= 32 * kSparseMaxW32 && I <= 8 * TPB * kSparseWords && chunks <= TPB && row_bytes % 16 == 0 &&
                        lds <= (size_t)(148 * 1024);
     if (!fused) {   // two launches: update, then the forward that reads the count on the device

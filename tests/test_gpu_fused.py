@@ -308,3 +308,38 @@ def test_fused_random_count_changes(I, H, dtype, has_gate, frac):
                 yp = plain.forward(x, "silu")
                 torch.cuda.synchronize()
                 assert torch.equal(yf, yp), (seed, t)
+
+
+@pytest.mark.parametrize("I,off", [(8, 1), (9, 0), (15, 3), (255, 0), (257, 5), (2049, 0), (3405, 1), (4098, 2), (8191, 0), (8193, 7),
+                                   (16383, 0), (16384, 1)])
+@pytest.mark.parametrize("B", [1, 3])
+def test_sizes_and_masks_at_any_alignment(I, off, B):
+    """Sizes that are no multiples of eight and masks that start anywhere: the last word of a mask, the last vector of a list, the
+    second halves of the double buffers.  Update alone, the layers of a launch together (one cache each for three shifted masks)
+    and the update + MLP call, against the oracle's order and against one another."""
+    H = 64
+    trace = syn.ragged_mask_trace(I + off, I, 14)
+    fused, plain, (gate, up, down), g = _pair(I, H, "float16", True, 3, torch.from_numpy(trace[0]))
+    third = st.WeightCache(torch.from_numpy(trace[0]).to(DEV), H, gate.to(DEV), up.to(DEV), down.to(DEV), True)
+    order = oracle.OracleWeightCache(trace[0], H, gate.float().numpy(), up.float().numpy(), down.float().numpy(), True)
+    stage = torch.zeros(off + 2 * (I + 1), dtype=torch.bool, device=DEV)
+    for t in range(1, len(trace)):
+        if not trace[t].any():
+            continue
+        views = [stage[off + k * (I + 1):off + k * (I + 1) + I] for k in range(2)]
+        for v in views:
+            v.copy_(torch.from_numpy(trace[t]))
+        x = torch.randn(B, H, generator=g).half().to(DEV)
+        yf = fused.update_and_forward(views[0], x, "silu")
+        st.weight_cache.update_layers_async([plain, third], views)
+        yp = plain.forward(x, "silu")
+        torch.cuda.synchronize()
+        assert torch.equal(yf, yp), t
+        order.update_active_weights(trace[t])
+        _same_state(fused, plain, t)
+        _same_state(plain, third, t)
+        assert plain.get_active_indices().cpu().tolist() == order.get_active_indices().tolist(), t
+        e = int(plain.sync_state()["epoch"])
+        assert torch.equal(plain.cur_mask[e].bool().cpu(), torch.from_numpy(trace[t]).bool()), t
+        idx = plain.get_active_indices()
+        assert torch.equal(plain.up_active[: len(idx)], plain.up_pool[idx]), t
