@@ -168,8 +168,11 @@ int st_predictor_mask_layers(const st_predictor_layer *layers, int64_t L, const 
  *           16-byte aligned; its first 16 bytes must be zero before the first
  *           call and are left zero by every call.  Calls that share a
  *           workspace must not overlap.
+ *   method | ST_MASK_INTO_ZEROS: the mask holds zeros already (st_predictor_mask
+ *           with thr = infinity and cmp_ge = 0 leaves them beside its scores);
+ *           faster for several rows, and no workspace is needed
  * ------------------------------------------------------------------------ */
-enum st_mask_method { ST_MASK_TOPK = 0, ST_MASK_STATISTICAL = 1 };
+enum st_mask_method { ST_MASK_TOPK = 0, ST_MASK_STATISTICAL = 1, ST_MASK_INTO_ZEROS = 0x100 };
 int64_t st_mask_select_workspace_bytes(int64_t B, int64_t I);
 int st_mask_select(const float *scores, int64_t B, int64_t I, int method, int64_t k, float z, uint8_t *mask,
                    float *cutoff, void *workspace, int64_t workspace_bytes, void *stream);

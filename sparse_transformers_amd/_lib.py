@@ -73,6 +73,8 @@ SIGNATURES = {
     "st_profile_collect": (_ci, [_vp, _vp, _ci]),
 }
 
+ST_MASK_INTO_ZEROS = 0x100
+
 KERNEL_KINDS = ["mlp_decode", "mlp_reduce", "cache_update", "mask_select", "pred_down", "pred_up_mask",
                 "mlp_prefill_gateup", "mlp_prefill_down", "mlp_batch_gateup", "mlp_batch_down",
                 "cache_update_decode"]

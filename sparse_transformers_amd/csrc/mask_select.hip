@@ -8,11 +8,11 @@
 //   sketch       approx_topk_threshold, sparse_transformers/csrc/approx_topk.h:10-88
 //
 // One block per row.  The row is read from HBM once; every thread keeps its scores in registers (rows of up
-// to 16384 scores) as order-preserving 32-bit keys.  The k-th largest key is found exactly by a radix select
-// (8-bit digits, most significant first, one LDS histogram per digit; once at most 64 keys share the
-// prefix one wave ranks them directly), so nothing is sorted.  With several rows every block leaves its row mask
-// in the workspace and the block that finishes last ORs them together; which block that is does not
-// change the result.
+// to 16384 scores) as order-preserving 32-bit keys.  The k-th largest key is found exactly, with nothing sorted: by one
+// histogram of the values and a ranking of the interval that holds it, or by a radix select (8-bit digits, most significant
+// first, one LDS histogram per digit; once at most 64 keys share the prefix one wave ranks them directly).  With several
+// rows every block leaves its row mask in the workspace and the block that finishes last ORs them together; which block that
+// is does not change the result.  A caller with a mask of zeros has the blocks set their rows' bytes in it instead.
 #include "st_common.h"
 
 namespace st {
@@ -40,8 +40,10 @@ struct SelShared {
     uint32_t hsum[256];
     uint32_t cand[kWave];
     uint32_t digit, rem, cnt, ncand;
+    __align__(16) uint32_t wave_hi[kSelWaves];
+    __align__(16) uint32_t wave_lo[kSelWaves];
     int wave_tot[kSelWaves];
-    double wave_sum[kSelWaves];
+    double wave_sum[2][kSelWaves];
     int last;
 };
 
@@ -130,17 +132,163 @@ __device__ __forceinline__ uint32_t radix_select_desc(Sweep sweep, uint32_t k, S
     return prefix;
 }
 
+template <int CTRL> __device__ __forceinline__ uint32_t dpp_u32(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
+}
+// largest value over the wave, the same in every lane
+__device__ __forceinline__ uint32_t wave_max(uint32_t v)
+{
+    v = max(v, dpp_u32<0xB1>(v));    // quad_perm [1,0,3,2]
+    v = max(v, dpp_u32<0x4E>(v));    // quad_perm [2,3,0,1]
+    v = max(v, dpp_u32<0x141>(v));   // row_half_mirror
+    v = max(v, dpp_u32<0x140>(v));   // row_mirror
+    auto row = [&](int l) __attribute__((always_inline)) { return (uint32_t)__builtin_amdgcn_readlane((int)v, l); };
+    return max(max(row(0), row(16)), max(row(32), row(48)));
+}
+// sum over the lanes below and this one (DPP row shifts, the row totals through scalar registers)
+__device__ __forceinline__ int wave_incl_sum(int v, int lane)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1, zeros from outside the row
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    const int t0 = __builtin_amdgcn_readlane(v, 15), t1 = __builtin_amdgcn_readlane(v, 31), t2 = __builtin_amdgcn_readlane(v, 47);
+    const int row = lane >> 4;
+    return v + (row >= 1 ? t0 : 0) + (row >= 2 ? t1 : 0) + (row >= 3 ? t2 : 0);
+}
+
+// The same key for a row of finite scores that every thread holds KPT of (index tid + 1024 u < I), by VALUE: 2048 equal
+// intervals between the row's smallest and largest score put a few scores into each (the top digit of the keys, sign and
+// exponent, takes a handful of values only), one histogram finds the interval that holds the k-th largest, and every wave
+// ranks what lies in it.  The map to intervals is monotone in the score, rounding included, so greater intervals hold
+// greater scores.  Five barriers, where two digits and a ranking take eleven.  False (uniform): no interval of at most 64
+// scores, or a range that the map does not take (infinities, NaN, all scores equal): radix_select_desc does those.
+// Predictor and selection, one row, replayed, by the digits / so: 30 % of 8192 (rank 128) 11.6 / 10.9 us, of 14336 (rank 256)
+// 15.9 / 15.0.
+template <int KPT>
+__device__ __forceinline__ bool value_select_desc(const float (&v)[KPT], int I, uint32_t k, SelShared &sh, int tid,
+                                                  uint32_t &kth_out, uint32_t &rem_out, uint32_t &cnt_out)
+{
+    constexpr int kBins = 256 * kHistCopies;
+    static_assert(kBins == 2 * kSelThreads, "two intervals per thread");
+    const int lane = tid & (kWave - 1), wave = tid >> 6;
+    sh.hist[tid] = 0u;
+    sh.hist[tid + kSelThreads] = 0u;
+    if (tid == 0) sh.ncand = 0u;
+    uint32_t hi = 0u, nlo = 0u;   // largest key, complement of the smallest
+#pragma unroll
+    for (int u = 0; u < KPT; ++u)
+        if (tid + u * kSelThreads < I) {
+            const uint32_t kv = order_key(v[u]);
+            hi = max(hi, kv);
+            nlo = max(nlo, ~kv);
+        }
+    hi = wave_max(hi);
+    nlo = wave_max(nlo);
+    if (lane == 0) { sh.wave_hi[wave] = hi; sh.wave_lo[wave] = nlo; }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kSelWaves; w += 4) {
+        const uint4 a = *reinterpret_cast<const uint4 *>(&sh.wave_hi[w]), c = *reinterpret_cast<const uint4 *>(&sh.wave_lo[w]);
+        hi = max(hi, max(max(a.x, a.y), max(a.z, a.w)));
+        nlo = max(nlo, max(max(c.x, c.y), max(c.z, c.w)));
+    }
+    hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)hi);
+    const uint32_t lo = ~(uint32_t)__builtin_amdgcn_readfirstlane((int)nlo);
+    const float flo = key_value(lo), range = key_value(hi) - flo;
+    if (hi > order_key(3.402823466e38f) || lo < order_key(-3.402823466e38f) || !(range >= 1e-30f && range <= 1e38f)) return false;
+    const float scale = (float)(kBins - 1) / range;
+    auto interval = [&](float f) __attribute__((always_inline)) {
+        const int b = (int)((f - flo) * scale);
+        return b < kBins ? b : kBins - 1;
+    };
+    int at[KPT];
+#pragma unroll
+    for (int u = 0; u < KPT; ++u) {
+        at[u] = interval(v[u]);
+        if (tid + u * kSelThreads < I) atomicAdd(&sh.hist[at[u]], 1u);
+    }
+    __syncthreads();
+    const uint2 c2 = *reinterpret_cast<const uint2 *>(&sh.hist[2 * tid]);
+    const int incl = wave_incl_sum((int)(c2.x + c2.y), lane);
+    if (lane == kWave - 1) sh.wave_tot[wave] = incl;
+    __syncthreads();
+    int upto = incl;   // scores in this thread's intervals and the lower ones
+#pragma unroll
+    for (int w = 0; w < kSelWaves; ++w) upto += w < wave ? sh.wave_tot[w] : 0;
+    uint32_t above = (uint32_t)(I - upto);
+#pragma unroll
+    for (int j = 1; j >= 0; --j) {
+        const uint32_t c = j ? c2.y : c2.x;
+        if (above < k && k <= above + c) { sh.digit = (uint32_t)(2 * tid + j); sh.rem = k - above; sh.cnt = c; }
+        above += c;
+    }
+    __syncthreads();
+    const int bin = (int)sh.digit;
+    const uint32_t rem = sh.rem, cnt = (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.cnt);
+    if (cnt > (uint32_t)kWave) return false;
+#pragma unroll
+    for (int u = 0; u < KPT; ++u)
+        if (tid + u * kSelThreads < I && at[u] == bin) sh.cand[atomicAdd(&sh.ncand, 1u)] = order_key(v[u]);
+    __syncthreads();
+    const uint32_t mine = (uint32_t)lane < cnt ? sh.cand[lane] : 0u;
+    uint32_t greater = 0u, equal = 0u;
+    for (uint32_t j = 0; j < cnt; ++j) {
+        const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)j);
+        greater += c > mine;
+        equal += c == mine;
+    }
+    const uint64_t is = __builtin_amdgcn_ballot_w64((uint32_t)lane < cnt && greater < rem && rem <= greater + equal);
+    const int l = __builtin_ctzll(is);   // (lanes that agree hold the same)
+    kth_out = (uint32_t)__builtin_amdgcn_readlane((int)mine, l);
+    rem_out = rem - (uint32_t)__builtin_amdgcn_readlane((int)greater, l);
+    cnt_out = (uint32_t)__builtin_amdgcn_readlane((int)equal, l);
+    return true;
+}
+
+template <int CTRL> __device__ __forceinline__ double dpp_add_f64(double v)
+{
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint64_t o = (uint64_t)dpp_u32<CTRL>((uint32_t)b) | (uint64_t)dpp_u32<CTRL>((uint32_t)(b >> 32)) << 32;
+    return v + __builtin_bit_cast(double, o);
+}
+__device__ __forceinline__ double wave_sum_f64(double v)
+{
+    v = dpp_add_f64<0xB1>(v);
+    v = dpp_add_f64<0x4E>(v);
+    v = dpp_add_f64<0x141>(v);
+    v = dpp_add_f64<0x140>(v);
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    auto row = [&](int l) __attribute__((always_inline)) {
+        const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, l), h = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), l);
+        return __builtin_bit_cast(double, lo | h << 32);
+    };
+    return (row(0) + row(16)) + (row(32) + row(48));
+}
+
 __device__ __forceinline__ double block_sum(double v, SelShared &sh, int tid)
 {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+    v = wave_sum_f64(v);
     __syncthreads();  // the previous reader of wave_sum is done
-    if ((tid & (kWave - 1)) == 0) sh.wave_sum[tid >> 6] = v;
+    if ((tid & (kWave - 1)) == 0) sh.wave_sum[0][tid >> 6] = v;
     __syncthreads();
     double s = 0.0;
 #pragma unroll
-    for (int w = 0; w < kSelWaves; ++w) s += sh.wave_sum[w];
+    for (int w = 0; w < kSelWaves; ++w) s += sh.wave_sum[0][w];
     return s;
+}
+
+// Both sums over the block, in every thread (once per kernel).
+__device__ __forceinline__ void block_sums(double &s, double &q, SelShared &sh, int tid)
+{
+    s = wave_sum_f64(s);
+    q = wave_sum_f64(q);
+    if ((tid & (kWave - 1)) == 0) { sh.wave_sum[0][tid >> 6] = s; sh.wave_sum[1][tid >> 6] = q; }
+    __syncthreads();
+    s = q = 0.0;
+#pragma unroll
+    for (int w = 0; w < kSelWaves; ++w) { s += sh.wave_sum[0][w]; q += sh.wave_sum[1][w]; }
 }
 
 // Exclusive prefix of one int per thread, threads in order.
@@ -164,6 +312,9 @@ __device__ __forceinline__ int block_excl_count(int v, SelShared &sh, int tid)
 // tid + u * 1024) in registers for all passes; a copy of the keys in LDS serves the one step that walks the
 // row in index order.  KPT == 0: rows of any length, every pass reads the keys from LDS (`in_lds`) or the
 // scores again from memory.
+// `into`: the mask holds zeros and the rows' blocks only set what they select, so that nothing is left to unite.  Predictor and
+// selection, replayed, the blocks' row masks united by the last one / so (and by value): top-k, four rows of 8192 15.4 / 12.8 us,
+// sixteen of 14336 24.5 / 19.7; statistical 12.7 / 10.6 and 20.2 / 16.2.
 template <int KPT>
 __global__ __launch_bounds__(kSelThreads) void mask_select_kernel(const float *__restrict__ scores,
                                                                   uint8_t *__restrict__ mask,
@@ -174,13 +325,18 @@ __global__ __launch_bounds__(kSelThreads) void mask_select_kernel(const float *_
 {
     // (pointers and sizes first: the first 14 dwords of the arguments are in scalar registers when the wave starts)
     const int method = method_word & 0xff, in_lds = (method_word >> 8) & 1;
+    const bool into = ((method_word >> 9) & 1) != 0;
     constexpr int NR = KPT > 0 ? KPT : 1;
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ SelShared sh;
     uint32_t *keys = reinterpret_cast<uint32_t *>(smem);
     const int tid = threadIdx.x, b = blockIdx.x;
     const float *row = scores + (size_t)b * I;
-    uint8_t *dst = B == 1 ? mask : rowmask + (size_t)b * ldm;
+    uint8_t *dst = B == 1 || into ? mask : rowmask + (size_t)b * ldm;
+    auto put = [&](int i, bool on) __attribute__((always_inline)) {
+        if (!into) dst[i] = on ? 1 : 0;
+        else if (on) dst[i] = 1;
+    };
 
     float v[NR];
     if constexpr (KPT > 0) {  // all loads of the row are in flight together
@@ -205,22 +361,29 @@ __global__ __launch_bounds__(kSelThreads) void mask_select_kernel(const float *_
     if (method == ST_MASK_TOPK) {
         const uint32_t k = k_in < 0 ? 0u : (k_in > I ? (uint32_t)I : (uint32_t)k_in);
         if (k == 0u || k == (uint32_t)I) {  // nothing / everything (uniform over the block)
-            each([&](int i, float) { dst[i] = k ? 1 : 0; });
+            each([&](int i, float) { put(i, k != 0u); });
         } else {
-            if (KPT > 0 || in_lds) {
-                if constexpr (KPT > 0) each([&](int i, float f) { keys[i] = order_key(f); });
-                else for (int i = tid; i < I; i += kSelThreads) keys[i] = order_key(row[i]);
-            }
+            if (KPT == 0 && in_lds)
+                for (int i = tid; i < I; i += kSelThreads) keys[i] = order_key(row[i]);
             auto sweep = [&](auto &&fn) __attribute__((always_inline)) {
                 each([&](int, float f) { fn(order_key(f)); });
             };
-            uint32_t rem, cnt;
-            const uint32_t kth = radix_select_desc(sweep, k, sh, tid, rem, cnt);
+            uint32_t rem = 0u, cnt = 0u, kth = 0u;
+            bool found = false;
+            if constexpr (KPT > 0) {
+                found = value_select_desc<KPT>(v, I, k, sh, tid, kth, rem, cnt);
+                if (!found) __syncthreads();   // (its readers of the shared words are done)
+            }
+            if (!found) kth = radix_select_desc(sweep, k, sh, tid, rem, cnt);
             if (cutoff && tid == 0) cutoff[b] = key_value(kth);
             if (rem == cnt) {  // every score equal to the k-th belongs to the k largest
-                each([&](int i, float f) { dst[i] = order_key(f) >= kth ? 1 : 0; });
+                each([&](int i, float f) { put(i, order_key(f) >= kth); });
             } else {
                 // only the first `rem` of the equal scores, by index: threads take contiguous index ranges
+                if constexpr (KPT > 0) {
+                    each([&](int i, float f) { keys[i] = order_key(f); });
+                    __syncthreads();
+                }
                 auto key = [&](int i) { return (KPT > 0 || in_lds) ? keys[i] : order_key(row[i]); };
                 const int per = (I + kSelThreads - 1) / kSelThreads;
                 const int i0 = tid * per < I ? tid * per : I, i1 = i0 + per < I ? i0 + per : I;
@@ -231,22 +394,25 @@ __global__ __launch_bounds__(kSelThreads) void mask_select_kernel(const float *_
                     const uint32_t kv = key(i);
                     bool on = kv > kth;
                     if (kv == kth) { on = (uint32_t)seen < rem; ++seen; }
-                    dst[i] = on ? 1 : 0;
+                    put(i, on);
                 }
             }
         }
     } else {
-        double s = 0.0;
-        each([&](int, float f) { s += (double)f; });
-        const double mean = block_sum(s, sh, tid) / (double)I;
-        double q = 0.0;
-        each([&](int, float f) { const double d = (double)f - mean; q += d * d; });
-        const double var = block_sum(q, sh, tid) / (double)I;
+        // sums of the scores' distances from the row's first one, and of their squares, in one sweep: the variance's
+        // cancellation is at most that distance's square against it, a factor of I, of doubles
+        const double first = (double)row[0];
+        double s = 0.0, q = 0.0;
+        each([&](int, float f) { const double d = (double)f - first; s += d; q += d * d; });
+        block_sums(s, q, sh, tid);
+        const double off = s / (double)I, mean = first + off;
+        double var = q / (double)I - off * off;
+        var = var < 0.0 ? 0.0 : var;
         const float cut = (float)mean + (float)sqrt(var) * z;
         if (cutoff && tid == 0) cutoff[b] = cut;
-        each([&](int i, float f) { dst[i] = f > cut ? 1 : 0; });
+        each([&](int i, float f) { put(i, f > cut); });
     }
-    if (B == 1) return;
+    if (B == 1 || into) return;
 
     // ---- union over rows by the block that finishes last
     for (int i = I + tid; i < ldm; i += kSelThreads) dst[i] = 0;  // padding of the row
@@ -431,13 +597,15 @@ extern "C" int st_mask_select(const float *scores, int64_t B, int64_t I, int met
 {
     using namespace st;
     ST_REQUIRE(scores && mask, "st_mask_select: null pointer");
+    const int into = method >= 0 && (method & ST_MASK_INTO_ZEROS) ? 1 : 0;
+    method &= ~ST_MASK_INTO_ZEROS;
     ST_REQUIRE(method == ST_MASK_TOPK || method == ST_MASK_STATISTICAL, "st_mask_select: unknown method %d", method);
     ST_REQUIRE(B >= 1 && B <= 4096, "st_mask_select: B=%lld out of range [1,4096]", (long long)B);
     ST_REQUIRE(I >= 1 && I <= (1 << 24), "st_mask_select: I=%lld out of range", (long long)I);
     const int ldm = (int)((I + 15) / 16 * 16);
     unsigned int *ticket = nullptr;
     uint8_t *rowmask = nullptr;
-    if (B > 1) {
+    if (B > 1 && !into) {
         ST_REQUIRE(workspace && workspace_bytes >= st_mask_select_workspace_bytes(B, I),
                    "st_mask_select: workspace of %lld bytes needed for B=%lld, I=%lld",
                    (long long)st_mask_select_workspace_bytes(B, I), (long long)B, (long long)I);
@@ -452,7 +620,7 @@ extern "C" int st_mask_select(const float *scores, int64_t B, int64_t I, int met
     }
     ProfScope ps(ST_K_MASK_SELECT, s);
     const dim3 grid((unsigned)B), block(kSelThreads);
-#define ST_SELECT_ARGS(in_lds) scores, mask, rowmask, cutoff, ticket, (int)B, (int)I, ldm, method | ((in_lds) << 8), (long)k, z
+#define ST_SELECT_ARGS(in_lds) scores, mask, rowmask, cutoff, ticket, (int)B, (int)I, ldm, method | ((in_lds) << 8) | (into << 9), (long)k, z
     if (I <= 8 * kSelThreads)
         ST_LAUNCH(ps, (mask_select_kernel<8>), grid, block, (size_t)I * 4, s, ST_SELECT_ARGS(1));
     else if (I <= 16 * kSelThreads)

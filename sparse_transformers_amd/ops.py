@@ -374,14 +374,17 @@ def select_workspace(device: torch.device, B: int, I: int) -> Optional[torch.Ten
 
 def mask_select(scores: torch.Tensor, method: str, k: int = 0, std_multiplier: float = 0.0,
                 out: Optional[torch.Tensor] = None, return_cutoff: bool = False,
-                workspace: Optional[torch.Tensor] = None):
+                workspace: Optional[torch.Tensor] = None, into_zeros: bool = False):
     """Union over rows of the per-row selection on fp32 ``scores`` [B, I].
 
     ``topk``: the k largest scores of every row (src/modeling_skip.py:208-211; equal scores are taken in
     index order).  ``statistical_topk``: score > mean + std * std_multiplier with the population standard
     deviation (src/modeling_skip.py:197-202).  Returns bool[I] (and the per-row cutoffs [B] on request).
+    ``into_zeros``: ``out`` is all False already, which spares several rows their workspace and the union of their masks.
     """
     dev = require_gpu(scores, out)
+    if into_zeros and out is None:
+        raise ValueError("into_zeros needs out")
     if method not in MASK_METHODS:
         raise ValueError(f"unknown sparsity method {method!r}")
     if scores.dim() != 2 or scores.dtype != torch.float32:
@@ -393,12 +396,12 @@ def mask_select(scores: torch.Tensor, method: str, k: int = 0, std_multiplier: f
         raise ValueError("out must be a contiguous bool[I] tensor")
     cutoff = torch.empty(B, dtype=torch.float32, device=dev) if return_cutoff else None
     ws = None
-    if B > 1:
+    if B > 1 and not into_zeros:
         ws = workspace if workspace is not None else _select_workspace(dev, B, I)
         if ws.dtype != torch.uint8 or not ws.is_cuda:
             raise ValueError("workspace must be a uint8 GPU tensor (see select_workspace)")
     rc = _lib.lib().st_mask_select(
-        scores.data_ptr(), B, I, MASK_METHODS[method], int(k), float(std_multiplier), mask.data_ptr(),
+        scores.data_ptr(), B, I, MASK_METHODS[method] | (_lib.ST_MASK_INTO_ZEROS if into_zeros else 0), int(k), float(std_multiplier), mask.data_ptr(),
         cutoff.data_ptr() if cutoff is not None else None, ws.data_ptr() if ws is not None else None,
         ws.numel() if ws is not None else 0, current_stream_ptr(dev))
     _lib.check(rc, "st_mask_select")

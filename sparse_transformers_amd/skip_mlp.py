@@ -16,7 +16,7 @@ from typing import List, Optional, Sequence
 import torch
 
 from .ops import (mask_select, mlp_workspace_bytes, predictor_mask, predictor_mask_layers, predictor_scores,
-                  select_workspace, sparse_mlp_forward)
+                  sparse_mlp_forward)
 from .weight_cache import WeightCache, update_layers_async
 
 
@@ -65,8 +65,7 @@ class FastLoRAProjection:
         ``naive`` (score >= 0) and ``threshold`` (score >= thr, or > thr) are fused into the predictor
         kernel.  ``topk`` and ``statistical_topk`` need a statistic of the whole row: the predictor kernel
         leaves its fp32 scores and a selection kernel (one block per row) finishes.  ``scores_ws`` (float32,
-        B*I elements) and, for several rows, ``select_ws`` (``ops.select_workspace``) make the call
-        allocation-free.
+        B*I elements) and ``out`` make the call allocation-free.
         """
         if method == "naive":
             return predictor_mask(x, self.down_weight, self.up_weight, 0.0, True, out=out, t_ws=t_ws,
@@ -76,12 +75,12 @@ class FastLoRAProjection:
                                   round_to_storage=self.round_to_storage)
         if method not in ("topk", "statistical_topk"):
             raise ValueError(f"unknown sparsity method {method!r}")
-        if scores_ws is None:
-            scores = self.forward(x)
-        else:   # caller-owned buffers: nothing is allocated (what a captured decode loop needs)
-            scores = predictor_mask(x, self.down_weight, self.up_weight, 0.0, True, out=out, t_ws=t_ws,
-                                    scores_out=scores_ws, round_to_storage=self.round_to_storage)[1]
-        return mask_select(scores, method, k=k, std_multiplier=std_multiplier, out=out, workspace=select_ws)
+        if type(self).forward is not FastLoRAProjection.forward:   # scores of a subclass's own
+            return mask_select(self.forward(x), method, k=k, std_multiplier=std_multiplier, out=out, workspace=select_ws)
+        # no score is above infinity: the mask comes back as the zeros that the selection then sets its bytes in
+        mask, scores = predictor_mask(x, self.down_weight, self.up_weight, float("inf"), False, return_scores=True, out=out,
+                                      t_ws=t_ws, scores_out=scores_ws, round_to_storage=self.round_to_storage)
+        return mask_select(scores, method, k=k, std_multiplier=std_multiplier, out=mask, into_zeros=True)
 
 
 def load_predictors(directory: str, num_layers: int, lora_pct: float, device=None, dtype=None) -> List["FastLoRAProjection"]:
@@ -236,7 +235,6 @@ class SparseDecodeLayer:
         self.method, self.k, self.std_multiplier = method, k, std_multiplier
         self.mask = torch.zeros(cache.intermediate_size, dtype=torch.bool, device=cache.device)
         self._scores_ws: Optional[torch.Tensor] = None
-        self._select_ws: Optional[torch.Tensor] = None
 
     @classmethod
     def from_sparsity(cls, predictor: FastLoRAProjection, cache: WeightCache, sparsity: float,
@@ -259,10 +257,9 @@ class SparseDecodeLayer:
             B, I = x_pred.reshape(-1, x_pred.shape[-1]).size(0), self.cache.intermediate_size
             if self._scores_ws is None or self._scores_ws.numel() < B * I:
                 self._scores_ws = torch.empty(B * I, dtype=torch.float32, device=self.cache.device)
-                self._select_ws = select_workspace(self.cache.device, B, I)
         return self.predictor.mask(x_pred, self.method, self.thr, self.ge, k=self.k,
                                    std_multiplier=self.std_multiplier, out=self.mask, t_ws=t_ws,
-                                   scores_ws=self._scores_ws, select_ws=self._select_ws)
+                                   scores_ws=self._scores_ws)
 
     def compute_mask_and_update(self, x_pred: torch.Tensor, mask_override: Optional[torch.Tensor] = None,
                                 t_ws: Optional[torch.Tensor] = None) -> None:

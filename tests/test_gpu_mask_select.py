@@ -90,6 +90,49 @@ def test_statistical_against_oracle(B, I, kind, z):
     assert not ((got != m) & ~near).any()
 
 
+@pytest.mark.parametrize("B,I,kind", [
+    (1, 1, "normal"), (2, 63, "normal"), (3, 1024, "normal"), (1, 1025, "wide"), (4, 8191, "normal"), (2, 8193, "normal"),
+    (1, 16384, "normal"), (3, 16384, "coarse"), (2, 40000, "normal"), (2, 5000, "outlier"), (2, 5000, "infinite"),
+    (2, 5000, "nan"), (2, 3000, "lowest"), (4, 4096, "constant"), (2, 4096, "steps"),
+])
+def test_selection_by_value_and_into_zeros(B, I, kind):
+    """The selection by intervals of the value where it applies and where it hands over to the digits (an interval with more than 64
+    scores, one score far out, infinities, NaN, the lowest of the type, all scores equal), at the edges of the row lengths;
+    into a mask of zeros like into any other.  Top-k bit for bit; NaN ranks as its bits do, above infinity."""
+    s = _scores(B * 7 + I, B, I, kind)
+    if kind == "outlier":
+        s[:, 17] = 3e37
+    elif kind == "infinite":
+        s[:, 5], s[:, 6] = np.inf, -np.inf
+    elif kind == "nan":
+        s[0, 9] = np.nan
+    elif kind == "lowest":
+        s[:, ::3] = np.finfo(np.float32).min
+    elif kind == "steps":
+        s = (np.arange(I, dtype=np.float32) // 65)[None].repeat(B, 0) * np.float32(0.5)
+    sd = torch.from_numpy(s).to(DEV)
+    t = np.where(np.isnan(s), np.float32(np.inf), s) if kind == "nan" else s
+    for k in sorted({1, max(1, I // 3), max(1, I - 1)}):
+        want = oracle.mask_topk(t, k)
+        for into in (False, True):
+            mask = torch.zeros(I, dtype=torch.bool, device=DEV) if into else torch.ones(I, dtype=torch.bool, device=DEV)
+            st.mask_select(sd, "topk", k=k, out=mask, into_zeros=into)
+            assert np.array_equal(mask.cpu().numpy(), want), (k, into)
+    for z in (0.4, -0.2):
+        a = st.mask_select(sd, "statistical_topk", std_multiplier=z)
+        b = st.mask_select(sd, "statistical_topk", std_multiplier=z, out=torch.zeros_like(a), into_zeros=True)
+        assert torch.equal(a, b)
+        if kind in ("infinite", "nan"):
+            assert not bool(a.any()) or kind == "nan"       # a mean or deviation that is no number selects nothing in its row
+        elif kind in ("normal", "outlier"):
+            d = s.astype(np.float64)
+            cut = (d.mean(1) + d.std(1) * z)[:, None]
+            sure = (np.abs(d - cut) > 1e-6 * np.abs(s).max(1, keepdims=True)).all(0)
+            assert np.array_equal(a.cpu().numpy()[sure], (d > cut).any(0)[sure])
+    with pytest.raises(ValueError):
+        st.mask_select(sd, "topk", k=1, into_zeros=True)
+
+
 def test_mask_select_errors():
     s = torch.zeros(2, 64, device=DEV)
     with pytest.raises(ValueError):
