@@ -19,7 +19,7 @@
 //             has to be transposed: blocks own (column group, row split), each
 //             wave stages 32 rows x 64 columns in LDS and reads the fragment
 //             with the transposing LDS load (fp32 needs neither).  Split-K partial rows are summed in a fixed order
-//             by kernel 3 (mlp_reduce_kernel).
+//             by kernel 3.
 // Unlike a per-CU fused kernel this writes no per-CU partial [B,H] rows (which
 // would cost B * 3 MB of extra traffic); h (B * n elements) is the only
 // intermediate.
@@ -848,6 +848,88 @@ __global__ __launch_bounds__(kBtThreads) void batch_down_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// kernel 3, and the GEMM kernels' third: the splits' partial rows, in their order (more than sixteen: first the z-th and the
+// (z + U)-th).  A round trip and little else: a thread takes four neighbouring results and has all splits' loads of them in flight
+// (U: how many, 16 at most at once).  Before, the batch kernels' went through mlp_reduce_kernel, whose blocks deal 256 partial
+// rows to sixteen groups of threads, and the GEMM kernels' through a loop that waited for each split.
+// Whole forward, us, before / now: batch kernels, 8 rows, H 4096, 3584 active 26.6 / 25.5; 16 rows, H 3072, 5900 33.3 / 32.4; 30
+// rows, H 4096, 2500 31.1 / 28.9; fp32, 8 rows, H 2048, 2500 24.6 / 23.0; GEMM kernels, 77 rows, H 2560, twelve splits 34.0 / 32.7,
+// 39 x 1920, sixteen 22.0 / 21.0.  Fewer than 16384 results are too few threads for that (4 rows, H 3072 24.9 / 25.1; 3 rows,
+// H 1152 11.7 / 11.9): the batch kernels keep the dealt form there.
+// ---------------------------------------------------------------------------
+template <typename T, int U>
+__global__ __launch_bounds__(256) void split_reduce_kernel(const float *__restrict__ partials, int splits, size_t stride,
+                                                           size_t total, int threads, T *__restrict__ out)
+{
+    const size_t i4 = ((size_t)blockIdx.x * threads + threadIdx.x) * 4;
+    if (i4 >= total) return;
+    const float *const p = partials + i4;
+    float4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = *reinterpret_cast<const float4 *>(p + (size_t)(u < splits ? u : splits - 1) * stride);
+    if (splits > U) {
+        float4 w[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) w[u] = *reinterpret_cast<const float4 *>(p + (size_t)(U + u < splits ? U + u : splits - 1) * stride);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool in = U + u < splits;
+            v[u].x = in ? v[u].x + w[u].x : v[u].x; v[u].y = in ? v[u].y + w[u].y : v[u].y;
+            v[u].z = in ? v[u].z + w[u].z : v[u].z; v[u].w = in ? v[u].w + w[u].w : v[u].w;
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float4 s = v[0];
+#pragma unroll
+    for (int u = 1; u < U; ++u) {   // (selects: with branches the last loads go out behind the first sums)
+        const bool in = u < splits;
+        s.x = in ? s.x + v[u].x : s.x; s.y = in ? s.y + v[u].y : s.y;
+        s.z = in ? s.z + v[u].z : s.z; s.w = in ? s.w + v[u].w : s.w;
+    }
+    T *const o = out + i4;
+    if constexpr (sizeof(T) == 2) {
+        if ((reinterpret_cast<uintptr_t>(out) & 7) == 0) {
+            const uint32_t lo = (uint32_t)from_float<T>(s.x).bits | ((uint32_t)from_float<T>(s.y).bits << 16);
+            const uint32_t hi = (uint32_t)from_float<T>(s.z).bits | ((uint32_t)from_float<T>(s.w).bits << 16);
+            *reinterpret_cast<uint2 *>(o) = make_uint2(lo, hi);
+            return;
+        }
+    }
+    o[0] = from_float<T>(s.x); o[1] = from_float<T>(s.y); o[2] = from_float<T>(s.z); o[3] = from_float<T>(s.w);
+}
+
+template <typename T>
+static int split_reduce_t(const float *partials, int splits, size_t stride, size_t total, void *out, hipStream_t stream)
+{
+    ProfScope ps(ST_K_MLP_REDUCE, stream);
+    const size_t quads = total / 4;
+    const int threads = quads >= (size_t)256 * device_cu_count() || splits <= 4 ? 256 : 64;   // (no CU without a block)
+    auto go = [&](auto kern) {
+        ST_LAUNCH(ps, kern, dim3((unsigned)((quads + threads - 1) / threads)), dim3(threads), 0, stream, partials, splits, stride,
+                  total, threads, static_cast<T *>(out));
+    };
+    const int u = splits <= 16 ? splits : (splits + 1) / 2;   // (32 splits at most; a load too many reads the last split again)
+    if (u <= 2) go(split_reduce_kernel<T, 2>);
+    else if (u <= 3) go(split_reduce_kernel<T, 3>);
+    else if (u <= 4) go(split_reduce_kernel<T, 4>);
+    else if (u <= 5) go(split_reduce_kernel<T, 5>);
+    else if (u <= 6) go(split_reduce_kernel<T, 6>);
+    else if (u <= 8) go(split_reduce_kernel<T, 8>);
+    else if (u <= 10) go(split_reduce_kernel<T, 10>);
+    else if (u <= 12) go(split_reduce_kernel<T, 12>);
+    else go(split_reduce_kernel<T, 16>);
+    ST_HIP(hipGetLastError());
+    return ST_OK;
+}
+
+int launch_split_reduce(int dtype, const float *partials, int splits, size_t stride, size_t total, void *out, hipStream_t stream)
+{
+    return dtype == ST_F32   ? split_reduce_t<float>(partials, splits, stride, total, out, stream)
+           : dtype == ST_F16 ? split_reduce_t<f16_t>(partials, splits, stride, total, out, stream)
+                             : split_reduce_t<bf16_t>(partials, splits, stride, total, out, stream);
+}
+
+// ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
 struct BatchShape { int ksw, np, cg, rs; bool special; };
@@ -987,6 +1069,13 @@ static int launch_any_pass(const T *x, int B, int H, const T *gate, const T *up,
     }
 }
 
+// Kernel 3 for rows [rs][ldb][H].
+static int launch_batch_reduce(int dtype, const float *partial, int rs, int ldb, int B, int H, void *out, hipStream_t stream)
+{
+    if ((size_t)B * H < 16384) return launch_mlp_reduce(dtype, partial, rs, ldb, B, H, out, stream);
+    return launch_split_reduce(dtype, partial, rs, (size_t)ldb * H, (size_t)B * H, out, stream);
+}
+
 // One pass over the weights per 32 rows of x; HT: the type h is held in.
 template <typename T, typename HT>
 static int launch_batch_any(const void *x_, int B, int H, const void *gate_, const void *up_, const void *down_, int n,
@@ -1008,7 +1097,7 @@ static int launch_batch_any(const void *x_, int B, int H, const void *gate_, con
                               : launch_any_pass<T, HT, 1>(x, bc, H, gate, up, down, n, n_dev, hbuf, ldh, partial, comb, ldc, act,
                                                           has_gate, &rs, stream);
         if (rc != ST_OK) return rc;
-        rc = launch_mlp_reduce(dtype, partial, rs, bc, bc, H, static_cast<T *>(out_) + (size_t)b0 * H, stream);
+        rc = launch_batch_reduce(dtype, partial, rs, bc, bc, H, static_cast<T *>(out_) + (size_t)b0 * H, stream);
         if (rc != ST_OK) return rc;
     }
     return ST_OK;
@@ -1052,7 +1141,7 @@ static int launch_batch_t(const void *x_, int B, int H, const void *gate_, const
         ST_HIP(hipGetLastError());
         // kernel 2 takes both tiles of x in one pass with two 64-column pieces per block (three would not leave
         // registers for a second set of accumulators); kernel 3 sums the row splits' partial rows
-        // [rs][16 or 32][H] in a fixed order (the streaming kernels' reduce kernel)
+        // [rs][16 or 32][H] in a fixed order
         T *out = static_cast<T *>(out_) + (size_t)b0 * H;
         int rs = s.rs, nbrows = kBtRows;
         if (bc > kBtRows) {
@@ -1067,7 +1156,7 @@ static int launch_batch_t(const void *x_, int B, int H, const void *gate_, const
         }
         if (rc != ST_OK) return rc;
         ST_HIP(hipGetLastError());
-        rc = launch_mlp_reduce(dtype, partial, rs, nbrows, bc, H, out, stream);
+        rc = launch_batch_reduce(dtype, partial, rs, nbrows, bc, H, out, stream);
         if (rc != ST_OK) return rc;
     }
     return ST_OK;

@@ -1421,29 +1421,6 @@ __global__ __launch_bounds__(kPwThreads) void prefill_down_few_kernel(const T *_
     pf_store_out<T>(acc, stg, lane, 16 * MI * wm, c0 + 64 * wn, M, H, Out, split_k == 1 ? nullptr : partial + (size_t)z * M * H);
 }
 
-// out[m, c] = sum over splits of partial[z][m][c]
-template <typename T>
-__global__ __launch_bounds__(256) void prefill_reduce_kernel(const float *__restrict__ partial, int split_k, int M,
-                                                             int H, T *__restrict__ out)
-{
-    const size_t i4 = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4, total = (size_t)M * H;
-    if (i4 >= total) return;
-    float4 s = *reinterpret_cast<const float4 *>(partial + i4);
-    for (int z = 1; z < split_k; ++z) {
-        const float4 v = *reinterpret_cast<const float4 *>(partial + (size_t)z * total + i4);
-        s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-    }
-    // (T is a 16-bit type here; M * H is a multiple of 4 and `out` a tensor's base, so the four results are one 8-byte store)
-    const uint32_t lo = (uint32_t)from_float<T>(s.x).bits | ((uint32_t)from_float<T>(s.y).bits << 16);
-    const uint32_t hi = (uint32_t)from_float<T>(s.z).bits | ((uint32_t)from_float<T>(s.w).bits << 16);
-    if ((reinterpret_cast<uintptr_t>(out) & 7) == 0) {
-        *reinterpret_cast<uint2 *>(out + i4) = make_uint2(lo, hi);
-    } else {
-        T *o = out + i4;
-        o[0] = from_float<T>(s.x); o[1] = from_float<T>(s.y); o[2] = from_float<T>(s.z); o[3] = from_float<T>(s.w);
-    }
-}
-
 int prefill_split_k(int M, int H, int n)
 {
     // Two blocks fit a CU, so the blocks run in rounds of 2 x CUs; a split costs its K stages plus about four
@@ -1619,13 +1596,8 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
         }
     }
     ST_HIP(hipGetLastError());
-    if (split_k > 1) {
-        ProfScope ps(ST_K_MLP_REDUCE, stream);
-        const size_t quads = ((size_t)M * H + 3) / 4;
-        ST_LAUNCH(ps, prefill_reduce_kernel<T>, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream,
-                           partial, split_k, M, H, static_cast<T *>(out));
-        ST_HIP(hipGetLastError());
-    }
+    if (split_k > 1)
+        return launch_split_reduce(__is_same(T, f16_t) ? ST_F16 : ST_BF16, partial, split_k, (size_t)M * H, (size_t)M * H, out, stream);
     return ST_OK;
 }
 

@@ -252,6 +252,9 @@ int mlp_grid();
 int launch_mlp_reduce(int dtype, const float *partials, int G, int NB, int bcount, int H, void *out,
                       hipStream_t stream);
 
+// out[i] = sum over z < splits of partials[z * stride + i], i < total (a multiple of 4), for a K split of the batch and GEMM kernels.
+int launch_split_reduce(int dtype, const float *partials, int splits, size_t stride, size_t total, void *out, hipStream_t stream);
+
 // Rows of x from which st_mlp_forward takes the GEMM kernels where the batch kernels are switched off or do not apply.
 constexpr int kPrefillMinRows = 32;
 // Two MFMA tiles: one pass of the batch kernels over the weights.

@@ -649,3 +649,22 @@ def test_batch_mfma_agrees_with_streaming_kernel():
     out4, _, _ = _run(x, cw, dn, "silu", True)
     ref = torch.cat([_run(x[i:i + 1], cw, dn, "silu", True)[0].clone() for i in range(4)]).float().cpu().numpy()
     assert_close(out4.float().cpu().numpy(), ref, "bfloat16", "batch vs streaming")
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("B,H,n", [(1, 64, 3), (4, 4096, 40), (16, 1024, 700), (17, 1024, 900), (32, 576, 1000), (9, 2048, 5000),
+                                   (31, 4160, 800), (3, 8192, 900), (100, 256, 6000), (100, 1152, 9000), (128, 2048, 4000)])
+def test_sums_of_splits(B, H, n, dtype):
+    """Every number of row splits the kernels behind a K split sum (two to sixteen by the width, twice that for narrow ones), with as
+    many results as make full blocks or not, into an output off its alignment.  Against float64, as above."""
+    td = getattr(torch, dtype)
+    g = torch.Generator().manual_seed(B + H + n)
+    gate, up, dn = ((torch.randn(n, H, generator=g) * H ** -0.5).to(td).to(DEV) for _ in range(3))
+    x = torch.randn(B, H, generator=g).to(td).to(DEV)
+    h = torch.nn.functional.silu(x.double() @ gate.double().t()) * (x.double() @ up.double().t())
+    store = torch.full((B * H + 1,), float("nan"), dtype=td, device=DEV)
+    out = store[1:].view(B, H)
+    mlp_forward_rows(x, gate, up, dn, n, None, out, None, "silu", True)
+    torch.cuda.synchronize()
+    assert_close(out.float().cpu().numpy(), (h @ dn.double()).cpu().numpy(), dtype, "out")
+    assert bool(torch.isnan(store[0]))
