@@ -377,17 +377,18 @@ __global__ __launch_bounds__(2 * BM * KS) void prefill_gateup_kernel(const T *__
 constexpr int kPwBM = 256, kPwThreads = 512, kPwBufs = 3;
 constexpr int kPwLds = 5 * 256 * kPfLd1;   // 16-byte units: the big tile's five buffers, 160 KB (the wide tile's three take 144)
 
-// kJ: 16-row tiles of up (and of gate) per wave
-template <typename T, bool HG, int kJ>
+// kJ: 16-row tiles of up (and of gate) per wave; kM: rows of x
+template <typename T, bool HG, int kJ, int kM = kPwBM>
 __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict__ X, const T *__restrict__ gate,
                                                  const T *__restrict__ up, int M, int H, int n, int n_pad, int j0, int m0,
                                                  T *__restrict__ Hh, long ldh, T *__restrict__ comb, long ldc, int act)
 {
     constexpr int kWR = 32 * kJ;                          // active rows of the tile
-    constexpr int kRows = kPwBM + (HG ? 2 : 1) * kWR;     // LDS rows of one buffer: x, gate, up
+    constexpr int kPairs = kM / 64;                       // pairs of 16-row fragments of x per wave
+    constexpr int kRows = kM + (HG ? 2 : 1) * kWR;        // LDS rows of one buffer: x, gate, up
     constexpr int kBuf = kRows * kPfLd1;                  // 16-byte units per buffer
     constexpr int kDma = kRows / 64;                      // 1 KB loads per wave and stage
-    constexpr int kGRow = kPwBM, kURow = kPwBM + (HG ? kWR : 0);
+    constexpr int kGRow = kM, kURow = kM + (HG ? kWR : 0);
     static_assert(kPwBufs * kBuf <= kPwLds, "LDS");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kh = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
@@ -403,7 +404,7 @@ __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict
         const int L = wave * kDma + j;
         const int r = 8 * L + (lane >> 3), c = (lane & 7) ^ pf_swz(r);
         int g;
-        if (8 * L < kPwBM) {
+        if (8 * L < kM) {
             g = m0 + r;
             g = g < M ? g : M - 1;
             dbase[j] = reinterpret_cast<const char *>(X);
@@ -429,23 +430,23 @@ __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict
         }
     };
 
-    f32x4_t ag[8][kJ], au[8][kJ];
+    f32x4_t ag[2 * kPairs][kJ], au[2 * kPairs][kJ];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 2 * kPairs; ++i)
 #pragma unroll
         for (int j = 0; j < kJ; ++j) {
             ag[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
             au[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
-    // fragments: the wave's k step of a stage is the kh-th 32 of its 64.  The 128 rows of x go through the MFMAs
-    // as four pairs of 16-row fragments, each pair against the wave's weight fragments.
+    // fragments: the wave's k step of a stage is the kh-th 32 of its 64.  Its 128 (64) rows of x go through the MFMAs
+    // as four (two) pairs of 16-row fragments, each pair against the wave's weight fragments.
     struct FragB { uint4 g[kJ], u[kJ]; };
     uint4 A[3][2];
     FragB Bc, Bn;
     auto rdA = [&](uint4 (&F)[2], int b, int pair) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-            F[i] = lds[b * kBuf + (128 * wm + 32 * pair + 16 * i + l16) * kPfLd1 + ((4 * kh + q) ^ fsw)];
+            F[i] = lds[b * kBuf + (kM / 2 * wm + 32 * pair + 16 * i + l16) * kPfLd1 + ((4 * kh + q) ^ fsw)];
     };
     auto rdB = [&](FragB &F, int b) __attribute__((always_inline)) {
 #pragma unroll
@@ -474,18 +475,26 @@ __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict
         const int x = u, y = (u + 1) % 3, z = (u + 2) % 3;
         const bool load = s + 2 < nk;
         if (load) dma(s + 2, z);
-        rdA(A[y], u, 1);
-        __builtin_amdgcn_sched_barrier(0);
-        mm(A[x], Bc, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        rdA(A[z], u, 2);
-        __builtin_amdgcn_sched_barrier(0);
-        mm(A[y], Bc, 1);
-        __builtin_amdgcn_sched_barrier(0);
-        rdA(A[x], u, 3);
-        __builtin_amdgcn_sched_barrier(0);
-        mm(A[z], Bc, 2);
-        __builtin_amdgcn_sched_barrier(0);
+        constexpr int kLast = kPairs - 1;
+        if constexpr (kPairs == 4) {
+            rdA(A[y], u, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            mm(A[x], Bc, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            rdA(A[z], u, 2);
+            __builtin_amdgcn_sched_barrier(0);
+            mm(A[y], Bc, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            rdA(A[x], u, 3);
+            __builtin_amdgcn_sched_barrier(0);
+            mm(A[z], Bc, 2);
+            __builtin_amdgcn_sched_barrier(0);
+        } else {
+            rdA(A[z], u, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            mm(A[x], Bc, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if (load) ST_WAIT_VM_LGKM0(kDma); else ST_WAIT_VM_LGKM0(0);
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
@@ -493,7 +502,7 @@ __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict
         rdB(Bn, y);
         rdA(A[y], y, 0);
         __builtin_amdgcn_sched_barrier(0);
-        mm(A[x], Bc, 3);
+        mm(A[kPairs == 4 ? x : z], Bc, kLast);
         __builtin_amdgcn_sched_barrier(0);
         Bc = Bn;
     };
@@ -519,23 +528,23 @@ __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict
     }
 
     ST_TL(2);
-    // The pair's sums: the wave with kh = 0 finishes the first 64 rows of the tile, the other the last 64; each
+    // The pair's sums: the wave with kh = 0 finishes the first half of the tile's rows, the other the second; each
     // hands the other half of its accumulators over through LDS (all stage buffers are free: the last stage ends
     // behind its barrier with no fragment read outstanding).
-    constexpr int kQuads = (HG ? 8 : 4) * kJ;   // accumulator quads per lane handed over
+    constexpr int kQuads = (HG ? 2 : 1) * kPairs * kJ;   // accumulator quads per lane handed over
     f32x4_t *red = reinterpret_cast<f32x4_t *>(lds);
-    f32x4_t fg[4][kJ], fu[4][kJ];
+    f32x4_t fg[kPairs][kJ], fu[kPairs][kJ];
     {
         f32x4_t *mine = red + (size_t)wave * kQuads * 64 + lane;
         auto hand = [&](int h) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < kPairs; ++i)
 #pragma unroll
                 for (int j = 0; j < kJ; ++j) {
-                    mine[(i * kJ + j) * 64] = au[4 * h + i][j];
-                    if (HG) mine[(4 * kJ + i * kJ + j) * 64] = ag[4 * h + i][j];
-                    fu[i][j] = au[4 * (1 - h) + i][j];
-                    if (HG) fg[i][j] = ag[4 * (1 - h) + i][j];
+                    mine[(i * kJ + j) * 64] = au[kPairs * h + i][j];
+                    if (HG) mine[(kPairs * kJ + i * kJ + j) * 64] = ag[kPairs * h + i][j];
+                    fu[i][j] = au[kPairs * (1 - h) + i][j];
+                    if (HG) fg[i][j] = ag[kPairs * (1 - h) + i][j];
                 }
         };
         if (kh == 0) hand(1); else hand(0);
@@ -544,18 +553,18 @@ __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict
     {
         const f32x4_t *other = red + (size_t)(wave ^ 4) * kQuads * 64 + lane;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < kPairs; ++i)
 #pragma unroll
             for (int j = 0; j < kJ; ++j) {
                 fu[i][j] += other[(i * kJ + j) * 64];
-                if (HG) fg[i][j] += other[(4 * kJ + i * kJ + j) * 64];
+                if (HG) fg[i][j] += other[(kPairs * kJ + i * kJ + j) * 64];
             }
     }
     __syncthreads();
 
     ST_TL(3);
-    T *stg = reinterpret_cast<T *>(lds) + (size_t)wave * 64 * (16 * kJ + 8);
-    pf_store_hidden<T, HG, kJ>(act, fg, fu, stg, lane, m0 + 128 * wm + 64 * kh, j0 + 16 * kJ * wn, M, n, n_pad, Hh, ldh, comb, ldc);
+    T *stg = reinterpret_cast<T *>(lds) + (size_t)wave * 16 * kPairs * (16 * kJ + 8);
+    pf_store_hidden<T, HG, kJ>(act, fg, fu, stg, lane, m0 + kM / 2 * wm + kM / 4 * kh, j0 + 16 * kJ * wn, M, n, n_pad, Hh, ldh, comb, ldc);
     ST_TL(4);
 }
 
@@ -699,22 +708,24 @@ __device__ __forceinline__ void gateup_big_tile(uint4 *lds, const T *__restrict_
 
 // How the active rows are dealt into tiles: big ones as long as they come in whole rounds over the CUs; what is left over
 // stays big when it keeps more than half of the CUs busy, and is halved into wide tiles (which take about 0.65 of the time)
-// when it does not; ungated, whose halves have no gate rows to split off, into quarters while those fit the CUs too.  Whole
-// forward, 2048 rows, H 3072, us, the rest big / halved: rest 112 of 256 CUs 217 / 203, 128 220 / 209, 144 225 / 243; no whole
-// round, 128 tiles 94 / 79, 136 95 / 113.  Ungated,
-// H 3072, 300 rows, halved / quartered: 48 tiles 68.8 / 58.7, 68 (two rounds of quarters) 75.8 / 92.0; 400 rows, H 4096, 64 99.9 / 91.4.
+// when it does not, into quarters while those fit the CUs too (ungated 256 rows of x x 64 active rows; gated, where 32 gate
+// and 32 up rows would leave each wave a single column of fragments, 128 rows of x x (64 + 64)).  Whole forward, us: 2048
+// rows, H 3072, the rest big / halved: rest 112 of 256 CUs 217 / 203, 128 220 / 209, 144 225 / 243; no whole round, 128 tiles
+// 94 / 79, 136 95 / 113.  Gated, halved / quartered: H 3072, 300 rows, 48 tiles 61.5 / 53.8, 64 66.0 / 59.2; 512 rows, 46
+// 73.3 / 63.0; H 4096, 256 rows, 63 98.0 / 88.7; 2048 rows, a rest of 40 585 / 571.  Ungated, H 3072, 300 rows, halved /
+// quartered: 48 tiles 68.8 / 58.7, 68 (two rounds of quarters) 75.8 / 92.0; 400 rows, H 4096, 64 99.9 / 91.4.
 struct GateupTiles { int big, small, parts; };   // big tiles, smaller ones, smaller ones per big one
-template <bool HG> __host__ __device__ __forceinline__ GateupTiles gateup_tiles(int n_pad, int rows, int mt, int cus)
+__host__ __device__ __forceinline__ GateupTiles gateup_tiles(int n_pad, int rows, int mt, int cus)
 {
     const int t = (n_pad + rows - 1) / rows * mt, rest = t % cus;
-    const int parts = !HG && 4 * rest <= cus ? 4 : 2 * rest <= cus ? 2 : 1;
+    const int parts = 4 * rest <= cus ? 4 : 2 * rest <= cus ? 2 : 1;
     return parts == 1 ? GateupTiles{t, 0, 1} : GateupTiles{t - rest, parts * rest, parts};
 }
 // The most blocks that any count up to the capacity's `t` big tiles asks for (both kinds in whole eights): the rest of the last
 // round, or any of a whole one before, in the parts that make most of it.
-template <bool HG> static int gateup_blocks(int t, int cus)
+static int gateup_blocks(int t, int cus)
 {
-    const int rest = t % cus, in4 = HG ? 0 : 4 * (rest < cus / 4 ? rest : cus / 4), in2 = 2 * (rest < cus / 2 ? rest : cus / 2);
+    const int rest = t % cus, in4 = 4 * (rest < cus / 4 ? rest : cus / 4), in2 = 2 * (rest < cus / 2 ? rest : cus / 2);
     return t - rest + (in4 > in2 ? in4 : in2 > rest ? in2 : rest) + kXcds;
 }
 
@@ -731,7 +742,7 @@ __global__ __launch_bounds__(kPwThreads) void prefill_gateup_wide_kernel(const T
     __shared__ uint4 lds[kPwLds];
     const int n = device_count(n_host, n_dev);
     const int n_pad = (n + kPfBK - 1) / kPfBK * kPfBK;
-    const GateupTiles tiles = gateup_tiles<HG>(n_pad, kBigRows, mt, cus);
+    const GateupTiles tiles = gateup_tiles(n_pad, kBigRows, mt, cus);
     const int big_blocks = (tiles.big + kXcds - 1) / kXcds * kXcds;
     ST_TL(0);
     if ((int)blockIdx.x < big_blocks) {
@@ -742,9 +753,12 @@ __global__ __launch_bounds__(kPwThreads) void prefill_gateup_wide_kernel(const T
         const int part = xcd_tile_id(blockIdx.x - big_blocks, tiles.small);
         if (part < 0) return;
         const int shift = tiles.parts == 4 ? 2 : 1, tile = tiles.big + (part >> shift);
-        const int j0 = tile / mt * kBigRows + (part & (tiles.parts - 1)) * (kBigRows >> shift), m0 = tile % mt * kPwBM;
-        if (j0 >= n_pad) return;
-        if (HG || tiles.parts == 4) gateup_wide_tile<T, HG, 2>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
+        const int cols = HG && tiles.parts == 4 ? 2 : tiles.parts;   // parts of a tile's active rows; the rest are of its rows of x
+        const int j0 = tile / mt * kBigRows + (part & (cols - 1)) * (kBigRows / cols);
+        const int m0 = tile % mt * kPwBM + (cols < tiles.parts ? ((part >> 1) & 1) * (kPwBM / 2) : 0);
+        if (j0 >= n_pad || m0 >= M) return;
+        if (HG && tiles.parts == 4) gateup_wide_tile<T, HG, 2, HG ? 128 : kPwBM>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
+        else if (HG || tiles.parts == 4) gateup_wide_tile<T, HG, 2>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
         else gateup_wide_tile<T, HG, HG ? 2 : 4>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
     }
 }
@@ -1554,7 +1568,7 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
         const int mt = big ? (M + 255) / 256 : quarters ? (M + 63) / 64 : mt128;
         // (the tiles are dealt out over the device's count)
         const int big_tiles = (int)((ldw + (has_gate ? 127 : 255)) / (has_gate ? 128 : 256)) * mt;
-        const int blocks = !big ? jt * mt : has_gate ? gateup_blocks<true>(big_tiles, cus) : gateup_blocks<false>(big_tiles, cus);
+        const int blocks = !big ? jt * mt : gateup_blocks(big_tiles, cus);
         const int grid = (blocks + kXcds - 1) / kXcds * kXcds;
         auto go = [&](auto kern, int threads) -> int {
             ST_LAUNCH(ps, kern, dim3(grid), dim3(threads), 0, stream, static_cast<const T *>(x),

@@ -335,8 +335,8 @@ def test_prefill_tiles_follow_the_device_count(M, n):
     (1030, 384, 8192, 3000, True),     # t = 120: all halved
     (1030, 384, 8192, 3201, True),     # t = 130: all big, the last row tile of x nearly empty
     (1030, 128, 8192, 6527, True),     # t = 255; two K stages
-    (1030, 256, 8192, 6529, True),     # t = 260: 256 big, 4 halved
-    (1030, 256, 8192, 8192, True),     # t = 320: 256 big, 64 halved
+    (1030, 256, 8192, 6529, True),     # t = 260: 256 big, 4 quartered
+    (1030, 256, 8192, 8192, True),     # t = 320: 256 big, 64 quartered
     (2030, 256, 8448, 8200, False),    # t = 264: 256 big, 8 quartered, of which the last two quarters are past the padded count
     (2030, 384, 8448, 8447, False),    # the same with all quarters
     (150, 256, 8448, 8447, False),     # t = 33: all quartered, one row tile
@@ -366,6 +366,17 @@ def test_prefill_big_tiles(M, H, I, n, gated):
     torch.cuda.synchronize()
     assert_close(out.float().cpu().numpy(), want.cpu().numpy(), "float16", f"{M} rows, {n} active")
     assert_close(comb[:, :n].float().cpu().numpy(), h.cpu().numpy(), "float16", f"intermediate, {M} rows, {n} active")
+
+
+@pytest.mark.parametrize("M,H,I,n", [
+    (129, 64, 9000, 1), (129, 64, 9000, 8192), (256, 192, 9000, 8129), (257, 128, 9000, 4095), (384, 256, 9000, 4033),
+    (385, 320, 9000, 4096), (1100, 128, 9000, 6700),
+])
+def test_prefill_quarters_of_gated_tiles(M, H, I, n):
+    """Rests of up to a quarter of the CUs, which go out as 128 rows of x by 64 active ones: one tile of them, the most, K loops
+    of one stage to five, rows of x that leave a tile's lower half out or with one row, counts that leave an active half out.
+    Checked as the tiles above are."""
+    test_prefill_big_tiles(M, H, I, n, True)
 
 
 @pytest.mark.parametrize("M,H,I,n,gated", [
