@@ -952,12 +952,18 @@ static bool batch_shape(int dtype, int H, BatchShape &s)
     return true;
 }
 
-// (three or four rows of fp32: whole forward, us, streaming / batch kernels, H 1024, 1500 active 12.8 / 15.3; H 1536, 1200 16.5 /
-// 17.0; H 1792, 1280 17.5 / 18.9; H 2048, 2500 26.4 / 23.5; H 2816, 2200 30.3 / 27.5.  Five: H 1280, 600, ungated 16.1 / 12.1)
+// Few rows at small hidden sizes stay with the streaming kernel, which takes four rows of 16 bits, or eight of fp32, in one pass
+// and is one launch (2.5 us of the host's, who sets the pace there) less.  Whole forward, us, streaming / batch kernels: fp16,
+// three rows, H 384, 768 active 11.0 / 11.2; H 640, 1280 11.6 / 11.5; H 896, 1760 12.4 / 12.1; H 1152, 2304 16.1 / 12.7; five
+// rows, H 384 13.3 / 11.3.  fp32, three or four rows, H 1024, 1500 active 12.8 / 15.3; H 1536, 1200 16.5 / 17.0; H 1792, 1280
+// 17.5 / 18.9; H 2048, 2500 26.4 / 23.5; seven, H 512, 1024 12.2 / 11.7; H 1024, 672 14.4 / 13.7 (three layers of a module
+// with their masks: 84.9 / 93.0 from the host); H 1536, 1002 20.3 / 17.5; twelve, H 512, 1024 21.8 / 11.9.
 bool batch_supported(int dtype, int B, int H)
 {
     BatchShape s;
-    return batch_shape(dtype, H, s) && !(dtype == ST_F32 && B <= 4 && H < 2048);
+    if (!batch_shape(dtype, H, s)) return false;
+    if (dtype == ST_F32) return !(B <= 4 && H < 2048) && !(B <= 8 && H <= 1024);
+    return s.special || !(B <= 4 && H < 1024);
 }
 
 static int64_t batch_ldh(int64_t n) { return (n + kBtTile - 1) / kBtTile * kBtTile; }

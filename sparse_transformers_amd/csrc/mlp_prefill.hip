@@ -370,7 +370,8 @@ __global__ __launch_bounds__(2 * BM * KS) void prefill_gateup_kernel(const T *__
 // per clock, whatever the number of loads in flight):
 //   wide  256 rows of x by 128 weight rows (64 + 64): 48 KB for 2 x 256 x 128 x 64 flops, about even; the two waves of a SIMD
 //         share a tile (wave kh takes the kh-th 32 of K into accumulators of its own; the pair is summed through LDS once at
-//         the end), three LDS buffers; ungated also by 64 weight rows
+//         the end), three LDS buffers; as the last round's quarters also 256 by 64 (ungated) and 128 by 128 (gated: 32 KB
+//         for half the flops)
 //   big   256 by 256 (128 + 128): 64 KB for twice the flops, MFMA bound; x in two LDS buffers, one stage ahead (L2 hits),
 //         the weights, which come from HBM, in three, two stages ahead: the whole 160 KB.  2048 rows, H 4096, 12902 of 14336
 //         active, bf16: 342-355 us against 400 in wide tiles alone (433 GFLOP; 270 without the loads)

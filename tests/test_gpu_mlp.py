@@ -590,6 +590,7 @@ def test_batch_mfma_vs_oracle(name, B, H, n, dtype, act, has_gate):
     (9, 1664, 6144, 1230, "bfloat16", True), (32, 896, 4500, 4096, "float16", True), (25, 1152, 9000, 8200, "bfloat16", True),
     (32, 1600, 5000, 4095, "float16", False), (31, 3200, 2000, 1999, "bfloat16", True), (12, 4736, 700, 333, "float16", True),
     (22, 16384, 100, 97, "bfloat16", False), (40, 1216, 3000, 2900, "float16", True),
+    (9, 48, 300, 257, "float32", False), (9, 16, 40, 1, "float32", True), (5, 64, 40, 16, "float16", True),
 ])
 def test_batch_any_width(B, H, I, n, dtype, gated):
     """The batch kernels for any width whose rows are multiples of 64 bytes, and fp32: remainders of the steps per wave, both
