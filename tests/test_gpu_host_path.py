@@ -255,6 +255,7 @@ def test_threads_and_streams():
     assert all(torch.equal(a, b) for g in got for a, b in zip(g, want))
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("I,H,gated,dtype", [(1, 64, True, torch.float32), (203, 72, False, torch.float16), (2048, 256, True, torch.bfloat16)])
 def test_cache_construction_forms(I, H, gated, dtype):
     """A cache built by the native path and by the general one, which takes every other form of the arguments (strided weights, a
