@@ -76,12 +76,13 @@ const char *st_last_error(void);
  *                      leaves in combined_proj_buffer
  *   workspace          scratch of st_mlp_workspace_bytes(B,H,n) bytes
  * All rows must be 16-byte aligned (H*sizeof(dtype) % 16 == 0). B <= 4096.
- * B <= 2 (and any B < 32 in fp32 or with a hidden size the MFMA kernels do not
- * cover) runs the streaming decode kernel; 3 <= B <= 32 in fp16 / bf16 with
- * H % 256 == 0 (H <= 16384) runs the MFMA batch kernels (still HBM-bound; one
- * pass over the weights per 32 rows of x for H in {2048, 3072, 4096}, per 16
- * rows otherwise); otherwise B >= 32 in fp16 / bf16 with H % 128 == 0
- * runs the MFMA GEMM kernels (then only columns [0,n) of `combined` carry results; when its rows are 16-byte
+ * B <= 2 runs the streaming decode kernel.  B >= 3 runs the MFMA batch kernels
+ * (still HBM-bound; one pass over the weights per 32 rows of x) where H % 64 == 0
+ * and H <= 16384, in fp32 H % 16 == 0 and H <= 8192, except that few rows at small
+ * hidden sizes (up to four below 1024, in fp32 below 2048; in fp32 up to eight to
+ * 1024) stay with the streaming kernel, which also takes every other H.  More than
+ * 32 rows in fp16 / bf16 with H % 128 == 0, and 32 where H % 256 != 0,
+ * run the MFMA GEMM kernels (then only columns [0,n) of `combined` carry results; when its rows are 16-byte
  * aligned and have room, the kernels keep their intermediate there and also zero the columns from n up to the next
  * multiple of 128).
  * ST_F64 (any B, H % 2 == 0): three plain kernels with every sum in double and in a fixed order, eight rows of x

@@ -479,17 +479,15 @@ int batch_min_rows()
     return v;
 }
 
-// Rows of x that take the GEMM kernels (mlp_prefill.hip) rather than the batch kernels: all beyond two MFMA tiles; of 17 to 32
-// those whose intermediate is held in the storage type either way, where the matrices are large (by their capacity, so that
-// the form does not change with the count).  Whole forward, us, batch / GEMM kernels: 32 rows, H 3840, 5000 of 10240 45.2 /
-// 39.1; 24 rows, H 4864, 6000 of 16384 56.3 / 45.1; 20 rows, H 4096, 2000 of 14336 26.3 / 27.7; 32 rows, H 2560, 3000 of 10240
-// 27.3 / 26.8, 20 rows 24.1 / 24.8; 24 rows, H 3072, 2867 of 8192 26.4 / 27.4.  32 rows where H is no multiple of 256: H 3200,
-// 5000 of 11200 48.4 / 34.3.  (17 to 31 rows there keep fp32 between the batch kernels.)
+// Rows of x that take the GEMM kernels (mlp_prefill.hip) rather than the batch kernels: all beyond two MFMA tiles, and two full
+// tiles where H is no multiple of 256 (32 rows, H 3200, 5000 of 11200 active, whole forward, us, batch / GEMM kernels 48.4 / 34.3).
+// Fewer rows stay with the batch kernels at every size, also where the GEMM kernels are faster (32 rows, H 3840, 5000 of 10240
+// 45.2 / 39.1; 24 rows, H 4864, 6000 of 16384 56.3 / 45.1): those leave the up projection out of `combined` and may write
+// past n columns of it, use the fast exponential, and split their sums by n, which a cache gives as its capacity and the
+// operator as the count.
 static bool gemm_rows(int dtype, int64_t B, int64_t H, int64_t n)
 {
-    if (dtype == ST_F32 || H % 128 != 0 || n < 1) return false;
-    if (B > kBatchMaxRows) return true;
-    return H % 256 != 0 ? B == kBatchMaxRows : B > 16 && n * H >= (int64_t)32 << 20;
+    return dtype != ST_F32 && H % 128 == 0 && n >= 1 && (B > kBatchMaxRows || (B == kBatchMaxRows && H % 256 != 0));
 }
 
 // Blocks per launch: one per CU by default; ST_MLP_GMULT (1..4) multiplies it.
@@ -623,7 +621,7 @@ extern "C" int64_t st_mlp_workspace_bytes(int64_t B, int64_t H, int64_t n)
         const int64_t batch = st::batch_workspace_bytes(H, n);
         decode = batch > decode ? batch : decode;
     }
-    if (B <= 16) return decode;   // (gemm_rows)
+    if (B < st::kPrefillMinRows) return decode;
     const int64_t prefill = st::prefill_workspace_bytes(B, H, n);
     return prefill > decode ? prefill : decode;
 }

@@ -451,7 +451,7 @@ def test_prefill_few_rows_infinite_last_row(M, H, I, n, gated):
     (24, 768, 44000, 6143, False),
 ])
 def test_prefill_of_17_to_32_rows(M, H, I, n, gated):
-    """The few-row form of one pair of tiles, where it takes rows that the batch kernels could: the checks of the two tests above.
+    """17 to 32 rows at both sides of the line between the batch kernels and the few-row form: the checks of the two tests above.
     (At most 2048 wide: rounding the intermediate to fp16 puts sqrt(n) * 0.05 * rms(h) * 1e-4 on a result, 0.0016 at rms(h) = 3.6 and
     8129 rows, against a bound of 0.02; at 4096, rms(h) near 10, two of 69632 results pass it.)"""
     test_prefill_few_rows(M, H, I, n, gated)
@@ -553,6 +553,35 @@ def test_prefill_leaves_the_parent_of_a_column_slice_alone():
                                      "relu", False)
     assert_close(out.float().cpu().numpy(), want, "float16", "out")
     assert_close(parent[:, :n].float().cpu().numpy(), wantc[:, :n], "float16", "combined view")
+
+
+@pytest.mark.parametrize("B,H,I,n,dtype,gated", [
+    (17, 4096, 11000, 11000, "float16", False), (24, 4096, 14336, 3500, "bfloat16", True), (31, 3840, 10240, 9001, "float16", True),
+    (32, 3072, 11000, 10999, "bfloat16", True), (24, 3072, 11000, 8200, "float16", False),
+])
+def test_17_to_32_rows_of_large_matrices(B, H, I, n, dtype, gated):
+    """17 to 32 rows where n * H passes 32 Mi: `combined` as a column slice gets act(gate) * up, the raw up projection behind it
+    when gated, and nothing is written outside the slice; the same bits with the count from the host or from the device.
+    Against float64 on weights that keep the intermediate of order one."""
+    td = getattr(torch, dtype)
+    g = torch.Generator().manual_seed(B + H + n)
+    gate, up, dn = ((torch.randn(I, H, generator=g) * H ** -0.5).to(td).to(DEV) for _ in range(3))
+    x = torch.randn(B, H, generator=g).to(td).to(DEV)
+    u = x.double() @ up[:n].double().t()
+    h = torch.nn.functional.silu(x.double() @ gate[:n].double().t()) * u if gated else torch.nn.functional.silu(u)
+    want, wantc = h @ dn[:n].double(), torch.cat([h, u], 1) if gated else h
+    first = None
+    for cap, n_dev in ((n, None), (I, torch.tensor([n], dtype=torch.int32, device=DEV))):
+        cols = (2 if gated else 1) * cap
+        parent = torch.full((B, (cols + 263) // 8 * 8), 7.0, dtype=td, device=DEV)
+        out = torch.empty(B, H, dtype=td, device=DEV)
+        mlp_forward_rows(x, gate if gated else None, up, dn, cap, n_dev, out, parent[:, :cols], "silu", gated)
+        torch.cuda.synchronize()
+        assert bool((parent[:, cols:] == 7.0).all()), "columns outside the view were written"
+        assert_close(out.float().cpu().numpy(), want.cpu().numpy(), dtype, "out")
+        assert_close(parent[:, :wantc.size(1)].float().cpu().numpy(), wantc.cpu().numpy(), dtype, "combined")
+        first = out if first is None else first
+        assert torch.equal(first, out)
 
 
 # ---- MFMA batch kernels (3 <= B <= 32, fp16 / bf16, hidden sizes that are multiples of 256) ----
