@@ -550,9 +550,9 @@ __global__ __launch_bounds__(kBtThreads) void batch_down_f32_kernel(
 }
 
 // Eight fp32 values of h as three 16-bit operands each that sum to them, for the MFMAs of kernel 2.  bf16 has fp32's range:
-// three parts of eight bits are the value.  fp16 has not: the chunk is scaled by a power of two that puts its largest finite
-// exponent at 2^14 (wave-uniform: one multiply-add per result takes it back), where three parts hold all 24 bits of
-// what is within 2^16 of the largest element and 2^-39 of the largest below that.  An infinity or NaN is its own first part.
+// three parts of eight bits are the value.  fp16 has not: each row of x is scaled, chunk by chunk, by a power of two that puts
+// its largest finite exponent at 2^14 (one multiply-add per result takes it back), where three parts hold all 24 bits of
+// what is within 2^16 of the row's largest element and 2^-39 of the largest below that.  An infinity or NaN is its own first part.
 template <typename T> struct SplitH;
 template <> struct SplitH<bf16_t> {
     static constexpr bool kScaled = false;
@@ -606,27 +606,20 @@ template <> struct SplitH<f16_t> {
     }
 };
 
-// largest value over the wave, in every lane's scalar registers
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
+// largest value over the four lanes that hold one row of an MFMA operand (lane % 16)
+__device__ __forceinline__ uint32_t row_max_u32(uint32_t v)
 {
-    auto step = [&](uint32_t o) __attribute__((always_inline)) { v = v > o ? v : o; };
-    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false));    // quad_perm [1,0,3,2]
-    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false));    // quad_perm [2,3,0,1]
-    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false));   // row_half_mirror
-    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, false));   // row_mirror
-    uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)v, 0);
-#pragma unroll
-    for (int l = 16; l < kWave; l += 16) {
-        const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)v, l);
-        m = m > o ? m : o;
-    }
-    return m;
+    const auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    v = a[0] > a[1] ? a[0] : a[1];
+    const auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return b[0] > b[1] ? b[0] : b[1];
 }
 
 // ---------------------------------------------------------------------------
 // kernel 2.  Block = (column group cg, row split rs); NP = 64-column pieces per
 // block; NX = tiles of 16 rows of x; HT = the type h is held in (the storage type behind
-// batch_gateup_kernel, fp32 behind batch_gateup_any_kernel: three MFMAs per tile and chunk of rows then).
+// batch_gateup_kernel, fp32 behind batch_gateup_any_kernel: three MFMAs per tile and chunk of rows then).  Where h is scaled
+// (fp16) the operands change places: a row of x is then a column of D, whose scale is the lane's own.
 // partial[(rs * ldb + b) * H + col], fp32.
 // ---------------------------------------------------------------------------
 template <typename T, typename HT, int NP, int NX>
@@ -635,7 +628,7 @@ __global__ __launch_bounds__(kBtThreads) void batch_down_kernel(
     const int *__restrict__ n_dev, float *__restrict__ partial, int CG, int RS, int ldb)
 {
     constexpr int NT = NP * 4;   // 16-column tiles per block
-    constexpr bool WIDE = __is_same(HT, float);
+    constexpr bool WIDE = __is_same(HT, float), SCALED = WIDE && SplitH<T>::kScaled;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid >> 6;
     const int c16 = lane & 15, q = lane >> 4;
@@ -693,7 +686,7 @@ __global__ __launch_bounds__(kBtThreads) void batch_down_kernel(
         }
         constexpr int PARTS = WIDE ? 3 : 1;
         uint4 hf[NX][PARTS];
-        float unscale = 1.f;
+        float unscale[NX];
         if constexpr (WIDE) {
             float hv[NX][8];
 #pragma unroll
@@ -710,23 +703,23 @@ __global__ __launch_bounds__(kBtThreads) void batch_down_kernel(
                         for (int t = 0; t < NX; ++t) hv[t][i] = 0.f;
                     }
             }
-            float scale = 1.f;
-            if constexpr (SplitH<T>::kScaled) {
-                uint32_t e = 15u << 23;
 #pragma unroll
-                for (int t = 0; t < NX; ++t)
+            for (int t = 0; t < NX; ++t) {
+                float scale = 1.f;
+                if constexpr (SCALED) {
+                    uint32_t e = 15u << 23;
 #pragma unroll
                     for (int i = 0; i < 8; ++i) {
                         uint32_t x = __float_as_uint(hv[t][i]) & 0x7f800000u;
                         x = x == 0x7f800000u ? 0u : x;
                         e = e > x ? e : x;
                     }
-                e = wave_max_u32(e);
-                scale = __uint_as_float((268u << 23) - e);      // 2^(141 - E)
-                unscale = __uint_as_float(e - (14u << 23));     // 2^(E - 141)
+                    e = row_max_u32(e);
+                    scale = __uint_as_float((268u << 23) - e);      // 2^(141 - E)
+                    unscale[t] = __uint_as_float(e - (14u << 23));  // 2^(E - 141)
+                }
+                SplitH<T>::run(hv[t], scale, hf[t]);
             }
-#pragma unroll
-            for (int t = 0; t < NX; ++t) SplitH<T>::run(hv[t], scale, hf[t]);
         } else {
 #pragma unroll
             for (int t = 0; t < NX; ++t) {
@@ -779,18 +772,18 @@ __global__ __launch_bounds__(kBtThreads) void batch_down_kernel(
 #pragma unroll
                         for (int t = 0; t < NX; ++t) {
                             const int lo = part > 0;
-                            f32x4_t &sum = SplitH<T>::kScaled ? d[lo][t][ct] : lo ? low[t][p * 4 + ct] : acc[t][p * 4 + ct];
-                            sum = Mfma<T>::run(hf[t][part], bf[ct], SplitH<T>::kScaled && part != 1 ? zero : sum);
+                            f32x4_t &sum = SCALED ? d[lo][t][ct] : lo ? low[t][p * 4 + ct] : acc[t][p * 4 + ct];
+                            sum = SCALED ? Mfma<T>::run(bf[ct], hf[t][part], part != 1 ? zero : sum) : Mfma<T>::run(hf[t][part], bf[ct], sum);
                         }
-                if constexpr (SplitH<T>::kScaled) {
+                if constexpr (SCALED) {
 #pragma unroll
                     for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
                         for (int t = 0; t < NX; ++t)
 #pragma unroll
                             for (int e = 0; e < 4; ++e) {
-                                acc[t][p * 4 + ct][e] = fmaf(d[0][t][ct][e], unscale, acc[t][p * 4 + ct][e]);
-                                low[t][p * 4 + ct][e] = fmaf(d[1][t][ct][e], unscale, low[t][p * 4 + ct][e]);
+                                acc[t][p * 4 + ct][e] = fmaf(d[0][t][ct][e], unscale[t], acc[t][p * 4 + ct][e]);
+                                low[t][p * 4 + ct][e] = fmaf(d[1][t][ct][e], unscale[t], low[t][p * 4 + ct][e]);
                             }
                 }
             }
@@ -828,21 +821,35 @@ __global__ __launch_bounds__(kBtThreads) void batch_down_kernel(
 #pragma unroll
     for (int t = 0; t < NX; ++t) {
         __syncthreads();
-        float *red = reinterpret_cast<float *>(lds_raw);   // [8][NT][4][64]
+        if constexpr (SCALED) {   // a lane holds four neighbouring columns of row lane % 16
+            f32x4_t *red = reinterpret_cast<f32x4_t *>(lds_raw);   // [8][NT][64]
 #pragma unroll
-        for (int i = 0; i < NT; ++i)
+            for (int i = 0; i < NT; ++i) red[(w * NT + i) * 64 + lane] = acc[t][i];
+            __syncthreads();
+            for (int idx = tid; idx < NT * 64; idx += kBtThreads) {
+                f32x4_t s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) red[((size_t)(w * NT + i) * 4 + e) * 64 + lane] = acc[t][i][e];
-        __syncthreads();
+                for (int ww = 0; ww < kBtWaves; ++ww) s += red[ww * NT * 64 + idx];
+                const int tile = idx >> 6, dl = idx & 63, b = 16 * t + (dl & 15);
+                if (b < B) *reinterpret_cast<f32x4_t *>(partial + ((size_t)rs * ldb + b) * H + col0 + 16 * tile + 4 * (dl >> 4)) = s;
+            }
+        } else {
+            float *red = reinterpret_cast<float *>(lds_raw);   // [8][NT][4][64]
 #pragma unroll
-        for (int m = 0; m < NT * 256 / kBtThreads; ++m) {
-            const int idx = tid + kBtThreads * m;
-            float s = 0.f;
+            for (int i = 0; i < NT; ++i)
 #pragma unroll
-            for (int ww = 0; ww < kBtWaves; ++ww) s += red[(size_t)ww * NT * 256 + idx];
-            const int tile = idx >> 8, e = (idx >> 6) & 3, dl = idx & 63;
-            const int b = 16 * t + 4 * (dl >> 4) + e;   // D rows are the rows of x
-            if (b < B) partial[((size_t)rs * ldb + b) * H + col0 + 16 * tile + (dl & 15)] = s;
+                for (int e = 0; e < 4; ++e) red[((size_t)(w * NT + i) * 4 + e) * 64 + lane] = acc[t][i][e];
+            __syncthreads();
+#pragma unroll
+            for (int m = 0; m < NT * 256 / kBtThreads; ++m) {
+                const int idx = tid + kBtThreads * m;
+                float s = 0.f;
+#pragma unroll
+                for (int ww = 0; ww < kBtWaves; ++ww) s += red[(size_t)ww * NT * 256 + idx];
+                const int tile = idx >> 8, e = (idx >> 6) & 3, dl = idx & 63;
+                const int b = 16 * t + 4 * (dl >> 4) + e;   // D rows are the rows of x
+                if (b < B) partial[((size_t)rs * ldb + b) * H + col0 + 16 * tile + (dl & 15)] = s;
+            }
         }
     }
 }

@@ -656,6 +656,29 @@ def test_batch_any_width(B, H, I, n, dtype, gated):
         assert_close(comb[:, n:].float().cpu().numpy(), hu.cpu().numpy(), dtype, "combined, up")
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16", "float32"])
+@pytest.mark.parametrize("B,H,n", [(5, 896, 700), (9, 960, 500), (16, 1152, 1111), (31, 1152, 2000), (12, 2048, 300)])
+def test_batch_rows_do_not_meet(B, H, n, dtype):
+    """A row's result has the same bits whatever the other rows of its tile hold: rows up to 2^20 larger, of zeros, with an infinity."""
+    td = getattr(torch, dtype)
+    g = torch.Generator().manual_seed(B + H)
+    gate, up, dn = ((torch.randn(n, H, generator=g) * H ** -0.5).to(td).to(DEV) for _ in range(3))
+    x = (torch.randn(B, H, generator=g) * 2.0 ** -7).to(td).to(DEV)
+    y = x.clone()
+    y[0] *= 2.0 ** 20 if dtype != "float16" else 2.0 ** 15
+    y[2] = 0.0
+    y[B - 1, 3] = float("inf")
+    outs = []
+    for v in (x, y):
+        out = torch.empty(B, H, dtype=td, device=DEV)
+        mlp_forward_rows(v, gate, up, dn, n, None, out, None, "silu", True)
+        torch.cuda.synchronize()
+        outs.append(out)
+    same = [b for b in range(B) if b not in (0, 2, B - 1)]
+    assert torch.equal(outs[0][same], outs[1][same])
+    assert not outs[1][2].any()
+
+
 def test_batch_mfma_device_count_and_determinism():
     """The batch kernels take the active count from device memory (rows past it may hold anything, here NaN),
     and repeat bit-identically."""
