@@ -8,9 +8,9 @@
 //   sketch       approx_topk_threshold, sparse_transformers/csrc/approx_topk.h:10-88
 //
 // One block per row.  The row is read from HBM once; every thread keeps its scores in registers (rows of up
-// to 16384 scores) as order-preserving 32-bit keys.  The k-th largest key is found exactly, with nothing sorted: by one
-// histogram of the values and a ranking of the interval that holds it, or by a radix select (8-bit digits, most significant
-// first, one LDS histogram per digit; once at most 64 keys share the prefix one wave ranks them directly).  With several
+// to 16384 scores) as order-preserving 32-bit keys.  The k-th largest key is found exactly, with nothing sorted, by a radix
+// select (10-bit digits, longer rows 8-bit ones, most significant first, one LDS histogram per digit; once at most 64 keys
+// share the prefix they are ranked directly).  With several
 // rows every block leaves its row mask in the workspace and the block that finishes last ORs them together; which block that
 // is does not change the result.  A caller with a mask of zeros has the blocks set their rows' bytes in it instead.
 #include "st_common.h"
@@ -35,13 +35,15 @@ __device__ __forceinline__ float key_value(uint32_t k)
 
 constexpr int kHistCopies = 8;  // a digit's counter exists once per lane % 8: equal digits in a wave spread over banks
 
+// of key_select_desc: digits, counters of each, and counters from one digit's first to its second (equal digits on other banks)
+constexpr int kKeyDigits = 1024, kKeyCopies = 8, kKeyPitch = kKeyDigits + kWave / kKeyCopies;
+constexpr size_t kKeyHistBytes = (size_t)kKeyPitch * kKeyCopies * 4;
+
 struct SelShared {
     uint32_t hist[256 * kHistCopies];
     uint32_t hsum[256];
     uint32_t cand[kWave];
     uint32_t digit, rem, cnt, ncand;
-    __align__(16) uint32_t wave_hi[kSelWaves];
-    __align__(16) uint32_t wave_lo[kSelWaves];
     int wave_tot[kSelWaves];
     double wave_sum[2][kSelWaves];
     int last;
@@ -136,16 +138,6 @@ template <int CTRL> __device__ __forceinline__ uint32_t dpp_u32(uint32_t v)
 {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
 }
-// largest value over the wave, the same in every lane
-__device__ __forceinline__ uint32_t wave_max(uint32_t v)
-{
-    v = max(v, dpp_u32<0xB1>(v));    // quad_perm [1,0,3,2]
-    v = max(v, dpp_u32<0x4E>(v));    // quad_perm [2,3,0,1]
-    v = max(v, dpp_u32<0x141>(v));   // row_half_mirror
-    v = max(v, dpp_u32<0x140>(v));   // row_mirror
-    auto row = [&](int l) __attribute__((always_inline)) { return (uint32_t)__builtin_amdgcn_readlane((int)v, l); };
-    return max(max(row(0), row(16)), max(row(32), row(48)));
-}
 // sum over the lanes below and this one (DPP row shifts, the row totals through scalar registers)
 __device__ __forceinline__ int wave_incl_sum(int v, int lane)
 {
@@ -158,79 +150,62 @@ __device__ __forceinline__ int wave_incl_sum(int v, int lane)
     return v + (row >= 1 ? t0 : 0) + (row >= 2 ? t1 : 0) + (row >= 3 ? t2 : 0);
 }
 
-// The same key for a row of finite scores that every thread holds KPT of (index tid + 1024 u < I), by VALUE: 2048 equal
-// intervals between the row's smallest and largest score put a few scores into each (the top digit of the keys, sign and
-// exponent, takes a handful of values only), one histogram finds the interval that holds the k-th largest, and every wave
-// ranks what lies in it.  The map to intervals is monotone in the score, rounding included, so greater intervals hold
-// greater scores.  Five barriers, where two digits and a ranking take eleven.  False (uniform): no interval of at most 64
-// scores, or a range that the map does not take (infinities, NaN, all scores equal): radix_select_desc does those.
-// Predictor and selection, one row, replayed, by the digits / so: 30 % of 8192 (rank 128) 11.6 / 10.9 us, of 14336 (rank 256)
-// 15.9 / 15.0.
+// The same for a row that every thread holds KPT keys of (index tid + 1024 u < I), by digits of 10 bits: the first is sign,
+// exponent and one bit of the mantissa, and a second one mostly leaves few enough to rank, which every wave does for itself.
+// What bounds it is the chain of barriers (eight; eleven with 8-bit digits, a sum of the counters by some waves and a ranking
+// by one) and, where many keys share a digit, the counters' addresses: lanes that share one take turns.  Top-k, 30 % of a row,
+// replayed, us, 8-bit digits / so: normal scores, 8192 6.80 / 6.40, 14336 9.28 / 8.24, four rows of 8192 8.80 / 8.41; of 14336, log-normal
+// 9.13 / 8.16, one score of 1e4 among normal ones 9.27 / 8.20, half of them zero 9.33 / 8.96, 60 % filled with -1e4 9.21 / 9.14.
+// Built and taken back: 2048 equal intervals of value between the row's ends, one histogram, the digits where more than 64
+// scores share the interval: normal 8192 5.50, 14336 8.64, but 14336 log-normal 18.6, one score of 1e4 20.2, of 30 12.2.  11-bit
+// digits of four counters each: normal 6.02 / 8.07, 60 % filled 10.1.
 template <int KPT>
-__device__ __forceinline__ bool value_select_desc(const float (&v)[KPT], int I, uint32_t k, SelShared &sh, int tid,
-                                                  uint32_t &kth_out, uint32_t &rem_out, uint32_t &cnt_out)
+__device__ __forceinline__ uint32_t key_select_desc(const uint32_t (&key)[KPT], int I, uint32_t k, uint32_t *hist, SelShared &sh,
+                                                    int tid, uint32_t &rem_out, uint32_t &cnt_out)
 {
-    constexpr int kBins = 256 * kHistCopies;
-    static_assert(kBins == 2 * kSelThreads, "two intervals per thread");
-    const int lane = tid & (kWave - 1), wave = tid >> 6;
-    sh.hist[tid] = 0u;
-    sh.hist[tid + kSelThreads] = 0u;
+    static_assert(kKeyDigits == kSelThreads, "one digit per thread");
+    const int lane = tid & (kWave - 1), wave = tid >> 6, mine_at = (tid & (kKeyCopies - 1)) * kKeyPitch;
+    auto own = [&](int c) __attribute__((always_inline)) -> uint32_t & { return hist[c * kKeyPitch + tid]; };
+#pragma unroll
+    for (int c = 0; c < kKeyCopies; ++c) own(c) = 0u;
     if (tid == 0) sh.ncand = 0u;
-    uint32_t hi = 0u, nlo = 0u;   // largest key, complement of the smallest
+    __syncthreads();
+    uint32_t prefix = 0u, pmask = 0u, rem = k, cnt = (uint32_t)I;
+#pragma unroll 1
+    for (int shift = 22;; shift = shift > 10 ? shift - 10 : 0) {
+        const uint32_t digits = shift ? kKeyDigits - 1 : 3u;
 #pragma unroll
-    for (int u = 0; u < KPT; ++u)
-        if (tid + u * kSelThreads < I) {
-            const uint32_t kv = order_key(v[u]);
-            hi = max(hi, kv);
-            nlo = max(nlo, ~kv);
+        for (int u = 0; u < KPT; ++u)
+            if (tid + u * kSelThreads < I && (key[u] & pmask) == prefix) atomicAdd(&hist[((key[u] >> shift) & digits) + mine_at], 1u);
+        __syncthreads();
+        uint32_t mine = 0u;
+#pragma unroll
+        for (int c = 0; c < kKeyCopies; ++c) mine += own(c);
+#pragma unroll
+        for (int c = 0; c < kKeyCopies; ++c) own(c) = 0u;
+        const int incl = wave_incl_sum((int)mine, lane);
+        if (lane == kWave - 1) sh.wave_tot[wave] = incl;
+        __syncthreads();
+        int upto = incl;   // keys with this thread's digit and the lower ones
+#pragma unroll
+        for (int w = 0; w < kSelWaves; ++w) upto += w < wave ? sh.wave_tot[w] : 0;
+        const uint32_t above = cnt - (uint32_t)upto;
+        if (above < rem && rem <= above + mine) { sh.digit = (uint32_t)tid; sh.rem = rem - above; sh.cnt = mine; }
+        __syncthreads();
+        prefix |= sh.digit << shift;
+        pmask |= digits << shift;
+        rem = sh.rem;
+        cnt = (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.cnt);
+        if (shift == 0) {
+            rem_out = rem;
+            cnt_out = cnt;
+            return prefix;
         }
-    hi = wave_max(hi);
-    nlo = wave_max(nlo);
-    if (lane == 0) { sh.wave_hi[wave] = hi; sh.wave_lo[wave] = nlo; }
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < kSelWaves; w += 4) {
-        const uint4 a = *reinterpret_cast<const uint4 *>(&sh.wave_hi[w]), c = *reinterpret_cast<const uint4 *>(&sh.wave_lo[w]);
-        hi = max(hi, max(max(a.x, a.y), max(a.z, a.w)));
-        nlo = max(nlo, max(max(c.x, c.y), max(c.z, c.w)));
+        if (cnt <= (uint32_t)kWave) break;
     }
-    hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)hi);
-    const uint32_t lo = ~(uint32_t)__builtin_amdgcn_readfirstlane((int)nlo);
-    const float flo = key_value(lo), range = key_value(hi) - flo;
-    if (hi > order_key(3.402823466e38f) || lo < order_key(-3.402823466e38f) || !(range >= 1e-30f && range <= 1e38f)) return false;
-    const float scale = (float)(kBins - 1) / range;
-    auto interval = [&](float f) __attribute__((always_inline)) {
-        const int b = (int)((f - flo) * scale);
-        return b < kBins ? b : kBins - 1;
-    };
-    int at[KPT];
-#pragma unroll
-    for (int u = 0; u < KPT; ++u) {
-        at[u] = interval(v[u]);
-        if (tid + u * kSelThreads < I) atomicAdd(&sh.hist[at[u]], 1u);
-    }
-    __syncthreads();
-    const uint2 c2 = *reinterpret_cast<const uint2 *>(&sh.hist[2 * tid]);
-    const int incl = wave_incl_sum((int)(c2.x + c2.y), lane);
-    if (lane == kWave - 1) sh.wave_tot[wave] = incl;
-    __syncthreads();
-    int upto = incl;   // scores in this thread's intervals and the lower ones
-#pragma unroll
-    for (int w = 0; w < kSelWaves; ++w) upto += w < wave ? sh.wave_tot[w] : 0;
-    uint32_t above = (uint32_t)(I - upto);
-#pragma unroll
-    for (int j = 1; j >= 0; --j) {
-        const uint32_t c = j ? c2.y : c2.x;
-        if (above < k && k <= above + c) { sh.digit = (uint32_t)(2 * tid + j); sh.rem = k - above; sh.cnt = c; }
-        above += c;
-    }
-    __syncthreads();
-    const int bin = (int)sh.digit;
-    const uint32_t rem = sh.rem, cnt = (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.cnt);
-    if (cnt > (uint32_t)kWave) return false;
 #pragma unroll
     for (int u = 0; u < KPT; ++u)
-        if (tid + u * kSelThreads < I && at[u] == bin) sh.cand[atomicAdd(&sh.ncand, 1u)] = order_key(v[u]);
+        if (tid + u * kSelThreads < I && (key[u] & pmask) == prefix) sh.cand[atomicAdd(&sh.ncand, 1u)] = key[u];
     __syncthreads();
     const uint32_t mine = (uint32_t)lane < cnt ? sh.cand[lane] : 0u;
     uint32_t greater = 0u, equal = 0u;
@@ -241,10 +216,9 @@ __device__ __forceinline__ bool value_select_desc(const float (&v)[KPT], int I, 
     }
     const uint64_t is = __builtin_amdgcn_ballot_w64((uint32_t)lane < cnt && greater < rem && rem <= greater + equal);
     const int l = __builtin_ctzll(is);   // (lanes that agree hold the same)
-    kth_out = (uint32_t)__builtin_amdgcn_readlane((int)mine, l);
     rem_out = rem - (uint32_t)__builtin_amdgcn_readlane((int)greater, l);
     cnt_out = (uint32_t)__builtin_amdgcn_readlane((int)equal, l);
-    return true;
+    return (uint32_t)__builtin_amdgcn_readlane((int)mine, l);
 }
 
 template <int CTRL> __device__ __forceinline__ double dpp_add_f64(double v)
@@ -313,8 +287,8 @@ __device__ __forceinline__ int block_excl_count(int v, SelShared &sh, int tid)
 // row in index order.  KPT == 0: rows of any length, every pass reads the keys from LDS (`in_lds`) or the
 // scores again from memory.
 // `into`: the mask holds zeros and the rows' blocks only set what they select, so that nothing is left to unite.  Predictor and
-// selection, replayed, the blocks' row masks united by the last one / so (and by value): top-k, four rows of 8192 15.4 / 12.8 us,
-// sixteen of 14336 24.5 / 19.7; statistical 12.7 / 10.6 and 20.2 / 16.2.
+// selection, replayed, the blocks' row masks united by the last one (and by 8-bit digits) / so: top-k, four rows of 8192 15.1 / 12.8
+// us, sixteen of 14336 24.2 / 19.4; statistical 12.5 / 10.4 and 19.9 / 16.0.
 template <int KPT>
 __global__ __launch_bounds__(kSelThreads) void mask_select_kernel(const float *__restrict__ scores,
                                                                   uint8_t *__restrict__ mask,
@@ -369,12 +343,14 @@ __global__ __launch_bounds__(kSelThreads) void mask_select_kernel(const float *_
                 each([&](int, float f) { fn(order_key(f)); });
             };
             uint32_t rem = 0u, cnt = 0u, kth = 0u;
-            bool found = false;
             if constexpr (KPT > 0) {
-                found = value_select_desc<KPT>(v, I, k, sh, tid, kth, rem, cnt);
-                if (!found) __syncthreads();   // (its readers of the shared words are done)
+                uint32_t key[KPT];
+#pragma unroll
+                for (int u = 0; u < KPT; ++u) key[u] = order_key(v[u]);
+                kth = key_select_desc<KPT>(key, I, k, keys, sh, tid, rem, cnt);
+            } else {
+                kth = radix_select_desc(sweep, k, sh, tid, rem, cnt);
             }
-            if (!found) kth = radix_select_desc(sweep, k, sh, tid, rem, cnt);
             if (cutoff && tid == 0) cutoff[b] = key_value(kth);
             if (rem == cnt) {  // every score equal to the k-th belongs to the k largest
                 each([&](int i, float f) { put(i, order_key(f) >= kth); });
@@ -621,10 +597,11 @@ extern "C" int st_mask_select(const float *scores, int64_t B, int64_t I, int met
     ProfScope ps(ST_K_MASK_SELECT, s);
     const dim3 grid((unsigned)B), block(kSelThreads);
 #define ST_SELECT_ARGS(in_lds) scores, mask, rowmask, cutoff, ticket, (int)B, (int)I, ldm, method | ((in_lds) << 8) | (into << 9), (long)k, z
+    const size_t lds = (size_t)I * 4 > kKeyHistBytes ? (size_t)I * 4 : kKeyHistBytes;   // keys, or the histogram before them
     if (I <= 8 * kSelThreads)
-        ST_LAUNCH(ps, (mask_select_kernel<8>), grid, block, (size_t)I * 4, s, ST_SELECT_ARGS(1));
+        ST_LAUNCH(ps, (mask_select_kernel<8>), grid, block, lds, s, ST_SELECT_ARGS(1));
     else if (I <= 16 * kSelThreads)
-        ST_LAUNCH(ps, (mask_select_kernel<16>), grid, block, (size_t)I * 4, s, ST_SELECT_ARGS(1));
+        ST_LAUNCH(ps, (mask_select_kernel<16>), grid, block, lds, s, ST_SELECT_ARGS(1));
     else if (I <= kSelMaxLdsKeys)
         ST_LAUNCH(ps, (mask_select_kernel<0>), grid, block, (size_t)I * 4, s, ST_SELECT_ARGS(1));
     else

@@ -96,9 +96,8 @@ def test_statistical_against_oracle(B, I, kind, z):
     (2, 5000, "nan"), (2, 3000, "lowest"), (4, 4096, "constant"), (2, 4096, "steps"),
 ])
 def test_selection_by_value_and_into_zeros(B, I, kind):
-    """The selection by intervals of the value where it applies and where it hands over to the digits (an interval with more than 64
-    scores, one score far out, infinities, NaN, the lowest of the type, all scores equal), at the edges of the row lengths;
-    into a mask of zeros like into any other.  Top-k bit for bit; NaN ranks as its bits do, above infinity."""
+    """Scores that lie close together, one far out, infinities, NaN, the lowest of the type, all scores equal, at the edges of the row
+    lengths; into a mask of zeros like into any other.  Top-k bit for bit; NaN ranks as its bits do, above infinity."""
     s = _scores(B * 7 + I, B, I, kind)
     if kind == "outlier":
         s[:, 17] = 3e37
@@ -131,6 +130,24 @@ def test_selection_by_value_and_into_zeros(B, I, kind):
             assert np.array_equal(a.cpu().numpy()[sure], (d > cut).any(0)[sure])
     with pytest.raises(ValueError):
         st.mask_select(sd, "topk", k=1, into_zeros=True)
+
+
+@pytest.mark.parametrize("B,I", [(1, 65), (2, 1023), (1, 1024), (3, 8191), (1, 8192), (2, 8193), (1, 16384)])
+@pytest.mark.parametrize("bits", [0, 2, 9, 10, 12, 20, 22, 31])
+def test_topk_digits(B, I, bits):
+    """Keys that agree in all but their last `bits` bits and fill those, so that the digits above leave everything and each level
+    of the select decides; more and fewer than 64 of a value, the first and the last of the row, cuts at 64 and 65 of a digit."""
+    rng = np.random.default_rng(I + bits)
+    key = (np.uint32(0x40500000) >> np.uint32(bits) << np.uint32(bits)) | rng.integers(0, 1 << bits, size=(B, I), dtype=np.uint32)
+    s = key.view(np.float32)
+    s = np.where(np.isfinite(s), s, np.float32(1.0))
+    if bits == 31:
+        s[:, ::2] *= np.float32(-1.0)
+    sd = torch.from_numpy(s).to(DEV)
+    for k in sorted({1, 2, 64, 65, I // 2, I - 64, I - 1} & set(range(1, I))):
+        got, cut = st.mask_select(sd, "topk", k=k, return_cutoff=True)
+        assert np.array_equal(got.cpu().numpy(), oracle.mask_topk(s, k)), k
+        assert np.array_equal(cut.cpu().numpy(), -np.sort(-s, axis=1)[:, k - 1]), k
 
 
 def test_mask_select_errors():
