@@ -375,15 +375,21 @@ __global__ __launch_bounds__(kSelThreads) void mask_select_kernel(const float *_
             }
         }
     } else {
-        // sums of the scores' distances from the row's first one, and of their squares, in one sweep: the variance's
-        // cancellation is at most that distance's square against it, a factor of I, of doubles
+        // sums of the scores' distances from the row's first one, and of their squares, in one sweep.  Where that score lies more
+        // than eight deviations out the differences below cancel (by up to I); such rows are summed again, plainly
         const double first = (double)row[0];
         double s = 0.0, q = 0.0;
         each([&](int, float f) { const double d = (double)f - first; s += d; q += d * d; });
         block_sums(s, q, sh, tid);
-        const double off = s / (double)I, mean = first + off;
-        double var = q / (double)I - off * off;
-        var = var < 0.0 ? 0.0 : var;
+        const double off = s / (double)I;
+        double mean = first + off, var = q / (double)I - off * off;
+        if (off * off > 64.0 * var) {   // (uniform: every thread has the same sums)
+            s = q = 0.0;
+            each([&](int, float f) { s += (double)f; });
+            mean = block_sum(s, sh, tid) / (double)I;
+            each([&](int, float f) { const double d = (double)f - mean; q += d * d; });
+            var = block_sum(q, sh, tid) / (double)I;
+        }
         const float cut = (float)mean + (float)sqrt(var) * z;
         if (cutoff && tid == 0) cutoff[b] = cut;
         each([&](int i, float f) { put(i, f > cut); });

@@ -3,8 +3,11 @@ threshold, against the oracle.  Top-k and the sketch threshold involve only comp
 match bit for bit, ties included; the statistical cut is a floating-point sum, so mask bits are compared
 outside a guard band around the cut that is much wider than the rounding difference (and asserted small)."""
 import base64
+import decimal
 import json
+import math
 import os
+from fractions import Fraction
 
 import numpy as np
 import pytest
@@ -130,6 +133,28 @@ def test_selection_by_value_and_into_zeros(B, I, kind):
             assert np.array_equal(a.cpu().numpy()[sure], (d > cut).any(0)[sure])
     with pytest.raises(ValueError):
         st.mask_select(sd, "topk", k=1, into_zeros=True)
+
+
+def test_statistical_cut_with_the_first_score_far_out():
+    """A row's first score thousands of deviations from the others: the cut is the float32 of the sums' 50 digits at every value
+    of it (a variance taken from sums about that score loses a factor of I of a double's bits)."""
+    I = 1 << 22
+    rest = np.random.default_rng(5).standard_normal(I - 1).astype(np.float32)
+    d = rest.astype(np.float64)                          # (squares of 24 bits are exact)
+    S, Q = Fraction(math.fsum(d)), Fraction(math.fsum(d * d))
+    row = torch.from_numpy(np.concatenate([np.zeros(1, np.float32), rest])).to(DEV)[None]
+    wrong = []
+    for f in np.linspace(9000, 11000, 600).astype(np.float32):
+        row[0, 0] = float(f)
+        _, cut = st.mask_select(row, "statistical_topk", std_multiplier=1.0, return_cutoff=True)
+        mean = (S + Fraction(float(f))) / I
+        var = (Q + Fraction(float(f)) ** 2) / I - mean ** 2
+        with decimal.localcontext() as ctx:
+            ctx.prec = 50
+            std = float((decimal.Decimal(var.numerator) / decimal.Decimal(var.denominator)).sqrt())
+        if np.float32(cut.item()) != np.float32(float(mean)) + np.float32(std):
+            wrong.append(float(f))
+    assert not wrong, (len(wrong), wrong[:4])
 
 
 @pytest.mark.parametrize("B,I", [(1, 65), (2, 1023), (1, 1024), (3, 8191), (1, 8192), (2, 8193), (1, 16384)])
