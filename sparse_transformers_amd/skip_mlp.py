@@ -65,7 +65,8 @@ class FastLoRAProjection:
         ``naive`` (score >= 0) and ``threshold`` (score >= thr, or > thr) are fused into the predictor
         kernel.  ``topk`` and ``statistical_topk`` need a statistic of the whole row: the predictor kernel
         leaves its fp32 scores and a selection kernel (one block per row) finishes.  ``scores_ws`` (float32,
-        B*I elements) and ``out`` make the call allocation-free.
+        B*I elements), ``t_ws`` (with it) and ``out`` make the call allocation-free.  Without ``scores_ws`` the scores are
+        ``self.forward``'s, where that is not this class's own, and ``select_ws`` unites their rows; no other call needs it.
         """
         if method == "naive":
             return predictor_mask(x, self.down_weight, self.up_weight, 0.0, True, out=out, t_ws=t_ws,
@@ -75,11 +76,13 @@ class FastLoRAProjection:
                                   round_to_storage=self.round_to_storage)
         if method not in ("topk", "statistical_topk"):
             raise ValueError(f"unknown sparsity method {method!r}")
-        if type(self).forward is not FastLoRAProjection.forward:   # scores of a subclass's own
+        if scores_ws is None and getattr(self.forward, "__func__", None) is not FastLoRAProjection.forward:
+            # scores of a subclass's or an instance's own
             return mask_select(self.forward(x), method, k=k, std_multiplier=std_multiplier, out=out, workspace=select_ws)
         # no score is above infinity: the mask comes back as the zeros that the selection then sets its bytes in
         mask, scores = predictor_mask(x, self.down_weight, self.up_weight, float("inf"), False, return_scores=True, out=out,
-                                      t_ws=t_ws, scores_out=scores_ws, round_to_storage=self.round_to_storage)
+                                      t_ws=t_ws if scores_ws is not None else None, scores_out=scores_ws,
+                                      round_to_storage=self.round_to_storage)
         return mask_select(scores, method, k=k, std_multiplier=std_multiplier, out=mask, into_zeros=True)
 
 

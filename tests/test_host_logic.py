@@ -367,3 +367,27 @@ def test_surplus_removal_tail_only_form():
         worst = max(worst, rounds)
         assert got == want, (trial, order, removed, added)
     assert worst >= 3      # the cases did reach chains of dependent surplus indices
+
+
+def test_row_statistic_masks_take_an_own_forward(monkeypatch):
+    """FastLoRAProjection.mask: scores of a ``forward`` set on the instance or by a subclass are the ones selected from, except with a
+    caller's scores buffer, which the kernels fill; a ``t_ws`` is looked at with that buffer only."""
+    from sparse_transformers_amd import skip_mlp
+
+    seen = []
+    monkeypatch.setattr(skip_mlp, "mask_select", lambda scores, method, **kw: seen.append((scores, kw.get("workspace"))))
+    monkeypatch.setattr(skip_mlp, "predictor_mask", lambda *a, **kw: ("zeros", ("kernel", kw["t_ws"], kw["scores_out"])))
+
+    class Own(skip_mlp.FastLoRAProjection):
+        def forward(self, x):
+            return "subclass"
+
+    weights = torch.zeros(2, 8), torch.zeros(16, 2)
+    plain, own, instance = skip_mlp.FastLoRAProjection(*weights), Own(*weights), skip_mlp.FastLoRAProjection(*weights)
+    instance.forward = lambda x: "instance"
+    for p, want in ((plain, ("kernel", None, None)), (own, "subclass"), (instance, "instance")):
+        for method in ("topk", "statistical_topk"):
+            p.mask(None, method, k=3, t_ws="t", select_ws="ws")
+            assert seen.pop() == (want, "ws" if isinstance(want, str) else None)
+            p.mask(None, method, k=3, t_ws="t", scores_ws="buffer", select_ws="ws")
+            assert seen.pop()[0] == ("kernel", "t", "buffer")
