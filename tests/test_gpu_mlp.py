@@ -2,6 +2,10 @@
 
 Tolerances (north star): fp32 1e-5 relative; fp16 / bf16 2e-2 absolute, 1e-2 relative, against an fp32
 evaluation of the dtype-rounded weights and inputs."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -13,6 +17,7 @@ from conftest import assert_close
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def _case(seed, B, H, n, dtype, has_gate, std=0.02, lead_shape=None):
@@ -732,3 +737,33 @@ def test_sums_of_splits(B, H, n, dtype):
     torch.cuda.synchronize()
     assert_close(out.float().cpu().numpy(), (h @ dn.double()).cpu().numpy(), dtype, "out")
     assert bool(torch.isnan(store[0]))
+
+
+def test_batch_kernels_can_be_switched_off():
+    """ST_MLP_BATCH_MIN above 32: no row count takes the batch kernels or their workspace (the variable is read once per process)."""
+    script = """
+import ctypes as C, torch
+from sparse_transformers_amd import _lib
+from sparse_transformers_amd.ops import mlp_forward_rows
+L = _lib.lib()
+for dtype, B, H in ((torch.float32, 33, 256), (torch.float32, 6, 2048), (torch.float16, 40, 192), (torch.float16, 16, 2048), (torch.float16, 40, 256)):
+    w = [torch.randn(300, H, device="cuda").to(dtype) * 0.05 for _ in range(3)]
+    x = torch.randn(B, H, device="cuda").to(dtype)
+    kinds, ms = (C.c_int32 * 64)(), (C.c_float * 64)()
+    _lib.check(L.st_profile_enable(64), "st_profile_enable")
+    mlp_forward_rows(x, *w, 300, None, torch.empty_like(x), None, "silu", True)
+    torch.cuda.synchronize()
+    names = {_lib.KERNEL_KINDS[kinds[i]] for i in range(L.st_profile_collect(kinds, ms, 64))}
+    L.st_profile_disable()
+    print("CALL", any("batch" in n for n in names), any("prefill" in n for n in names), L.st_mlp_workspace_bytes(40, 64, 16384))
+"""
+    lines = {}
+    for value in ("33", "40", "3"):
+        p = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, timeout=100,
+                           env={**os.environ, "ST_MLP_BATCH_MIN": value, "PYTHONPATH": ROOT}, cwd=ROOT)
+        assert p.returncode == 0, p.stderr[-2000:]
+        lines[value] = [l.split()[1:] for l in p.stdout.splitlines() if l.startswith("CALL")]
+    for value in ("33", "40"):
+        assert [l[:2] for l in lines[value]] == [["False", "False"]] * 4 + [["False", "True"]], lines
+        assert lines[value][0][2] < lines["3"][0][2]
+    assert [l[0] for l in lines["3"]] == ["True"] * 4 + ["False"], lines
