@@ -282,7 +282,8 @@ int st_cache_sync_state(st_cache *c, int32_t *state_out, void *stream);
  * updated cache -- weight_cache.h:229-359 then sparse_mlp_op.cpp:53-192 /
  * src/modeling_skip.py:114-117, i.e. what SkipDecoderLayer.forward does per
  * layer (src/modeling_skip.py:234-261) -- enqueued as one call.  For B <= 2
- * (16-byte aligned rows, 8 <= I <= 16384) this is
+ * (16-byte aligned rows, 8 <= I <= 16384; two rows of matrices up to 16 MiB only
+ * with I % 8 == 0 and an 8-byte aligned mask) this is
  * ONE kernel in which every block works out where the rows of the positions
  * it owns come from and streams them, taking rows whose index changed from
  * the pool and writing them back on the way; otherwise it is

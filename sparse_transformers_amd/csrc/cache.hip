@@ -137,39 +137,48 @@ __device__ __forceinline__ uint32_t pack_bits8(uint64_t ones)
     return (uint32_t)((ones * 0x0102040810204080ull) >> 56);
 }
 
-// Eight bytes of a mask and four entries of an index list at any alignment: sizes that are no multiples of eight put the second
-// half of the double buffers, and the masks of a stack's layers, anywhere.  (The loads are the same instructions.)  The last
-// word of such a mask, or the last vector of a list, is the one that ends with it; mask_tail and list_tail shift its first
-// elements down, at the place of use: shifted where it is loaded, the load would be waited for there.  I >= 8; what lies
-// past I reads as zero in a mask and as anything in a list.  I 3405, H 896, bf16, eight rows, a stack of four layers: 86 us with
-// the updates byte by byte, layer by layer; 70 so, in one launch.  One or two rows of x also get the fused kernel.
-__device__ __forceinline__ uint64_t load_mask(const uint8_t *m, int e, int I)
+// Eight bytes of a mask and four entries of an index list.  AL: the size is a multiple of eight and the buffers are aligned for
+// words.  Otherwise at any alignment: sizes that are no multiples of eight put the second half of the double buffers, and the
+// masks of a stack's layers, anywhere.  (The loads are the same instructions.)  The last word of such a mask, or the last
+// vector of a list, is the one that ends with it; mask_tail and list_tail shift its first elements down, at the place of use:
+// shifted where it is loaded, the load would be waited for there.  I >= 8; what lies past I reads as zero in a mask and as
+// anything in a list.  I 3405, H 896, bf16, eight rows, a stack of four layers: 86 us with the updates byte by byte, layer by
+// layer; 70 so, in one launch.  One or two rows of x also get the fused kernel.  With one form for both, which is a tenth more
+// code to fetch, aligned calls of that kernel were slower: H 896, I 2688, bf16, one / two rows 13.9 / 18.4 us, and
+// 14.1 / 18.9 so.
+template <bool AL> __device__ __forceinline__ uint64_t load_mask(const uint8_t *m, int e, int I)
 {
+    if constexpr (AL) return *reinterpret_cast<const uint64_t *>(m + e);
     uint64_t v;
     __builtin_memcpy(&v, m + (e < I - 8 ? e : I - 8), 8);
     return v;
 }
-__device__ __forceinline__ uint64_t mask_tail(uint64_t v, int e, int I)
+template <bool AL> __device__ __forceinline__ uint64_t mask_tail(uint64_t v, int e, int I)
 {
+    if constexpr (AL) return v;
     const int over = e + 8 - I;   // (words past the end, all of whose elements are, come out as anything)
     return v >> (8 * (over > 0 ? over : 0) & 63);
 }
-__device__ __forceinline__ void store_mask(uint8_t *m, int e, int I, uint64_t v)
+template <bool AL> __device__ __forceinline__ void store_mask(uint8_t *m, int e, int I, uint64_t v)
 {
-    if (e + 8 <= I) {
+    if constexpr (AL) {
+        *reinterpret_cast<uint64_t *>(m + e) = v;
+    } else if (e + 8 <= I) {
         __builtin_memcpy(m + e, &v, 8);
     } else {
         for (int k = 0; k < I - e; ++k) m[e + k] = (uint8_t)(v >> (8 * k));
     }
 }
 typedef int list4_t __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ int4 load_list(const int32_t *l, int p, int I)
+template <bool AL> __device__ __forceinline__ int4 load_list(const int32_t *l, int p, int I)
 {
+    if constexpr (AL) return *reinterpret_cast<const int4 *>(l + p);
     const list4_t v = *reinterpret_cast<const list4_t *>(l + (p < I - 4 ? p : I - 4));
     return make_int4(v.x, v.y, v.z, v.w);
 }
-__device__ __forceinline__ int4 list_tail(int4 c, int p, int I)
+template <bool AL> __device__ __forceinline__ int4 list_tail(int4 c, int p, int I)
 {
+    if constexpr (AL) return c;
     if (I & 3) {   // uniform
         const int over = p + 4 - I;
         const bool one = over > 0 && (over & 1), two = over > 0 && (over & 2);
@@ -266,12 +275,12 @@ __device__ __forceinline__ void surplus_ends(P place, Q stays, int base, int n, 
 // contains block barriers.  VEC (I >= 8): masks are read as 8-byte words and indices as 16-byte vectors; both bookkeeping
 // buffers are requested together with the ticket, so the front costs one memory round trip.  MARK: the
 // dirty bitmap is kept on the fast path too.
-// NW: 8-element words per thread of the vector path (I <= 8 NW threads); the registers of the front loads follow from it.
+// NW: 8-element words per thread of the vector path (I <= 8 NW threads); the registers of the front loads follow from it.  AL: as above.
 //
 // Barrier sequence: 1 after the LDS fill; 2 in the diff scan;
 // [unchanged mask: done]; 1 after the lists; 1 after phases 1 and 2; [surplus removals: those of surplus_count and surplus_ends and 1
 // behind it, 2 in the compaction scan, 1 after the compaction].
-template <bool VEC, int PT, int NW, bool MARK>
+template <bool VEC, int PT, int NW, bool MARK, bool AL>
 __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, PlanShared *ps,
                                            const uint8_t *__restrict__ new_mask, uint8_t *__restrict__ cur_mask2,
                                            int32_t *__restrict__ indices2, int32_t *__restrict__ state, int I,
@@ -279,11 +288,12 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
 {
     constexpr int TPB = PT;
     uint16_t *pos_l = reinterpret_cast<uint16_t *>(smem);  // index -> position
-    uint16_t *idx_l = pos_l + ((I + 7) & ~7);              // position -> index
+    const int span = AL ? I : (I + 7) & ~7;                // (the last words and vectors are written whole)
+    uint16_t *idx_l = pos_l + span;                        // position -> index
     // added indices ascending from the front, removed indices ascending from the
     // back (k-th removed at lists[I-1-k]); the two never meet: na + nr <= I.
     // After the plan the same array holds the positions to rewrite.
-    uint16_t *lists = idx_l + ((I + 7) & ~7);
+    uint16_t *lists = idx_l + span;
     uint32_t *dirty = reinterpret_cast<uint32_t *>(lists + I + (I & 1));  // bit per position
     const int dirty_words = (I + 31) >> 5;
     uint8_t *flag_l = reinterpret_cast<uint8_t *>(dirty + ((dirty_words + 1) & ~1));  // bit0 new, bit1 old; 8-byte aligned
@@ -315,13 +325,13 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
         for (int w = 0; w < NW; ++w) {
             const int e = e0 + 8 * w;
             if (e < e1) {
-                v_new[w] = load_mask(new_mask, e, I);
-                v_cur0[w] = load_mask(cur_mask2, e, I);
-                v_cur1[w] = load_mask(cur_mask2 + I, e, I);
-                v_i0a[w] = load_list(indices2, e, I);
-                v_i0b[w] = load_list(indices2, e + 4, I);
-                v_i1a[w] = load_list(indices2 + I, e, I);
-                v_i1b[w] = load_list(indices2 + I, e + 4, I);
+                v_new[w] = load_mask<AL>(new_mask, e, I);
+                v_cur0[w] = load_mask<AL>(cur_mask2, e, I);
+                v_cur1[w] = load_mask<AL>(cur_mask2 + I, e, I);
+                v_i0a[w] = load_list<AL>(indices2, e, I);
+                v_i0b[w] = load_list<AL>(indices2, e + 4, I);
+                v_i1a[w] = load_list<AL>(indices2 + I, e, I);
+                v_i1b[w] = load_list<AL>(indices2 + I, e + 4, I);
             }
         }
         n_both[0] = state[ST_STATE_N_BUF0];
@@ -342,9 +352,9 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
             const int e = e0 + 8 * w;
             w_new[w] = w_cur[w] = 0;
             if (e < e1) {
-                w_new[w] = nonzero_bytes(mask_tail(v_new[w], e, I));
-                w_cur[w] = nonzero_bytes(mask_tail(ep ? v_cur1[w] : v_cur0[w], e, I));
-                const int4 a = list_tail(ep ? v_i1a[w] : v_i0a[w], e, I), b4 = list_tail(ep ? v_i1b[w] : v_i0b[w], e + 4, I);
+                w_new[w] = nonzero_bytes(mask_tail<AL>(v_new[w], e, I));
+                w_cur[w] = nonzero_bytes(mask_tail<AL>(ep ? v_cur1[w] : v_cur0[w], e, I));
+                const int4 a = list_tail<AL>(ep ? v_i1a[w] : v_i0a[w], e, I), b4 = list_tail<AL>(ep ? v_i1b[w] : v_i0b[w], e + 4, I);
                 uint4 packed;
                 packed.x = (uint32_t)(a.x & 0xffff) | ((uint32_t)a.y << 16);
                 packed.y = (uint32_t)(a.z & 0xffff) | ((uint32_t)a.w << 16);
@@ -510,7 +520,7 @@ __device__ __forceinline__ void cache_plan(PlanView &pv, unsigned char *smem, Pl
 #pragma unroll
             for (int w = 0; w < NW; ++w) {
                 const int e = e0 + 8 * w;
-                if (e < e1) store_mask(mask_out, e, I, n_new > 0 ? w_new[w] : w_cur[w]);
+                if (e < e1) store_mask<AL>(mask_out, e, I, n_new > 0 ? w_new[w] : w_cur[w]);
             }
         } else {
             for (int i = tid; i < I; i += TPB) mask_out[i] = n_new > 0 ? (flag_l[i] & 1) : (flag_l[i] >> 1);
@@ -650,7 +660,7 @@ constexpr size_t update_lds_bytes(int I)
 // barriers when removals do not outnumber additions.  Every block plans for itself (as a launch of its own the plan would
 // cost a kernel boundary) and copies its share of the items.
 // Masks in 8-byte words, lists in 16-byte vectors, at any alignment (I >= 8); I <= 8 NW TPB.
-template <int TPB, int NW, typename Tab>
+template <int TPB, int NW, typename Tab, bool AL>
 __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__restrict__ new_mask,
                                                            uint8_t *__restrict__ cur_mask2,
                                                            int32_t *__restrict__ indices2, int32_t *__restrict__ state,
@@ -689,17 +699,17 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
     uint64_t v_new[NW], v_cur0[NW], v_cur1[NW];
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-        const int e = 8 * (tid * words + w);
-        v_new[w] = load_mask(new_mask, e, I);
-        v_cur0[w] = load_mask(cur_mask2, e, I);
-        v_cur1[w] = load_mask(cur_mask2 + I, e, I);
+        const int e = !AL || (w < words && 8 * (tid * words + w) < I) ? 8 * (tid * words + w) : 0;
+        v_new[w] = load_mask<AL>(new_mask, e, I);
+        v_cur0[w] = load_mask<AL>(cur_mask2, e, I);
+        v_cur1[w] = load_mask<AL>(cur_mask2 + I, e, I);
     }
     int4 v_i0[NV], v_i1[NV];
 #pragma unroll
     for (int q = 0; q < NV; ++q) {
         const int p = 4 * (tid + TPB * q), pc = p < idx_cap ? p : 0;   // (idx_cap: a multiple of 8, or I)
-        v_i0[q] = load_list(indices2, pc, I);
-        v_i1[q] = load_list(indices2 + I, pc, I);
+        v_i0[q] = load_list<AL>(indices2, pc, I);
+        v_i1[q] = load_list<AL>(indices2 + I, pc, I);
     }
     const int n_buf0 = state[ST_STATE_N_BUF0], n_buf1 = state[ST_STATE_N_BUF1];
     const int serial_old = state[ST_STATE_SERIAL], valid_old = state[ST_STATE_VALID];
@@ -714,8 +724,8 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
     for (int w = 0; w < NW; ++w) {
         const int e = 8 * (tid * words + w);
         const bool in = w < words && e < I;
-        w_new[w] = in ? nonzero_bytes(mask_tail(v_new[w], e, I)) : 0ull;
-        w_cur[w] = in ? nonzero_bytes(mask_tail(ep ? v_cur1[w] : v_cur0[w], e, I)) : 0ull;
+        w_new[w] = in ? nonzero_bytes(mask_tail<AL>(v_new[w], e, I)) : 0ull;
+        w_cur[w] = in ? nonzero_bytes(mask_tail<AL>(ep ? v_cur1[w] : v_cur0[w], e, I)) : 0ull;
         cnt += (uint32_t)__popcll(w_new[w] & ~w_cur[w]) + ((uint32_t)__popcll(w_cur[w] & ~w_new[w]) << 16);
     }
     ST_TL(1);
@@ -781,8 +791,8 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
             const int p0 = 4 * (tid + TPB * q);
             int4 c = ep ? v_i1[q] : v_i0[q];
             if (n > idx_cap && p0 >= idx_cap && p0 < n)   // more positions in use than the caller expected (one more round trip)
-                c = load_list(indices2 + (size_t)ep * I, p0, I);
-            c = list_tail(c, p0, I);
+                c = load_list<AL>(indices2 + (size_t)ep * I, p0, I);
+            c = list_tail<AL>(c, p0, I);
             const int e4[4] = {c.x, c.y, c.z, c.w};
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
@@ -848,7 +858,7 @@ __global__ __launch_bounds__(TPB) void cache_update_kernel(const uint8_t *__rest
 #pragma unroll
             for (int w = 0; w < NW; ++w) {
                 const int e = 8 * (tid * words + w);
-                if (w < words && e < I) store_mask(mask_out, e, I, n_new > 0 ? w_new[w] : w_cur[w]);
+                if (w < words && e < I) store_mask<AL>(mask_out, e, I, n_new > 0 ? w_new[w] : w_cur[w]);
             }
             uint32_t mine = 0;
             if (S_all > 0)
@@ -898,7 +908,7 @@ __global__ __launch_bounds__(TPB) void cache_update_bytes_kernel(const uint8_t *
     __shared__ PlanShared ps;
     const int tid = threadIdx.x;
     PlanView pv;
-    cache_plan<false, TPB, 1, false>(pv, smem, &ps, new_mask, cur_mask2, indices2, state, I, tid);
+    cache_plan<false, TPB, 1, false, true>(pv, smem, &ps, new_mask, cur_mask2, indices2, state, I, tid);
     if (tid == 0 && pv.writer) tell_count(host, pv.n_new);
     if (pv.changed) {
         // (the index of a rewritten position, beside the position: the map of the plan is not needed any more)
@@ -946,7 +956,7 @@ struct SparseShared {
     int found, paired_tail, replay_ok, fast_ok, nchg;   // surplus removals (removed > added)
 };
 
-template <typename T, int RB, int TPB, int NB = 1, int NW = 1, int SPECN = RB / 2>
+template <typename T, int RB, int TPB, int NB, int NW, int SPECN, bool AL>
 __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
     const uint8_t *__restrict__ new_mask, uint8_t *__restrict__ cur_mask2, int32_t *__restrict__ indices2,
     int32_t *__restrict__ state, int I, int launch_word, const T *__restrict__ x, int H, int n_hint,
@@ -1002,10 +1012,10 @@ __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
     uint64_t v_new[NW], v_c0[NW], v_c1[NW];
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-        const int e = (tid * nw_rt + w) * 8;
-        v_new[w] = load_mask(new_mask, e, I);
-        v_c0[w] = load_mask(cur_mask2, e, I);
-        v_c1[w] = load_mask(cur_mask2 + I, e, I);
+        const int e = !AL || (tid * nw_rt + w) * 8 + 8 <= I ? (tid * nw_rt + w) * 8 : I - 8;
+        v_new[w] = load_mask<AL>(new_mask, e, I);
+        v_c0[w] = load_mask<AL>(cur_mask2, e, I);
+        v_c1[w] = load_mask<AL>(cur_mask2 + I, e, I);
     }
     // The plan is worked out by ONE wave, the last of the block (with 6 KB rows a wave that owns no columns), while
     // the others already request rows; its lanes own the block's positions.
@@ -1025,8 +1035,8 @@ __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
     const bool scan_in = scan_p + kSparseScan <= scan_cap;
     const int scan_pc = scan_in ? scan_p : 0;
     static_assert(kSparseScan == 4, "one 16-byte load per bookkeeping buffer");
-    const int4 sc0 = load_list(indices2, scan_pc, I);
-    const int4 sc1 = load_list(indices2 + I, scan_pc, I);
+    const int4 sc0 = load_list<AL>(indices2, scan_pc, I);
+    const int4 sc1 = load_list<AL>(indices2 + I, scan_pc, I);
     uint4 xr[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b)
@@ -1076,8 +1086,8 @@ __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
     for (int w = 0; w < NW; ++w) {
         const int bi = tid * nw_rt + w;            // byte of the bitmaps = elements [8 bi, 8 bi + 8)
         const bool in = w < nw_rt && bi * 8 < I;
-        w_new[w] = in ? nonzero_bytes(mask_tail(v_new[w], bi * 8, I)) : 0ull;
-        w_cur[w] = in ? nonzero_bytes(mask_tail(ep ? v_c1[w] : v_c0[w], bi * 8, I)) : 0ull;
+        w_new[w] = in ? nonzero_bytes(mask_tail<AL>(v_new[w], bi * 8, I)) : 0ull;
+        w_cur[w] = in ? nonzero_bytes(mask_tail<AL>(ep ? v_c1[w] : v_c0[w], bi * 8, I)) : 0ull;
         if (w < nw_rt && bi < W32 * 4) {
             reinterpret_cast<uint8_t *>(sh.newbits)[bi] = (uint8_t)pack_bits8(w_new[w]);
             reinterpret_cast<uint8_t *>(sh.oldbits)[bi] = (uint8_t)pack_bits8(w_cur[w]);
@@ -1491,7 +1501,7 @@ __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
             for (int w = 0; w < NW; ++w) {
                 const int bi = tid * nw_rt + w;
                 if (w < nw_rt && bi * 8 < I && (bi % G) == blk)
-                    store_mask(mask_out, bi * 8, I, n > 0 ? w_new[w] : w_cur[w]);
+                    store_mask<AL>(mask_out, bi * 8, I, n > 0 ? w_new[w] : w_cur[w]);
             }
             if (blk == 0 && arriver) {
                 state[ST_STATE_N_BUF0 + (ep ^ 1)] = n;
@@ -1518,7 +1528,7 @@ __global__ __launch_bounds__(TPB) void cache_sparse_decode_kernel(
     } else {
         // ---- too many surplus removals for the replay above: the per-index plan
         PlanView pv;
-        cache_plan<true, TPB, NW, true>(pv, smem, &plan_shared, new_mask, cur_mask2, indices2, state, I, tid);
+        cache_plan<true, TPB, NW, true, AL>(pv, smem, &plan_shared, new_mask, cur_mask2, indices2, state, I, tid);
         n = pv.n_new;
         if (plan_wave) {
             int s = -1;
@@ -2306,6 +2316,12 @@ static st::UpdateLayer update_layer(const st_cache *c, const uint8_t *mask)
     return y;
 }
 
+// Masks as 8-byte words, index lists as 16-byte vectors, with no rest?
+static bool update_is_aligned(const st_cache *c, const uint8_t *mask)
+{
+    return c->I % 8 == 0 && (uintptr_t)mask % 8 == 0 && (uintptr_t)c->b.cur_mask % 8 == 0 && (uintptr_t)c->b.indices % 16 == 0;
+}
+
 // The count an update last told the host, 0 if none has yet.  A guess: later updates may be on their way.
 static int seen_count(const st_cache *c) { return *const_cast<const volatile int32_t *>(&c->host->count); }
 
@@ -2333,6 +2349,8 @@ static int launch_update(st_cache *const *caches, const uint8_t *const *masks, i
         return v ? atoi(v) : 0;
     }();
     const bool words_fit = I >= 8;
+    bool aligned = true;
+    for (int l = 0; l < L; ++l) aligned = aligned && update_is_aligned(caches[l], masks[l]);
     // 512-thread blocks (ST_CACHE_TPB=512) leave room on the CU for a kernel of another stream, but
     // measure slower on their own; they cover I <= 12288.
     const bool small = L == 1 && want_tpb == 512 && words_fit && I <= 8 * 512 * 3;
@@ -2367,18 +2385,27 @@ static int launch_update(st_cache *const *caches, const uint8_t *const *masks, i
         const int most = device_cu_count() * 3 / 4;
         int grid = blocks ? blocks : device_cu_count() / L;
         grid = grid < 4 ? 4 : grid > most ? most : grid;
-        rc = words == 1   ? launch(cache_update_kernel<1024, 1, UpdateLayers>, grid, lds, idx_cap, cp, c->host, tab)
-             : words == 2 ? launch(cache_update_kernel<1024, 2, UpdateLayers>, grid, lds, idx_cap, cp, c->host, tab)
-                          : launch(cache_update_kernel<1024, 3, UpdateLayers>, grid, lds, idx_cap, cp, c->host, tab);
+        auto go = [&](auto al) -> int {
+            constexpr bool AL = decltype(al)::value;
+            return words == 1   ? launch(cache_update_kernel<1024, 1, UpdateLayers, AL>, grid, lds, idx_cap, cp, c->host, tab)
+                   : words == 2 ? launch(cache_update_kernel<1024, 2, UpdateLayers, AL>, grid, lds, idx_cap, cp, c->host, tab)
+                                : launch(cache_update_kernel<1024, 3, UpdateLayers, AL>, grid, lds, idx_cap, cp, c->host, tab);
+        };
+        rc = aligned ? go(std::true_type{}) : go(std::false_type{});
     } else {
         const int grid = blocks ? blocks : device_cu_count() * 3 / 4;   // (measured against 1/4, 3/8, 1/2 and all of the CUs)
         const size_t lds = update_lds_bytes(I);
         const int idx_cap = update_idx_cap(c);
-        rc = !words_fit   ? launch(cache_update_bytes_kernel<1024>, grid, plan_lds_bytes(I), cp, c->host)
-             : small      ? launch(cache_update_kernel<512, 3, NoLayers>, grid, lds, idx_cap, cp, c->host, NoLayers{})
-             : words == 1 ? launch(cache_update_kernel<1024, 1, NoLayers>, grid, lds, idx_cap, cp, c->host, NoLayers{})
-             : words == 2 ? launch(cache_update_kernel<1024, 2, NoLayers>, grid, lds, idx_cap, cp, c->host, NoLayers{})
-                          : launch(cache_update_kernel<1024, 3, NoLayers>, grid, lds, idx_cap, cp, c->host, NoLayers{});
+        auto go = [&](auto al) -> int {
+            constexpr bool AL = decltype(al)::value;
+            return small        ? launch(cache_update_kernel<512, 3, NoLayers, AL>, grid, lds, idx_cap, cp, c->host, NoLayers{})
+                   : words == 1 ? launch(cache_update_kernel<1024, 1, NoLayers, AL>, grid, lds, idx_cap, cp, c->host, NoLayers{})
+                   : words == 2 ? launch(cache_update_kernel<1024, 2, NoLayers, AL>, grid, lds, idx_cap, cp, c->host, NoLayers{})
+                                : launch(cache_update_kernel<1024, 3, NoLayers, AL>, grid, lds, idx_cap, cp, c->host, NoLayers{});
+        };
+        rc = !words_fit ? launch(cache_update_bytes_kernel<1024>, grid, plan_lds_bytes(I), cp, c->host)
+             : aligned  ? go(std::true_type{})
+                        : go(std::false_type{});
     }
     if (rc != ST_OK) return rc;
     ST_HIP(hipGetLastError());
@@ -2475,9 +2502,13 @@ extern "C" int st_cache_update_forward(st_cache *c, const uint8_t *mask, const v
     const size_t lds = plan_bytes + (size_t)(ngrp - 1) * NBF * H * 4;
     const int G = mlp_grid();
     static const bool fused_off = [] { const char *v = getenv("ST_CACHE_FUSED"); return v && atoi(v) == 0; }();
+    const bool aligned = update_is_aligned(c, mask);
     // One kernel for one or two rows of x when a block owns at most kSparseMaxQ positions, the masks fit the
-    // kernel's bitmaps and a row fits one pass of a thread group; everything else runs as two calls.
-    const bool fused = !fused_off && B <= 2 && I >= 8 && G <= 0xffff && (I + G - 1) / G <= kSparseMaxQ &&
+    // kernel's bitmaps and a row fits one pass of a thread group; everything else runs as two calls, as do two rows of small
+    // matrices without alignment.  Replayed, us, one kernel / two calls: fp16, H 512, I 1537 19.0 / 17.5; H 896, 2689 19.0 / 17.8;
+    // H 1536, 5001 19.3 / 19.0; H 1792, 5001 19.0 / 19.4; H 2048, 8189 20.9 / 22.2; fp32, H 1024, 4001 18.2 / 18.0; one after the
+    // other from the host 0.2 to 1.6 us less for the calls up to H 2048, 5001.
+    const bool fused = !fused_off && B <= 2 && I >= 8 && !(B == 2 && !aligned && (int64_t)I * row_bytes <= (int64_t)16 << 20) && G <= 0xffff && (I + G - 1) / G <= kSparseMaxQ &&
                        I <= 32 * kSparseMaxW32 && I <= 8 * TPB * kSparseWords && chunks <= TPB && row_bytes % 16 == 0 &&
                        lds <= (size_t)(148 * 1024);
     if (!fused) {   // two launches: update, then the forward that reads the count on the device
@@ -2517,14 +2548,15 @@ extern "C" int st_cache_update_forward(st_cache *c, const uint8_t *mask, const v
         // a group has at most three rows; two rows of x: six when that is one batch, else five.
         const int rpg = ((hint + G - 1) / G + ngrp - 1) / ngrp;   // rows per thread group on the caller's guess
         const bool seven = c->dtype != ST_F32 && B == 1 && (rpg + 6) / 7 < (rpg + 5) / 6;
-#define ST_SPARSE_NW(TYPE, ROWS, NBX)                                                                               \
-    rc = I <= 8 * TPB ? launch(cache_sparse_decode_kernel<TYPE, ROWS, TPB, NBX, 1>, xt, ct)                         \
-                      : launch(cache_sparse_decode_kernel<TYPE, ROWS, TPB, NBX, 2>, xt, ct)
+#define ST_SPARSE_SPEC(TYPE, ROWS, NBX, SPEC)                                                                       \
+    rc = aligned ? I <= 8 * TPB ? launch(cache_sparse_decode_kernel<TYPE, ROWS, TPB, NBX, 1, SPEC, true>, xt, ct)   \
+                                : launch(cache_sparse_decode_kernel<TYPE, ROWS, TPB, NBX, 2, SPEC, true>, xt, ct)   \
+         : I <= 8 * TPB         ? launch(cache_sparse_decode_kernel<TYPE, ROWS, TPB, NBX, 1, SPEC, false>, xt, ct)  \
+                                : launch(cache_sparse_decode_kernel<TYPE, ROWS, TPB, NBX, 2, SPEC, false>, xt, ct)
+#define ST_SPARSE_NW(TYPE, ROWS, NBX) ST_SPARSE_SPEC(TYPE, ROWS, NBX, ROWS / 2)
 // (three rows in flight: two of them ahead of the plan -- with so few rows per block nearly everything waits for the plan
 // otherwise; measured +4 % tok/s on the 10 %-active workloads against one, and against all three)
-#define ST_SPARSE_NW3(TYPE)                                                                                         \
-    rc = I <= 8 * TPB ? launch(cache_sparse_decode_kernel<TYPE, 3, TPB, 1, 1, 2>, xt, ct)                           \
-                      : launch(cache_sparse_decode_kernel<TYPE, 3, TPB, 1, 2, 2>, xt, ct)
+#define ST_SPARSE_NW3(TYPE) ST_SPARSE_SPEC(TYPE, 3, 1, 2)
 #define ST_SPARSE_LAUNCH(TYPE)                                                                                      \
     do {                                                                                                            \
         const TYPE *xt = static_cast<const TYPE *>(x);                                                              \
@@ -2541,6 +2573,7 @@ extern "C" int st_cache_update_forward(st_cache *c, const uint8_t *mask, const v
 #undef ST_SPARSE_LAUNCH
 #undef ST_SPARSE_NW
 #undef ST_SPARSE_NW3
+#undef ST_SPARSE_SPEC
         if (rc != ST_OK) return rc;
     }
     ST_HIP(hipGetLastError());

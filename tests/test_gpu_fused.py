@@ -311,13 +311,12 @@ def test_fused_random_count_changes(I, H, dtype, has_gate, frac):
 
 
 @pytest.mark.parametrize("I,off", [(8, 1), (9, 0), (15, 3), (255, 0), (257, 5), (2049, 0), (3405, 1), (4098, 2), (8191, 0), (8193, 7),
-                                   (16383, 0), (16384, 1)])
-@pytest.mark.parametrize("B", [1, 3])
-def test_sizes_and_masks_at_any_alignment(I, off, B):
+                                   (16383, 0), (16384, 1), (16, 0), (4096, 7)])
+@pytest.mark.parametrize("B", [1, 2, 3])
+def test_sizes_and_masks_at_any_alignment(I, off, B, H=64):
     """Sizes that are no multiples of eight and masks that start anywhere: the last word of a mask, the last vector of a list, the
     second halves of the double buffers.  Update alone, the layers of a launch together (one cache each for three shifted masks)
     and the update + MLP call, against the oracle's order and against one another."""
-    H = 64
     trace = syn.ragged_mask_trace(I + off, I, 14)
     fused, plain, (gate, up, down), g = _pair(I, H, "float16", True, 3, torch.from_numpy(trace[0]))
     third = st.WeightCache(torch.from_numpy(trace[0]).to(DEV), H, gate.to(DEV), up.to(DEV), down.to(DEV), True)
@@ -343,3 +342,9 @@ def test_sizes_and_masks_at_any_alignment(I, off, B):
         assert torch.equal(plain.cur_mask[e].bool().cpu(), torch.from_numpy(trace[t]).bool()), t
         idx = plain.get_active_indices()
         assert torch.equal(plain.up_active[: len(idx)], plain.up_pool[idx]), t
+
+
+@pytest.mark.parametrize("I,off", [(5461, 0), (5462, 0), (5464, 3), (5456, 4)])
+def test_two_rows_without_alignment(I, off):
+    """Two rows of x on both sides of the line (16 MiB a matrix) from which they take one kernel without alignment too."""
+    test_sizes_and_masks_at_any_alignment(I, off, 2, H=1536)
