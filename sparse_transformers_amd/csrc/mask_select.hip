@@ -289,17 +289,16 @@ __device__ __forceinline__ int block_excl_count(int v, SelShared &sh, int tid)
 // `into`: the mask holds zeros and the rows' blocks only set what they select, so that nothing is left to unite.  Predictor and
 // selection, replayed, the blocks' row masks united by the last one (and by 8-bit digits) / so: top-k, four rows of 8192 15.1 / 12.8
 // us, sixteen of 14336 24.2 / 19.4; statistical 12.5 / 10.4 and 19.9 / 16.0.
-template <int KPT>
+template <int KPT, int METHOD>
 __global__ __launch_bounds__(kSelThreads) void mask_select_kernel(const float *__restrict__ scores,
                                                                   uint8_t *__restrict__ mask,
                                                                   uint8_t *__restrict__ rowmask,
                                                                   float *__restrict__ cutoff,
                                                                   unsigned int *__restrict__ ticket, int B, int I,
-                                                                  int ldm, int method_word, long k_in, float z)
+                                                                  int ldm, int flags, long k_in, float z)
 {
     // (pointers and sizes first: the first 14 dwords of the arguments are in scalar registers when the wave starts)
-    const int method = method_word & 0xff, in_lds = (method_word >> 8) & 1;
-    const bool into = ((method_word >> 9) & 1) != 0;
+    const bool in_lds = (flags & 1) != 0, into = (flags & 2) != 0;
     constexpr int NR = KPT > 0 ? KPT : 1;
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ SelShared sh;
@@ -328,11 +327,11 @@ __global__ __launch_bounds__(kSelThreads) void mask_select_kernel(const float *_
                 if (tid + u * kSelThreads < I) fn(tid + u * kSelThreads, v[u]);
         } else {
             for (int i = tid; i < I; i += kSelThreads)
-                fn(i, in_lds && method == ST_MASK_TOPK ? key_value(keys[i]) : row[i]);
+                fn(i, in_lds && METHOD == ST_MASK_TOPK ? key_value(keys[i]) : row[i]);
         }
     };
 
-    if (method == ST_MASK_TOPK) {
+    if constexpr (METHOD == ST_MASK_TOPK) {
         const uint32_t k = k_in < 0 ? 0u : (k_in > I ? (uint32_t)I : (uint32_t)k_in);
         if (k == 0u || k == (uint32_t)I) {  // nothing / everything (uniform over the block)
             each([&](int i, float) { put(i, k != 0u); });
@@ -385,9 +384,9 @@ __global__ __launch_bounds__(kSelThreads) void mask_select_kernel(const float *_
         double mean = first + off, var = q / (double)I - off * off;
         if (off * off > 64.0 * var) {   // (uniform: every thread has the same sums)
             s = q = 0.0;
-            each([&](int, float f) { s += (double)f; });
+            for (int i = tid; i < I; i += kSelThreads) s += (double)row[i];
             mean = block_sum(s, sh, tid) / (double)I;
-            each([&](int, float f) { const double d = (double)f - mean; q += d * d; });
+            for (int i = tid; i < I; i += kSelThreads) { const double d = (double)row[i] - mean; q += d * d; }
             var = block_sum(q, sh, tid) / (double)I;
         }
         const float cut = (float)mean + (float)sqrt(var) * z;
@@ -596,23 +595,23 @@ extern "C" int st_mask_select(const float *scores, int64_t B, int64_t I, int met
         rowmask = static_cast<uint8_t *>(workspace) + 16;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    {
-        const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(mask_select_kernel<0>), kSelMaxLdsKeys * 4);
-        if (rc != ST_OK) return rc;
-    }
     ProfScope ps(ST_K_MASK_SELECT, s);
-    const dim3 grid((unsigned)B), block(kSelThreads);
-#define ST_SELECT_ARGS(in_lds) scores, mask, rowmask, cutoff, ticket, (int)B, (int)I, ldm, method | ((in_lds) << 8) | (into << 9), (long)k, z
-    const size_t lds = (size_t)I * 4 > kKeyHistBytes ? (size_t)I * 4 : kKeyHistBytes;   // keys, or the histogram before them
-    if (I <= 8 * kSelThreads)
-        ST_LAUNCH(ps, (mask_select_kernel<8>), grid, block, lds, s, ST_SELECT_ARGS(1));
-    else if (I <= 16 * kSelThreads)
-        ST_LAUNCH(ps, (mask_select_kernel<16>), grid, block, lds, s, ST_SELECT_ARGS(1));
-    else if (I <= kSelMaxLdsKeys)
-        ST_LAUNCH(ps, (mask_select_kernel<0>), grid, block, (size_t)I * 4, s, ST_SELECT_ARGS(1));
-    else
-        ST_LAUNCH(ps, (mask_select_kernel<0>), grid, block, 0, s, ST_SELECT_ARGS(0));
-#undef ST_SELECT_ARGS
+    auto go = [&](auto kern, size_t lds) {
+        ST_LAUNCH(ps, kern, dim3((unsigned)B), dim3(kSelThreads), lds, s, scores, mask, rowmask, cutoff, ticket, (int)B, (int)I, ldm,
+                  (lds > 0 ? 1 : 0) | (into ? 2 : 0), (long)k, z);
+    };
+    const size_t keys = (size_t)I * 4, lds = keys > kKeyHistBytes ? keys : kKeyHistBytes;   // keys, or the histogram before them
+    if (method == ST_MASK_TOPK) {
+        const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(mask_select_kernel<0, ST_MASK_TOPK>), kSelMaxLdsKeys * 4);
+        if (rc != ST_OK) return rc;
+        if (I <= 8 * kSelThreads) go(mask_select_kernel<8, ST_MASK_TOPK>, lds);
+        else if (I <= 16 * kSelThreads) go(mask_select_kernel<16, ST_MASK_TOPK>, lds);
+        else go(mask_select_kernel<0, ST_MASK_TOPK>, I <= kSelMaxLdsKeys ? keys : 0);
+    } else {
+        if (I <= 8 * kSelThreads) go(mask_select_kernel<8, ST_MASK_STATISTICAL>, 0);
+        else if (I <= 16 * kSelThreads) go(mask_select_kernel<16, ST_MASK_STATISTICAL>, 0);
+        else go(mask_select_kernel<0, ST_MASK_STATISTICAL>, 0);
+    }
     ST_HIP(hipGetLastError());
     return ST_OK;
 }
