@@ -81,6 +81,6 @@ def assert_close(got: np.ndarray, want: np.ndarray, dtype: str, what: str = ""):
     t = TOL[dtype]
     scale = float(np.max(np.abs(want))) if want.size else 0.0
     atol = t.get("atol", t.get("atol_rel", 0.0) * max(scale, 1e-30))
-    err = np.abs(got - want)
-    bad = err > atol + t["rtol"] * np.abs(want)
+    err = np.where(got == want, 0.0, np.abs(got - want))   # (infinities)
+    bad = ~(err <= atol + t["rtol"] * np.abs(want))        # a NaN is outside, too
     assert not bad.any(), f"{what}: {int(bad.sum())} of {bad.size} outside tolerance; max err {err.max():.3e}, scale {scale:.3e}"

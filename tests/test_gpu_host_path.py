@@ -257,7 +257,7 @@ def test_threads_and_streams():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("I,H,gated,dtype", [(1, 64, True, torch.float32), (203, 72, False, torch.float16), (2048, 256, True, torch.bfloat16)])
-def test_cache_construction_forms(I, H, gated, dtype):
+def test_cache_construction_forms(I, H, gated, dtype, monkeypatch):
     """A cache built by the native path and by the general one, which takes every other form of the arguments (strided weights, a
     mask of numbers or on the host), hold the same; sizes and types that do not fit are refused by either."""
     g = torch.Generator(device=DEV).manual_seed(I)
@@ -265,7 +265,9 @@ def test_cache_construction_forms(I, H, gated, dtype):
     mask = torch.rand(I, generator=g, device=DEV) < 0.7
     mask[0] = True
     native = st._lib.native()
-    fast = st.WeightCache(mask, H, gate if gated else None, up, down, gated)
+    with monkeypatch.context() as m:
+        m.setattr(st.WeightCache, "_build", None)          # only the native path can make it
+        fast = st.WeightCache(mask, H, gate if gated else None, up, down, gated)
     strided = down.t().contiguous().t()
     for args in ((mask.float(), H, gate, up, down), (mask.cpu(), H, gate, up, down), (mask, H, gate, up, strided)):
         if args[4] is strided and I == 1:
