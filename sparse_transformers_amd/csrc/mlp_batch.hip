@@ -619,7 +619,9 @@ __device__ __forceinline__ uint32_t row_max_u32(uint32_t v)
 // kernel 2.  Block = (column group cg, row split rs); NP = 64-column pieces per
 // block; NX = tiles of 16 rows of x; HT = the type h is held in (the storage type behind
 // batch_gateup_kernel, fp32 behind batch_gateup_any_kernel: three MFMAs per tile and chunk of rows then).  Where h is scaled
-// (fp16) the operands change places: a row of x is then a column of D, whose scale is the lane's own.
+// (fp16) the operands change places: a row of x is then a column of D, whose scale is the lane's own.  With fp32 h two forms do not
+// fit the registers beside two chunks in flight: bf16 with two tiles of x keeps 112 bytes a lane of the chunks' h in scratch,
+// fp16 with two pieces spills 12 registers (of batch_gateup_any_kernel, fp32 with two tiles and x from memory three).
 // partial[(rs * ldb + b) * H + col], fp32.
 // ---------------------------------------------------------------------------
 template <typename T, typename HT, int NP, int NX>

@@ -715,22 +715,25 @@ __device__ __forceinline__ void gateup_big_tile(uint4 *lds, const T *__restrict_
 // 94 / 79, 136 95 / 113.  Gated, halved / quartered: H 3072, 300 rows, 48 tiles 61.5 / 53.8, 64 66.0 / 59.2; 512 rows, 46
 // 73.3 / 63.0; H 4096, 256 rows, 63 98.0 / 88.7; 2048 rows, a rest of 40 585 / 571.  Ungated, H 3072, 300 rows, halved /
 // quartered: 48 tiles 68.8 / 58.7, 68 (two rounds of quarters) 75.8 / 92.0; 400 rows, H 4096, 64 99.9 / 91.4.
+// `most`: the most parts of a tile, 4 or 2.  Gated, the kernel that knows quarters is another one than that with halves only, whose
+// halves run without their code in 48.7 us instead of 49.1 (512 rows, H 3072, 6554 active); the host picks by its guess of the
+// count.  A wrong guess takes the slower of the two; a result's sum is the same in any tile, bit for bit.
 struct GateupTiles { int big, small, parts; };   // big tiles, smaller ones, smaller ones per big one
-__host__ __device__ __forceinline__ GateupTiles gateup_tiles(int n_pad, int rows, int mt, int cus)
+__host__ __device__ __forceinline__ GateupTiles gateup_tiles(int n_pad, int rows, int mt, int cus, int most)
 {
     const int t = (n_pad + rows - 1) / rows * mt, rest = t % cus;
-    const int parts = 4 * rest <= cus ? 4 : 2 * rest <= cus ? 2 : 1;
+    const int parts = most == 4 && 4 * rest <= cus ? 4 : 2 * rest <= cus ? 2 : 1;
     return parts == 1 ? GateupTiles{t, 0, 1} : GateupTiles{t - rest, parts * rest, parts};
 }
 // The most blocks that any count up to the capacity's `t` big tiles asks for (both kinds in whole eights): the rest of the last
 // round, or any of a whole one before, in the parts that make most of it.
-static int gateup_blocks(int t, int cus)
+static int gateup_blocks(int t, int cus, int most)
 {
-    const int rest = t % cus, in4 = 4 * (rest < cus / 4 ? rest : cus / 4), in2 = 2 * (rest < cus / 2 ? rest : cus / 2);
+    const int rest = t % cus, in4 = most == 4 ? 4 * (rest < cus / 4 ? rest : cus / 4) : 0, in2 = 2 * (rest < cus / 2 ? rest : cus / 2);
     return t - rest + (in4 > in2 ? in4 : in2 > rest ? in2 : rest) + kXcds;
 }
 
-template <typename T, bool HG>
+template <typename T, bool HG, int MOST>
 __global__ __launch_bounds__(kPwThreads) void prefill_gateup_wide_kernel(const T *__restrict__ X,
                                                                          const T *__restrict__ gate,
                                                                          const T *__restrict__ up,
@@ -743,7 +746,7 @@ __global__ __launch_bounds__(kPwThreads) void prefill_gateup_wide_kernel(const T
     __shared__ uint4 lds[kPwLds];
     const int n = device_count(n_host, n_dev);
     const int n_pad = (n + kPfBK - 1) / kPfBK * kPfBK;
-    const GateupTiles tiles = gateup_tiles(n_pad, kBigRows, mt, cus);
+    const GateupTiles tiles = gateup_tiles(n_pad, kBigRows, mt, cus, MOST);
     const int big_blocks = (tiles.big + kXcds - 1) / kXcds * kXcds;
     ST_TL(0);
     if ((int)blockIdx.x < big_blocks) {
@@ -754,12 +757,17 @@ __global__ __launch_bounds__(kPwThreads) void prefill_gateup_wide_kernel(const T
         const int part = xcd_tile_id(blockIdx.x - big_blocks, tiles.small);
         if (part < 0) return;
         const int shift = tiles.parts == 4 ? 2 : 1, tile = tiles.big + (part >> shift);
-        const int cols = HG && tiles.parts == 4 ? 2 : tiles.parts;   // parts of a tile's active rows; the rest are of its rows of x
+        const int cols = HG ? 2 : tiles.parts;   // parts of a tile's active rows; the rest are of its rows of x
         const int j0 = tile / mt * kBigRows + (part & (cols - 1)) * (kBigRows / cols);
-        const int m0 = tile % mt * kPwBM + (cols < tiles.parts ? ((part >> 1) & 1) * (kPwBM / 2) : 0);
-        if (j0 >= n_pad || m0 >= M) return;
-        if (HG && tiles.parts == 4) gateup_wide_tile<T, HG, 2, HG ? 128 : kPwBM>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
-        else if (HG || tiles.parts == 4) gateup_wide_tile<T, HG, 2>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
+        const int m0 = tile % mt * kPwBM + (HG && MOST == 4 && tiles.parts == 4 ? ((part >> 1) & 1) * (kPwBM / 2) : 0);
+        if (j0 >= n_pad || (HG && MOST == 4 && m0 >= M)) return;
+        if constexpr (HG && MOST == 4) {
+            if (tiles.parts == 4) {
+                gateup_wide_tile<T, HG, 2, 128>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
+                return;
+            }
+        }
+        if (HG || tiles.parts == 4) gateup_wide_tile<T, HG, 2>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
         else gateup_wide_tile<T, HG, HG ? 2 : 4>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
     }
 }
@@ -1569,7 +1577,10 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
         const int mt = big ? (M + 255) / 256 : quarters ? (M + 63) / 64 : mt128;
         // (the tiles are dealt out over the device's count)
         const int big_tiles = (int)((ldw + (has_gate ? 127 : 255)) / (has_gate ? 128 : 256)) * mt;
-        const int blocks = !big ? jt * mt : gateup_blocks(big_tiles, cus);
+        const int guess = n_dev && n_hint > 0 && n_hint < n ? n_hint : n;
+        const int rest = (guess + kPfBK - 1) / kPfBK * kPfBK / 128 * mt % cus;   // of the gated tiles, whose active rows are 128
+        const int most = !has_gate || (rest > 0 && 4 * rest <= cus) ? 4 : 2;
+        const int blocks = !big ? jt * mt : gateup_blocks(big_tiles, cus, most);
         const int grid = (blocks + kXcds - 1) / kXcds * kXcds;
         auto go = [&](auto kern, int threads) -> int {
             ST_LAUNCH(ps, kern, dim3(grid), dim3(threads), 0, stream, static_cast<const T *>(x),
@@ -1578,7 +1589,8 @@ static int launch_prefill_t(const void *x, int M, int H, const void *gate, const
             return ST_OK;
         };
         int rc;
-        if (big) rc = has_gate ? go(prefill_gateup_wide_kernel<T, true>, kPwThreads) : go(prefill_gateup_wide_kernel<T, false>, kPwThreads);
+        if (big && has_gate) rc = most == 4 ? go(prefill_gateup_wide_kernel<T, true, 4>, kPwThreads) : go(prefill_gateup_wide_kernel<T, true, 2>, kPwThreads);
+        else if (big) rc = go(prefill_gateup_wide_kernel<T, false, 4>, kPwThreads);
         else if (quarters) rc = has_gate ? go(prefill_gateup_kernel<T, true, 64, 2, 4, 1>, 512) : go(prefill_gateup_kernel<T, false, 64, 2, 4, 1>, 512);
         else if (halves) rc = has_gate ? go(prefill_gateup_kernel<T, true, 128, 2, 2, 1>, 512) : go(prefill_gateup_kernel<T, false, 128, 2, 2, 1>, 512);
         else if (wide_halves) rc = has_gate ? go(prefill_gateup_kernel<T, true, 128, 2, 2, 2>, 512) : go(prefill_gateup_kernel<T, false, 128, 2, 2, 2>, 512);

@@ -67,7 +67,7 @@ def round_to(a: np.ndarray, dtype: str) -> np.ndarray:
     return t.to(getattr(torch, dtype)).to(torch.float32).numpy()
 
 
-# tolerances of the north star: fp32 1e-5 relative; fp16/bf16 2e-2 absolute / 1e-2 relative
+# tolerances: fp32 1e-5 relative; fp16/bf16 2e-2 absolute / 1e-2 relative
 TOL = {"float32": dict(rtol=1e-5, atol_rel=1e-5), "float16": dict(rtol=1e-2, atol=2e-2),
        "bfloat16": dict(rtol=1e-2, atol=2e-2),
        # double precision against a float64 library evaluation: summation order only

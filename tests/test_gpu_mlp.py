@@ -1,6 +1,6 @@
 """Fused sparse MLP on the GPU vs the oracle (float64-accumulating CPU restatement), through the C ABI.
 
-Tolerances (north star): fp32 1e-5 relative; fp16 / bf16 2e-2 absolute, 1e-2 relative, against an fp32
+Tolerances: fp32 1e-5 relative; fp16 / bf16 2e-2 absolute, 1e-2 relative, against an fp32
 evaluation of the dtype-rounded weights and inputs."""
 import os
 import subprocess
@@ -382,6 +382,25 @@ def test_prefill_quarters_of_gated_tiles(M, H, I, n):
     of one stage to five, rows of x that leave a tile's lower half out or with one row, counts that leave an active half out.
     Checked as the tiles above are."""
     test_prefill_big_tiles(M, H, I, n, True)
+
+
+@pytest.mark.parametrize("M,n", [(300, 3000), (300, 4096), (300, 4097), (512, 6500), (1030, 6529)])
+def test_prefill_guess_of_the_count_picks_the_kernel_only(M, n, H=256, I=9000):
+    """Counts whose rest of gated tiles goes out in quarters, in halves or whole, under guesses that pick either kernel: the same bits."""
+    g = torch.Generator().manual_seed(M + n)
+    gate, up, dn = ((torch.randn(I, H, generator=g) * 0.05).half().to(DEV) for _ in range(3))
+    x = torch.randn(M, H, generator=g).half().to(DEV)
+    outs = []
+    for hint in (0, n, 3000, 6500, I):
+        out = torch.full((M, H), float("nan"), dtype=torch.float16, device=DEV)
+        comb = torch.full((M, 2 * I), float("nan"), dtype=torch.float16, device=DEV)
+        mlp_forward_rows(x, gate, up, dn, I, torch.tensor([n], dtype=torch.int32, device=DEV), out, comb, "silu", True, n_hint=hint)
+        torch.cuda.synchronize()
+        outs.append((out, comb[:, :n]))
+    h = torch.nn.functional.silu(x.float() @ gate[:n].float().t()) * (x.float() @ up[:n].float().t())
+    assert_close(outs[0][1].float().cpu().numpy(), h.cpu().numpy(), "float16", "intermediate")
+    for o, c in outs[1:]:
+        assert torch.equal(o, outs[0][0]) and torch.equal(c, outs[0][1])
 
 
 @pytest.mark.parametrize("M,H,I,n,gated", [
