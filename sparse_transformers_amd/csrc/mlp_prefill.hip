@@ -378,8 +378,9 @@ __global__ __launch_bounds__(2 * BM * KS) void prefill_gateup_kernel(const T *__
 constexpr int kPwBM = 256, kPwThreads = 512, kPwBufs = 3;
 constexpr int kPwLds = 5 * 256 * kPfLd1;   // 16-byte units: the big tile's five buffers, 160 KB (the wide tile's three take 144)
 
-// kJ: 16-row tiles of up (and of gate) per wave; kM: rows of x
-template <typename T, bool HG, int kJ, int kM = kPwBM>
+// kJ: 16-row tiles of up (and of gate) per wave; kM: rows of x; MOST: of the kernel (below; a copy for each, so that one's code does
+// not depend on the other's)
+template <typename T, bool HG, int MOST, int kJ, int kM = kPwBM>
 __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict__ X, const T *__restrict__ gate,
                                                  const T *__restrict__ up, int M, int H, int n, int n_pad, int j0, int m0,
                                                  T *__restrict__ Hh, long ldh, T *__restrict__ comb, long ldc, int act)
@@ -570,7 +571,7 @@ __device__ __forceinline__ void gateup_wide_tile(uint4 *lds, const T *__restrict
 }
 
 // The big tile: every wave runs all of K over a 128 x 64 tile of its own (waves 2 x 4).
-template <typename T, bool HG>
+template <typename T, bool HG, int MOST>
 __device__ __forceinline__ void gateup_big_tile(uint4 *lds, const T *__restrict__ X, const T *__restrict__ gate,
                                                 const T *__restrict__ up, int M, int H, int n, int n_pad, int j0, int m0,
                                                 T *__restrict__ Hh, long ldh, T *__restrict__ comb, long ldc, int act)
@@ -715,14 +716,14 @@ __device__ __forceinline__ void gateup_big_tile(uint4 *lds, const T *__restrict_
 // 94 / 79, 136 95 / 113.  Gated, halved / quartered: H 3072, 300 rows, 48 tiles 61.5 / 53.8, 64 66.0 / 59.2; 512 rows, 46
 // 73.3 / 63.0; H 4096, 256 rows, 63 98.0 / 88.7; 2048 rows, a rest of 40 585 / 571.  Ungated, H 3072, 300 rows, halved /
 // quartered: 48 tiles 68.8 / 58.7, 68 (two rounds of quarters) 75.8 / 92.0; 400 rows, H 4096, 64 99.9 / 91.4.
-// `most`: the most parts of a tile, 4 or 2.  Gated, the kernel that knows quarters is another one than that with halves only, whose
+// MOST: the most parts of a tile, 4 or 2.  Gated, the kernel that knows quarters is another one than that with halves only, whose
 // halves run without their code in 48.7 us instead of 49.1 (512 rows, H 3072, 6554 active); the host picks by its guess of the
 // count.  A wrong guess takes the slower of the two; a result's sum is the same in any tile, bit for bit.
 struct GateupTiles { int big, small, parts; };   // big tiles, smaller ones, smaller ones per big one
-__host__ __device__ __forceinline__ GateupTiles gateup_tiles(int n_pad, int rows, int mt, int cus, int most)
+template <int MOST> __host__ __device__ __forceinline__ GateupTiles gateup_tiles(int n_pad, int rows, int mt, int cus)
 {
     const int t = (n_pad + rows - 1) / rows * mt, rest = t % cus;
-    const int parts = most == 4 && 4 * rest <= cus ? 4 : 2 * rest <= cus ? 2 : 1;
+    const int parts = (MOST == 4 ? 4 * rest <= cus : false) ? 4 : 2 * rest <= cus ? 2 : 1;
     return parts == 1 ? GateupTiles{t, 0, 1} : GateupTiles{t - rest, parts * rest, parts};
 }
 // The most blocks that any count up to the capacity's `t` big tiles asks for (both kinds in whole eights): the rest of the last
@@ -746,29 +747,24 @@ __global__ __launch_bounds__(kPwThreads) void prefill_gateup_wide_kernel(const T
     __shared__ uint4 lds[kPwLds];
     const int n = device_count(n_host, n_dev);
     const int n_pad = (n + kPfBK - 1) / kPfBK * kPfBK;
-    const GateupTiles tiles = gateup_tiles(n_pad, kBigRows, mt, cus, MOST);
+    const GateupTiles tiles = gateup_tiles<MOST>(n_pad, kBigRows, mt, cus);
     const int big_blocks = (tiles.big + kXcds - 1) / kXcds * kXcds;
     ST_TL(0);
     if ((int)blockIdx.x < big_blocks) {
         const int tile = xcd_tile_id(blockIdx.x, tiles.big);   // row tiles of x fastest: they share the weight rows
         if (tile >= 0)
-            gateup_big_tile<T, HG>(lds, X, gate, up, M, H, n, n_pad, tile / mt * kBigRows, tile % mt * kPwBM, Hh, ldh, comb, ldc, act);
+            gateup_big_tile<T, HG, MOST>(lds, X, gate, up, M, H, n, n_pad, tile / mt * kBigRows, tile % mt * kPwBM, Hh, ldh, comb, ldc, act);
     } else {
         const int part = xcd_tile_id(blockIdx.x - big_blocks, tiles.small);
         if (part < 0) return;
         const int shift = tiles.parts == 4 ? 2 : 1, tile = tiles.big + (part >> shift);
-        const int cols = HG ? 2 : tiles.parts;   // parts of a tile's active rows; the rest are of its rows of x
+        const int cols = HG && tiles.parts == 4 ? 2 : tiles.parts;   // parts of a tile's active rows; the rest are of its rows of x
         const int j0 = tile / mt * kBigRows + (part & (cols - 1)) * (kBigRows / cols);
-        const int m0 = tile % mt * kPwBM + (HG && MOST == 4 && tiles.parts == 4 ? ((part >> 1) & 1) * (kPwBM / 2) : 0);
-        if (j0 >= n_pad || (HG && MOST == 4 && m0 >= M)) return;
-        if constexpr (HG && MOST == 4) {
-            if (tiles.parts == 4) {
-                gateup_wide_tile<T, HG, 2, 128>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
-                return;
-            }
-        }
-        if (HG || tiles.parts == 4) gateup_wide_tile<T, HG, 2>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
-        else gateup_wide_tile<T, HG, HG ? 2 : 4>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
+        const int m0 = tile % mt * kPwBM + (cols < tiles.parts ? ((part >> 1) & 1) * (kPwBM / 2) : 0);
+        if (j0 >= n_pad || m0 >= M) return;
+        if (HG && tiles.parts == 4) gateup_wide_tile<T, HG, MOST, 2, HG ? 128 : kPwBM>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
+        else if (HG || tiles.parts == 4) gateup_wide_tile<T, HG, MOST, 2>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
+        else gateup_wide_tile<T, HG, MOST, HG ? 2 : 4>(lds, X, gate, up, M, H, n, n_pad, j0, m0, Hh, ldh, comb, ldc, act);
     }
 }
 
